@@ -41,7 +41,6 @@ constexpr unsigned kErrStall = 4u;     // a persistent launch's grid barrier tim
 
 struct RepDev {
   double lx, ly, lz;     // box
-  double hx, hy, hz;     // half box (lx/2.0 ...)
   double sx, sy, sz;     // sweep-grid cell side (lx/gx ...)
   double ix, iy, iz;     // 1.0 / sx ...: the sweep grid's cell index is (int)(t * ix)
   double dr_max;         // displacement width

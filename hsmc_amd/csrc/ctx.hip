@@ -106,7 +106,6 @@ int lcap_for(long bound) { return bound <= 128 ? 128 : (bound <= 192 ? 192 : 256
 void fill_repdev(const RepHost &h, RepDev &d) {
   const hsmc_gpu_replica &p = h.p;
   d.lx = p.lx; d.ly = p.ly; d.lz = p.lz;
-  d.hx = p.lx / 2.0; d.hy = p.ly / 2.0; d.hz = p.lz / 2.0;
   d.sx = p.lx / h.gx; d.sy = p.ly / h.gy; d.sz = p.lz / h.gz;
   d.ix = 1.0 / d.sx; d.iy = 1.0 / d.sy; d.iz = 1.0 / d.sz;
   d.dr_max = p.dr_max;

@@ -307,7 +307,7 @@ __global__ void k_pack_net(const float *__restrict__ P, MlpDev *__restrict__ net
 // ---- descriptors -------------------------------------------------------------
 struct NGrid {  // CSR observable grid (side >= 1.5) over one replica
   int nx, ny, nz;
-  double sx, sy, sz, lx, ly, lz, hx, hy, hz;
+  double sx, sy, sz, ix, iy, iz, lx, ly, lz;  // ix = 1.0 / sx ...
   const int *start;
   const double *px, *py, *pz;
 };
@@ -364,8 +364,8 @@ __device__ __forceinline__ void nearest12(const NGrid &g, double qx, double qy, 
   constexpr int CH = 8;
 #pragma unroll
   for (int k = 0; k < NIN; ++k) best[k] = far2;
-  const int cx = plain_cell(qx, g.sx, g.nx), cy = plain_cell(qy, g.sy, g.ny),
-            cz = plain_cell(qz, g.sz, g.nz);
+  const int cx = search_cell(qx, g.ix, g.nx), cy = search_cell(qy, g.iy, g.ny),
+            cz = search_cell(qz, g.iz, g.nz);
   int ra0[9], ra1[9], rb0[9], rb1[9];
 #pragma unroll
   for (int r = 0; r < 9; ++r) {
@@ -388,7 +388,7 @@ __device__ __forceinline__ void nearest12(const NGrid &g, double qx, double qy, 
 #pragma unroll
       for (int u = 0; u < CH; ++u) {
         if (p + u < p1)
-          take12((float)dist2(qx, qy, qz, ox[u], oy[u], oz[u], g.lx, g.ly, g.lz, g.hx, g.hy, g.hz),
+          take12((float)dist2(qx, qy, qz, ox[u], oy[u], oz[u], g.lx, g.ly, g.lz),
                  best);
       }
     }
@@ -568,9 +568,9 @@ k_voxel_scores_tiled(NGrid g, Vox vx, float far2, double smin, const MlpDev *__r
     const int c = (wrap_index(lo[0] + kx, g.nx) * g.ny + wrap_index(lo[1] + ky, g.ny)) * g.nz +
                   wrap_index(lo[2] + kz, g.nz);
     for (int p = g.start[c]; p < g.start[c + 1]; ++p) {
-      const double dx = min_image(g.px[p] - ccx, g.lx, g.hx);
-      const double dy = min_image(g.py[p] - ccy, g.ly, g.hy);
-      const double dz = min_image(g.pz[p] - ccz, g.lz, g.hz);
+      const double dx = min_image(g.px[p] - ccx, g.lx, g.lx / 2.0);
+      const double dy = min_image(g.py[p] - ccy, g.ly, g.ly / 2.0);
+      const double dz = min_image(g.pz[p] - ccz, g.lz, g.lz / 2.0);
       if (fabs(dx) <= ex && fabs(dy) <= ey && fabs(dz) <= ez) {
         const int slot = atomicAdd(&ncand, 1);
         if (slot < TCAP) {
@@ -635,7 +635,7 @@ k_voxel_scores_tiled(NGrid g, Vox vx, float far2, double smin, const MlpDev *__r
 // No global atomics: the tile counts are prefix-summed instead.  Scores are
 // written for free voxels only; the flags tell the others apart.
 struct Box3 {
-  double lx, ly, lz, hx, hy, hz;
+  double lx, ly, lz;
 };
 
 // First candidate voxel index for centres (i + 0.5) * v within r of p: the
@@ -677,11 +677,11 @@ k_mark_blocked(const double *__restrict__ x, const double *__restrict__ y,
   // layer k's index and dx^2 once and each layer reads them from that lane.
   const int kx = lane & 7;
   const int ixk = wrap_voxel(lx + kx, vx.mx);
-  const double dxk = min_image((ixk + 0.5) * vx.vx - px, b.lx, b.hx);
+  const double dxk = image_mag((ixk + 0.5) * vx.vx - px, b.lx);
   const double dx2k = dxk * dxk;
   const int iy = wrap_voxel(ly + (lane >> 3), vx.my), iz = wrap_voxel(lz + (lane & 7), vx.mz);
-  const double dy = min_image((iy + 0.5) * vx.vy - py, b.ly, b.hy);
-  const double dz = min_image((iz + 0.5) * vx.vz - pz, b.lz, b.hz);
+  const double dy = image_mag((iy + 0.5) * vx.vy - py, b.ly);
+  const double dz = image_mag((iz + 0.5) * vx.vz - pz, b.lz);
   const double dy2 = dy * dy, dz2 = dz * dz;
   const long col = (long)iy * vx.mz + iz, layer = (long)vx.my * vx.mz;
 #pragma unroll
@@ -876,8 +876,8 @@ __global__ void k_cdf_add(double *__restrict__ cdf, long V, const double *__rest
 // rest): almost every proposed point overlaps a sphere, and usually one of
 // those.
 __device__ __forceinline__ bool widom_free(const NGrid &g1, double qx, double qy, double qz) {
-  const int cx = plain_cell(qx, g1.sx, g1.nx), cy = plain_cell(qy, g1.sy, g1.ny),
-            cz = plain_cell(qz, g1.sz, g1.nz);
+  const int cx = search_cell(qx, g1.ix, g1.nx), cy = search_cell(qy, g1.iy, g1.ny),
+            cz = search_cell(qz, g1.iz, g1.nz);
   auto cell_of = [&](int j, bool &ok) {
     int dx, dy, dz;
     stencil_by_distance(j, dx, dy, dz);
@@ -888,8 +888,7 @@ __device__ __forceinline__ bool widom_free(const NGrid &g1, double qx, double qy
   };
   auto hit = [&](int b, int e) {
     for (int p = b; p < e; ++p)
-      if (dist2(qx, qy, qz, g1.px[p], g1.py[p], g1.pz[p], g1.lx, g1.ly, g1.lz, g1.hx, g1.hy,
-                g1.hz) < 1.0)
+      if (dist2(qx, qy, qz, g1.px[p], g1.py[p], g1.pz[p], g1.lx, g1.ly, g1.lz) < 1.0)
         return true;
     return false;
   };
@@ -1039,11 +1038,11 @@ namespace {
 
 __global__ void k_grid_count2(const double *__restrict__ x, const double *__restrict__ y,
                               const double *__restrict__ z, int n, int nx, int ny, int nz,
-                              double sx, double sy, double sz, int *__restrict__ cnt,
+                              double ix, double iy, double iz, int *__restrict__ cnt,
                               int *__restrict__ cellof) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int c = (plain_cell(x[i], sx, nx) * ny + plain_cell(y[i], sy, ny)) * nz + plain_cell(z[i], sz, nz);
+  const int c = (search_cell(x[i], ix, nx) * ny + search_cell(y[i], iy, ny)) * nz + search_cell(z[i], iz, nz);
   cellof[i] = c;
   atomicAdd(&cnt[c], 1);
 }
@@ -1068,12 +1067,12 @@ __global__ void k_grid_scatter2(const double *__restrict__ x, const double *__re
 // [n, 2n], and both grids index one position array of 2n entries.
 struct CellDims {
   int nx, ny, nz;
-  double sx, sy, sz;
+  double ix, iy, iz;  // reciprocal cell sides
 };
 
 __device__ __forceinline__ int cell_in(const CellDims &d, double x, double y, double z) {
-  return (plain_cell(x, d.sx, d.nx) * d.ny + plain_cell(y, d.sy, d.ny)) * d.nz +
-         plain_cell(z, d.sz, d.nz);
+  return (search_cell(x, d.ix, d.nx) * d.ny + search_cell(y, d.iy, d.ny)) * d.nz +
+         search_cell(z, d.iz, d.nz);
 }
 
 __global__ void k_grid_count_pair(const double *__restrict__ x, const double *__restrict__ y,
@@ -1133,8 +1132,8 @@ void set_grid(NGrid &g, const RepHost &h, double cut, const int *start, const do
   g.ny = grid_cells_for2(h.p.ly, cut);
   g.nz = grid_cells_for2(h.p.lz, cut);
   g.sx = h.p.lx / g.nx; g.sy = h.p.ly / g.ny; g.sz = h.p.lz / g.nz;
+  g.ix = 1.0 / g.sx; g.iy = 1.0 / g.sy; g.iz = 1.0 / g.sz;
   g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
-  g.hx = h.p.lx / 2.0; g.hy = h.p.ly / 2.0; g.hz = h.p.lz / 2.0;
   g.start = start;
   g.px = pos; g.py = pos + stride; g.pz = pos + 2 * stride;
 }
@@ -1166,8 +1165,8 @@ int build_ngrid_pair(hsmc_gpu_ctx *ctx, int replica, double cut_a, double cut_b,
   set_grid(ga, h, cut_a, start, pos, stride);
   set_grid(gb, h, cut_b, start + Ca, pos, stride);
   if (cached) return HSMC_OK;
-  const CellDims da{ga.nx, ga.ny, ga.nz, ga.sx, ga.sy, ga.sz};
-  const CellDims db{gb.nx, gb.ny, gb.nz, gb.sx, gb.sy, gb.sz};
+  const CellDims da{ga.nx, ga.ny, ga.nz, ga.ix, ga.iy, ga.iz};
+  const CellDims db{gb.nx, gb.ny, gb.nz, gb.ix, gb.iy, gb.iz};
   const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
   HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * 2 * (C + 1), ctx->stream));
   hipLaunchKernelGGL(k_grid_count_pair, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z,
@@ -1202,14 +1201,14 @@ int build_ngrid(hsmc_gpu_ctx *ctx, int replica, double cut, int slot0, NGrid &g)
   const double sx = h.p.lx / nx, sy = h.p.ly / ny, sz = h.p.lz / nz;
   g.nx = nx; g.ny = ny; g.nz = nz;
   g.sx = sx; g.sy = sy; g.sz = sz;
+  g.ix = 1.0 / sx; g.iy = 1.0 / sy; g.iz = 1.0 / sz;
   g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
-  g.hx = h.p.lx / 2.0; g.hy = h.p.ly / 2.0; g.hz = h.p.lz / 2.0;
   g.start = start;
   g.px = pos; g.py = pos + N; g.pz = pos + 2 * (size_t)N;
   if (cached) return HSMC_OK;
   HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * 2 * (C + 1), ctx->stream));
   hipLaunchKernelGGL(k_grid_count2, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z, N,
-                     nx, ny, nz, sx, sy, sz, cnt, cellof);
+                     nx, ny, nz, g.ix, g.iy, g.iz, cnt, cellof);
   exclusive_scan(ctx->stream, cnt, (int)C, start, part);
   hipLaunchKernelGGL(k_grid_scatter2, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z,
                      N, cellof, start, fill, pos, pos + N, pos + 2 * (size_t)N);
@@ -1333,7 +1332,7 @@ int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, const NGrid &g, const
   int *off = cnt + tiles;
   int *part = off + tiles + 1;
   const int N = rh.p.n_part;
-  Box3 b3{rh.p.lx, rh.p.ly, rh.p.lz, rh.p.lx / 2.0, rh.p.ly / 2.0, rh.p.lz / 2.0};
+  Box3 b3{rh.p.lx, rh.p.ly, rh.p.lz};
   hipLaunchKernelGGL(k_mark_blocked, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, ctx->stream,
                      ctx->d_x + rh.poff, ctx->d_y + rh.poff, ctx->d_z + rh.poff, N, vx, b3, r, flag);
   hipLaunchKernelGGL(k_free_tiles, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, ctx->stream, vx,

@@ -27,18 +27,23 @@ enum Slot { S_CNT = 0, S_START, S_CELLOF, S_IDS, S_PX, S_PY, S_PZ, S_FILL, S_Q0,
 struct Grid {
   int nx, ny, nz;
   double sx, sy, sz;
-  double lx, ly, lz, hx, hy, hz;
+  double ix, iy, iz;  // 1.0 / sx ...
+  double lx, ly, lz;
   const int *start;   // C + 1
   const int *ids;     // N, particle id by sorted position
   const double *px, *py, *pz;
 };
 
+// EXACT: the reference's cells (cell_part_idx, for cell_list) and sx its cell
+// side; otherwise a search grid and sx the reciprocal of its side.
+template <bool EXACT>
 __global__ void k_grid_count(const double *__restrict__ x, const double *__restrict__ y,
                              const double *__restrict__ z, int n, int nx, int ny, int nz, double sx,
                              double sy, double sz, int *__restrict__ cnt, int *__restrict__ cellof) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int c = (plain_cell(x[i], sx, nx) * ny + plain_cell(y[i], sy, ny)) * nz + plain_cell(z[i], sz, nz);
+  auto cell = [](double p, double s, int g) { return EXACT ? plain_cell(p, s, g) : search_cell(p, s, g); };
+  const int c = (cell(x[i], sx, nx) * ny + cell(y[i], sy, ny)) * nz + cell(z[i], sz, nz);
   cellof[i] = c;
   atomicAdd(&cnt[c], 1);
 }
@@ -199,8 +204,8 @@ __device__ __forceinline__ bool for_stencil(const Grid &g, int cx, int cy, int c
 // leaves after one round trip for the ranges and one for the spheres.
 __device__ __forceinline__ bool point_overlaps(const Grid &g, double qx, double qy, double qz,
                                                int skip_id) {
-  const int cx = plain_cell(qx, g.sx, g.nx), cy = plain_cell(qy, g.sy, g.ny),
-            cz = plain_cell(qz, g.sz, g.nz);
+  const int cx = search_cell(qx, g.ix, g.nx), cy = search_cell(qy, g.iy, g.ny),
+            cz = search_cell(qz, g.iz, g.nz);
   auto cell_of = [&](int j, bool &ok) {
     int dx, dy, dz;
     stencil_by_distance(j, dx, dy, dz);
@@ -214,7 +219,7 @@ __device__ __forceinline__ bool point_overlaps(const Grid &g, double qx, double 
       // the id and the position load together; the skip is tested after
       const int id = g.ids[p];
       const double d2 =
-          dist2(qx, qy, qz, g.px[p], g.py[p], g.pz[p], g.lx, g.ly, g.lz, g.hx, g.hy, g.hz);
+          dist2(qx, qy, qz, g.px[p], g.py[p], g.pz[p], g.lx, g.ly, g.lz);
       if (id != skip_id && d2 < 1.0) return true;
     }
     return false;
@@ -394,8 +399,7 @@ k_widom_cells(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, int p
         for (int e = 0; e < T4; e += 4) {
 #pragma unroll 1
           for (int i = 0; i < 4; ++i)
-            m = fmin(m, dist2(qx, qy, qz, Lx[e + i], Ly[e + i], Lz[e + i], g.lx, g.ly, g.lz, g.hx,
-                              g.hy, g.hz));
+            m = fmin(m, dist2(qx, qy, qz, Lx[e + i], Ly[e + i], Lz[e + i], g.lx, g.ly, g.lz));
           if (__all(m < 1.0 || !mine)) break;
         }
       }
@@ -418,7 +422,7 @@ __global__ void k_overlap_scaled(Grid g, const double *__restrict__ x, const dou
   const int i = idx[k];
   const double sf = sfv[k];
   const double ax = x[i], ay = y[i], az = z[i];
-  const int cx = plain_cell(ax, g.sx, g.nx), cy = plain_cell(ay, g.sy, g.ny), cz = plain_cell(az, g.sz, g.nz);
+  const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
   const bool ov = for_stencil(g, cx, cy, cz, [&](int b, int e) {
     for (int p = b; p < e; ++p) {
       if (g.ids[p] == i) continue;
@@ -438,12 +442,12 @@ k_any_overlap_scaled(Grid g, int n, const double *__restrict__ sfv, int nsf, dou
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
-  const int cx = plain_cell(ax, g.sx, g.nx), cy = plain_cell(ay, g.sy, g.ny), cz = plain_cell(az, g.sz, g.nz);
+  const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
   unsigned long long m = 0;
   for_stencil(g, cx, cy, cz, [&](int b, int e) {
     for (int q = b; q < e; ++q) {
       if (q <= p) continue;  // each unordered pair once
-      const double s0 = dist2(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz, g.hx, g.hy, g.hz);
+      const double s0 = dist2(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz);
       if (s0 >= cut2) continue;
       for (int k = 0; k < nsf; ++k)
         if (dist2_scaled(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz, sfv[k]) < 1.0)
@@ -476,10 +480,10 @@ k_pair_hist(Grid g, int n, double dr_bin, int nbins, double rmax_eff, double cut
   unsigned long long bad = 0;
   if (p < n) {
     const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
-    const int cx = plain_cell(ax, g.sx, g.nx), cy = plain_cell(ay, g.sy, g.ny), cz = plain_cell(az, g.sz, g.nz);
+    const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
     for_stencil(g, cx, cy, cz, [&](int b, int e) {
       for (int q = max(b, p + 1); q < e; ++q) {
-        const double s = dist2(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz, g.hx, g.hy, g.hz);
+        const double s = dist2(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz);
         if (s >= cut2) continue;
         const double dr = sqrt(s);
         if (dr < rmax_eff) {
@@ -526,7 +530,7 @@ __device__ __forceinline__ void pair_tile(const Grid &g, double px, double py, d
   for (int j = j0; j < nq; ++j) {
     double s;
     if constexpr (MI) {
-      s = dist2(px, py, pz, tx[j], ty[j], tz[j], g.lx, g.ly, g.lz, g.hx, g.hy, g.hz);
+      s = dist2(px, py, pz, tx[j], ty[j], tz[j], g.lx, g.ly, g.lz);
     } else {
       const double dx = px - tx[j], dy = py - ty[j], dz = pz - tz[j];
       s = dx * dx + dy * dy + dz * dz;
@@ -650,8 +654,8 @@ int build_grid(hsmc_gpu_ctx *ctx, int replica, double cut, Grid &g) {
     return HSMC_ERR_NO_MEMORY;
   g.nx = nx; g.ny = ny; g.nz = nz;
   g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
-  g.hx = h.p.lx / 2.0; g.hy = h.p.ly / 2.0; g.hz = h.p.lz / 2.0;
   g.sx = h.p.lx / nx; g.sy = h.p.ly / ny; g.sz = h.p.lz / nz;
+  g.ix = 1.0 / g.sx; g.iy = 1.0 / g.sy; g.iz = 1.0 / g.sz;
   g.start = start; g.ids = ids; g.px = px; g.py = py; g.pz = pz;
   if (ctx->aux_replica == replica && ctx->aux_version == ctx->version && ctx->aux_n[0] == nx &&
       ctx->aux_n[1] == ny && ctx->aux_n[2] == nz)
@@ -660,8 +664,8 @@ int build_grid(hsmc_gpu_ctx *ctx, int replica, double cut, Grid &g) {
   HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * C, ctx->stream));
   HSMC_HIP(ctx, hipMemsetAsync(fill, 0, sizeof(int) * C, ctx->stream));
   const unsigned blocks = (unsigned)((N + 255) / 256);
-  hipLaunchKernelGGL(k_grid_count, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny, nz,
-                     g.sx, g.sy, g.sz, cnt, cellof);
+  hipLaunchKernelGGL(k_grid_count<false>, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
+                     nz, g.ix, g.iy, g.iz, cnt, cellof);
   exclusive_scan(ctx->stream, cnt, (int)C, start, part);
   hipLaunchKernelGGL(k_grid_scatter, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, cellof,
                      start, fill, ids, px, py, pz);
@@ -775,8 +779,8 @@ int overlap_scan_in_workspace(hsmc_gpu_ctx *ctx, int replica, const double *sf, 
   Grid g;
   g.nx = nx; g.ny = ny; g.nz = nz;
   g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
-  g.hx = h.p.lx / 2.0; g.hy = h.p.ly / 2.0; g.hz = h.p.lz / 2.0;
   g.sx = h.p.lx / nx; g.sy = h.p.ly / ny; g.sz = h.p.lz / nz;
+  g.ix = 1.0 / g.sx; g.iy = 1.0 / g.sy; g.iz = 1.0 / g.sz;
   g.start = start; g.ids = ids; g.px = px; g.py = py; g.pz = pz;
   // counts and fill counters are adjacent regions: one clearing kernel
   const long zero_words = (long)((l.start - l.cnt) / sizeof(unsigned int));
@@ -788,8 +792,8 @@ int overlap_scan_in_workspace(hsmc_gpu_ctx *ctx, int replica, const double *sf, 
   hipLaunchKernelGGL(k_store_sf, dim3(1), dim3(64), 0, ctx->stream, t, n_sf, dsf);
   const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
   const unsigned blocks = (unsigned)((N + 255) / 256);
-  hipLaunchKernelGGL(k_grid_count, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny, nz,
-                     g.sx, g.sy, g.sz, cnt, cellof);
+  hipLaunchKernelGGL(k_grid_count<false>, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
+                     nz, g.ix, g.iy, g.iz, cnt, cellof);
   exclusive_scan(ctx->stream, cnt, (int)C, start, (int *)(ws + l.part));
   hipLaunchKernelGGL(k_grid_scatter, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, cellof,
                      start, fill, ids, px, py, pz);
@@ -834,7 +838,7 @@ int hsmc_gpu_cell_list(hsmc_gpu_ctx *ctx, int replica, int nx, int ny, int nz, i
     HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * C, ctx->stream));
     HSMC_HIP(ctx, hipMemsetAsync(fill, 0, sizeof(int) * C, ctx->stream));
     const unsigned blocks = (unsigned)((N + 255) / 256);
-    hipLaunchKernelGGL(k_grid_count, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
+    hipLaunchKernelGGL(k_grid_count<true>, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
                        nz, sx, sy, sz, cnt, cellof);
     exclusive_scan(ctx->stream, cnt, (int)C, start, part);
     hipLaunchKernelGGL(k_grid_scatter, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, cellof,

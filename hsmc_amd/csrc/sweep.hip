@@ -412,7 +412,7 @@ __device__ __forceinline__ void phase_cell(
         const int q = lane + j * LPC;
         if (q < T) {
           const bool hit =
-              dist2(nx, ny, nz, px[j], py[j], pz[j], rp.lx, rp.ly, rp.lz, rp.hx, rp.hy, rp.hz) < 1.0;
+              dist2(nx, ny, nz, px[j], py[j], pz[j], rp.lx, rp.ly, rp.lz) < 1.0;
           ov |= hit & (q != (int)e);
         }
       }
