@@ -58,6 +58,30 @@ def test_mlp_gradient_matches_oracle():
     assert np.linalg.norm(g - g64) <= 0.05 * np.linalg.norm(g64)
 
 
+@pytest.mark.parametrize("n", [1, 15, 64, 65, 16384, 16449, 40000])
+def test_mlp_forward_and_gradient_at_tile_edges(n):
+    """Row counts around the kernels' tiles: 16 rows per wave, 64 per
+    workgroup and pass, 16384 in one pass of all workgroups.  A BF16 value
+    one rounding away (2^-8) in each of a gradient entry's three rounded
+    factors bounds its distance from the oracle by 3 / 256 of the largest."""
+    ctx, _ = _ctx_with(4, 0.5, 0)
+    rng = np.random.default_rng(n)
+    p = (rng.standard_normal(M.NPARAM) * 0.2).astype(np.float32)
+    net = gpu.Mlp(ctx)
+    net.set(p)
+    x = rng.standard_normal((n, 12)).astype(np.float32)
+    t = rng.standard_normal(n).astype(np.float32)
+    ref, _ = M.forward(p.astype(np.float64), x.astype(np.float64), bf=True)
+    assert np.max(np.abs(net.forward(x) - ref)) <= 2e-3 * max(1.0, np.max(np.abs(ref)))
+    loss, g = net.gradient(x, t)
+    rl, rg = M.loss_and_grad(p.astype(np.float64), x.astype(np.float64), t.astype(np.float64), bf=True)
+    assert abs(loss - rl) <= 3 / 256 * rl
+    assert np.max(np.abs(g - rg)) <= 3 / 256 * np.max(np.abs(rg))
+    # sums in a fixed order: the same bits again
+    loss2, g2 = net.gradient(x, t)
+    assert loss2 == loss and np.array_equal(g2, g)
+
+
 def test_descriptors_match_brute_force():
     ctx, L = _ctx_with(6, 0.8, 20)
     conf = ctx.download()
