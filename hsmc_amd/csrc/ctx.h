@@ -49,6 +49,10 @@ struct RepDev {
   uint32_t k0, k1;       // Philox key
 };
 
+// Results of an observable: a histogram's bins (at most 8192) and its
+// out-of-range count.
+constexpr int kResults = 8192 + 1;
+
 // Entries of the one-replica sweep table: one per sweep of a batch (at most
 // 512 sweeps per graph) and one past the last.
 constexpr int kSweepTable = 520;
@@ -115,6 +119,15 @@ struct hsmc_gpu_ctx {
   // after each batch of sweeps, so later batches are not launched onto a
   // cell list that has already overflowed
   volatile unsigned int *h_err = nullptr;
+  // results of an observable, stored by its last kernel in pinned memory
+  unsigned long long *h_acc = nullptr;
+  // the observable grids' cell counts: their buffer's size when it was last
+  // used and how many of its counts are zero
+  size_t counts_bytes = 0;
+  long counts_clear = 0;
+  // squared-distance edges of the histogram bins kept on the device
+  double edge_dr = 0.0;
+  int edge_bins = 0;
   hsmc_gpu_tuning tune{32, 8, 32, 0};
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -186,10 +199,10 @@ int overlap_scan_in_workspace(hsmc_gpu_ctx *ctx, int replica, const double *sf, 
 // Look up the allocation-free scratch array's address on `device` (current).
 int noalloc_scratch_init(int device);
 // Exclusive prefix sum of in[0..n) into out[0..n] (out[n] = total), three
-// launches on stream s; part is a device workspace of scan_workspace_ints(n)
-// ints.
+// launches on stream s at most; part is a device workspace of
+// scan_workspace_ints(n) ints.  With clear, in is left at zero.
 long scan_workspace_ints(long n);
-void exclusive_scan(hipStream_t s, const int *in, int n, int *out, int *part);
+void exclusive_scan(hipStream_t s, int *in, int n, int *out, int *part, bool clear);
 
 }  // namespace hsmc
 

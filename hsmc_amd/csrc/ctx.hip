@@ -374,7 +374,9 @@ int hsmc_gpu_create(hsmc_gpu_ctx **out, int device, int n_replicas,
       hipMalloc(&ctx->d_z, sizeof(double) * ptot) != hipSuccess ||
       hipMalloc(&ctx->d_sweep, sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc(&ctx->d_err, sizeof(unsigned int)) != hipSuccess ||
-      hipMalloc(&ctx->d_bar, 2 * sizeof(unsigned int)) != hipSuccess)
+      hipMalloc(&ctx->d_bar, 2 * sizeof(unsigned int)) != hipSuccess ||
+      hipHostMalloc((void **)&ctx->h_acc, sizeof(unsigned long long) * kResults,
+                    hipHostMallocDefault) != hipSuccess)
     return fail(HSMC_ERR_NO_MEMORY);
   if (hipDeviceGetAttribute(&ctx->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
     return fail(HSMC_ERR_HIP);
@@ -412,6 +414,7 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
   for (int i = 0; i < hsmc_gpu_ctx::kScratch; ++i)
     if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
   if (ctx->h_err) (void)hipHostFree((void *)ctx->h_err);
+  if (ctx->h_acc) (void)hipHostFree(ctx->h_acc);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

@@ -1249,7 +1249,7 @@ int build_ngrid_pair(hsmc_gpu_ctx *ctx, int replica, double cut_a, double cut_b,
   HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * 2 * (C + 1), ctx->stream));
   hipLaunchKernelGGL(k_grid_count_pair, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z,
                      N, da, db, (int)Ca, cnt, cellof);
-  exclusive_scan(ctx->stream, cnt, (int)C, start, part);
+  exclusive_scan(ctx->stream, cnt, (int)C, start, part, false);
   hipLaunchKernelGGL(k_grid_scatter_pair, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y,
                      z, N, cellof, start, fill, pos, pos + stride, pos + 2 * stride);
   HSMC_HIP(ctx, hipGetLastError());
@@ -1287,7 +1287,7 @@ int build_ngrid(hsmc_gpu_ctx *ctx, int replica, double cut, int slot0, NGrid &g)
   HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * 2 * (C + 1), ctx->stream));
   hipLaunchKernelGGL(k_grid_count2, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z, N,
                      nx, ny, nz, g.ix, g.iy, g.iz, cnt, cellof);
-  exclusive_scan(ctx->stream, cnt, (int)C, start, part);
+  exclusive_scan(ctx->stream, cnt, (int)C, start, part, false);
   hipLaunchKernelGGL(k_grid_scatter2, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z,
                      N, cellof, start, fill, pos, pos + N, pos + 2 * (size_t)N);
   HSMC_HIP(ctx, hipGetLastError());
@@ -1419,7 +1419,7 @@ int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, const NGrid &g, const
                      ctx->d_x + rh.poff, ctx->d_y + rh.poff, ctx->d_z + rh.poff, N, vx, b3, r, flag);
   hipLaunchKernelGGL(k_free_tiles, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, ctx->stream, vx,
                      flag, slots, cnt, tiles);
-  exclusive_scan(ctx->stream, cnt, (int)tiles, off, part);
+  exclusive_scan(ctx->stream, cnt, (int)tiles, off, part, false);
   hipLaunchKernelGGL(k_gather_free, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, ctx->stream,
                      slots, cnt, off, list, tiles);
   HSMC_HIP(ctx, hipGetLastError());

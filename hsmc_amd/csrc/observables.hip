@@ -21,8 +21,8 @@ using namespace hsmc;
 
 namespace {
 
-enum Slot { S_CNT = 0, S_START, S_CELLOF, S_IDS, S_PX, S_PY, S_PZ, S_FILL, S_Q0, S_Q1, S_Q2, S_OUT0, S_OUT1,
-            S_PART };
+enum Slot { S_CNT = 0, S_START, S_CELLOF, S_IDS, S_PX, S_PY, S_PZ, S_Q0, S_Q1, S_Q2, S_OUT0,
+            S_PART, S_BINS, S_SUMS };
 
 struct Grid {
   int nx, ny, nz;
@@ -32,6 +32,8 @@ struct Grid {
   const int *start;   // C + 1
   const int *ids;     // N, particle id by sorted position
   const double *px, *py, *pz;
+  __device__ __forceinline__ int begin(int c) const { return start[c]; }
+  __device__ __forceinline__ int end(int c) const { return start[c + 1]; }
 };
 
 // EXACT: the reference's cells (cell_part_idx, for cell_list) and sx its cell
@@ -39,46 +41,53 @@ struct Grid {
 template <bool EXACT>
 __global__ void k_grid_count(const double *__restrict__ x, const double *__restrict__ y,
                              const double *__restrict__ z, int n, int nx, int ny, int nz, double sx,
-                             double sy, double sz, int *__restrict__ cnt, int *__restrict__ cellof) {
+                             double sy, double sz, int *__restrict__ cnt, int2 *__restrict__ cellof) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   auto cell = [](double p, double s, int g) { return EXACT ? plain_cell(p, s, g) : search_cell(p, s, g); };
   const int c = (cell(x[i], sx, nx) * ny + cell(y[i], sy, ny)) * nz + cell(z[i], sz, nz);
-  cellof[i] = c;
-  atomicAdd(&cnt[c], 1);
+  cellof[i] = make_int2(c, atomicAdd(&cnt[c], 1));  // its cell and its place there
 }
 
 // Exclusive prefix sum of cnt[0..n) into start[0..n], one workgroup.  Each
 // pass covers 32 * 1024 entries: a thread loads its 32 consecutive entries
-// at once (all loads in flight together), the block scans the thread sums,
-// and a carry links the passes.
-__global__ void __launch_bounds__(1024) k_scan1(const int *__restrict__ cnt, int n, int *__restrict__ start) {
+// at once (all loads in flight together), the waves scan the thread sums in
+// registers and the 16 wave totals go through LDS; a carry links the passes.
+// CLEAR: the counts are set to zero once read, for the next grid.
+template <bool CLEAR>
+__global__ void __launch_bounds__(1024) k_scan1(int *__restrict__ cnt, int n, int *__restrict__ start) {
   constexpr int K = 32;
-  __shared__ int part[1024];
-  const int t = threadIdx.x;
+  __shared__ int tot[2][16];
+  const int t = threadIdx.x, w = t >> 6;
   int carry = 0;
-  for (int base = 0; base < n; base += K * 1024) {
-    const int b = base + t * K;
+  for (int base = 0, pass = 0; base < n; base += K * 1024, ++pass) {
+    // short scans spread over all threads: k entries each, at most K
+    const int k1 = min(K, (n - base + 1023) / 1024);
+    const int b = base + t * k1;
     int v[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = (b + k < n) ? cnt[b + k] : 0;
     int s = 0;
 #pragma unroll
-    for (int k = 0; k < K; ++k) s += v[k];
-    part[t] = s;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-      const int u = (t >= d) ? part[t - d] : 0;
-      __syncthreads();
-      part[t] += u;
-      __syncthreads();
+    for (int k = 0; k < K; ++k) {
+      v[k] = (k < k1 && b + k < n) ? cnt[b + k] : 0;
+      s += v[k];
     }
-    int run = carry + part[t] - s;
-    const int total = part[1023];
-    __syncthreads();  // part is rewritten by the next pass
+    const int incl = group_inclusive_sum<64>(s);
+    if ((t & 63) == 63) tot[pass & 1][w] = incl;
+    __syncthreads();  // one barrier a pass: the next pass writes the other row
+    int before = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int u = tot[pass & 1][i];
+      before += i < w ? u : 0;
+      total += u;
+    }
+    int run = carry + before + incl - s;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      if (b + k < n) start[b + k] = run;
+      if (k < k1 && b + k < n) {
+        start[b + k] = run;
+        if (CLEAR) cnt[b + k] = 0;
+      }
       run += v[k];
     }
     carry += total;
@@ -92,8 +101,12 @@ __global__ void __launch_bounds__(1024) k_scan1(const int *__restrict__ cnt, int
 // offset.  Three short launches in place of one workgroup walking the whole
 // array.
 constexpr int kScanTile = 4096;
+// Up to here k_scan1 alone: one pass over n entries takes 3 us, the three
+// launches 9 us.
+constexpr int kScanOne = 32 * 1024;
 
-__global__ void __launch_bounds__(256) k_scan_tile(const int *__restrict__ in, int n,
+template <bool CLEAR>
+__global__ void __launch_bounds__(256) k_scan_tile(int *__restrict__ in, int n,
                                                    int *__restrict__ out, int *__restrict__ part) {
   __shared__ int wsum[4];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -118,7 +131,10 @@ __global__ void __launch_bounds__(256) k_scan_tile(const int *__restrict__ in, i
   int run = woff + incl - s;
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-    if (base + k < n) out[base + k] = run;
+    if (base + k < n) {
+      out[base + k] = run;
+      if (CLEAR) in[base + k] = 0;
+    }
     run += v[k];
   }
   if (t == 255) part[blockIdx.x] = woff + incl;
@@ -136,14 +152,13 @@ __global__ void __launch_bounds__(256) k_scan_add(int *__restrict__ out, int n,
 }
 
 __global__ void k_grid_scatter(const double *__restrict__ x, const double *__restrict__ y,
-                               const double *__restrict__ z, int n, const int *__restrict__ cellof,
-                               const int *__restrict__ start, int *__restrict__ fill,
-                               int *__restrict__ ids, double *__restrict__ px,
+                               const double *__restrict__ z, int n, const int2 *__restrict__ cellof,
+                               const int *__restrict__ start, int *__restrict__ ids, double *__restrict__ px,
                                double *__restrict__ py, double *__restrict__ pz) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int c = cellof[i];
-  const int pos = start[c] + atomicAdd(&fill[c], 1);
+  const int2 c = cellof[i];
+  const int pos = start[c.x] + c.y;
   ids[pos] = i;
   px[pos] = x[i];
   py[pos] = y[i];
@@ -202,7 +217,8 @@ __device__ __forceinline__ bool for_stencil(const Grid &g, int cx, int cy, int c
 // cell, then the 6 sharing a face, then the rest), with the ranges of the
 // first 7 loaded together: a point that overlaps usually does so there, and
 // leaves after one round trip for the ranges and one for the spheres.
-__device__ __forceinline__ bool point_overlaps(const Grid &g, double qx, double qy, double qz,
+template <bool SKIP, class G>
+__device__ __forceinline__ bool point_overlaps(const G &g, double qx, double qy, double qz,
                                                int skip_id) {
   const int cx = search_cell(qx, g.ix, g.nx), cy = search_cell(qy, g.iy, g.ny),
             cz = search_cell(qz, g.iz, g.nz);
@@ -217,10 +233,10 @@ __device__ __forceinline__ bool point_overlaps(const Grid &g, double qx, double 
   auto scan = [&](int b, int e) {
     for (int p = b; p < e; ++p) {
       // the id and the position load together; the skip is tested after
-      const int id = g.ids[p];
-      const double d2 =
-          dist2(qx, qy, qz, g.px[p], g.py[p], g.pz[p], g.lx, g.ly, g.lz);
-      if (id != skip_id && d2 < 1.0) return true;
+      int id = 0;
+      if constexpr (SKIP) id = g.ids[p];
+      const double d2 = dist2(qx, qy, qz, g.px[p], g.py[p], g.pz[p], g.lx, g.ly, g.lz);
+      if ((!SKIP || id != skip_id) && d2 < 1.0) return true;
     }
     return false;
   };
@@ -229,9 +245,9 @@ __device__ __forceinline__ bool point_overlaps(const Grid &g, double qx, double 
 #pragma unroll
   for (int j = 0; j < 7; ++j) c7[j] = cell_of(j, ok7[j]);
 #pragma unroll
-  for (int j = 0; j < 7; ++j) b7[j] = g.start[c7[j]];
+  for (int j = 0; j < 7; ++j) b7[j] = g.begin(c7[j]);
 #pragma unroll
-  for (int j = 0; j < 7; ++j) e7[j] = g.start[c7[j] + 1];
+  for (int j = 0; j < 7; ++j) e7[j] = g.end(c7[j]);
 #pragma unroll
   for (int j = 0; j < 7; ++j)
     if (!ok7[j]) e7[j] = b7[j];  // a cell the stencil leaves out (tiny grids): empty
@@ -241,7 +257,7 @@ __device__ __forceinline__ bool point_overlaps(const Grid &g, double qx, double 
   for (int j = 7; j < 27; ++j) {
     bool ok;
     const int c = cell_of(j, ok);
-    if (ok && scan(g.start[c], g.start[c + 1])) return true;
+    if (ok && scan(g.begin(c), g.end(c))) return true;
   }
   return false;
 }
@@ -250,14 +266,62 @@ __global__ void k_overlap_batch(Grid g, const int *__restrict__ idx, const doubl
                                 int m, unsigned char *__restrict__ out) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= m) return;
-  out[k] = point_overlaps(g, q[3 * k], q[3 * k + 1], q[3 * k + 2], idx[k]) ? 1 : 0;
+  out[k] = point_overlaps<true>(g, q[3 * k], q[3 * k + 1], q[3 * k + 2], idx[k]) ? 1 : 0;
 }
 
 __global__ void k_widom_points(Grid g, const double *__restrict__ q, int m,
                                unsigned char *__restrict__ out) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= m) return;
-  out[k] = point_overlaps(g, q[3 * k], q[3 * k + 1], q[3 * k + 2], -1) ? 0 : 1;
+  out[k] = point_overlaps<false>(g, q[3 * k], q[3 * k + 1], q[3 * k + 2], -1) ? 0 : 1;
+}
+
+// ---- results of a launch ----------------------------------------------------
+// Each workgroup stores its counts in its own row of `part` and one more
+// kernel adds the rows up into the context's pinned host memory, so a call is
+// its kernels and one wait: nothing to clear, no copy.  (An atomic on one
+// address from workgroups on different XCDs takes about 0.1 us, one after
+// the other: 512 workgroups adding to shared counts took 70 us longer.)
+
+// Column sums of rows x cols counts: 64 columns a workgroup, 16 interleaved
+// groups of rows; with several workgroups along y each takes its share of
+// the rows and stores its own row of sums.
+template <class T>
+__global__ void __launch_bounds__(1024)
+k_sum_rows(const T *__restrict__ part, int rows, int cols, unsigned long long *__restrict__ out) {
+  __shared__ unsigned long long s[16][64];
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
+  const int cc = min(c, cols - 1);
+  unsigned long long v = 0;
+#pragma unroll 8
+  for (int r = blockIdx.y * 16 + q; r < rows; r += 16 * gridDim.y) v += part[(size_t)r * cols + cc];
+  s[q][lane] = v;
+  __syncthreads();
+  if (q) return;
+#pragma unroll
+  for (int k = 1; k < 16; ++k) v += s[k][lane];
+  if (c < cols) out[(size_t)blockIdx.y * cols + c] = v;
+}
+
+// Sum (or OR) of n 64-bit values; with err, the sticky error bits too.
+template <bool OR>
+__global__ void __launch_bounds__(1024)
+k_sum_all(const unsigned long long *__restrict__ part, int n, const unsigned *__restrict__ err,
+          unsigned long long *__restrict__ host) {
+  __shared__ unsigned long long s[16];
+  unsigned long long v = 0;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < n; i += 1024) v = OR ? v | part[i] : v + part[i];
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long u = __shfl_xor(v, o, 64);
+    v = OR ? v | u : v + u;
+  }
+  if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int k = 1; k < 16; ++k) v = OR ? v | s[k] : v + s[k];
+  host[0] = v;
+  if (err) host[1] = *err;
 }
 
 __device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long v) {
@@ -276,9 +340,12 @@ __device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long v
 // widom_insertion (compute_widom_chem_pot.c:44-71) on a Philox stream:
 // point i has counter {i_lo, i_hi, sample_lo, 0x5749xxxx}, coordinates
 // u/(2^32-1) * L (widom_rand_pos, :73-80).
-__global__ void __launch_bounds__(256)
-k_widom_uniform(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, long long first,
-                long long n, unsigned long long *__restrict__ hits) {
+constexpr int kWidomUniformBlocks = 8192;
+
+template <class G>
+__device__ __forceinline__ void uniform_points(const G &g, uint32_t k0, uint32_t k1,
+                                               unsigned long long sample, long long first,
+                                               long long n, unsigned long long *__restrict__ part) {
   unsigned long long h = 0;
   const long long stride = (long long)gridDim.x * blockDim.x;
   const uint32_t c3 = 0x57490000u | (uint32_t)((sample >> 32) & 0xFFFFu);
@@ -289,10 +356,77 @@ k_widom_uniform(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, lon
     const double qx = u32_unit_closed(u[0]) * g.lx;
     const double qy = u32_unit_closed(u[1]) * g.ly;
     const double qz = u32_unit_closed(u[2]) * g.lz;
-    if (!point_overlaps(g, qx, qy, qz, -1)) ++h;
+    if (!point_overlaps<false>(g, qx, qy, qz, -1)) ++h;
   }
   const unsigned long long s = block_sum_u64(h);
-  if (threadIdx.x == 0 && s) atomicAdd(hits, s);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
+}
+
+__global__ void __launch_bounds__(256)
+k_widom_uniform(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, long long first,
+                long long n, unsigned long long *__restrict__ part) {
+  uniform_points(g, k0, k1, sample, first, n, part);
+}
+
+// The same for systems whose grid and positions fit in 64 KB of LDS: every
+// workgroup files the spheres itself (a few us, beside the three launches of
+// a grid in memory) and its points' scattered reads stay on the chip.
+constexpr int kWidomLdsThreads = 512, kWidomLdsBlocks = 1024;
+
+struct LdsGrid {  // after filing, last[c] is the end of cell c and so the start of cell c + 1
+  int nx, ny, nz;
+  double ix, iy, iz, lx, ly, lz;
+  const int *last;
+  const double *px, *py, *pz;
+  __device__ __forceinline__ int begin(int c) const { return c ? last[c - 1] : 0; }
+  __device__ __forceinline__ int end(int c) const { return last[c]; }
+};
+
+size_t widom_lds_bytes(long N, long C) { return sizeof(double) * 3 * N + sizeof(int) * C; }
+
+__global__ void __launch_bounds__(kWidomLdsThreads)
+k_widom_uniform_lds(Grid gg, int N, const double *__restrict__ x, const double *__restrict__ y,
+                    const double *__restrict__ z, uint32_t k0, uint32_t k1,
+                    unsigned long long sample, long long first, long long n,
+                    unsigned long long *__restrict__ part) {
+  extern __shared__ double lds_pos[];
+  __shared__ int tot[kWidomLdsThreads / 64];
+  double *px = lds_pos, *py = px + N, *pz = py + N;
+  int *cnt = reinterpret_cast<int *>(pz + N);
+  const int t = threadIdx.x, C = gg.nx * gg.ny * gg.nz;
+  for (int c = t; c < C; c += kWidomLdsThreads) cnt[c] = 0;
+  __syncthreads();
+  auto cell = [&](double a, double b, double c) {
+    return (search_cell(a, gg.ix, gg.nx) * gg.ny + search_cell(b, gg.iy, gg.ny)) * gg.nz +
+           search_cell(c, gg.iz, gg.nz);
+  };
+  for (int i = t; i < N; i += kWidomLdsThreads) atomicAdd(&cnt[cell(x[i], y[i], z[i])], 1);
+  __syncthreads();
+  // counts to starts: a run of consecutive cells per thread
+  const int per = (C + kWidomLdsThreads - 1) / kWidomLdsThreads, c0 = min(t * per, C), c1 = min(c0 + per, C);
+  int s = 0;
+  for (int c = c0; c < c1; ++c) s += cnt[c];
+  const int incl = group_inclusive_sum<64>(s);
+  if ((t & 63) == 63) tot[t >> 6] = incl;
+  __syncthreads();
+  int run = incl - s;
+  for (int w = 0; w < (t >> 6); ++w) run += tot[w];
+  for (int c = c0; c < c1; ++c) {
+    const int k = cnt[c];
+    cnt[c] = run;
+    run += k;
+  }
+  __syncthreads();
+  for (int i = t; i < N; i += kWidomLdsThreads) {
+    const double a = x[i], b = y[i], c = z[i];
+    const int p = atomicAdd(&cnt[cell(a, b, c)], 1);
+    px[p] = a;
+    py[p] = b;
+    pz[p] = c;
+  }
+  __syncthreads();
+  const LdsGrid g{gg.nx, gg.ny, gg.nz, gg.ix, gg.iy, gg.iz, gg.lx, gg.ly, gg.lz, cnt, px, py, pz};
+  uniform_points(g, k0, k1, sample, first, n, part);
 }
 
 // Cell-stratified uniform insertion: every cell of the observable grid
@@ -312,10 +446,11 @@ k_widom_uniform(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, lon
 // the walk as soon as a ballot shows every point overlapping.
 constexpr int kWidomCellsLcap = 256;   // bound of spheres in a 27-cell stencil (host-checked)
 constexpr int kWidomCellsWaves = 4;    // waves per workgroup
+constexpr int kWidomCellsBlocks = 1 << 16;
 
 __global__ void __launch_bounds__(64 * kWidomCellsWaves)
 k_widom_cells(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, int per_cell,
-              unsigned long long *__restrict__ hits, unsigned *__restrict__ err) {
+              unsigned long long *__restrict__ part, unsigned *__restrict__ err) {
   __shared__ double sx_[kWidomCellsWaves][kWidomCellsLcap];
   __shared__ double sy_[kWidomCellsWaves][kWidomCellsLcap];
   __shared__ double sz_[kWidomCellsWaves][kWidomCellsLcap];
@@ -408,8 +543,8 @@ k_widom_cells(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, int p
     }
     __builtin_amdgcn_wave_barrier();  // the list is rewritten for the next cell
   }
-  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);
-  if (lane == 0 && h) atomicAdd(hits, h);
+  const unsigned long long s = block_sum_u64(h);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 // check_overlap(idx, sf, sf, sf) (moves.c:157-212) for each query.
@@ -434,30 +569,6 @@ __global__ void k_overlap_scaled(Grid g, const double *__restrict__ x, const dou
   out[k] = ov ? 1 : 0;
 }
 
-// Any pair overlapping after scaling by sf[k]: bit k of *mask.  Pairs whose
-// unscaled squared distance exceeds cut2 cannot overlap for any sf[k].
-__global__ void __launch_bounds__(256)
-k_any_overlap_scaled(Grid g, int n, const double *__restrict__ sfv, int nsf, double cut2,
-                     unsigned long long *__restrict__ mask) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
-  const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
-  unsigned long long m = 0;
-  for_stencil(g, cx, cy, cz, [&](int b, int e) {
-    for (int q = b; q < e; ++q) {
-      if (q <= p) continue;  // each unordered pair once
-      const double s0 = dist2(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz);
-      if (s0 >= cut2) continue;
-      for (int k = 0; k < nsf; ++k)
-        if (dist2_scaled(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz, sfv[k]) < 1.0)
-          m |= (1ull << k);
-    }
-    return false;
-  });
-  if (m) atomicOr(mask, m);
-}
-
 __global__ void k_pair_dist(const double *__restrict__ x, const double *__restrict__ y,
                             const double *__restrict__ z, const int *__restrict__ ii,
                             const int *__restrict__ jj, int m, double sf, double lx, double ly,
@@ -468,137 +579,312 @@ __global__ void k_pair_dist(const double *__restrict__ x, const double *__restri
   out[k] = sqrt(dist2_scaled(x[i], y[i], z[i], x[j], y[j], z[j], lx, ly, lz, sf));
 }
 
-// Pair histogram: every unordered pair with dr < rmax_eff, bin
+// ---- pair kernels --------------------------------------------------------
+// What a histogram kernel asks of a pair: dr < rmax_eff and bin
 // (int)((dr - 1.0) / dr_bin) (compute_rdf.c:118-124, compute_press.c:150-155).
-__global__ void __launch_bounds__(256)
-k_pair_hist(Grid g, int n, double dr_bin, int nbins, double rmax_eff, double cut2,
-            unsigned long long *__restrict__ counts, unsigned long long *__restrict__ oor) {
-  extern __shared__ unsigned int hist[];
-  for (int b = threadIdx.x; b < nbins; b += blockDim.x) hist[b] = 0;
+// dr, the difference and the quotient are correctly rounded and so grow with
+// the squared distance s: dr < rmax_eff is s < smax, and the bin is b when
+// edge[b] <= s < edge[b + 1], with smax and the edges the first doubles past
+// each step, which the host finds with the formula itself.  A pair is binned
+// by an FP32 estimate corrected against the edges, about 15 instructions in
+// place of the 50 of an FP64 square root and division.
+struct Bins {
+  double dr_bin, rmax_eff, smax;
+  float inv_bin;
+  int n;
+  const double *edge;  // n + 1 entries, or null: few bins, binned by the formula
+};
+
+// The kernels' LDS: nbins counts, then the edges.
+__device__ __forceinline__ double *hist_edges(unsigned int *hist, int n) {
+  return reinterpret_cast<double *>(hist + ((n + 1) & ~1));
+}
+
+__device__ __forceinline__ void hist_begin(const Bins &bn, unsigned int *hist) {
+  for (int b = threadIdx.x; b < bn.n; b += blockDim.x) hist[b] = 0;
+  if (bn.edge) {
+    double *e = hist_edges(hist, bn.n);
+    for (int b = threadIdx.x; b <= bn.n; b += blockDim.x) e[b] = bn.edge[b];
+  }
   __syncthreads();
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  unsigned long long bad = 0;
-  if (p < n) {
-    const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
-    const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
-    for_stencil(g, cx, cy, cz, [&](int b, int e) {
-      for (int q = max(b, p + 1); q < e; ++q) {
-        const double s = dist2(ax, ay, az, g.px[q], g.py[q], g.pz[q], g.lx, g.ly, g.lz);
-        if (s >= cut2) continue;
-        const double dr = sqrt(s);
-        if (dr < rmax_eff) {
-          const int bin = (int)((dr - 1.0) / dr_bin);
-          if (bin >= 0 && bin < nbins)
-            atomicAdd(&hist[bin], 1u);
-          else
-            ++bad;
+}
+
+template <bool EDGES>
+__device__ __forceinline__ void bin_pair(const Bins &bn, unsigned int *hist, double s,
+                                         unsigned int &bad) {
+  if (!(s < bn.smax)) return;
+  int b;
+  bool in;
+  if constexpr (EDGES) {
+    const double *e = hist_edges(hist, bn.n);
+    b = (int)((__builtin_amdgcn_sqrtf((float)s) - 1.0f) * bn.inv_bin);
+    b = min(max(b, 0), bn.n - 1);
+    const double lo = e[b], hi = e[b + 1];
+    in = s >= lo && s < hi;
+    if (!in) {  // next to an edge, or out of the bins' range
+      while (b > 0 && s < e[b]) --b;
+      while (b < bn.n - 1 && s >= e[b + 1]) ++b;
+      in = s >= e[b] && s < e[b + 1];
+    }
+  } else {
+    b = (int)((sqrt(s) - 1.0) / bn.dr_bin);
+    in = b >= 0 && b < bn.n;
+  }
+  if (in)
+    atomicAdd(&hist[b], 1u);
+  else
+    ++bad;
+}
+
+// The workgroup's counts, and its pairs out of the bins' range, in its row.
+__device__ __forceinline__ void hist_end(const Bins &bn, const unsigned int *hist, unsigned int bad,
+                                         unsigned int *__restrict__ part) {
+  unsigned int *row = part + (size_t)blockIdx.x * (bn.n + 1);
+  const unsigned long long out = block_sum_u64(bad);  // with the barrier before the counts are read
+  for (int b = threadIdx.x; b < bn.n; b += blockDim.x) row[b] = hist[b];
+  if (threadIdx.x == 0) row[bn.n] = (unsigned int)out;
+}
+
+// Scale factors of one scan, passed by value (no host-to-device copy).
+struct SfTable {
+  double v[64];
+};
+
+// Bits k of the factors at which a pair overlaps after scaling.  s0 is its
+// unscaled squared distance: at cut2 and beyond no factor makes it overlap.
+__device__ __forceinline__ void scaled_pair(const SfTable &sf, int nsf, double cut2, double s0,
+                                            double ax, double ay, double az, double bx, double by,
+                                            double bz, double lx, double ly, double lz,
+                                            unsigned long long &m) {
+  if (s0 >= cut2) return;
+  for (int k = 0; k < nsf; ++k)
+    if (dist2_scaled(ax, ay, az, bx, by, bz, lx, ly, lz, sf.v[k]) < 1.0) m |= 1ull << k;
+}
+
+__device__ __forceinline__ void mask_end(unsigned long long m, unsigned long long *__restrict__ part) {
+  __shared__ unsigned long long red[16];
+  for (int o = 32; o > 0; o >>= 1) m |= __shfl_xor(m, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int k = 1; k < (int)(blockDim.x >> 6); ++k) m |= red[k];
+  part[blockIdx.x] = m;
+}
+
+// All pairs of N spheres without a grid, for systems of up to kAllPairs
+// spheres (kAllPairsWide for a cutoff of kWide and more): a wave takes 64 spheres, one a lane, against a run of JC spheres
+// read through the scalar cache (their index is the same in every lane), and
+// keeps the pairs of a later sphere.  f(squared distance, ...) of each pair.
+// A grid costs three launches and a stencil walk of dependent loads; all
+// 8 M pairs of 4000 spheres are 15 FP64 instructions each on the whole GPU:
+// contact histogram 11.5 us (27.0 with a thread per sphere on a grid, and the
+// grid 26), g(r) to 5 diameters 14.5 us (130 with a wave per pair of cells),
+// 20 scale factors 12.2 us (28.0).  Whole calls, all pairs against the grid:
+// contacts 29.8 / 33.9 us at N = 4000, 34.9 / 34.1 at 5324, 41.8 / 34.9 at
+// 6912; g(r) 51.5 / 54.5 us at 6912, about 62 / 62 at 8000.
+constexpr int kAllPairs = 5120, kAllPairsWide = 7168;
+constexpr double kWide = 4.0;
+constexpr int kPairThreads = 512, kPairBlocks = 2048;
+
+template <int JC, class F>
+__device__ __forceinline__ void all_pairs(const double *__restrict__ x, const double *__restrict__ y,
+                                          const double *__restrict__ z, int n, double lx, double ly,
+                                          double lz, F &&f) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kPairThreads / 64) + (threadIdx.x >> 6)));
+  const int waves = gridDim.x * (kPairThreads / 64);
+  // tile a of 64 spheres meets tiles a .. nt - 1; tiles a and nt - 1 - a
+  // together meet nt + 1, so task t of the half-by-(nt + 1) rectangle is one
+  // pair of tiles (the middle tile of an odd number comes up twice: its
+  // second half of tasks is left out), JC spheres of the later tile at a time
+  const int nt = (n + 63) / 64, tasks = (nt + 1) / 2 * (nt + 1) * (64 / JC);
+  for (int t = wave; t < tasks; t += waves) {
+    const int u = t / (64 / JC), p = u / (nt + 1), r = u % (nt + 1);
+    const bool low = r < nt - p;
+    if (!low && nt - 1 - p == p) continue;
+    const int a = low ? p : nt - 1 - p, b = low ? p + r : r - 1;
+    const int i0 = 64 * a, j0 = 64 * b + (t % (64 / JC)) * JC, j1 = min(j0 + JC, n);
+    const int i = i0 + lane;
+    const int ic = min(i, n - 1);
+    const int after = i < n ? i : n;  // a lane past the end keeps no pair
+    const double ax = x[ic], ay = y[ic], az = z[ic];
+#pragma unroll 8
+    for (int j = j0; j < j1; ++j) {
+      const double bx = x[j], by = y[j], bz = z[j];
+      const double s = dist2(ax, ay, az, bx, by, bz, lx, ly, lz);
+      if (j > after) f(s, ax, ay, az, bx, by, bz);
+    }
+  }
+}
+
+template <int JC, bool EDGES>
+__global__ void __launch_bounds__(kPairThreads)
+k_hist_all(const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
+           int n, double lx, double ly, double lz, Bins bn, unsigned int *__restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) unsigned int hist[];
+  hist_begin(bn, hist);
+  unsigned int bad = 0;
+  all_pairs<JC>(x, y, z, n, lx, ly, lz, [&](double s, double, double, double, double, double, double) {
+    bin_pair<EDGES>(bn, hist, s, bad);
+  });
+  hist_end(bn, hist, bad, part);
+}
+
+template <int JC>
+__global__ void __launch_bounds__(kPairThreads)
+k_scaled_all(const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
+             int n, double lx, double ly, double lz, SfTable sf, int nsf, double cut2,
+             unsigned long long *__restrict__ part) {
+  unsigned long long m = 0;
+  all_pairs<JC>(x, y, z, n, lx, ly, lz,
+                [&](double s, double ax, double ay, double az, double bx, double by, double bz) {
+                  scaled_pair(sf, nsf, cut2, s, ax, ay, az, bx, by, bz, lx, ly, lz, m);
+                });
+  mask_end(m, part);
+}
+
+// Pairs of larger systems on a grid whose side is at least cutoff / S and
+// which has at least 2 S + 1 cells an axis.  A workgroup takes a cell A: the
+// cells of A's stencil that follow it (half of the (2S+1)^3, each pair of
+// cells once) are runs along z of consecutive entries of the sorted arrays,
+// two where a row wraps.  The runs' spheres go one to a lane, loaded
+// contiguously, and the spheres of A, the same for every lane, come through
+// the scalar cache.  f(squared distance, ...) of each pair.
+// g(r) to 5 diameters at N = 32000 on 12^3 cells: 52 us (244 us with a wave
+// per pair of cells 5 wide and each pair binned by square root and division).
+// (Four cells a workgroup of 1024 left fewer counts to add up but 75 us of
+// uneven work where single cells take 53.)
+constexpr int kRowThreads = 256, kRowBlocks = 2048;
+
+template <int S, class F>
+__device__ __forceinline__ void row_pairs(const Grid &g, F &&f) {
+  constexpr int ROWS = 2 * S * (S + 1) + 1, RUNS = 2 * ROWS;  // rows after A's, and A's own
+  __shared__ int run_b[64], run_off[64];
+  const int t = threadIdx.x;
+  const int C = g.nx * g.ny * g.nz;
+  for (int A = blockIdx.x; A < C; A += gridDim.x) {
+    const int bA = g.start[A], eA = g.start[A + 1];
+    if (bA == eA) continue;  // the whole workgroup
+    const int cx = A / (g.ny * g.nz), cy = (A / g.nz) % g.ny, cz = A % g.nz;
+    __syncthreads();  // the previous cell's runs are no longer read
+    if (t < 64) {
+      int b = 0, len = 0;
+      if (t < RUNS) {
+        // row 0 is A's own (A and the cells after it along z); row k >= 1
+        // the k-th offset (dx, dy) after (0, 0)
+        const int k = t >> 1, d = k + S;
+        const int dx = d / (2 * S + 1), dy = d % (2 * S + 1) - S;
+        const int z0 = k ? cz - S : cz, z1 = cz + S;
+        const int base = (wrap_index(cx + dx, g.nx) * g.ny + wrap_index(cy + dy, g.ny)) * g.nz;
+        int a0, a1;
+        if ((t & 1) == 0) {  // the part inside [0, nz)
+          a0 = max(z0, 0), a1 = min(z1, g.nz - 1);
+        } else if (z0 < 0) {           // the part that wraps
+          a0 = z0 + g.nz, a1 = g.nz - 1;
+        } else {
+          a0 = 0, a1 = z1 - g.nz;
+        }
+        if (a1 >= a0) {
+          b = g.start[base + a0];
+          len = g.start[base + a1 + 1] - b;
         }
       }
-      return false;
-    });
-  }
-  __syncthreads();
-  for (int b = threadIdx.x; b < nbins; b += blockDim.x)
-    if (hist[b]) atomicAdd(&counts[b], (unsigned long long)hist[b]);
-  const unsigned long long s = block_sum_u64(bad);
-  if (threadIdx.x == 0 && s) atomicAdd(oor, s);
-}
-
-// The same pair histogram on cell pairs, for grids whose cells hold many
-// spheres (the g(r) cutoff of several diameters), where one thread per
-// sphere leaves most of the GPU without waves.  One wave per (cell A,
-// stencil cell B) with B at or after A in cell order: B's sorted positions
-// are staged in LDS a tile at a time and each lane tests its sphere of A
-// against the tile.  Positions are sorted by cell, so "q after p in sorted
-// order" is the per-sphere kernel's rule and every pair is counted once,
-// with the same arithmetic (reference sphere first).
-constexpr int kPairTile = 256;
-
-size_t pair_tiled_lds(int nbins) {
-  return ((sizeof(unsigned int) * (size_t)nbins + 7) & ~(size_t)7) + 3 * sizeof(double) * kPairTile;
-}
-
-// One lane's sphere (px, py, pz) against tile entries [j0, nq): the per-pair
-// arithmetic of k_pair_hist; MI = false leaves out the minimum image where
-// it cannot change a difference.
-template <bool MI>
-__device__ __forceinline__ void pair_tile(const Grid &g, double px, double py, double pz,
-                                          const double *tx, const double *ty, const double *tz,
-                                          int j0, int nq, double cut2, double rmax_eff,
-                                          double dr_bin, int nbins, unsigned int *hist,
-                                          unsigned long long &bad) {
-  for (int j = j0; j < nq; ++j) {
-    double s;
-    if constexpr (MI) {
-      s = dist2(px, py, pz, tx[j], ty[j], tz[j], g.lx, g.ly, g.lz);
-    } else {
-      const double dx = px - tx[j], dy = py - ty[j], dz = pz - tz[j];
-      s = dx * dx + dy * dy + dz * dz;
+      const int incl = group_inclusive_sum<64>(len);
+      run_b[t] = b;
+      run_off[t] = incl - len;
     }
-    if (s >= cut2) continue;
-    const double dr = sqrt(s);
-    if (dr < rmax_eff) {
-      const int bin = (int)((dr - 1.0) / dr_bin);
-      if (bin >= 0 && bin < nbins)
-        atomicAdd(&hist[bin], 1u);
-      else
-        ++bad;
-    }
-  }
-}
-
-__global__ void __launch_bounds__(64)
-k_pair_hist_tiled(Grid g, int nbins, double dr_bin, double rmax_eff, double cut2,
-                  unsigned long long *__restrict__ counts, unsigned long long *__restrict__ oor) {
-  extern __shared__ unsigned long long smem_u64[];
-  unsigned int *hist = (unsigned int *)smem_u64;
-  double *tx = (double *)((unsigned char *)smem_u64 + ((sizeof(unsigned int) * (size_t)nbins + 7) & ~(size_t)7));
-  double *ty = tx + kPairTile, *tz = ty + kPairTile;
-  const int lane = threadIdx.x;
-  const int cA = (int)(blockIdx.x / 27u), st = (int)(blockIdx.x % 27u);
-  const int dx = st / 9 - 1, dy = (st / 3) % 3 - 1, dz = st % 3 - 1;
-  if (!stencil_axis_ok(dx, g.nx) || !stencil_axis_ok(dy, g.ny) || !stencil_axis_ok(dz, g.nz)) return;
-  const int ax = cA / (g.ny * g.nz), ay = (cA / g.nz) % g.ny, az = cA % g.nz;
-  const int cB = (wrap_index(ax + dx, g.nx) * g.ny + wrap_index(ay + dy, g.ny)) * g.nz +
-                 wrap_index(az + dz, g.nz);
-  if (cB < cA) return;  // counted from B's side
-  const int bA = g.start[cA], eA = g.start[cA + 1], bB = g.start[cB], eB = g.start[cB + 1];
-  if (bA == eA || bB == eB) return;
-  // No wrap between A and B on any axis, and at least 5 cells per axis: every
-  // coordinate difference is within 2 sides (plus rounding of the cell
-  // index) <= 0.4 L, below half a box, where the minimum image returns it
-  // unchanged, so the tile skips it (the same doubles either way).
-  const bool direct = g.nx >= 5 && g.ny >= 5 && g.nz >= 5 && ax + dx >= 0 && ax + dx < g.nx &&
-                      ay + dy >= 0 && ay + dy < g.ny && az + dz >= 0 && az + dz < g.nz;
-  for (int b = lane; b < nbins; b += 64) hist[b] = 0;
-  unsigned long long bad = 0;
-  for (int p0 = bA; p0 < eA; p0 += 64) {
-    const int p = p0 + lane;
-    const bool act = p < eA;
-    const double px = act ? g.px[p] : 0.0, py = act ? g.py[p] : 0.0, pz = act ? g.pz[p] : 0.0;
-    for (int q0 = bB; q0 < eB; q0 += kPairTile) {
-      const int nq = min(kPairTile, eB - q0);
-      __syncthreads();  // the previous tile is no longer read
-      for (int j = lane; j < nq; j += 64) {
-        tx[j] = g.px[q0 + j];
-        ty[j] = g.py[q0 + j];
-        tz[j] = g.pz[q0 + j];
+    __syncthreads();
+    const int total = run_off[63];  // runs past RUNS are empty
+    // without a wrap every difference is within (S + 1) sides, under half a
+    // box of 2 S + 3 cells: the minimum image changes none of them
+    const bool direct = g.nx >= 2 * S + 3 && g.ny >= 2 * S + 3 && g.nz >= 2 * S + 3 && cx + S < g.nx &&
+                        cy >= S && cy + S < g.ny && cz >= S && cz + S < g.nz;
+    for (int j = t; j < total; j += kRowThreads) {
+      int r = 0;
+#pragma unroll
+      for (int w = 32; w > 0; w >>= 1)
+        if (run_off[r + w] <= j) r += w;  // the last run that starts at or before j
+      const int q = run_b[r] + j - run_off[r];
+      const double qx = g.px[q], qy = g.py[q], qz = g.pz[q];
+      const int before = q < eA && q >= bA ? q : eA;  // in A itself the spheres before q
+      if (direct) {
+#pragma unroll 2
+        for (int p = bA; p < eA; ++p) {
+          const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
+          const double dx = ax - qx, dy = ay - qy, dz = az - qz;
+          if (p < before) f(dx * dx + dy * dy + dz * dz, ax, ay, az, qx, qy, qz);
+        }
+      } else {
+#pragma unroll 1
+        for (int p = bA; p < eA; ++p) {
+          const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
+          const double s = dist2(ax, ay, az, qx, qy, qz, g.lx, g.ly, g.lz);
+          if (p < before) f(s, ax, ay, az, qx, qy, qz);
+        }
       }
-      __syncthreads();
-      if (!act) continue;
-      // in A's own cell only the spheres after p; in a later cell all
-      const int j0 = max(0, p + 1 - q0);
-      if (direct)
-        pair_tile<false>(g, px, py, pz, tx, ty, tz, j0, nq, cut2, rmax_eff, dr_bin, nbins, hist, bad);
-      else
-        pair_tile<true>(g, px, py, pz, tx, ty, tz, j0, nq, cut2, rmax_eff, dr_bin, nbins, hist, bad);
     }
   }
-  __syncthreads();
-  for (int b = lane; b < nbins; b += 64)
-    if (hist[b]) atomicAdd(&counts[b], (unsigned long long)hist[b]);
-  for (int o = 32; o > 0; o >>= 1) bad += __shfl_down(bad, o, 64);
-  if (lane == 0 && bad) atomicAdd(oor, bad);
+}
+
+template <int S, bool EDGES>
+__global__ void __launch_bounds__(kRowThreads)
+k_hist_rows(Grid g, Bins bn, unsigned int *__restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) unsigned int hist[];
+  hist_begin(bn, hist);
+  unsigned int bad = 0;
+  row_pairs<S>(g, [&](double s, double, double, double, double, double, double) {
+    bin_pair<EDGES>(bn, hist, s, bad);
+  });
+  hist_end(bn, hist, bad, part);
+}
+
+__global__ void __launch_bounds__(kRowThreads)
+k_scaled_rows(Grid g, SfTable sf, int nsf, double cut2,
+             unsigned long long *__restrict__ part) {
+  unsigned long long m = 0;
+  row_pairs<1>(g, [&](double s, double ax, double ay, double az, double bx, double by, double bz) {
+    scaled_pair(sf, nsf, cut2, s, ax, ay, az, bx, by, bz, g.lx, g.ly, g.lz, m);
+  });
+  mask_end(m, part);
+}
+
+// The same on a grid of fewer cells along an axis (long thin boxes): one
+// thread per sphere walks the distinct cells of its 27-cell stencil.
+template <class F>
+__device__ __forceinline__ void sphere_pairs(const Grid &g, int n, F &&f) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
+  const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
+  for_stencil(g, cx, cy, cz, [&](int b, int e) {
+    for (int q = max(b, p + 1); q < e; ++q) {  // each unordered pair once
+      const double bx = g.px[q], by = g.py[q], bz = g.pz[q];
+      f(dist2(ax, ay, az, bx, by, bz, g.lx, g.ly, g.lz), ax, ay, az, bx, by, bz);
+    }
+    return false;
+  });
+}
+
+template <bool EDGES>
+__global__ void __launch_bounds__(256)
+k_hist_spheres(Grid g, int n, Bins bn, unsigned int *__restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) unsigned int hist[];
+  hist_begin(bn, hist);
+  unsigned int bad = 0;
+  sphere_pairs(g, n, [&](double s, double, double, double, double, double, double) {
+    bin_pair<EDGES>(bn, hist, s, bad);
+  });
+  hist_end(bn, hist, bad, part);
+}
+
+__global__ void __launch_bounds__(256)
+k_scaled_spheres(Grid g, int n, SfTable sf, int nsf, double cut2,
+             unsigned long long *__restrict__ part) {
+  unsigned long long m = 0;
+  sphere_pairs(g, n, [&](double s, double ax, double ay, double az, double bx, double by, double bz) {
+    scaled_pair(sf, nsf, cut2, s, ax, ay, az, bx, by, bz, g.lx, g.ly, g.lz, m);
+  });
+  mask_end(m, part);
 }
 
 }  // namespace
@@ -610,16 +896,21 @@ long scan_workspace_ints(long n) {
   return 2 * tiles + 1;
 }
 
-void exclusive_scan(hipStream_t s, const int *in, int n, int *out, int *part) {
-  const int tiles = (int)((n + kScanTile - 1) / kScanTile);
-  if (tiles == 0) {
+void exclusive_scan(hipStream_t s, int *in, int n, int *out, int *part, bool clear) {
+  if (n == 0) {
     hipLaunchKernelGGL(k_scan_empty, dim3(1), dim3(64), 0, s, out);
     return;
   }
+  if (n <= kScanOne) {
+    hipLaunchKernelGGL(clear ? k_scan1<true> : k_scan1<false>, dim3(1), dim3(1024), 0, s, in, n, out);
+    return;
+  }
+  const int tiles = (int)(((long)n + kScanTile - 1) / kScanTile);
   int *offs = part + tiles;  // tiles + 1 entries: exclusive offsets and the total
-  hipLaunchKernelGGL(k_scan_tile, dim3((unsigned)tiles), dim3(256), 0, s, in, n, out, part);
-  hipLaunchKernelGGL(k_scan1, dim3(1), dim3(1024), 0, s, part, tiles, offs);
-  hipLaunchKernelGGL(k_scan_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, out, n, offs, tiles);
+  hipLaunchKernelGGL(clear ? k_scan_tile<true> : k_scan_tile<false>, dim3((unsigned)tiles), dim3(256), 0, s,
+                     in, n, out, part);
+  hipLaunchKernelGGL(k_scan1<false>, dim3(1), dim3(1024), 0, s, part, tiles, offs);
+  hipLaunchKernelGGL(k_scan_add, dim3((unsigned)(((long)n + 255) / 256)), dim3(256), 0, s, out, n, offs, tiles);
 }
 
 }  // namespace hsmc
@@ -633,43 +924,61 @@ int grid_cells_for(double L, double cut) {
   return n;
 }
 
+// Cells of a search grid of side at least `cut` over a replica's box.
+void set_grid(const RepHost &h, double cut, Grid &g) {
+  g.nx = grid_cells_for(h.p.lx, cut); g.ny = grid_cells_for(h.p.ly, cut); g.nz = grid_cells_for(h.p.lz, cut);
+  g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
+  g.sx = h.p.lx / g.nx; g.sy = h.p.ly / g.ny; g.sz = h.p.lz / g.nz;
+  g.ix = 1.0 / g.sx; g.iy = 1.0 / g.sy; g.iz = 1.0 / g.sz;
+}
+
+// The C counts of a grid at zero, and in *clear how many of the buffer's are
+// once the grid is built: every build's prefix sum leaves the counts it read
+// at zero, so only those of a buffer not yet used that far are cleared here.
+// Until the build notes *clear (its launches went well), none count as zero.
+int clear_counts(hsmc_gpu_ctx *ctx, int *cnt, long C, long *clear) {
+  const bool same = ctx->counts_bytes == ctx->scratch_bytes[S_CNT];  // a buffer only ever grows
+  const long have = same ? ctx->counts_clear : 0;
+  ctx->counts_bytes = ctx->scratch_bytes[S_CNT];
+  ctx->counts_clear = 0;
+  *clear = std::max(have, C);
+  if (have < C) HSMC_HIP(ctx, hipMemsetAsync(cnt + have, 0, sizeof(int) * (C - have), ctx->stream));
+  return HSMC_OK;
+}
+
 // Build (or reuse) the observable grid of `replica` for cutoff `cut`.
 int build_grid(hsmc_gpu_ctx *ctx, int replica, double cut, Grid &g) {
   const RepHost &h = ctx->reps[replica];
   const int N = h.p.n_part;
-  const int nx = grid_cells_for(h.p.lx, cut), ny = grid_cells_for(h.p.ly, cut),
-            nz = grid_cells_for(h.p.lz, cut);
+  set_grid(h, cut, g);
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
   const long C = (long)nx * ny * nz;
   if (C > (1L << 28)) return HSMC_ERR_NOT_SUPPORTED;
   int *cnt = (int *)scratch(ctx, S_CNT, sizeof(int) * C);
-  int *fill = (int *)scratch(ctx, S_FILL, sizeof(int) * C);
   int *start = (int *)scratch(ctx, S_START, sizeof(int) * (C + 1));
-  int *cellof = (int *)scratch(ctx, S_CELLOF, sizeof(int) * N);
+  int2 *cellof = (int2 *)scratch(ctx, S_CELLOF, sizeof(int2) * N);
   int *ids = (int *)scratch(ctx, S_IDS, sizeof(int) * N);
   double *px = (double *)scratch(ctx, S_PX, sizeof(double) * N);
   double *py = (double *)scratch(ctx, S_PY, sizeof(double) * N);
   double *pz = (double *)scratch(ctx, S_PZ, sizeof(double) * N);
   int *part = (int *)scratch(ctx, S_PART, sizeof(int) * scan_workspace_ints(C));
-  if (!cnt || !fill || !start || !cellof || !ids || !px || !py || !pz || !part)
+  if (!cnt || !start || !cellof || !ids || !px || !py || !pz || !part)
     return HSMC_ERR_NO_MEMORY;
-  g.nx = nx; g.ny = ny; g.nz = nz;
-  g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
-  g.sx = h.p.lx / nx; g.sy = h.p.ly / ny; g.sz = h.p.lz / nz;
-  g.ix = 1.0 / g.sx; g.iy = 1.0 / g.sy; g.iz = 1.0 / g.sz;
   g.start = start; g.ids = ids; g.px = px; g.py = py; g.pz = pz;
   if (ctx->aux_replica == replica && ctx->aux_version == ctx->version && ctx->aux_n[0] == nx &&
       ctx->aux_n[1] == ny && ctx->aux_n[2] == nz)
     return HSMC_OK;
   const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
-  HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * C, ctx->stream));
-  HSMC_HIP(ctx, hipMemsetAsync(fill, 0, sizeof(int) * C, ctx->stream));
+  long clear = 0;
+  if (clear_counts(ctx, cnt, C, &clear)) return HSMC_ERR_HIP;
   const unsigned blocks = (unsigned)((N + 255) / 256);
   hipLaunchKernelGGL(k_grid_count<false>, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
                      nz, g.ix, g.iy, g.iz, cnt, cellof);
-  exclusive_scan(ctx->stream, cnt, (int)C, start, part);
+  exclusive_scan(ctx->stream, cnt, (int)C, start, part, true);
   hipLaunchKernelGGL(k_grid_scatter, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, cellof,
-                     start, fill, ids, px, py, pz);
+                     start, ids, px, py, pz);
   HSMC_HIP(ctx, hipGetLastError());
+  ctx->counts_clear = clear;
   ctx->aux_replica = replica;
   ctx->aux_version = ctx->version;
   ctx->aux_n[0] = nx; ctx->aux_n[1] = ny; ctx->aux_n[2] = nz;
@@ -677,17 +986,74 @@ int build_grid(hsmc_gpu_ctx *ctx, int replica, double cut, Grid &g) {
   return HSMC_OK;
 }
 
-bool bad_replica(const hsmc_gpu_ctx *ctx, int r) { return !ctx || r < 0 || r >= ctx->R; }
+constexpr int kWidomLdsSpheres = 2048;
+constexpr int kSmallRuns = 4096;   // all_pairs: shorter runs for the smallest systems
+constexpr double kRowSide = 2.0;   // row_pairs: smallest cell side worth a workgroup
 
-// Scale factors of one scan, passed by value (no host-to-device copy).
-struct SfTable {
-  double v[64];
-};
-
-__global__ void k_store_sf(SfTable t, int n, double *__restrict__ dst) {
-  const int k = threadIdx.x;
-  if (k < n) dst[k] = t.v[k];
+unsigned all_pairs_blocks(int N) {
+  const long nt = (N + 63) / 64, waves = (nt + 1) / 2 * (nt + 1) * (N <= kSmallRuns ? 4 : 1);
+  return (unsigned)std::min((waves + kPairThreads / 64 - 1) / (kPairThreads / 64), (long)kPairBlocks);
 }
+
+// The column sums of the workgroups' rows into the pinned results; above 256
+// rows in two steps (1728 rows of 401 counts in one step took 35 us).
+int sum_rows(hsmc_gpu_ctx *ctx, const unsigned int *part, int rows, int cols) {
+  const dim3 wg(1024);
+  const unsigned cb = (unsigned)((cols + 63) / 64);
+  if (rows <= 256) {
+    hipLaunchKernelGGL(k_sum_rows<unsigned int>, dim3(cb), wg, 0, ctx->stream, part, rows, cols, ctx->h_acc);
+  } else {
+    const int mid = std::min(64, (rows + 63) / 64);
+    unsigned long long *sums = (unsigned long long *)scratch(ctx, S_SUMS, sizeof(unsigned long long) * mid * cols);
+    if (!sums) return HSMC_ERR_NO_MEMORY;
+    hipLaunchKernelGGL(k_sum_rows<unsigned int>, dim3(cb, mid), wg, 0, ctx->stream, part, rows, cols, sums);
+    hipLaunchKernelGGL(k_sum_rows<unsigned long long>, dim3(cb), wg, 0, ctx->stream, sums, mid, cols, ctx->h_acc);
+  }
+  HSMC_HIP(ctx, hipGetLastError());
+  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  return HSMC_OK;
+}
+
+bool cells_at_least(const hsmc_gpu_replica &p, double side, int n) {
+  return grid_cells_for(p.lx, side) >= n && grid_cells_for(p.ly, side) >= n &&
+         grid_cells_for(p.lz, side) >= n;
+}
+
+// First double at which the monotone condition holds, from a guess a few
+// units in the last place away.
+template <class Cond>
+double first_double(double guess, Cond &&holds) {
+  while (guess > 0.0 && holds(guess)) guess = nextafter(guess, 0.0);
+  while (!holds(guess)) guess = nextafter(guess, INFINITY);
+  return guess;
+}
+
+// Edges of the bins (int)((dr - 1.0) / dr_bin) in squared distance, on the
+// device: edge[b] is the first s of bin b or later.  Kept by bin width (a
+// run bins every sample alike), made longer when more bins are asked for.
+int bin_edges(hsmc_gpu_ctx *ctx, double dr_bin, int nbins, const double **edge) {
+  double *d = (double *)scratch(ctx, S_BINS, sizeof(double) * (nbins + 1));
+  if (!d) return HSMC_ERR_NO_MEMORY;
+  if (ctx->edge_bins < nbins || ctx->edge_dr != dr_bin) {
+    std::vector<double> e(nbins + 1);
+    for (int b = 0; b <= nbins; ++b) {
+      const double r = b == 0 ? std::max(0.0, 1.0 - dr_bin) : 1.0 + b * dr_bin;
+      // truncation towards zero puts quotients in (-1, 0) in bin 0
+      e[b] = first_double(r * r, [&](double s) {
+        const double q = (sqrt(s) - 1.0) / dr_bin;
+        return b == 0 ? q > -1.0 : q >= (double)b;
+      });
+    }
+    HSMC_HIP(ctx, hipMemcpyAsync(d, e.data(), sizeof(double) * (nbins + 1), hipMemcpyHostToDevice, ctx->stream));
+    HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->edge_dr = dr_bin;
+    ctx->edge_bins = nbins;
+  }
+  *edge = d;
+  return HSMC_OK;
+}
+
+bool bad_replica(const hsmc_gpu_ctx *ctx, int r) { return !ctx || r < 0 || r >= ctx->R; }
 
 __global__ void k_zero_words(unsigned int *__restrict__ p, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -696,11 +1062,11 @@ __global__ void k_zero_words(unsigned int *__restrict__ p, long n) {
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Workspace layout of the scan: counts, fill counters and starts of the
-// grid's C cells, cell and id of the N spheres, their sorted positions, the
-// scale table and the result mask, each region 256-B aligned.
+// Workspace layout of the scan: counts and starts of the grid's C cells, cell
+// (and place in it) and id of the N spheres, their sorted positions and
+// the workgroups' result masks, each region 256-B aligned.
 struct ScanLayout {
-  size_t cnt, fill, start, cellof, ids, px, py, pz, sf, mask, part, bytes;
+  size_t cnt, start, cellof, ids, px, py, pz, mask, part, bytes;
 };
 
 ScanLayout scan_layout(long N, long C) {
@@ -712,15 +1078,13 @@ ScanLayout scan_layout(long N, long C) {
     return at;
   };
   l.cnt = take(sizeof(int) * C);
-  l.fill = take(sizeof(int) * C);
   l.start = take(sizeof(int) * (C + 1));
-  l.cellof = take(sizeof(int) * N);
+  l.cellof = take(sizeof(int2) * N);
   l.ids = take(sizeof(int) * N);
   l.px = take(sizeof(double) * N);
   l.py = take(sizeof(double) * N);
   l.pz = take(sizeof(double) * N);
-  l.sf = take(sizeof(double) * 64);
-  l.mask = take(sizeof(unsigned long long));
+  l.mask = take(sizeof(unsigned long long) * ((N + 255) / 256));  // one per workgroup
   l.part = take(sizeof(int) * scan_workspace_ints(C));
   l.bytes = o;
   return l;
@@ -762,8 +1126,9 @@ int overlap_scan_in_workspace(hsmc_gpu_ctx *ctx, int replica, const double *sf, 
   if (st) return st;
   const RepHost &h = ctx->reps[replica];
   const int N = h.p.n_part;
-  const int nx = grid_cells_for(h.p.lx, cut), ny = grid_cells_for(h.p.ly, cut),
-            nz = grid_cells_for(h.p.lz, cut);
+  Grid g;
+  set_grid(h, cut, g);
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
   const long C = (long)nx * ny * nz;
   const ScanLayout l = scan_layout(N, C);
   if (l.bytes > ws_bytes) {
@@ -771,38 +1136,31 @@ int overlap_scan_in_workspace(hsmc_gpu_ctx *ctx, int replica, const double *sf, 
                       std::to_string(ws_bytes) + " available";
     return HSMC_ERR_NOT_SUPPORTED;
   }
-  int *cnt = (int *)(ws + l.cnt), *fill = (int *)(ws + l.fill), *start = (int *)(ws + l.start);
-  int *cellof = (int *)(ws + l.cellof), *ids = (int *)(ws + l.ids);
+  int *cnt = (int *)(ws + l.cnt), *start = (int *)(ws + l.start);
+  int2 *cellof = (int2 *)(ws + l.cellof);
+  int *ids = (int *)(ws + l.ids);
   double *px = (double *)(ws + l.px), *py = (double *)(ws + l.py), *pz = (double *)(ws + l.pz);
-  double *dsf = (double *)(ws + l.sf);
   unsigned long long *dmask = (unsigned long long *)(ws + l.mask);
-  Grid g;
-  g.nx = nx; g.ny = ny; g.nz = nz;
-  g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
-  g.sx = h.p.lx / nx; g.sy = h.p.ly / ny; g.sz = h.p.lz / nz;
-  g.ix = 1.0 / g.sx; g.iy = 1.0 / g.sy; g.iz = 1.0 / g.sz;
   g.start = start; g.ids = ids; g.px = px; g.py = py; g.pz = pz;
-  // counts and fill counters are adjacent regions: one clearing kernel
-  const long zero_words = (long)((l.start - l.cnt) / sizeof(unsigned int));
+  const long zero_words = C;
   hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((zero_words + 255) / 256)), dim3(256), 0, ctx->stream,
                      (unsigned int *)cnt, zero_words);
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, ctx->stream, (unsigned int *)dmask, 2L);
   SfTable t{};
   for (int k = 0; k < n_sf; ++k) t.v[k] = sf[k];
-  hipLaunchKernelGGL(k_store_sf, dim3(1), dim3(64), 0, ctx->stream, t, n_sf, dsf);
   const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
   const unsigned blocks = (unsigned)((N + 255) / 256);
   hipLaunchKernelGGL(k_grid_count<false>, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
                      nz, g.ix, g.iy, g.iz, cnt, cellof);
-  exclusive_scan(ctx->stream, cnt, (int)C, start, (int *)(ws + l.part));
+  exclusive_scan(ctx->stream, cnt, (int)C, start, (int *)(ws + l.part), false);
   hipLaunchKernelGGL(k_grid_scatter, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, cellof,
-                     start, fill, ids, px, py, pz);
-  hipLaunchKernelGGL(k_any_overlap_scaled, dim3(blocks), dim3(256), 0, ctx->stream, g, N, dsf, n_sf,
+                     start, ids, px, py, pz);
+  hipLaunchKernelGGL(k_scaled_spheres, dim3(blocks), dim3(256), 0, ctx->stream, g, N, t, n_sf,
                      cut * cut, dmask);
+  hipLaunchKernelGGL(k_sum_all<true>, dim3(1), dim3(1024), 0, ctx->stream, dmask, (int)blocks,
+                     (const unsigned *)nullptr, ctx->h_acc);
   HSMC_HIP(ctx, hipGetLastError());
-  unsigned long long mask = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&mask, dmask, sizeof(mask), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  const unsigned long long mask = ctx->h_acc[0];
   for (int k = 0; k < n_sf; ++k) no_overlap[k] = ((mask >> k) & 1ull) ? 0 : 1;
   return HSMC_OK;
 }
@@ -822,30 +1180,30 @@ int hsmc_gpu_cell_list(hsmc_gpu_ctx *ctx, int replica, int nx, int ny, int nz, i
   const int N = h.p.n_part;
   if (part_cell) {
     int *cnt = (int *)scratch(ctx, S_CNT, sizeof(int) * C);
-    int *fill = (int *)scratch(ctx, S_FILL, sizeof(int) * C);
     int *start = (int *)scratch(ctx, S_START, sizeof(int) * (C + 1));
-    int *cellof = (int *)scratch(ctx, S_CELLOF, sizeof(int) * N);
+    int2 *cellof = (int2 *)scratch(ctx, S_CELLOF, sizeof(int2) * N);
     int *ids = (int *)scratch(ctx, S_IDS, sizeof(int) * N);
     double *px = (double *)scratch(ctx, S_PX, sizeof(double) * N);
     double *py = (double *)scratch(ctx, S_PY, sizeof(double) * N);
     double *pz = (double *)scratch(ctx, S_PZ, sizeof(double) * N);
     int *rows = (int *)scratch(ctx, S_OUT0, sizeof(int) * C * max_part);
     int *part = (int *)scratch(ctx, S_PART, sizeof(int) * scan_workspace_ints(C));
-    if (!cnt || !fill || !start || !cellof || !ids || !px || !py || !pz || !rows || !part)
+    if (!cnt || !start || !cellof || !ids || !px || !py || !pz || !rows || !part)
       return HSMC_ERR_NO_MEMORY;
     ctx->aux_replica = -1;  // the CSR scratch now holds this grid
     const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
-    HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * C, ctx->stream));
-    HSMC_HIP(ctx, hipMemsetAsync(fill, 0, sizeof(int) * C, ctx->stream));
+  long clear = 0;
+  if (clear_counts(ctx, cnt, C, &clear)) return HSMC_ERR_HIP;
     const unsigned blocks = (unsigned)((N + 255) / 256);
     hipLaunchKernelGGL(k_grid_count<true>, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
                        nz, sx, sy, sz, cnt, cellof);
-    exclusive_scan(ctx->stream, cnt, (int)C, start, part);
+    exclusive_scan(ctx->stream, cnt, (int)C, start, part, true);
     hipLaunchKernelGGL(k_grid_scatter, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, cellof,
-                       start, fill, ids, px, py, pz);
+                     start, ids, px, py, pz);
     hipLaunchKernelGGL(k_part_cell, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, ctx->stream,
                        start, (int)C, ids, max_part, rows, ctx->d_err);
     HSMC_HIP(ctx, hipGetLastError());
+    ctx->counts_clear = clear;
     HSMC_HIP(ctx, hipMemcpyAsync(part_cell, rows, sizeof(int) * C * max_part,
                                  hipMemcpyDeviceToHost, ctx->stream));
     HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -931,22 +1289,44 @@ int hsmc_gpu_any_overlap_scaled(hsmc_gpu_ctx *ctx, int replica, const double *sf
     if (!(sf[k] > 0.0)) return HSMC_ERR_BAD_ARG;
     smin = std::min(smin, sf[k]);
   }
-  const double cut = (1.0 / smin) * (1.0 + 1e-6);
-  Grid g;
-  int st = build_grid(ctx, replica, cut, g);
-  if (st) return st;
-  const int N = ctx->reps[replica].p.n_part;
-  double *dsf = (double *)scratch(ctx, S_Q1, sizeof(double) * n_sf);
-  unsigned long long *dmask = (unsigned long long *)scratch(ctx, S_OUT1, sizeof(unsigned long long));
-  if (!dsf || !dmask) return HSMC_ERR_NO_MEMORY;
-  HSMC_HIP(ctx, hipMemcpyAsync(dsf, sf, sizeof(double) * n_sf, hipMemcpyHostToDevice, ctx->stream));
-  HSMC_HIP(ctx, hipMemsetAsync(dmask, 0, sizeof(unsigned long long), ctx->stream));
-  hipLaunchKernelGGL(k_any_overlap_scaled, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, g, N,
-                     dsf, n_sf, cut * cut, dmask);
+  const double cut = (1.0 / smin) * (1.0 + 1e-6), cut2 = cut * cut;
+  const RepHost &h = ctx->reps[replica];
+  const int N = h.p.n_part;
+  SfTable t{};
+  for (int k = 0; k < n_sf; ++k) t.v[k] = sf[k];
+  unsigned blocks;
+  unsigned long long *part;
+  if (N <= kAllPairs) {
+    const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
+    blocks = all_pairs_blocks(N);
+    part = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * blocks);
+    if (!part) return HSMC_ERR_NO_MEMORY;
+    hipLaunchKernelGGL(N <= kSmallRuns ? k_scaled_all<16> : k_scaled_all<64>, dim3(blocks),
+                       dim3(kPairThreads), 0, ctx->stream, x, y, z, N, h.p.lx, h.p.ly, h.p.lz, t, n_sf,
+                       cut2, part);
+  } else {
+    // cells of a few spheres give row_pairs' lanes work
+    const double side = std::max(cut, kRowSide);
+    const bool rows = cells_at_least(h.p, side, 3);
+    Grid g;
+    int st = build_grid(ctx, replica, rows ? side : cut, g);
+    if (st) return st;
+    const long C = (long)g.nx * g.ny * g.nz;
+    blocks = rows ? (unsigned)std::min(C, (long)kRowBlocks) : (unsigned)((N + 255) / 256);
+    part = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * blocks);
+    if (!part) return HSMC_ERR_NO_MEMORY;
+    if (rows)
+      hipLaunchKernelGGL(k_scaled_rows, dim3(blocks), dim3(kRowThreads), 0, ctx->stream, g, t, n_sf,
+                         cut2, part);
+    else
+      hipLaunchKernelGGL(k_scaled_spheres, dim3(blocks), dim3(256), 0, ctx->stream, g, N, t, n_sf, cut2,
+                         part);
+  }
+  hipLaunchKernelGGL(k_sum_all<true>, dim3(1), dim3(1024), 0, ctx->stream, part, (int)blocks,
+                     (const unsigned *)nullptr, ctx->h_acc);
   HSMC_HIP(ctx, hipGetLastError());
-  unsigned long long mask = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&mask, dmask, sizeof(mask), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  const unsigned long long mask = ctx->h_acc[0];
   for (int k = 0; k < n_sf; ++k) no_overlap[k] = ((mask >> k) & 1ull) ? 0 : 1;
   return HSMC_OK;
 }
@@ -986,30 +1366,59 @@ static int pair_hist(hsmc_gpu_ctx *ctx, int replica, double dr_bin, int nbins, d
     return HSMC_ERR_BAD_ARG;
   }
   const double cut = rmax_eff * (1.0 + 1e-9);
-  Grid g;
-  int st = build_grid(ctx, replica, cut, g);
-  if (st) return st;
   const int N = h.p.n_part;
-  unsigned long long *dcounts = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * (nbins + 1));
-  if (!dcounts) return HSMC_ERR_NO_MEMORY;
-  HSMC_HIP(ctx, hipMemsetAsync(dcounts, 0, sizeof(unsigned long long) * (nbins + 1), ctx->stream));
-  const double cut2 = (rmax_eff * (1.0 + 1e-6)) * (rmax_eff * (1.0 + 1e-6));
-  const long C = (long)g.nx * g.ny * g.nz;
-  if (N >= 16 * C && pair_tiled_lds(nbins) <= 64 * 1024 && 27 * C < (1L << 31)) {
-    // cells of 16 spheres or more on average: one wave per cell pair
-    hipLaunchKernelGGL(k_pair_hist_tiled, dim3((unsigned)(27 * C)), dim3(64), pair_tiled_lds(nbins),
-                       ctx->stream, g, nbins, dr_bin, rmax_eff, cut2, dcounts, dcounts + nbins);
+  Bins bn{dr_bin, rmax_eff, 0.0, (float)(1.0 / dr_bin), nbins, nullptr};
+  bn.smax = first_double(rmax_eff * rmax_eff, [&](double s) { return !(sqrt(s) < rmax_eff); });
+  // the edges for the many bins of g(r); a contact histogram's few pairs are
+  // binned by the formula, and above 2048 bins the edges would leave LDS
+  const bool edges = nbins > 16 && nbins <= 2048;
+  if (edges) {
+    int st = bin_edges(ctx, dr_bin, nbins, &bn.edge);
+    if (st) return st;
+  }
+  const size_t lds = sizeof(unsigned int) * (((size_t)nbins + 1) & ~(size_t)1) +
+                     (edges ? sizeof(double) * ((size_t)nbins + 1) : 0);
+  unsigned blocks;
+  auto rows_of = [&]() {
+    return (unsigned int *)scratch(ctx, S_OUT0, sizeof(unsigned int) * ((size_t)nbins + 1) * blocks);
+  };
+  unsigned int *part;
+  if (N <= (rmax_eff < kWide ? kAllPairs : kAllPairsWide)) {
+    const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
+    blocks = all_pairs_blocks(N);
+    part = rows_of();
+    if (!part) return HSMC_ERR_NO_MEMORY;
+    auto fn = N <= kSmallRuns ? (edges ? k_hist_all<16, true> : k_hist_all<16, false>)
+                              : (edges ? k_hist_all<64, true> : k_hist_all<64, false>);
+    hipLaunchKernelGGL(fn, dim3(blocks), dim3(kPairThreads), lds, ctx->stream, x, y, z, N, h.p.lx,
+                       h.p.ly, h.p.lz, bn, part);
   } else {
-    hipLaunchKernelGGL(k_pair_hist, dim3((N + 255) / 256), dim3(256), sizeof(unsigned int) * nbins,
-                       ctx->stream, g, N, dr_bin, nbins, rmax_eff, cut2, dcounts, dcounts + nbins);
+    // a stencil of 5^3 cells of half the cutoff has 0.58 of the volume of
+    // 3^3 cells of the cutoff, as long as those cells hold some spheres
+    const bool two = rmax_eff >= kWide && cells_at_least(h.p, cut / 2.0, 5);
+    const double side = two ? cut / 2.0 : std::max(cut, kRowSide);
+    const bool rows = two || cells_at_least(h.p, side, 3);
+    Grid g;
+    int st = build_grid(ctx, replica, rows ? side : cut, g);
+    if (st) return st;
+    const long C = (long)g.nx * g.ny * g.nz;
+    blocks = rows ? (unsigned)std::min(C, (long)kRowBlocks) : (unsigned)((N + 255) / 256);
+    part = rows_of();
+    if (!part) return HSMC_ERR_NO_MEMORY;
+    if (rows) {
+      auto fn = two ? (edges ? k_hist_rows<2, true> : k_hist_rows<2, false>)
+                    : (edges ? k_hist_rows<1, true> : k_hist_rows<1, false>);
+      hipLaunchKernelGGL(fn, dim3(blocks), dim3(kRowThreads), lds, ctx->stream, g, bn, part);
+    } else {
+      hipLaunchKernelGGL(edges ? k_hist_spheres<true> : k_hist_spheres<false>, dim3(blocks), dim3(256),
+                         lds, ctx->stream, g, N, bn, part);
+    }
   }
   HSMC_HIP(ctx, hipGetLastError());
-  std::vector<unsigned long long> hc(nbins + 1);
-  HSMC_HIP(ctx, hipMemcpyAsync(hc.data(), dcounts, sizeof(unsigned long long) * (nbins + 1),
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  for (int b = 0; b < nbins; ++b) counts[b] = (int64_t)hc[b];
-  if (oor) *oor = (int64_t)hc[nbins];
+  int st = sum_rows(ctx, part, (int)blocks, nbins + 1);
+  if (st) return st;
+  for (int b = 0; b < nbins; ++b) counts[b] = (int64_t)ctx->h_acc[b];
+  if (oor) *oor = (int64_t)ctx->h_acc[nbins];
   return HSMC_OK;
 }
 
@@ -1060,24 +1469,32 @@ int hsmc_gpu_widom_uniform(hsmc_gpu_ctx *ctx, int replica, uint64_t seed, uint64
   if (bad_replica(ctx, replica) || n < 0 || first < 0 || !hits) return HSMC_ERR_BAD_ARG;
   *hits = 0;
   if (n == 0) return HSMC_OK;
+  const RepHost &h = ctx->reps[replica];
+  const int N = h.p.n_part;
   Grid g;
-  int st = build_grid(ctx, replica, 1.0 + 1e-9, g);
-  if (st) return st;
-  unsigned long long *dh = (unsigned long long *)scratch(ctx, S_OUT1, sizeof(unsigned long long));
-  if (!dh) return HSMC_ERR_NO_MEMORY;
-  HSMC_HIP(ctx, hipMemsetAsync(dh, 0, sizeof(unsigned long long), ctx->stream));
-  const long long per_block = 256LL * 16;
-  long long blocks = (n + per_block - 1) / per_block;
-  if (blocks > 65536) blocks = 65536;
-  if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(k_widom_uniform, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, g,
-                     (uint32_t)seed, (uint32_t)(seed >> 32), (unsigned long long)sample,
-                     (long long)first, (long long)n, dh);
+  set_grid(h, 1.0 + 1e-9, g);
+  const size_t lds = widom_lds_bytes(N, (long)g.nx * g.ny * g.nz);
+  const bool in_lds = N <= kWidomLdsSpheres && lds <= 64 * 1024;
+  const long long wg = in_lds ? kWidomLdsThreads : 256, most = in_lds ? kWidomLdsBlocks : kWidomUniformBlocks;
+  const long long blocks = std::min((n + wg - 1) / wg, most);
+  unsigned long long *part = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * blocks);
+  if (!part) return HSMC_ERR_NO_MEMORY;
+  if (in_lds) {
+    hipLaunchKernelGGL(k_widom_uniform_lds, dim3((unsigned)blocks), dim3((unsigned)wg), lds, ctx->stream, g, N,
+                       ctx->d_x + h.poff, ctx->d_y + h.poff, ctx->d_z + h.poff, (uint32_t)seed,
+                       (uint32_t)(seed >> 32), (unsigned long long)sample, (long long)first, (long long)n, part);
+  } else {
+    int st = build_grid(ctx, replica, 1.0 + 1e-9, g);
+    if (st) return st;
+    hipLaunchKernelGGL(k_widom_uniform, dim3((unsigned)blocks), dim3((unsigned)wg), 0, ctx->stream, g,
+                       (uint32_t)seed, (uint32_t)(seed >> 32), (unsigned long long)sample,
+                       (long long)first, (long long)n, part);
+  }
+  hipLaunchKernelGGL(k_sum_all<false>, dim3(1), dim3(1024), 0, ctx->stream, part, (int)blocks,
+                     (const unsigned *)nullptr, ctx->h_acc);
   HSMC_HIP(ctx, hipGetLastError());
-  unsigned long long hv = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&hv, dh, sizeof(hv), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  *hits = (int64_t)hv;
+  *hits = (int64_t)ctx->h_acc[0];
   return HSMC_OK;
 }
 
@@ -1106,19 +1523,18 @@ int hsmc_gpu_widom_cells(hsmc_gpu_ctx *ctx, int replica, uint64_t seed, uint64_t
     ctx->last_error = "observable-grid cells too wide for the stratified insertion kernel";
     return HSMC_ERR_NOT_SUPPORTED;
   }
-  unsigned long long *dh = (unsigned long long *)scratch(ctx, S_OUT1, sizeof(unsigned long long));
-  if (!dh) return HSMC_ERR_NO_MEMORY;
-  HSMC_HIP(ctx, hipMemsetAsync(dh, 0, sizeof(unsigned long long), ctx->stream));
-  const long blocks = std::min((C + kWidomCellsWaves - 1) / kWidomCellsWaves, 1L << 20);
+  const long blocks = std::min((C + kWidomCellsWaves - 1) / kWidomCellsWaves, (long)kWidomCellsBlocks);
+  unsigned long long *part = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * blocks);
+  if (!part) return HSMC_ERR_NO_MEMORY;
   hipLaunchKernelGGL(k_widom_cells, dim3((unsigned)blocks), dim3(64 * kWidomCellsWaves), 0, ctx->stream, g,
                      (uint32_t)seed, (uint32_t)(seed >> 32), (unsigned long long)sample, (int)per_cell,
-                     dh, ctx->d_err);
+                     part, ctx->d_err);
+  hipLaunchKernelGGL(k_sum_all<false>, dim3(1), dim3(1024), 0, ctx->stream, part, (int)blocks, ctx->d_err,
+                     ctx->h_acc);
   HSMC_HIP(ctx, hipGetLastError());
-  unsigned long long hv = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&hv, dh, sizeof(hv), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  *hits = (int64_t)hv;
-  return check_device_errors(ctx);
+  *hits = (int64_t)ctx->h_acc[0];
+  return ctx->h_acc[1] ? check_device_errors(ctx) : HSMC_OK;  // the kernel's view of the sticky bits
 }
 
 }  // extern "C"

@@ -1,0 +1,170 @@
+"""Pair histograms, scaled-overlap flags and uniform insertions at the sizes
+where their kernels change: with and without a neighbour grid, tile edges of
+the all-pairs kernels, the 3^3 and 5^3 stencils and their fallback on thin
+boxes, bins by formula and by edges, spheres filed in LDS or in memory.
+Every result is compared with FP64 numpy over all pairs, bit for bit."""
+import math
+
+import numpy as np
+import pytest
+
+from hsmc_amd import gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def _context(xyz, box):
+    conf = np.zeros((len(xyz), 4))
+    conf[:, 0] = np.arange(len(xyz))
+    conf[:, 1:] = xyz
+    ctx = gpu.Context([dict(n=len(xyz), box=tuple(box))])
+    ctx.upload(conf)
+    return ctx
+
+
+def _image(d, L):
+    return np.where(d > L / 2, d - L, np.where(d < -L / 2, d + L, d))
+
+
+def _near_pairs(xyz, box, reach):
+    """(i, j, squared distance) of the pairs i < j closer than about reach."""
+    out = []
+    for a in range(0, len(xyz), 256):
+        s = 0.0
+        for k in range(3):
+            d = _image(xyz[a:a + 256, None, k] - xyz[None, :, k], box[k])
+            s = s + d * d if k else d * d
+        i, j = np.nonzero(s < reach * reach * (1 + 1e-9))
+        keep = j > i + a
+        out.append((i[keep] + a, j[keep], s[i[keep], j[keep]]))
+    return tuple(np.concatenate(v) for v in zip(*out))
+
+
+def _histogram(s, dr_bin, nbins, rmax):
+    dr = np.sqrt(s)
+    b = ((dr[dr < rmax] - 1.0) / dr_bin).astype(np.int64)   # truncation, as in C
+    ok = (b >= 0) & (b < nbins)
+    return np.bincount(b[ok], minlength=nbins), int((~ok).sum())
+
+
+BOXES = {
+    # cubic boxes at density 0.8; N around the all-pairs tiles (64), run
+    # lengths (4096) and the steps to a grid (5120, 7168)
+    **{f"cube-{n}": (n, None) for n in (1, 2, 63, 64, 65, 127, 129, 1000, 4096, 4097, 5120, 5121, 7168, 7169)},
+    # a grid with fewer than 3 cells along x; exactly 3 of side 2 and more;
+    # exactly 5 of half a cutoff of 4.4 and more
+    "thin-2": (8300, (4.5, 4.6)), "thin-3": (8400, (7.0, 8.3)), "thin-5": (8500, (11.1, 13.9)),
+}
+
+
+@pytest.mark.parametrize("name", list(BOXES))
+def test_histograms_match_all_pairs(name):
+    n, thin = BOXES[name]
+    vol = max(n / 0.8, 75.0)
+    box = np.array([vol ** (1 / 3)] * 3 if thin is None else [thin[0], thin[1], vol / (thin[0] * thin[1])])
+    rng = np.random.default_rng(n)
+    xyz = rng.random((n, 3)) * box   # overlapping points too: bins below 0 count as out of range
+    xyz[0] = box                     # coordinates at the edge itself
+    half = min(box) / 2
+    reach = min(5.5, half)
+    _, _, s = _near_pairs(xyz, box, reach)
+    ctx = _context(xyz, box)
+    # (bin width, bins, cutoff): contact; formula / edges (16, 17); edges in
+    # LDS / not (2048, 2049); more bins than the cutoff reaches; fewer
+    for dr_bin, nbins, rmax in ((0.01, 5, 1.05), (0.02, 16, 1.32), (0.02, 17, 1.34), (0.01, 400, 5.0),
+                                (0.002, 2048, 5.096), (0.002, 2049, 5.098), (0.01, 300, 2.1),
+                                (0.013, 40, 4.4)):
+        rmax = min(rmax, half)
+        if rmax <= 1.0:
+            continue
+        want = _histogram(s, dr_bin, nbins, rmax)
+        got = ctx.rdf_counts(dr_bin, nbins, rmax)
+        assert np.array_equal(got[0], want[0]), (dr_bin, nbins, rmax)
+        assert got[1] == want[1], (dr_bin, nbins, rmax)
+    ctx.close()
+
+
+def test_histogram_bins_at_their_edges():
+    """Pairs whose distance is within a few units in the last place of a bin
+    edge fall in the bin the formula gives: 64 spheres far apart on a line in
+    y and z, partners at 1 + b dr_bin and its neighbours along x."""
+    dr_bin, nbins = 0.01, 64
+    box = np.array([8.0, 24.0, 24.0])
+    xyz = []
+    for b in range(nbins):
+        y, z = 1.5 * (b % 8) + 6.0 * (b % 2), 1.5 * (b // 8)
+        d = 1.0 + b * dr_bin
+        for _ in range(b % 5):
+            d = np.nextafter(d, 0.0 if b % 2 else 9.0)
+        xyz += [(0.0, y, z), (d, y, z)]
+    xyz = np.array(xyz)
+    i, j, s = _near_pairs(xyz, box, 2.0)
+    ctx = _context(xyz, box)
+    for n in (10, 30, nbins):
+        want = _histogram(s, dr_bin, n, 1.0 + nbins * dr_bin)
+        got = ctx.rdf_counts(dr_bin, n, 1.0 + nbins * dr_bin)
+        assert np.array_equal(got[0], want[0]) and got[1] == want[1], n
+    ctx.close()
+
+
+@pytest.mark.parametrize("shape,drop", [((4, 4, 4), 1), ((8, 8, 16), 0), ((16, 16, 16), 0),
+                                        ((16, 16, 17), 5), ((16, 16, 20), 0), ((16, 16, 21), 3),
+                                        ((4, 45, 50), 2), ((6, 38, 40), 7)])
+def test_scaled_flags_match_all_pairs(shape, drop):
+    """64 compressions on a jittered cubic lattice whose closest pair lies
+    inside their range."""
+    a = 1.012
+    box = a * np.array(shape)
+    rng = np.random.default_rng(sum(shape))
+    sites = np.stack(np.meshgrid(*(np.arange(k) for k in shape), indexing="ij"), -1).reshape(-1, 3)
+    sites = sites[np.sort(rng.permutation(len(sites))[drop:])]
+    xyz = (sites * a + rng.uniform(-0.0035, 0.0035, sites.shape)) % box
+    ctx = _context(xyz, box)
+    i, j, s = _near_pairs(xyz, box, 1.03)
+    sf = np.linspace(1.0, 0.985, 64)
+    want = []
+    for f in sf:
+        t = 0.0
+        for k in range(3):
+            d = _image((xyz[i, k] - xyz[j, k]) * f, box[k] * f)
+            t = t + d * d if k else d * d
+        want.append(not np.any(t < 1.0))
+    assert want[0] and not want[-1]
+    assert np.array_equal(ctx.any_overlap_scaled(sf), np.array(want, dtype=np.uint8))
+    assert ctx.any_overlap_scaled([sf[20]])[0] == want[20]
+    ctx.close()
+
+
+def _uniform(seed, n):
+    """Points 0..n-1 of the uniform insertions' Philox4x32-10 stream."""
+    mask = np.uint64(0xFFFFFFFF)
+    c = [np.arange(n, dtype=np.uint64), np.zeros(n, np.uint64), np.zeros(n, np.uint64),
+         np.full(n, 0x57490000, np.uint64)]
+    k0, k1 = seed & 0xFFFFFFFF, (seed >> 32) & 0xFFFFFFFF
+    for _ in range(10):
+        a, b = np.uint64(0xD2511F53) * c[0], np.uint64(0xCD9E8D57) * c[2]
+        c = [(b >> np.uint64(32)) ^ c[1] ^ np.uint64(k0), b & mask,
+             (a >> np.uint64(32)) ^ c[3] ^ np.uint64(k1), a & mask]
+        k0, k1 = (k0 + 0x9E3779B9) & 0xFFFFFFFF, (k1 + 0xBB67AE85) & 0xFFFFFFFF
+    return np.stack([w.astype(np.float64) / 4294967295.0 for w in c[:3]], 1)
+
+
+@pytest.mark.parametrize("n,rho", [(1, 0.01), (108, 0.7), (511, 0.3), (2048, 0.45), (2049, 0.45),
+                                   (1500, 0.12), (700, 0.02)])
+def test_uniform_insertions_filed_in_lds_or_memory(n, rho):
+    """Hits of the points themselves, decided over all spheres in numpy;
+    N = 2048 / 2049 and dilute boxes (many cells) are the two sides of the
+    LDS rule.  5000 points leave the last workgroup partly idle."""
+    rng = np.random.default_rng(n)
+    L = (n / rho) ** (1 / 3)
+    xyz = rng.random((n, 3)) * L
+    ctx = _context(xyz, (L, L, L))
+    pts = _uniform(31 + (n << 33), 5000) * L
+    near = np.full(len(pts), np.inf)
+    for a in range(0, n, 64):
+        s = sum(_image(pts[:, None, k] - xyz[None, a:a + 64, k], L) ** 2 for k in range(3))
+        near = np.minimum(near, s.min(1))
+    assert np.min(np.abs(near - 1.0)) > 1e-9   # no point for which the order of the sum matters
+    for m in (1, 511, 5000):
+        assert ctx.widom_uniform(31 + (n << 33), 0, 0, m) == int((near[:m] >= 1.0).sum())
+    ctx.close()
