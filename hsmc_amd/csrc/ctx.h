@@ -129,6 +129,16 @@ struct hsmc_gpu_ctx {
   double edge_dr = 0.0;
   int edge_bins = 0;
   hsmc_gpu_tuning tune{32, 8, 32, 0};
+  // the launch shape was set by hand: sweeps run in that shape even where the
+  // resident kernel would take them
+  bool tune_set = false;
+  // sweeps since the move counters were last folded into the host totals, as
+  // far as the resident kernel made them (a counter takes at most
+  // 2^32 attempts)
+  unsigned long long resident_sweeps = 0;
+  // the launched sweeps' count buffers may hold an earlier sweep's counts
+  // (the resident kernel ran, or the sweep counter moved)
+  bool counts_stale = false;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   int graph_sweeps = 0;
@@ -179,6 +189,14 @@ int layout(hsmc_gpu_ctx *ctx);
 size_t phase_lds_bytes(int cap, int lcap, int cpb);
 // n checkerboard sweeps of every replica (enqueued on the context stream)
 int run_sweeps(hsmc_gpu_ctx *ctx, int n);
+// Resident sweeps (resident.hip): whether the context's replicas run that
+// way, in what shape, and n sweeps of all of them.
+struct ResidentShape {
+  int lpc = 0, threads = 0;
+  size_t bytes = 0;
+};
+bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape);
+int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, int n);
 // File the current by-id positions into the cell slots of the last sweep's
 // grid (the cell list the volume-move scan reads after positions changed).
 int rebin_last_sweep(hsmc_gpu_ctx *ctx);

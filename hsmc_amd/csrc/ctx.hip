@@ -84,6 +84,7 @@ int fold_counters(hsmc_gpu_ctx *ctx) {
     ctx->tot_acc[r] += sa;
     ctx->tot_left[r] += sl;
   }
+  ctx->resident_sweeps = 0;
   return HSMC_OK;
 }
 

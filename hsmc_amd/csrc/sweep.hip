@@ -30,6 +30,7 @@
 
 #include "ctx.h"
 #include "device_common.h"
+#include "sweep_draws.h"
 
 using namespace hsmc;
 
@@ -45,35 +46,6 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Shift of the sweep grid for one sweep: 3 uniform draws in [0, side).
-__device__ __forceinline__ void sweep_shift(const RepDev &rp, unsigned long long sweep,
-                                            double &shx, double &shy, double &shz) {
-  uint32_t u[4];
-  philox4x32_10(0xFFFFFFFFu, 0u, (uint32_t)sweep, (uint32_t)(sweep >> 32), rp.k0, rp.k1, u);
-  shx = ((double)u[0] * 0x1p-32) * rp.sx;
-  shy = ((double)u[1] * 0x1p-32) * rp.sy;
-  shz = ((double)u[2] * 0x1p-32) * rp.sz;
-}
-
-// Order of the 8 sublattices in one sweep: a Fisher-Yates order of 0..7
-// drawn from one Philox block, kept as 8 nibbles (nibble p = sublattice of
-// phase p).
-__device__ __forceinline__ uint32_t sweep_order(const RepDev &rp, unsigned long long sweep) {
-  uint32_t u[4];
-  philox4x32_10(0xFFFFFFFEu, 0u, (uint32_t)sweep, (uint32_t)(sweep >> 32), rp.k0, rp.k1, u);
-  uint32_t pk = 0x76543210u;
-#pragma unroll
-  for (int h = 0; h < 7; ++h) {
-    const int i = 7 - h;
-    const uint32_t half = (u[h >> 1] >> (16 * (h & 1))) & 0xFFFFu;
-    const int j = (int)((half * (uint32_t)(i + 1)) >> 16);
-    const uint32_t vi = (pk >> (4 * i)) & 0xFu, vj = (pk >> (4 * j)) & 0xFu;
-    pk &= ~((0xFu << (4 * i)) | (0xFu << (4 * j)));
-    pk |= (vi << (4 * j)) | (vj << (4 * i));
-  }
-  return pk;
 }
 
 // Work item i of a sweep's rebin: clear cell i of the next sweep's count
@@ -685,6 +657,11 @@ __global__ void k_advance(unsigned long long *sweep_base, int n) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *sweep_base += (unsigned long long)n;
 }
 
+__global__ void k_zero_counts(int *__restrict__ cnt, long n) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) cnt[i] = 0;
+}
+
 // The phase kernel's occupant pick for attempts t < count of one cell, any n.
 __global__ void __launch_bounds__(256)
 k_occupant_picks(uint32_t k0, uint32_t k1, uint32_t cell, unsigned long long sweep, uint32_t n,
@@ -900,6 +877,14 @@ bool same_launch_shape(const hsmc_gpu_tuning &a, const hsmc_gpu_tuning &b) {
 
 }  // namespace
 
+// Both count buffers at zero, as a launched sweep expects the one it fills.
+static void fresh_counts(hsmc_gpu_ctx *ctx) {
+  if (!ctx->counts_stale) return;
+  hipLaunchKernelGGL(k_zero_counts, dim3((unsigned)((2 * ctx->Ctot + 255) / 256)), dim3(256), 0, ctx->stream,
+                     ctx->d_cnt, 2 * ctx->Ctot);
+  ctx->counts_stale = false;
+}
+
 namespace hsmc {
 // After each batch of sweeps the device's error bits are copied to pinned
 // host memory without waiting; a batch is launched only while the copies
@@ -910,6 +895,30 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
   if (n <= 0) return HSMC_OK;
   if (*ctx->h_err) return check_device_errors(ctx);
   ctx->version++;
+  ResidentShape shape;
+  if (!ctx->tune_set && resident_shape(ctx, &shape)) {
+    // launches of at most 4096 sweeps, so that an error stops a long call
+    constexpr int per = 4096;
+    for (int done = 0; done < n; done += per) {
+      if (*ctx->h_err) return check_device_errors(ctx);
+      const int k = std::min(per, n - done);
+      // a counter entry gathers the attempts of C / 8 / groups cells, below
+      // 256 a sweep: 2^24 sweeps stay below 2^32
+      if (ctx->resident_sweeps + k > (1u << 24)) {
+        int st = fold_counters(ctx);
+        if (st) return st;
+      }
+      int st = launch_resident(ctx, shape, k);
+      if (st) return st;
+      ctx->resident_sweeps += k;
+      HSMC_HIP(ctx, hipMemcpyAsync((void *)ctx->h_err, ctx->d_err, sizeof(unsigned int),
+                                   hipMemcpyDeviceToHost, ctx->stream));
+    }
+    ctx->cells_version = 0;  // no cell list in memory
+    ctx->counts_stale = true;
+    return HSMC_OK;
+  }
+  fresh_counts(ctx);
   if (ctx->tune.persistent) {  // cooperative launches of whole sweeps
     const int per = ctx->tune.sweeps_per_graph > 0 ? ctx->tune.sweeps_per_graph : 64;
     for (int done = 0; done < n; done += per) {
@@ -1002,8 +1011,10 @@ int hsmc_gpu_time_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, float *ms) {
   // capture outside the timed region: the batch graph, and a graph of
   // exactly the remaining n mod sweeps_per_graph sweeps (the whole call when
   // it is shorter than a batch), so every timed sweep is a graph replay
-  // (persistent launches capture nothing)
-  const int K = ctx->tune.persistent ? 0 : ctx->tune.sweeps_per_graph;
+  // (persistent launches and resident sweeps capture nothing)
+  ResidentShape shape;
+  const bool resident = !ctx->tune_set && resident_shape(ctx, &shape);
+  const int K = ctx->tune.persistent || resident ? 0 : ctx->tune.sweeps_per_graph;
   if (K > 0 && n_sweeps >= K &&
       (!ctx->gexec || ctx->graph_sweeps != K || !same_launch_shape(ctx->graph_tune, ctx->tune))) {
     int st = capture_graph(ctx, K);
@@ -1031,6 +1042,7 @@ int hsmc_gpu_time_phase_kernel(hsmc_gpu_ctx *ctx, int n_sweeps, float *avg_ms, i
   // once per 8 launches
   hipEvent_t ev[16];
   for (int i = 0; i < 16; ++i) HSMC_HIP(ctx, hipEventCreate(&ev[i]));
+  fresh_counts(ctx);
   double total = 0.0;
   int count = 0;
   for (int s = 0; s < n_sweeps; ++s) {
@@ -1109,14 +1121,16 @@ int hsmc_gpu_set_sweep_counter(hsmc_gpu_ctx *ctx, uint64_t sweep) {
   // attempts are N * (sweep - sweep_at_reset): move the origin with the counter
   ctx->sweep_at_reset += want - now;
   // the last sweep's cell list is found by the counter's parity: refile it
-  // before anything reads it
+  // before anything reads it, and clear it before it is filled again
   ctx->cells_version = 0;
+  ctx->counts_stale = true;
   return HSMC_OK;
 }
 
 int hsmc_gpu_set_tuning(hsmc_gpu_ctx *ctx, const hsmc_gpu_tuning *t) {
   if (!ctx || !t || !tuning_ok(ctx, *t)) return HSMC_ERR_BAD_ARG;
   ctx->tune = *t;
+  ctx->tune_set = true;
   drop_graph(ctx);
   return HSMC_OK;
 }
@@ -1145,8 +1159,28 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
   HSMC_HIP(ctx, hipMemcpyAsync(&sweep0, ctx->d_sweep, sizeof(sweep0), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   const hsmc_gpu_tuning start = ctx->tune;
+  const bool start_set = ctx->tune_set;
   hsmc_gpu_tuning winner = start;
   float best_ms = 1e30f;
+  // the resident kernel, where the replicas fit it, stands beside the launch
+  // shapes; when it wins the tuning stays as it was and is not in force
+  bool resident = false;
+  {
+    ResidentShape shape;
+    if (resident_shape(ctx, &shape)) {
+      ctx->tune_set = false;
+      float ms = 0.f;
+      int st = hsmc_gpu_time_sweeps(ctx, std::max(2, sweeps_per_trial / 4), &ms);
+      if (st == HSMC_OK) st = hsmc_gpu_time_sweeps(ctx, sweeps_per_trial, &ms);
+      if (st != HSMC_OK) {
+        ctx->tune_set = start_set;
+        return st;
+      }
+      best_ms = ms;
+      resident = true;
+    }
+  }
+  ctx->tune_set = true;
   const int lpcs[2] = {32, 64};
   const int cpbs[4] = {1, 2, 4, 8};
   const int graphs[3] = {0, 16, 64};
@@ -1163,14 +1197,17 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
         if (st == HSMC_OK) st = hsmc_gpu_time_sweeps(ctx, sweeps_per_trial, &ms);
         if (st != HSMC_OK) {
           ctx->tune = start;
+          ctx->tune_set = start_set;
           return st;
         }
         if (ms < best_ms) {
           best_ms = ms;
           winner = t;
+          resident = false;
         }
       }
   ctx->tune = winner;
+  ctx->tune_set = !resident;
   drop_graph(ctx);
   HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_x, save, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
   HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_y, save + P, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
