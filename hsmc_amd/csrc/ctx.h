@@ -119,6 +119,9 @@ struct hsmc_gpu_ctx {
   // after each batch of sweeps, so later batches are not launched onto a
   // cell list that has already overflowed
   volatile unsigned int *h_err = nullptr;
+  // pinned memory of the volume moves (proposals in, decisions out)
+  void *h_npt = nullptr;
+  size_t h_npt_bytes = 0;
   // results of an observable, stored by its last kernel in pinned memory
   unsigned long long *h_acc = nullptr;
   // the observable grids' cell counts: their buffer's size when it was last
@@ -185,6 +188,12 @@ int hip_fail(hsmc_gpu_ctx *ctx, hipError_t e, const char *what);
 void *scratch(hsmc_gpu_ctx *ctx, int slot, size_t bytes);
 // (Re)build replica offsets, the sweep grids, and the device cell arrays.
 int layout(hsmc_gpu_ctx *ctx);
+// Device parameters of one replica from its box, grid and offsets.
+void fill_repdev(const RepHost &h, RepDev &d);
+// Whether the replicas' present boxes keep every sweep grid and capacity;
+// if so their records go to rd (when given), the host's copy of replica 0's
+// follows, and a one-replica graph that carries another one is dropped.
+bool layout_keeps(hsmc_gpu_ctx *ctx, std::vector<RepDev> *rd = nullptr);
 // LDS bytes of one sublattice-phase workgroup of cpb cells
 size_t phase_lds_bytes(int cap, int lcap, int cpb);
 // n checkerboard sweeps of every replica (enqueued on the context stream)

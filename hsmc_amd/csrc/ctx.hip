@@ -103,7 +103,6 @@ long stencil_list_bound(const RepDev &d) {
 
 int lcap_for(long bound) { return bound <= 128 ? 128 : (bound <= 192 ? 192 : 256); }
 
-// Device parameters of one replica from its box, grid and offsets.
 void fill_repdev(const RepHost &h, RepDev &d) {
   const hsmc_gpu_replica &p = h.p;
   d.lx = p.lx; d.ly = p.ly; d.lz = p.lz;
@@ -124,13 +123,7 @@ void fill_repdev(const RepHost &h, RepDev &d) {
 bool needs_big_cells(const RepDev &d) { return d.sx >= 1.1547 || d.sy >= 1.1547 || d.sz >= 1.1547; }
 bool cells_too_wide(const RepDev &d) { return d.sx >= 1.5 || d.sy >= 1.5 || d.sz >= 1.5; }
 
-// Box or step-size change that keeps every replica's sweep grid, the slot
-// capacity and the stencil-list bound: only the parameter table changes.
-// The cell arrays and counters stay valid (the next sweep re-bins every
-// sphere), and so does a captured graph of a batch (its kernels read the
-// table at run time); a one-replica graph carries replica 0's record as a
-// kernel argument and is dropped when that record changes.
-bool layout_in_place(hsmc_gpu_ctx *ctx) {
+bool layout_keeps(hsmc_gpu_ctx *ctx, std::vector<RepDev> *out) {
   if (!ctx->d_cnt || !ctx->d_reps) return false;
   std::vector<RepDev> rd(ctx->R);
   bool big = false;
@@ -150,6 +143,19 @@ bool layout_in_place(hsmc_gpu_ctx *ctx) {
   if ((big ? 16 : 8) != ctx->cap || lcap_for(tmax) != ctx->lcap) return false;
   if (ctx->R == 1 && memcmp(&ctx->rep0, &rd[0], sizeof(RepDev)) != 0) drop_graph(ctx);
   ctx->rep0 = rd[0];
+  if (out) *out = std::move(rd);
+  return true;
+}
+
+// Box or step-size change that keeps every replica's sweep grid, the slot
+// capacity and the stencil-list bound: only the parameter table changes.
+// The cell arrays and counters stay valid (the next sweep re-bins every
+// sphere), and so does a captured graph of a batch (its kernels read the
+// table at run time); a one-replica graph carries replica 0's record as a
+// kernel argument and is dropped when that record changes.
+bool layout_in_place(hsmc_gpu_ctx *ctx) {
+  std::vector<RepDev> rd;
+  if (!layout_keeps(ctx, &rd)) return false;
   if (hipMemcpyAsync(ctx->d_reps, rd.data(), sizeof(RepDev) * ctx->R, hipMemcpyHostToDevice,
                      ctx->stream) != hipSuccess ||
       hipStreamSynchronize(ctx->stream) != hipSuccess)  // rd is freed on return
@@ -416,6 +422,7 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
     if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
   if (ctx->h_err) (void)hipHostFree((void *)ctx->h_err);
   if (ctx->h_acc) (void)hipHostFree(ctx->h_acc);
+  if (ctx->h_npt) (void)hipHostFree(ctx->h_npt);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

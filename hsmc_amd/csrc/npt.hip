@@ -10,11 +10,13 @@
 //   r' < exp(-beta P (V' - V) + (N + 1) ln(V'/V)) (moves.c:117-121), and then
 //   positions and box are scaled by sf (moves.c:129-142).
 // Both kernels leave the NpT distribution invariant, so their composition
-// samples it.  Volume moves are done in rounds: round t holds the t-th move of
-// every replica that draws more than t, and one kernel checks every
-// compression of the round at once.
+// samples it.  In rounds, round t holds the t-th move of every replica that
+// draws more than t, and one kernel checks every compression of the round.
 //
-// The scan reads the cell list the last sweep left (the sweep grid: cells of
+// Replicas of up to 4096 spheres make all of a sweep's moves in one launch
+// (k_volume_moves), larger ones round by round with the scan below.
+//
+// That scan reads the cell list the last sweep left (the sweep grid: cells of
 // side > 1 holding every sphere, filed by the sweep's rebin and kept by its
 // moves, none of which leaves its cell).  A pair closer than 1/sf before
 // scaling lies in neighbouring cells whenever the cell side is at least 1/sf,
@@ -25,6 +27,7 @@
 // its seed (counter: sweep, round, 0, "NPT\0"), so its run does not depend
 // on the other replicas of the batch.
 #include <math.h>
+#include <string.h>
 
 #include <algorithm>
 #include <vector>
@@ -36,7 +39,7 @@ using namespace hsmc;
 
 namespace {
 
-constexpr int S_SF = 40, S_BOX = 41, S_FLAG = 42, S_BLK = 43;
+constexpr int S_FLAG = 15, S_BLK = 16, S_MOVE = 17;  // context scratch slots
 constexpr uint32_t kNptTag = 0x4E505400u;  // "NPT\0"
 
 // Any pair of a replica with a proposed compression (sf[r] > 0) closer than 1
@@ -62,6 +65,7 @@ k_vol_overlap(const RepDev *__restrict__ reps, const SweepDev *__restrict__ swp,
   const int i = i0 + (int)threadIdx.x;
   if (i >= rp.poff + rp.N) return;
   const double sf = sfr[r];
+  if (!(sf > 0.0)) return;  // the whole block
   if (__hip_atomic_load(&flags[r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   const unsigned long long sweep = *sweep_next - 1ull;
   const int *cntb = cnt + (size_t)(sweep & 1ull) * C;
@@ -114,19 +118,226 @@ k_vol_overlap(const RepDev *__restrict__ reps, const SweepDev *__restrict__ swp,
   if (ov) atomicOr(&flags[r], 1);
 }
 
-// Scale the spheres of replicas with sf[r] > 0 into their new boxes
-// (moves.c:134-140: coordinates times sf, then apply_pbc in the new box).
-__global__ void k_scale_batch(const int *__restrict__ prep, int P, double *__restrict__ x,
-                              double *__restrict__ y, double *__restrict__ z,
-                              const double *__restrict__ sfr, const double *__restrict__ box) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P) return;
-  const int r = prep[i];
-  const double sf = sfr[r];
-  if (!(sf > 0.0)) return;
-  x[i] = wrap_once(x[i] * sf, box[3 * r]);
-  y[i] = wrap_once(y[i] * sf, box[3 * r + 1]);
-  z[i] = wrap_once(z[i] * sf, box[3 * r + 2]);
+// A volume move as the host proposes it: its scale factor, whether the
+// acceptance rule passes (decided before the scan: it does not depend on
+// it), and the replica's record in the new box.
+struct VolNode {
+  double sf;
+  int rule, pad;
+  RepDev rec;
+};
+
+// One round of volume moves on the device: the replicas whose move passed
+// the scan (flags) and the rule take their new record and their spheres
+// their scaled positions (moves.c:134-140: coordinates times sf, then
+// apply_pbc in the new box).  Block b takes the 256 spheres from blk[b] on,
+// all of one replica.  The flags go to the host's copy.
+__global__ void __launch_bounds__(256)
+k_vol_apply(const int *__restrict__ blk, const int *__restrict__ prep, const VolNode *__restrict__ node,
+            const int *__restrict__ flags, RepDev *__restrict__ reps, double *__restrict__ x,
+            double *__restrict__ y, double *__restrict__ z, int *__restrict__ host_flags) {
+  const int i0 = blk[blockIdx.x], r = prep[i0];
+  const VolNode &nd = node[r];
+  const double sf = nd.sf;
+  const int hit = flags[r], first = nd.rec.poff;
+  if (i0 == first && threadIdx.x == 0) host_flags[r] = hit;
+  if (!(sf > 0.0) || hit || !nd.rule) return;
+  const int i = i0 + (int)threadIdx.x;
+  if (i < first + nd.rec.N) {
+    x[i] = wrap_once(x[i] * sf, nd.rec.lx);
+    y[i] = wrap_once(y[i] * sf, nd.rec.ly);
+    z[i] = wrap_once(z[i] * sf, nd.rec.lz);
+  }
+  if (i0 == first && threadIdx.x == 0) reps[r] = nd.rec;
+}
+
+// Several volume moves of small replicas in one launch, a workgroup each.
+// Which move follows depends on the one before, so the host lays a replica's
+// next moves out as a binary tree (node k: accepted 2 k + 1, else 2 k + 2)
+// with its own log, exp and pow, and the kernel walks it.
+//
+// One scan serves all the moves: the smallest squared distance s of any pair,
+// on a search grid filed in LDS whose cells cover the strongest compression
+// of the tree.  A move by sf makes an overlap when s sf^2 < 1, and an
+// accepted one scales s by sf^2; the rounding of coordinates and products
+// moves s by less than kNear (a coordinate's is 2^-53 of the box edge), and
+// only where s sf^2 lies within kNear of 1 are the pairs tested one by one
+// with the reference's arithmetic.  Latency-bound, 23 us for the 32 x N = 256
+// of the published table (40 us with a scan per move); a sweep's volume moves
+// took about 400 us as rounds of transfers and waits.
+constexpr int kVolDepth = 4;               // moves per launch at most
+constexpr int kVolThreads = 1024;
+constexpr int kVolPer = 4;                 // spheres per thread at most
+constexpr int kVolSpheres = kVolThreads * kVolPer;
+constexpr int kVolAxis = 16;               // search-grid cells per axis at most
+constexpr double kNear = 1e-9;             // for box edges up to 10^5
+
+struct VolPlan {
+  int steps, first;  // moves of this launch and the replica's first node
+};
+
+__device__ __forceinline__ int search_cells(double L, double cut) {
+  int n = (int)(L / cut);
+  n = n < 1 ? 1 : (n > kVolAxis ? kVolAxis : n);
+  while (n > 1 && L / n < cut) --n;
+  return n;
+}
+
+__global__ void __launch_bounds__(kVolThreads)
+k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
+               const VolNode *__restrict__ nodes, double *__restrict__ gx, double *__restrict__ gy,
+               double *__restrict__ gz, int *__restrict__ result) {
+  extern __shared__ double vol_lds[];
+  __shared__ int tot[kVolThreads / 64];
+  __shared__ double low[kVolThreads / 64];
+  __shared__ VolNode tree[(1 << kVolDepth) - 1];
+  const int r = blockIdx.x, t = threadIdx.x, w = t >> 6;
+  const int steps = plan[r].steps;
+  if (steps == 0) return;
+  // the moves lie in host memory: read once, side by side
+  constexpr int words = sizeof(VolNode) / 8;
+  static_assert(sizeof(VolNode) % 8 == 0 && words * ((1 << kVolDepth) - 1) <= kVolThreads, "one read");
+  const int count = (1 << steps) - 1;
+  if (t < words * count)
+    reinterpret_cast<unsigned long long *>(tree)[t] =
+        reinterpret_cast<const unsigned long long *>(nodes + plan[r].first)[t];
+  const int N = reps[r].N, poff = reps[r].poff;
+  double lx = reps[r].lx, ly = reps[r].ly, lz = reps[r].lz;
+  double x[kVolPer], y[kVolPer], z[kVolPer];
+#pragma unroll
+  for (int u = 0; u < kVolPer; ++u) {
+    const int i = min(t + u * kVolThreads, N - 1);
+    x[u] = gx[poff + i];
+    y[u] = gy[poff + i];
+    z[u] = gz[poff + i];
+  }
+  double *px = vol_lds, *py = px + N, *pz = py + N;
+  int *cnt = reinterpret_cast<int *>(pz + N);  // once filed, the end of each cell
+  __syncthreads();
+  int nx = 1, ny = 1, nz = 1;
+  double ix = 0.0, iy = 0.0, iz = 0.0;  // reciprocal cell sides
+  // file the spheres in cells of side at least cut
+  auto file = [&](double cut) {
+    nx = search_cells(lx, cut);
+    ny = search_cells(ly, cut);
+    nz = search_cells(lz, cut);
+    ix = nx / lx;
+    iy = ny / ly;
+    iz = nz / lz;
+    const int C = nx * ny * nz;
+    __syncthreads();  // an earlier filing is no longer read
+    for (int c = t; c < C; c += kVolThreads) cnt[c] = 0;
+    __syncthreads();
+    int ci[kVolPer], at[kVolPer];
+#pragma unroll
+    for (int u = 0; u < kVolPer; ++u) {
+      if (t + u * kVolThreads < N) {
+        ci[u] = (search_cell(x[u], ix, nx) * ny + search_cell(y[u], iy, ny)) * nz + search_cell(z[u], iz, nz);
+        at[u] = atomicAdd(&cnt[ci[u]], 1);
+      }
+    }
+    __syncthreads();
+    const int per = (C + kVolThreads - 1) / kVolThreads, c0 = min(t * per, C), c1 = min(c0 + per, C);
+    int s = 0;
+    for (int c = c0; c < c1; ++c) s += cnt[c];
+    const int incl = group_inclusive_sum<64>(s);
+    if ((t & 63) == 63) tot[w] = incl;
+    __syncthreads();
+    int run = incl - s;
+    for (int k = 0; k < w; ++k) run += tot[k];
+    for (int c = c0; c < c1; ++c) {
+      run += cnt[c];
+      cnt[c] = run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kVolPer; ++u) {
+      if (t + u * kVolThreads < N) {
+        const int p = (ci[u] ? cnt[ci[u] - 1] : 0) + at[u];
+        px[p] = x[u];
+        py[p] = y[u];
+        pz[p] = z[u];
+      }
+    }
+    __syncthreads();
+  };
+  // the least f(pair) over the pairs of a 27-cell stencil, each once (the
+  // spheres after p in filed order), in every thread
+  auto least = [&](auto &&f) {
+    double m = 1e300;
+    for (int p = t; p < N; p += kVolThreads) {
+      const double ax = px[p], ay = py[p], az = pz[p];
+      const int cx = search_cell(ax, ix, nx), cy = search_cell(ay, iy, ny), cz = search_cell(az, iz, nz);
+      for (int d = 0; d < 27; ++d) {
+        const int dx = d / 9 - 1, dy = (d / 3) % 3 - 1, dz = d % 3 - 1;
+        if (!stencil_axis_ok(dx, nx) || !stencil_axis_ok(dy, ny) || !stencil_axis_ok(dz, nz)) continue;
+        const int c = (wrap_index(cx + dx, nx) * ny + wrap_index(cy + dy, ny)) * nz + wrap_index(cz + dz, nz);
+        const int e = cnt[c];
+        for (int q = max(c ? cnt[c - 1] : 0, p + 1); q < e; ++q) m = fmin(m, f(ax, ay, az, px[q], py[q], pz[q]));
+      }
+    }
+    for (int o = 32; o > 0; o >>= 1) m = fmin(m, __shfl_xor(m, o, 64));
+    __syncthreads();  // low is no longer read
+    if ((t & 63) == 0) low[w] = m;
+    __syncthreads();
+    for (int k = 0; k < kVolThreads / 64; ++k) m = fmin(m, low[k]);
+    return m;
+  };
+  double sf_min = 1.0;  // along any path: at most kVolDepth compressions in a row
+  {
+    double least_sf = 1.0;
+    for (int k = 0; k < count; ++k) least_sf = fmin(least_sf, tree[k].sf);
+    for (int k = 0; k < steps; ++k) sf_min *= least_sf;
+  }
+  file((1.0 / sf_min) * (1.0 + 1e-6));
+  // pairs the grid does not hold are farther apart than 1 / sf_min
+  double s = fmin(least([&](double ax, double ay, double az, double bx, double by, double bz) {
+                    return dist2(ax, ay, az, bx, by, bz, lx, ly, lz);
+                  }),
+                  (1.0 + 1e-6) / (sf_min * sf_min));
+  int cur = 0, bits = 0, moved = 0;
+  for (int k = 0; k < steps; ++k) {
+    const double sf = tree[cur].sf, after = s * sf * sf;
+    bool hit = false;
+    if (sf < 1.0) {  // an expansion makes no overlap
+      hit = after < 1.0;
+      if (fabs(after - 1.0) < kNear) {
+        file((1.0 / sf) * (1.0 + 1e-6));
+        hit = least([&](double ax, double ay, double az, double bx, double by, double bz) {
+                return dist2_scaled(ax, ay, az, bx, by, bz, lx, ly, lz, sf);
+              }) < 1.0;
+      }
+    }
+    const bool accept = !hit && tree[cur].rule;
+    bits |= (hit ? 1 : 0) << k | (accept ? 1 : 0) << (16 + k);
+    if (accept) {
+      lx = tree[cur].rec.lx;
+      ly = tree[cur].rec.ly;
+      lz = tree[cur].rec.lz;
+#pragma unroll
+      for (int u = 0; u < kVolPer; ++u) {
+        x[u] = wrap_once(x[u] * sf, lx);
+        y[u] = wrap_once(y[u] * sf, ly);
+        z[u] = wrap_once(z[u] * sf, lz);
+      }
+      s = after;
+      moved = cur + 1;
+    }
+    cur = 2 * cur + (accept ? 1 : 2);
+  }
+  if (moved) {
+#pragma unroll
+    for (int u = 0; u < kVolPer; ++u) {
+      const int i = t + u * kVolThreads;
+      if (i < N) {
+        gx[poff + i] = x[u];
+        gy[poff + i] = y[u];
+        gz[poff + i] = z[u];
+      }
+    }
+    if (t == 0) reps[r] = tree[moved - 1].rec;
+  }
+  if (t == 0) result[r] = bits;
 }
 
 __global__ void k_zero_flags(int *__restrict__ f, int n) {
@@ -169,23 +380,279 @@ int hsmc_gpu_box(const hsmc_gpu_ctx *ctx, int replica, double out[3]) {
   return HSMC_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// Pinned host memory of at least `bytes`, which kernels read and write.
+void *pinned(hsmc_gpu_ctx *ctx, size_t bytes) {
+  if (ctx->h_npt_bytes >= bytes) return ctx->h_npt;
+  (void)hipStreamSynchronize(ctx->stream);
+  if (ctx->h_npt) (void)hipHostFree(ctx->h_npt);
+  ctx->h_npt = nullptr;
+  ctx->h_npt_bytes = 0;
+  bytes += bytes / 2;
+  if (hipHostMalloc(&ctx->h_npt, bytes, hipHostMallocDefault) != hipSuccess) {
+    ctx->h_npt = nullptr;
+    return nullptr;
+  }
+  ctx->h_npt_bytes = bytes;
+  return ctx->h_npt;
+}
+
+// First sphere of each 256-sphere block, every block inside one replica, on
+// the device (the particle counts of a context do not change).
+int sphere_blocks(hsmc_gpu_ctx *ctx, const int **blk, int *n) {
+  size_t count = 0;
+  for (const RepHost &h : ctx->reps) count += (size_t)(h.p.n_part + 255) / 256;
+  const bool had = ctx->scratch_bytes[S_BLK] > 0;
+  int *d = (int *)scratch(ctx, S_BLK, sizeof(int) * count);
+  if (!d) return HSMC_ERR_NO_MEMORY;
+  if (!had) {
+    std::vector<int> b;
+    b.reserve(count);
+    for (const RepHost &h : ctx->reps)
+      for (long i = h.poff; i < h.poff + h.p.n_part; i += 256) b.push_back((int)i);
+    HSMC_HIP(ctx, hipMemcpyAsync(d, b.data(), sizeof(int) * count, hipMemcpyHostToDevice, ctx->stream));
+    HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  }
+  *blk = d;
+  *n = (int)count;
+  return HSMC_OK;
+}
+
+// Whether the sweep grid's cells cover the scaled cutoff 1/sf.
+bool sweep_grid_covers(const RepHost &h, double sf) {
+  const double side = std::min(h.p.lx / h.gx, std::min(h.p.ly / h.gy, h.p.lz / h.gz));
+  return side >= (1.0 / sf) * (1.0 + 1e-9);
+}
+
+// Enqueue the scan of the replicas with sf[r] > 0 (in device memory) on the
+// last sweep's cell list, flags on the device.
+int enqueue_scan(hsmc_gpu_ctx *ctx, const double *sf, int *d_flag, const int *blk, int nblk) {
+  if (ctx->cells_version != ctx->version) {  // positions changed since the last sweep, or no list in memory
+    int st = rebin_last_sweep(ctx);
+    if (st) return st;
+  }
+  const int R = ctx->R;
+  hipLaunchKernelGGL(k_zero_flags, dim3((R + 255) / 256), dim3(256), 0, ctx->stream, d_flag, R);
+  hipLaunchKernelGGL(k_vol_overlap, dim3((unsigned)nblk), dim3(256), 0, ctx->stream, ctx->d_reps,
+                     ctx->d_swp + (ctx->R == 1 ? ctx->swp_last : 0), ctx->R, ctx->d_prep, blk, (int)ctx->Ctot,
+                     ctx->d_cnt, ctx->d_slot, ctx->cap, ctx->d_sweep, ctx->d_x, ctx->d_y, ctx->d_z, sf,
+                     d_flag);
+  HSMC_HIP(ctx, hipGetLastError());
+  return HSMC_OK;
+}
+
+__global__ void k_copy_flags(const int *__restrict__ f, int n, const unsigned *__restrict__ err,
+                             int *__restrict__ host) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) host[i] = f[i];
+  if (i == n) host[n] = (int)*err;
+}
+
+// A replica's volume move from its present box (moves.c:91-121): the
+// proposal and the acceptance rule.
+struct Box {
+  double lx, ly, lz;
+};
+
+VolNode propose(const RepHost &h, const Box &b, unsigned long long sweep, int t, double press, double dv_max,
+                Box *next) {
+  uint32_t u[4];
+  draws(h, sweep, (uint32_t)t + 1u, u);
+  const double vol = b.lx * b.ly * b.lz;
+  const double log_vol_new = log(vol) + (unit_closed(u[0]) - 0.5) * dv_max;
+  const double vnew = exp(log_vol_new);
+  VolNode n{};
+  n.sf = pow(vnew / vol, 1. / 3.);
+  const double boltz = exp(press * (vol - vnew) + (h.p.n_part + 1) * log(vnew / vol));
+  n.rule = !(unit_closed(u[1]) >= boltz);
+  next->lx = b.lx * n.sf;
+  next->ly = b.ly * n.sf;
+  next->lz = b.lz * n.sf;
+  RepHost hh = h;
+  hh.p.lx = next->lx;
+  hh.p.ly = next->ly;
+  hh.p.lz = next->lz;
+  fill_repdev(hh, n.rec);
+  return n;
+}
+
+void count_move(uint64_t *vc, bool overlap, bool accepted) {
+  if (!vc) return;
+  vc[0] += 1;
+  vc[accepted ? 1 : (overlap ? 2 : 3)] += 1;
+}
+
+// After accepted moves: the boxes are in ctx->reps and the records and
+// positions on the device already; the layout follows where a grid changed.
+int boxes_changed(hsmc_gpu_ctx *ctx) {
+  ctx->version++;
+  if (layout_keeps(ctx)) return HSMC_OK;
+  return layout(ctx);
+}
+
+// The volume moves of one sweep, steps[r] of replica r, for replicas that
+// fit k_volume_moves.
+int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::vector<int> &steps, int rounds,
+                       const double *press, const double *dv_max, uint64_t *vol_counts) {
+  const int R = ctx->R;
+  int n_max = 0;
+  for (const RepHost &h : ctx->reps) n_max = std::max(n_max, h.p.n_part);
+  const size_t lds = sizeof(double) * 3 * n_max + sizeof(int) * kVolAxis * kVolAxis * kVolAxis;
+  if (lds > 60 * 1024)  // with the kernel's own few KB above 64 KB
+    HSMC_HIP(ctx, hipFuncSetAttribute((const void *)k_volume_moves, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  for (int t0 = 0; t0 < rounds; t0 += kVolDepth) {
+    // each replica's tree of this launch's moves
+    std::vector<VolNode> nodes;
+    std::vector<VolPlan> plan(R);
+    std::vector<Box> at;
+    for (int r = 0; r < R; ++r) {
+      const RepHost &h = ctx->reps[r];
+      const int k = std::max(0, std::min(kVolDepth, steps[r] - t0));
+      plan[r] = VolPlan{k, (int)nodes.size()};
+      if (k == 0) continue;
+      const int n = (1 << k) - 1;
+      at.assign(2 * n + 1, Box{h.p.lx, h.p.ly, h.p.lz});
+      for (int i = 0, depth = 0; i < n; ++i) {
+        if (i == (2 << depth) - 1) ++depth;
+        nodes.push_back(propose(h, at[i], sweep, t0 + depth, press[r], dv_max[r], &at[2 * i + 1]));
+        at[2 * i + 2] = at[i];
+      }
+    }
+    const size_t o_node = (sizeof(VolPlan) * R + 15) & ~(size_t)15;
+    const size_t o_res = o_node + sizeof(VolNode) * nodes.size();
+    unsigned char *host = (unsigned char *)pinned(ctx, o_res + sizeof(int) * R);
+    if (!host) return HSMC_ERR_NO_MEMORY;
+    memcpy(host, plan.data(), sizeof(VolPlan) * R);
+    memcpy(host + o_node, nodes.data(), sizeof(VolNode) * nodes.size());
+    const int *res = (const int *)(host + o_res);
+    hipLaunchKernelGGL(k_volume_moves, dim3((unsigned)R), dim3(kVolThreads), lds, ctx->stream, ctx->d_reps,
+                       (const VolPlan *)host, (const VolNode *)(host + o_node), ctx->d_x, ctx->d_y, ctx->d_z,
+                       (int *)(host + o_res));
+    HSMC_HIP(ctx, hipGetLastError());
+    HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    bool any = false;
+    for (int r = 0; r < R; ++r) {
+      int cur = 0;
+      for (int k = 0; k < plan[r].steps; ++k) {
+        const bool acc = (res[r] >> (16 + k)) & 1, ov = (res[r] >> k) & 1;
+        count_move(vol_counts ? vol_counts + 4 * (size_t)r : nullptr, ov, acc);
+        if (acc) {
+          const RepDev &rec = nodes[plan[r].first + cur].rec;
+          hsmc_gpu_replica &p = ctx->reps[r].p;
+          p.lx = rec.lx;
+          p.ly = rec.ly;
+          p.lz = rec.lz;
+          any = true;
+        }
+        cur = 2 * cur + (acc ? 1 : 2);
+      }
+    }
+    if (any) {
+      int st = boxes_changed(ctx);
+      if (st) return st;
+    }
+  }
+  return HSMC_OK;
+}
+
+// The same round by round for any replicas: round t holds the t-th move of
+// every replica that makes more than t, scanned on the last sweep's cells.
+int volume_moves_rounds(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::vector<int> &steps, int rounds,
+                        const double *press, const double *dv_max, uint64_t *vol_counts) {
+  const int R = ctx->R;
+  const int *blk = nullptr;
+  int nblk = 0, st = sphere_blocks(ctx, &blk, &nblk);
+  if (st) return st;
+  int *d_flag = (int *)scratch(ctx, S_FLAG, sizeof(int) * R);
+  if (!d_flag) return HSMC_ERR_NO_MEMORY;
+  const size_t o_sf = sizeof(VolNode) * R, o_res = o_sf + sizeof(double) * R;
+  unsigned char *host = (unsigned char *)pinned(ctx, o_res + sizeof(int) * R);
+  if (!host) return HSMC_ERR_NO_MEMORY;
+  VolNode *node = (VolNode *)host;
+  double *sf = (double *)(host + o_sf);
+  const int *flag = (const int *)(host + o_res);
+  // the blocks of a round read their replica's move from device memory
+  unsigned char *dev = (unsigned char *)scratch(ctx, S_MOVE, o_res);
+  if (!dev) return HSMC_ERR_NO_MEMORY;
+  std::vector<uint8_t> decided(R);  // overlap found by the single scan
+  for (int t = 0; t < rounds; ++t) {
+    bool scan = false;
+    for (int r = 0; r < R; ++r) {
+      const RepHost &h = ctx->reps[r];
+      decided[r] = 0;
+      sf[r] = 0.0;
+      Box next;
+      if (steps[r] <= t) {
+        node[r] = VolNode{};
+        fill_repdev(h, node[r].rec);
+        continue;
+      }
+      node[r] = propose(h, Box{h.p.lx, h.p.ly, h.p.lz}, sweep, t, press[r], dv_max[r], &next);
+      // an expansion cannot create an overlap in a configuration that has none
+      if (!(node[r].sf < 1.0)) continue;
+      if (sweep_grid_covers(h, node[r].sf)) {
+        sf[r] = node[r].sf;
+        scan = true;
+      } else {
+        uint8_t ok = 1;
+        st = hsmc_gpu_any_overlap_scaled(ctx, r, &node[r].sf, 1, &ok);
+        if (st) return st;
+        decided[r] = !ok;
+        if (decided[r]) node[r].rule = 0;
+      }
+    }
+    HSMC_HIP(ctx, hipMemcpyAsync(dev, host, o_res, hipMemcpyHostToDevice, ctx->stream));
+    if (scan) {
+      st = enqueue_scan(ctx, (const double *)(dev + o_sf), d_flag, blk, nblk);
+      if (st) return st;
+    } else {
+      hipLaunchKernelGGL(k_zero_flags, dim3((R + 255) / 256), dim3(256), 0, ctx->stream, d_flag, R);
+    }
+    hipLaunchKernelGGL(k_vol_apply, dim3((unsigned)nblk), dim3(256), 0, ctx->stream, blk, ctx->d_prep,
+                       (const VolNode *)dev, d_flag, ctx->d_reps, ctx->d_x, ctx->d_y, ctx->d_z, (int *)(host + o_res));
+    HSMC_HIP(ctx, hipGetLastError());
+    HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    bool any = false;
+    for (int r = 0; r < R; ++r) {
+      if (steps[r] <= t) continue;
+      const bool ov = decided[r] || flag[r], acc = !ov && node[r].rule;
+      count_move(vol_counts ? vol_counts + 4 * (size_t)r : nullptr, ov, acc);
+      if (!acc) continue;
+      hsmc_gpu_replica &p = ctx->reps[r].p;
+      p.lx = node[r].rec.lx;
+      p.ly = node[r].rec.ly;
+      p.lz = node[r].rec.lz;
+      any = true;
+    }
+    if (any) {
+      st = boxes_changed(ctx);
+      if (st) return st;
+    }
+  }
+  return HSMC_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int hsmc_gpu_any_overlap_scaled_batch(hsmc_gpu_ctx *ctx, const double *sf, uint8_t *no_overlap) {
   if (!ctx || !sf || !no_overlap) return HSMC_ERR_BAD_ARG;
   const int R = ctx->R;
-  double *d_sf = (double *)scratch(ctx, S_SF, sizeof(double) * R);
   int *d_flag = (int *)scratch(ctx, S_FLAG, sizeof(int) * R);
-  if (!d_sf || !d_flag) return HSMC_ERR_NO_MEMORY;
+  if (!d_flag) return HSMC_ERR_NO_MEMORY;
   // replicas whose sweep-grid cells cover the scaled cutoff 1/sf are scanned
-  // together on the sweep grid; the others on their own grid of side 1/sf
-  std::vector<double> sf_dev(R, 0.0);
+  // together on the sweep grid; the others one by one
+  std::vector<double> on_grid(R, 0.0);
   bool any = false;
   for (int r = 0; r < R; ++r) {
     no_overlap[r] = 1;
     if (!(sf[r] > 0.0)) continue;
-    const RepHost &h = ctx->reps[r];
-    const double side = std::min(h.p.lx / h.gx, std::min(h.p.ly / h.gy, h.p.lz / h.gz));
-    if (side >= (1.0 / sf[r]) * (1.0 + 1e-9)) {
-      sf_dev[r] = sf[r];
+    if (sweep_grid_covers(ctx->reps[r], sf[r])) {
+      on_grid[r] = sf[r];
       any = true;
     } else {
       int st = hsmc_gpu_any_overlap_scaled(ctx, r, &sf[r], 1, &no_overlap[r]);
@@ -193,32 +660,24 @@ int hsmc_gpu_any_overlap_scaled_batch(hsmc_gpu_ctx *ctx, const double *sf, uint8
     }
   }
   if (!any) return HSMC_OK;
-  if (ctx->cells_version != ctx->version) {  // positions changed since the last sweep
-    int st = rebin_last_sweep(ctx);
-    if (st) return st;
-  }
-  // first sphere of each 256-sphere block of the replicas scanned here
-  std::vector<int> blk;
-  for (int r = 0; r < R; ++r) {
-    if (!(sf_dev[r] > 0.0)) continue;
-    const RepHost &h = ctx->reps[r];
-    for (long b = h.poff; b < h.poff + h.p.n_part; b += 256) blk.push_back((int)b);
-  }
-  int *d_blk = (int *)scratch(ctx, S_BLK, sizeof(int) * blk.size());
-  if (!d_blk) return HSMC_ERR_NO_MEMORY;
-  HSMC_HIP(ctx, hipMemcpyAsync(d_sf, sf_dev.data(), sizeof(double) * R, hipMemcpyHostToDevice, ctx->stream));
-  HSMC_HIP(ctx, hipMemcpyAsync(d_blk, blk.data(), sizeof(int) * blk.size(), hipMemcpyHostToDevice, ctx->stream));
-  hipLaunchKernelGGL(k_zero_flags, dim3((R + 255) / 256), dim3(256), 0, ctx->stream, d_flag, R);
-  hipLaunchKernelGGL(k_vol_overlap, dim3((unsigned)blk.size()), dim3(256), 0, ctx->stream, ctx->d_reps,
-                     ctx->d_swp + (ctx->R == 1 ? ctx->swp_last : 0), ctx->R, ctx->d_prep, d_blk, (int)ctx->Ctot, ctx->d_cnt, ctx->d_slot,
-                     ctx->cap, ctx->d_sweep, ctx->d_x, ctx->d_y, ctx->d_z, d_sf, d_flag);
+  const int *blk = nullptr;
+  int nblk = 0, st = sphere_blocks(ctx, &blk, &nblk);
+  if (st) return st;
+  unsigned char *host = (unsigned char *)pinned(ctx, sizeof(double) * R + sizeof(int) * (R + 1));
+  if (!host) return HSMC_ERR_NO_MEMORY;
+  memcpy(host, on_grid.data(), sizeof(double) * R);
+  int *flag = (int *)(host + sizeof(double) * R);
+  double *d_sf = (double *)scratch(ctx, S_MOVE, sizeof(double) * R);
+  if (!d_sf) return HSMC_ERR_NO_MEMORY;
+  HSMC_HIP(ctx, hipMemcpyAsync(d_sf, host, sizeof(double) * R, hipMemcpyHostToDevice, ctx->stream));
+  st = enqueue_scan(ctx, d_sf, d_flag, blk, nblk);
+  if (st) return st;
+  hipLaunchKernelGGL(k_copy_flags, dim3((unsigned)(R / 256 + 1)), dim3(256), 0, ctx->stream, d_flag, R, ctx->d_err, flag);
   HSMC_HIP(ctx, hipGetLastError());
-  std::vector<int> hf(R);
-  HSMC_HIP(ctx, hipMemcpyAsync(hf.data(), d_flag, sizeof(int) * R, hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   for (int r = 0; r < R; ++r)
-    if (sf_dev[r] > 0.0) no_overlap[r] = hf[r] ? 0 : 1;
-  return check_device_errors(ctx);
+    if (on_grid[r] > 0.0) no_overlap[r] = flag[r] ? 0 : 1;
+  return flag[R] ? check_device_errors(ctx) : HSMC_OK;
 }
 
 int hsmc_gpu_npt_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, const double *press,
@@ -228,19 +687,12 @@ int hsmc_gpu_npt_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, const double *press,
   for (int r = 0; r < R; ++r)
     if (!(press[r] >= 0.0) || !(dv_max[r] > 0.0) || !std::isfinite(press[r])) return HSMC_ERR_BAD_ARG;
   if (n_sweeps == 0) return HSMC_OK;
-  double *d_sf = (double *)scratch(ctx, S_SF, sizeof(double) * R);
-  double *d_box = (double *)scratch(ctx, S_BOX, sizeof(double) * 3 * R);
-  int *d_flag = (int *)scratch(ctx, S_FLAG, sizeof(int) * R);
-  if (!d_sf || !d_box || !d_flag) return HSMC_ERR_NO_MEMORY;
   unsigned long long sweep0 = 0;
   HSMC_HIP(ctx, hipMemcpyAsync(&sweep0, ctx->d_sweep, sizeof(sweep0), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-
-  std::vector<int> steps(R), flag(R);
-  std::vector<uint8_t> no_ov(R);
-  std::vector<double> sf(R), vnew(R), sf_dev(R), box(3 * R);
-  std::vector<uint32_t> acc_word(R);
-  const unsigned blocks = (unsigned)((ctx->Ptot + 255) / 256);
+  bool small = true;
+  for (const RepHost &h : ctx->reps) small = small && h.p.n_part <= kVolSpheres;
+  std::vector<int> steps(R);
   for (int sw = 0; sw < n_sweeps; ++sw) {
     int st = run_sweeps(ctx, 1);
     if (st) return st;
@@ -252,72 +704,9 @@ int hsmc_gpu_npt_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, const double *press,
       steps[r] = volume_steps(ctx->reps[r].p.n_part, u[0]);
       rounds = std::max(rounds, steps[r]);
     }
-    for (int t = 0; t < rounds; ++t) {
-      // proposals (moves.c:91-102)
-      bool any_compression = false;
-      for (int r = 0; r < R; ++r) {
-        sf[r] = 0.0;
-        if (steps[r] <= t) continue;
-        const hsmc_gpu_replica &p = ctx->reps[r].p;
-        uint32_t u[4];
-        draws(ctx->reps[r], s, (uint32_t)t + 1u, u);
-        const double vol = p.lx * p.ly * p.lz;
-        const double log_vol_new = log(vol) + (unit_closed(u[0]) - 0.5) * dv_max[r];
-        vnew[r] = exp(log_vol_new);
-        sf[r] = pow(vnew[r] / vol, 1. / 3.);
-        acc_word[r] = u[1];
-        if (sf[r] < 1.0) any_compression = true;
-      }
-      // overlap scan of the compressions: an expansion cannot create an
-      // overlap in a configuration that has none
-      std::fill(flag.begin(), flag.end(), 0);
-      if (any_compression) {
-        for (int r = 0; r < R; ++r) sf_dev[r] = (sf[r] > 0.0 && sf[r] < 1.0) ? sf[r] : 0.0;
-        st = hsmc_gpu_any_overlap_scaled_batch(ctx, sf_dev.data(), no_ov.data());
-        if (st) return st;
-        for (int r = 0; r < R; ++r)
-          if (sf_dev[r] > 0.0) flag[r] = no_ov[r] ? 0 : 1;
-      }
-      // acceptance (moves.c:114-127)
-      bool any_accepted = false;
-      for (int r = 0; r < R; ++r) {
-        sf_dev[r] = 0.0;
-        if (!(sf[r] > 0.0)) continue;
-        hsmc_gpu_replica &p = ctx->reps[r].p;
-        uint64_t *vc = vol_counts ? vol_counts + 4 * (size_t)r : nullptr;
-        if (vc) vc[0] += 1;
-        if (flag[r]) {
-          if (vc) vc[2] += 1;
-          continue;
-        }
-        const double vol = p.lx * p.ly * p.lz;
-        const double boltz = exp(press[r] * (vol - vnew[r]) + (p.n_part + 1) * log(vnew[r] / vol));
-        if (unit_closed(acc_word[r]) >= boltz) {
-          if (vc) vc[3] += 1;
-          continue;
-        }
-        if (vc) vc[1] += 1;
-        p.lx *= sf[r];
-        p.ly *= sf[r];
-        p.lz *= sf[r];
-        sf_dev[r] = sf[r];
-        box[3 * r] = p.lx;
-        box[3 * r + 1] = p.ly;
-        box[3 * r + 2] = p.lz;
-        any_accepted = true;
-      }
-      if (any_accepted) {
-        HSMC_HIP(ctx, hipMemcpyAsync(d_sf, sf_dev.data(), sizeof(double) * R, hipMemcpyHostToDevice, ctx->stream));
-        HSMC_HIP(ctx, hipMemcpyAsync(d_box, box.data(), sizeof(double) * 3 * R, hipMemcpyHostToDevice, ctx->stream));
-        hipLaunchKernelGGL(k_scale_batch, dim3(blocks), dim3(256), 0, ctx->stream, ctx->d_prep,
-                           (int)ctx->Ptot, ctx->d_x, ctx->d_y, ctx->d_z, d_sf, d_box);
-        HSMC_HIP(ctx, hipGetLastError());
-        // the host copies of sf/box are reused next round: wait for the copies
-        HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        st = layout(ctx);
-        if (st) return st;
-      }
-    }
+    st = small ? volume_moves_small(ctx, s, steps, rounds, press, dv_max, vol_counts)
+               : volume_moves_rounds(ctx, s, steps, rounds, press, dv_max, vol_counts);
+    if (st) return st;
   }
   return check_device_errors(ctx);
 }

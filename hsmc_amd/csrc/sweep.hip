@@ -662,6 +662,11 @@ __global__ void k_zero_counts(int *__restrict__ cnt, long n) {
   if (i < n) cnt[i] = 0;
 }
 
+__global__ void k_zero_last_counts(int *__restrict__ cnt, int C, const unsigned long long *__restrict__ sweep_next) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < C) cnt[(size_t)((*sweep_next - 1ull) & 1ull) * C + c] = 0;
+}
+
 // The phase kernel's occupant pick for attempts t < count of one cell, any n.
 __global__ void __launch_bounds__(256)
 k_occupant_picks(uint32_t k0, uint32_t k1, uint32_t cell, unsigned long long sweep, uint32_t n,
@@ -972,12 +977,8 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
 int rebin_last_sweep(hsmc_gpu_ctx *ctx) {
   // the last sweep done is *d_sweep - 1; its count buffer is refilled from
   // zero and the rebin clears the other buffer as a sweep's rebin does
-  unsigned long long next = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&next, ctx->d_sweep, sizeof(next), hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  const int buf = (int)((next - 1ull) & 1ull);
-  HSMC_HIP(ctx, hipMemsetAsync(ctx->d_cnt + (size_t)buf * ctx->Ctot, 0, sizeof(int) * ctx->Ctot,
-                               ctx->stream));
+  hipLaunchKernelGGL(k_zero_last_counts, dim3((unsigned)((ctx->Ctot + 255) / 256)), dim3(256), 0, ctx->stream,
+                     ctx->d_cnt, (int)ctx->Ctot, ctx->d_sweep);
   const long work = std::max(ctx->Ptot, ctx->Ctot);
   hipLaunchKernelGGL(ctx->R == 1 ? k_rebin<true> : k_rebin<false>,
                      dim3((unsigned)((work + 255) / 256)), dim3(256), 0, ctx->stream,

@@ -274,3 +274,36 @@ def test_c5_full_size_npt_workload():
         dec = ctx.overlap_scaled(idx, np.full(len(idx), s), r)
         want = np.array([o.check_overlap(int(i), s) for i in idx], dtype=np.uint8)
         assert np.array_equal(dec, want), s
+
+
+def test_npt_moves_in_one_launch_equal_moves_in_rounds():
+    """Volume moves of small replicas walk a tree in one launch; a replica of
+    more than 4096 spheres in the batch makes every replica's moves go round
+    by round.  Boxes, positions and counts agree bit for bit: 12 replicas of
+    N = 32 to 1372 over 120 sweeps (some sweeps with more than the four moves
+    of one launch), steps wide enough that sweep grids change, and compressions
+    beyond the sweep grid's cutoff."""
+    small = [(2, 0.35, 900 + k, 0.2) for k in range(5)] + [(2, 0.12, 905, 0.2),  # from 6 cells an axis to 4
+                                                          (3, 0.55, 950, 0.15), (4, 0.60, 951, 0.12),
+                                                          (5, 0.70, 952, 0.1), (7, 0.80, 953, 0.1),
+                                                          (4, 0.05, 954, 0.5), (3, 0.80, 955, 0.1)]
+    press = [0.6] * 5 + [0.9, 2.2, 2.9, 4.5, 7.0, 0.06, 6.5]
+    dv = [0.3] * 6 + [0.05, 0.03, 0.02, 0.008, 0.4, 0.04]
+    one = make(small)
+    rounds = make(small + [(11, 0.5, 99, 0.1)])
+    boxes0 = [one.box(r) for r in range(one.R)]
+    grids0 = [one.grid(r) for r in range(one.R)]
+    a = one.npt_sweeps(120, press, dv)
+    b = rounds.npt_sweeps(120, press + [1.7], dv + [0.004])
+    assert np.array_equal(a, b[:-1])
+    assert np.array_equal(a[:, 0], a[:, 1] + a[:, 2] + a[:, 3])
+    assert a[:, 1].sum() > 0 and a[:, 2].sum() > 0 and a[:, 3].sum() > 0
+    for r in range(one.R):
+        assert one.box(r) == rounds.box(r), r
+        assert np.array_equal(one.download(r), rounds.download(r)), r
+        assert one.counters(r) == rounds.counters(r), r
+    assert any(one.box(r) != boxes0[r] for r in range(one.R))
+    assert any(one.grid(r) != grids0[r] for r in range(one.R))
+    assert all(one.any_overlap_scaled_batch(1.0) == 1)
+    one.close()
+    rounds.close()
