@@ -119,9 +119,15 @@ struct hsmc_gpu_ctx {
   // after each batch of sweeps, so later batches are not launched onto a
   // cell list that has already overflowed
   volatile unsigned int *h_err = nullptr;
-  // pinned memory of the volume moves (proposals in, decisions out)
-  void *h_npt = nullptr;
-  size_t h_npt_bytes = 0;
+  // pinned host memory, grown on demand: volume moves (proposals in,
+  // decisions out), configuration rows in transit, folded move counters
+  static constexpr int kPinned = 3;
+  void *pin[kPinned] = {};
+  size_t pin_bytes[kPinned] = {};
+  // the move counters are all in the host totals and sweep_now is the sweep
+  // counter: nothing has swept since they were last read
+  bool folded = false;
+  unsigned long long sweep_now = 0;
   // results of an observable, stored by its last kernel in pinned memory
   unsigned long long *h_acc = nullptr;
   // the observable grids' cell counts: their buffer's size when it was last
@@ -188,6 +194,9 @@ int hip_fail(hsmc_gpu_ctx *ctx, hipError_t e, const char *what);
 void *scratch(hsmc_gpu_ctx *ctx, int slot, size_t bytes);
 // (Re)build replica offsets, the sweep grids, and the device cell arrays.
 int layout(hsmc_gpu_ctx *ctx);
+// Pinned host memory `slot` of at least `bytes`, which kernels read and write.
+enum PinnedSlot { P_MOVES, P_ROWS, P_COUNTERS };
+void *pinned(hsmc_gpu_ctx *ctx, PinnedSlot slot, size_t bytes);
 // Device parameters of one replica from its box, grid and offsets.
 void fill_repdev(const RepHost &h, RepDev &d);
 // Whether the replicas' present boxes keep every sweep grid and capacity;

@@ -39,6 +39,24 @@ void *scratch(hsmc_gpu_ctx *ctx, int slot, size_t bytes) {
   return ctx->scratch[slot];
 }
 
+void *pinned(hsmc_gpu_ctx *ctx, PinnedSlot slot, size_t bytes) {
+  if (ctx->pin_bytes[slot] >= bytes) return ctx->pin[slot];
+  if (ctx->pin[slot]) {
+    (void)hipStreamSynchronize(ctx->stream);
+    (void)hipHostFree(ctx->pin[slot]);
+    ctx->pin[slot] = nullptr;
+    ctx->pin_bytes[slot] = 0;
+  }
+  const size_t want = bytes + bytes / 4;
+  if (hipHostMalloc(&ctx->pin[slot], want, hipHostMallocDefault) != hipSuccess) {
+    ctx->pin[slot] = nullptr;
+    ctx->last_error = "pinned allocation failed";
+    return nullptr;
+  }
+  ctx->pin_bytes[slot] = want;
+  return ctx->pin[slot];
+}
+
 int sweep_grid_cells(double L) {
   const double minside = 1.0 + 1e-9;
   int g = (int)floor(L / minside);
@@ -60,31 +78,56 @@ void drop_graph(hsmc_gpu_ctx *ctx) {
   ctx->graph_r_sweeps = 0;
 }
 
+// One replica per workgroup: its move counters summed over its active cells
+// (cells / 8 entries from aoff on; the padding behind them is never written)
+// into out[2 r], out[2 r + 1], and cleared; the sweep counter and the sticky
+// error bits behind them.
+__global__ void __launch_bounds__(256)
+k_fold_counters(const RepDev *__restrict__ reps, int R, unsigned int *__restrict__ cacc,
+                unsigned int *__restrict__ cleft, const unsigned long long *__restrict__ sweep,
+                const unsigned int *__restrict__ err, unsigned long long *__restrict__ out) {
+  __shared__ unsigned long long s[2][4];
+  const int r = blockIdx.x, a0 = reps[r].aoff, a1 = a0 + reps[r].gx * reps[r].gy * reps[r].gz / 8;
+  unsigned long long sa = 0, sl = 0;
+  for (int a = a0 + (int)threadIdx.x; a < a1; a += 256) {
+    sa += cacc[a];
+    sl += cleft[a];
+    cacc[a] = 0u;
+    cleft[a] = 0u;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    sa += __shfl_xor(sa, o, 64);
+    sl += __shfl_xor(sl, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s[0][threadIdx.x >> 6] = sa;
+    s[1][threadIdx.x >> 6] = sl;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const unsigned long long *v = s[threadIdx.x];
+    out[2 * r + threadIdx.x] = v[0] + v[1] + v[2] + v[3];
+    if (r == 0) out[2 * R + threadIdx.x] = threadIdx.x ? (unsigned long long)*err : *sweep;
+  }
+}
+
+// Add the device counters into the host totals, all replicas at once; free
+// while nothing has swept since.
 int fold_counters(hsmc_gpu_ctx *ctx) {
-  // the counters are indexed by active-cell index (Atot entries, replica r
-  // owning [aoff, aoff + cells/8) and padding up to a multiple of 8 that no
-  // kernel writes)
-  if (!ctx->d_cacc || ctx->Atot == 0) return HSMC_OK;
-  std::vector<unsigned int> a(ctx->Atot), l(ctx->Atot);
-  HSMC_HIP(ctx, hipMemcpyAsync(a.data(), ctx->d_cacc, sizeof(unsigned int) * ctx->Atot,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipMemcpyAsync(l.data(), ctx->d_cleft, sizeof(unsigned int) * ctx->Atot,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipMemsetAsync(ctx->d_cacc, 0, sizeof(unsigned int) * ctx->Atot, ctx->stream));
-  HSMC_HIP(ctx, hipMemsetAsync(ctx->d_cleft, 0, sizeof(unsigned int) * ctx->Atot, ctx->stream));
+  if (ctx->folded || !ctx->d_cacc || ctx->Atot == 0) return HSMC_OK;
+  unsigned long long *out = (unsigned long long *)pinned(ctx, P_COUNTERS, sizeof(unsigned long long) * (2 * (size_t)ctx->R + 2));
+  if (!out) return HSMC_ERR_NO_MEMORY;
+  hipLaunchKernelGGL(k_fold_counters, dim3((unsigned)ctx->R), dim3(256), 0, ctx->stream, ctx->d_reps, ctx->R, ctx->d_cacc,
+                     ctx->d_cleft, ctx->d_sweep, ctx->d_err, out);
+  HSMC_HIP(ctx, hipGetLastError());
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   for (int r = 0; r < ctx->R; ++r) {
-    const RepHost &h = ctx->reps[r];
-    const long n = (long)h.gx * h.gy * h.gz / 8;
-    unsigned long long sa = 0, sl = 0;
-    for (long c = h.aoff; c < h.aoff + n; ++c) {
-      sa += a[c];
-      sl += l[c];
-    }
-    ctx->tot_acc[r] += sa;
-    ctx->tot_left[r] += sl;
+    ctx->tot_acc[r] += out[2 * r];
+    ctx->tot_left[r] += out[2 * r + 1];
   }
   ctx->resident_sweeps = 0;
+  ctx->sweep_now = out[2 * ctx->R];
+  ctx->folded = out[2 * ctx->R + 1] == 0;  // with an error pending, the next reader reports it
   return HSMC_OK;
 }
 
@@ -261,10 +304,10 @@ int layout(hsmc_gpu_ctx *ctx) {
 }
 
 int check_device_errors(hsmc_gpu_ctx *ctx) {
-  unsigned int e = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&e, ctx->d_err, sizeof(e), hipMemcpyDeviceToHost, ctx->stream));
+  HSMC_HIP(ctx, hipMemcpyAsync((void *)ctx->h_err, ctx->d_err, sizeof(unsigned int), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  if (ctx->h_err) *ctx->h_err = 0u;
+  const unsigned int e = *ctx->h_err;
+  *ctx->h_err = 0u;
   if (e) {
     unsigned int zero = 0;
     HSMC_HIP(ctx, hipMemcpy(ctx->d_err, &zero, sizeof(zero), hipMemcpyHostToDevice));
@@ -292,6 +335,34 @@ __global__ void k_scale(double *__restrict__ x, double *__restrict__ y, double *
   y[i] = wrap_once(y[i] * sf, ly);
   z[i] = wrap_once(z[i] * sf, lz);
 }
+
+// Rows {id, x, y, z} of particles first .. first + n - 1 to pinned host
+// memory (with the sticky error bits), and the positions back from such rows.
+__global__ void __launch_bounds__(256)
+k_rows_out(const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
+           long first, int n, const unsigned int *__restrict__ err, double4 *__restrict__ rows,
+           unsigned long long *__restrict__ host_err) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k == 0) *host_err = *err;
+  if (k >= n) return;
+  const long i = first + k;
+  rows[k] = make_double4((double)i, x[i], y[i], z[i]);
+}
+
+__global__ void __launch_bounds__(256)
+k_rows_in(const double4 *__restrict__ rows, long first, int n, double *__restrict__ x,
+          double *__restrict__ y, double *__restrict__ z) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const double4 q = rows[k];
+  x[first + k] = q.y;
+  y[first + k] = q.z;
+  z[first + k] = q.w;
+}
+
+// Rows in transit go through two pinned buffers of at most this many, so
+// that one is copied on the host while a kernel fills or empties the other.
+constexpr int kRowChunk = 1 << 15;
 
 bool valid_box(double L) { return L > 2.0 && std::isfinite(L); }
 
@@ -422,7 +493,8 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
     if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
   if (ctx->h_err) (void)hipHostFree((void *)ctx->h_err);
   if (ctx->h_acc) (void)hipHostFree(ctx->h_acc);
-  if (ctx->h_npt) (void)hipHostFree(ctx->h_npt);
+  for (void *p : ctx->pin)
+    if (p) (void)hipHostFree(p);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -432,31 +504,35 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
 
 int hsmc_gpu_sync(hsmc_gpu_ctx *ctx) {
   if (!ctx) return HSMC_ERR_BAD_ARG;
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return check_device_errors(ctx);
+  return check_device_errors(ctx);  // waits for the stream
 }
 
 int hsmc_gpu_upload(hsmc_gpu_ctx *ctx, int replica, const double *conf4) {
   if (!ctx || replica < 0 || replica >= ctx->R || !conf4) return HSMC_ERR_BAD_ARG;
   const RepHost &h = ctx->reps[replica];
   const int n = h.p.n_part;
-  std::vector<double> x(n), y(n), z(n);
-  for (int i = 0; i < n; ++i) {
-    x[i] = conf4[4 * (size_t)i + 1];
-    y[i] = conf4[4 * (size_t)i + 2];
-    z[i] = conf4[4 * (size_t)i + 3];
-    if (!(x[i] >= 0.0 && x[i] <= h.p.lx && y[i] >= 0.0 && y[i] <= h.p.ly && z[i] >= 0.0 &&
-          z[i] <= h.p.lz)) {
+  for (size_t i = 0; i < (size_t)n; ++i) {
+    const double *q = conf4 + 4 * i;
+    if (!(q[1] >= 0.0 && q[1] <= h.p.lx && q[2] >= 0.0 && q[2] <= h.p.ly && q[3] >= 0.0 &&
+          q[3] <= h.p.lz)) {
       ctx->last_error = "particle outside [0, L] (apply_pbc range)";
       return HSMC_ERR_BAD_ARG;
     }
   }
-  HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_x + h.poff, x.data(), sizeof(double) * n,
-                               hipMemcpyHostToDevice, ctx->stream));
-  HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_y + h.poff, y.data(), sizeof(double) * n,
-                               hipMemcpyHostToDevice, ctx->stream));
-  HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_z + h.poff, z.data(), sizeof(double) * n,
-                               hipMemcpyHostToDevice, ctx->stream));
+  const int chunk = std::min(n, kRowChunk);
+  double4 *rows = (double4 *)pinned(ctx, P_ROWS, sizeof(double4) * 2 * (size_t)chunk + sizeof(unsigned long long));
+  if (!rows) return HSMC_ERR_NO_MEMORY;
+  const hipEvent_t ev[2] = {ctx->ev0, ctx->ev1};
+  for (int first = 0, c = 0; first < n; first += chunk, ++c) {
+    const int m = std::min(chunk, n - first);
+    double4 *buf = rows + (size_t)(c & 1) * chunk;
+    if (c >= 2) HSMC_HIP(ctx, hipEventSynchronize(ev[c & 1]));  // the kernel that read this buffer
+    memcpy(buf, conf4 + 4 * (size_t)first, sizeof(double4) * m);
+    hipLaunchKernelGGL(k_rows_in, dim3((m + 255) / 256), dim3(256), 0, ctx->stream, buf, (long)first, m,
+                       ctx->d_x + h.poff, ctx->d_y + h.poff, ctx->d_z + h.poff);
+    if (n > 2 * chunk) HSMC_HIP(ctx, hipEventRecord(ev[c & 1], ctx->stream));
+  }
+  HSMC_HIP(ctx, hipGetLastError());
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   ctx->version++;
   return HSMC_OK;
@@ -465,22 +541,30 @@ int hsmc_gpu_upload(hsmc_gpu_ctx *ctx, int replica, const double *conf4) {
 int hsmc_gpu_download(hsmc_gpu_ctx *ctx, int replica, double *conf4) {
   if (!ctx || replica < 0 || replica >= ctx->R || !conf4) return HSMC_ERR_BAD_ARG;
   const RepHost &h = ctx->reps[replica];
-  const int n = h.p.n_part;
-  std::vector<double> x(n), y(n), z(n);
-  HSMC_HIP(ctx, hipMemcpyAsync(x.data(), ctx->d_x + h.poff, sizeof(double) * n,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipMemcpyAsync(y.data(), ctx->d_y + h.poff, sizeof(double) * n,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipMemcpyAsync(z.data(), ctx->d_z + h.poff, sizeof(double) * n,
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  for (int i = 0; i < n; ++i) {
-    conf4[4 * (size_t)i] = (double)i;
-    conf4[4 * (size_t)i + 1] = x[i];
-    conf4[4 * (size_t)i + 2] = y[i];
-    conf4[4 * (size_t)i + 3] = z[i];
+  const int n = h.p.n_part, chunk = std::min(n, kRowChunk);
+  double4 *rows = (double4 *)pinned(ctx, P_ROWS, sizeof(double4) * 2 * (size_t)chunk + sizeof(unsigned long long));
+  if (!rows) return HSMC_ERR_NO_MEMORY;
+  unsigned long long *err = (unsigned long long *)(rows + 2 * (size_t)chunk);
+  const hipEvent_t ev[2] = {ctx->ev0, ctx->ev1};
+  const int chunks = (n + chunk - 1) / chunk;
+  for (int c = 0; c <= chunks; ++c) {
+    if (c < chunks) {
+      const int m = std::min(chunk, n - c * chunk);
+      hipLaunchKernelGGL(k_rows_out, dim3((m + 255) / 256), dim3(256), 0, ctx->stream, ctx->d_x + h.poff,
+                         ctx->d_y + h.poff, ctx->d_z + h.poff, (long)c * chunk, m, ctx->d_err,
+                         rows + (size_t)(c & 1) * chunk, err);
+      HSMC_HIP(ctx, hipGetLastError());
+      if (chunks > 1) HSMC_HIP(ctx, hipEventRecord(ev[c & 1], ctx->stream));
+    }
+    if (c == 0) continue;
+    // copy out the chunk before, while the kernel fills the other buffer
+    if (chunks > 1) HSMC_HIP(ctx, hipEventSynchronize(ev[(c - 1) & 1]));
+    else HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    const int first = (c - 1) * chunk;
+    memcpy(conf4 + 4 * (size_t)first, rows + (size_t)((c - 1) & 1) * chunk,
+           sizeof(double4) * (size_t)std::min(chunk, n - first));
   }
-  return check_device_errors(ctx);
+  return *err ? check_device_errors(ctx) : HSMC_OK;
 }
 
 int hsmc_gpu_set_particles(hsmc_gpu_ctx *ctx, int replica, const int32_t *idx,

@@ -384,22 +384,6 @@ int hsmc_gpu_box(const hsmc_gpu_ctx *ctx, int replica, double out[3]) {
 
 namespace {
 
-// Pinned host memory of at least `bytes`, which kernels read and write.
-void *pinned(hsmc_gpu_ctx *ctx, size_t bytes) {
-  if (ctx->h_npt_bytes >= bytes) return ctx->h_npt;
-  (void)hipStreamSynchronize(ctx->stream);
-  if (ctx->h_npt) (void)hipHostFree(ctx->h_npt);
-  ctx->h_npt = nullptr;
-  ctx->h_npt_bytes = 0;
-  bytes += bytes / 2;
-  if (hipHostMalloc(&ctx->h_npt, bytes, hipHostMallocDefault) != hipSuccess) {
-    ctx->h_npt = nullptr;
-    return nullptr;
-  }
-  ctx->h_npt_bytes = bytes;
-  return ctx->h_npt;
-}
-
 // First sphere of each 256-sphere block, every block inside one replica, on
 // the device (the particle counts of a context do not change).
 int sphere_blocks(hsmc_gpu_ctx *ctx, const int **blk, int *n) {
@@ -523,7 +507,7 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
     }
     const size_t o_node = (sizeof(VolPlan) * R + 15) & ~(size_t)15;
     const size_t o_res = o_node + sizeof(VolNode) * nodes.size();
-    unsigned char *host = (unsigned char *)pinned(ctx, o_res + sizeof(int) * R);
+    unsigned char *host = (unsigned char *)pinned(ctx, P_MOVES, o_res + sizeof(int) * R);
     if (!host) return HSMC_ERR_NO_MEMORY;
     memcpy(host, plan.data(), sizeof(VolPlan) * R);
     memcpy(host + o_node, nodes.data(), sizeof(VolNode) * nodes.size());
@@ -569,7 +553,7 @@ int volume_moves_rounds(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::
   int *d_flag = (int *)scratch(ctx, S_FLAG, sizeof(int) * R);
   if (!d_flag) return HSMC_ERR_NO_MEMORY;
   const size_t o_sf = sizeof(VolNode) * R, o_res = o_sf + sizeof(double) * R;
-  unsigned char *host = (unsigned char *)pinned(ctx, o_res + sizeof(int) * R);
+  unsigned char *host = (unsigned char *)pinned(ctx, P_MOVES, o_res + sizeof(int) * R);
   if (!host) return HSMC_ERR_NO_MEMORY;
   VolNode *node = (VolNode *)host;
   double *sf = (double *)(host + o_sf);
@@ -663,7 +647,7 @@ int hsmc_gpu_any_overlap_scaled_batch(hsmc_gpu_ctx *ctx, const double *sf, uint8
   const int *blk = nullptr;
   int nblk = 0, st = sphere_blocks(ctx, &blk, &nblk);
   if (st) return st;
-  unsigned char *host = (unsigned char *)pinned(ctx, sizeof(double) * R + sizeof(int) * (R + 1));
+  unsigned char *host = (unsigned char *)pinned(ctx, P_MOVES, sizeof(double) * R + sizeof(int) * (R + 1));
   if (!host) return HSMC_ERR_NO_MEMORY;
   memcpy(host, on_grid.data(), sizeof(double) * R);
   int *flag = (int *)(host + sizeof(double) * R);

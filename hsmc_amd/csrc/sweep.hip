@@ -900,6 +900,7 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
   if (n <= 0) return HSMC_OK;
   if (*ctx->h_err) return check_device_errors(ctx);
   ctx->version++;
+  ctx->folded = false;
   ResidentShape shape;
   if (!ctx->tune_set && resident_shape(ctx, &shape)) {
     // launches of at most 4096 sweeps, so that an error stops a long call
@@ -1044,6 +1045,7 @@ int hsmc_gpu_time_phase_kernel(hsmc_gpu_ctx *ctx, int n_sweeps, float *avg_ms, i
   hipEvent_t ev[16];
   for (int i = 0; i < 16; ++i) HSMC_HIP(ctx, hipEventCreate(&ev[i]));
   fresh_counts(ctx);
+  ctx->folded = false;
   double total = 0.0;
   int count = 0;
   for (int s = 0; s < n_sweeps; ++s) {
@@ -1088,15 +1090,13 @@ int hsmc_gpu_counters(hsmc_gpu_ctx *ctx, int replica, uint64_t out[4]) {
   if (!ctx || replica < 0 || replica >= ctx->R || !out) return HSMC_ERR_BAD_ARG;
   int st = fold_counters(ctx);
   if (st) return st;
-  unsigned long long sw = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&sw, ctx->d_sweep, sizeof(sw), hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  const unsigned long long sw = ctx->sweep_now;
   // every occupant of every cell makes one attempt per sweep: N per sweep
   out[0] = (uint64_t)ctx->reps[replica].p.n_part * (sw - ctx->sweep_at_reset);
   out[1] = ctx->tot_acc[replica];
   out[2] = ctx->tot_left[replica];
   out[3] = sw;
-  return check_device_errors(ctx);
+  return ctx->folded ? HSMC_OK : check_device_errors(ctx);
 }
 
 int hsmc_gpu_reset_counters(hsmc_gpu_ctx *ctx) {
@@ -1105,9 +1105,7 @@ int hsmc_gpu_reset_counters(hsmc_gpu_ctx *ctx) {
   if (st) return st;
   std::fill(ctx->tot_acc.begin(), ctx->tot_acc.end(), 0ull);
   std::fill(ctx->tot_left.begin(), ctx->tot_left.end(), 0ull);
-  HSMC_HIP(ctx, hipMemcpyAsync(&ctx->sweep_at_reset, ctx->d_sweep, sizeof(unsigned long long),
-                               hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->sweep_at_reset = ctx->sweep_now;
   return HSMC_OK;
 }
 
@@ -1125,6 +1123,7 @@ int hsmc_gpu_set_sweep_counter(hsmc_gpu_ctx *ctx, uint64_t sweep) {
   // before anything reads it, and clear it before it is filled again
   ctx->cells_version = 0;
   ctx->counts_stale = true;
+  ctx->folded = false;
   return HSMC_OK;
 }
 

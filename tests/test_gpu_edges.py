@@ -87,3 +87,54 @@ def test_reference_exit_conditions(sys500):
     ctx.sweeps(5)
     ctx.sync()
     assert ctx.any_overlap_scaled([1.0])[0] == 1
+
+
+@pytest.mark.parametrize("n", [1, 255, 32768, 32769, 65536, 65537, 100001])
+def test_rows_in_transit(n):
+    """Configurations cross in chunks of 32768 rows through two buffers: every
+    row arrives, up and down, as it was, beside another replica's."""
+    L = max(5.0, (n / 0.3) ** (1 / 3))
+    rng = np.random.default_rng(n)
+    conf = np.zeros((n, 4))
+    conf[:, 0] = np.arange(n)
+    conf[:, 1:] = rng.random((n, 3)) * L
+    other = conf[:300].copy()
+    ctx = gpu.Context([dict(n=len(other), box=(L, L, L)), dict(n=n, box=(L, L, L))])
+    ctx.upload(other, 0)
+    ctx.upload(conf, 1)
+    assert np.array_equal(ctx.download(1), conf)
+    assert np.array_equal(ctx.download(0), other)
+    bad = conf.copy()
+    bad[n - 1, 3] = L * 1.001
+    assert _code(lambda: ctx.upload(bad, 1)) == BAD_ARG
+    assert np.array_equal(ctx.download(1), conf)   # a refused upload changes nothing
+    ctx.close()
+
+
+def test_counters_are_current_after_every_kind_of_sweep():
+    """Counters read between sweeps, resets, tuning and box changes: attempts
+    are N per sweep and what was counted before is kept."""
+    conf, box = gpu.lattice(2, 5, 0.7)
+    ctx = gpu.Context([dict(n=500, box=box, dr_max=0.1, seed=r) for r in (1, 2)])
+    for r in (0, 1):
+        ctx.upload(conf, r)
+    total, last = 0, [0, 0]
+    for step in (lambda: ctx.sweeps(3), lambda: ctx.sweeps(70), lambda: ctx.time_phase_kernel(2),
+                 lambda: ctx.set_tuning(32, 2, 4), lambda: ctx.sweeps(9), lambda: ctx.time_sweeps(5),
+                 lambda: ctx.npt_sweeps(3, 4.0, 0.01), lambda: ctx.scale(1.01, [1.01 * b for b in ctx.box(0)], 0),
+                 lambda: ctx.autotune(8), lambda: ctx.sweeps(1)):
+        before = ctx.counters(1)["sweeps"]
+        step()
+        for r in (0, 1):
+            c = ctx.counters(r)
+            assert c == ctx.counters(r)
+            assert c["attempts"] == 500 * c["sweeps"] and c["sweeps"] >= before
+            assert last[r] <= c["accepted"] <= c["attempts"]
+            assert (c["accepted"] > last[r]) == (c["sweeps"] > before)
+            last[r] = c["accepted"]
+    sweeps = ctx.counters()["sweeps"]
+    assert sweeps == 3 + 70 + 2 + 9 + 5 + 3 + 1
+    ctx.reset_counters()
+    ctx.sweeps(2)
+    assert ctx.counters()["attempts"] == 1000 and ctx.counters()["sweeps"] == sweeps + 2
+    ctx.close()
