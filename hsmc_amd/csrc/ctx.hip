@@ -366,6 +366,24 @@ constexpr int kRowChunk = 1 << 15;
 
 bool valid_box(double L) { return L > 2.0 && std::isfinite(L); }
 
+// A few moved particles, by value: no copy and no wait.
+constexpr int kFewMoves = 8;
+
+struct FewMoves {
+  double q[kFewMoves][3];
+  int idx[kFewMoves];
+};
+
+__global__ void k_set_few(double *__restrict__ x, double *__restrict__ y, double *__restrict__ z, FewMoves f,
+                          int m) {
+  if (threadIdx.x != 0) return;
+  for (int k = 0; k < m; ++k) {  // in order: a particle given twice ends at its last place
+    x[f.idx[k]] = f.q[k][0];
+    y[f.idx[k]] = f.q[k][1];
+    z[f.idx[k]] = f.q[k][2];
+  }
+}
+
 __global__ void k_set_particles(double *__restrict__ x, double *__restrict__ y,
                                 double *__restrict__ z, const int *__restrict__ idx,
                                 const double *__restrict__ q, int m) {
@@ -579,6 +597,18 @@ int hsmc_gpu_set_particles(hsmc_gpu_ctx *ctx, int replica, const int32_t *idx,
     if (!(q[0] >= 0.0 && q[0] <= h.p.lx && q[1] >= 0.0 && q[1] <= h.p.ly && q[2] >= 0.0 &&
           q[2] <= h.p.lz))
       return HSMC_ERR_BAD_ARG;
+  }
+  if (m <= kFewMoves) {
+    FewMoves f{};
+    for (int k = 0; k < m; ++k) {
+      for (int a = 0; a < 3; ++a) f.q[k][a] = xyz[3 * k + a];
+      f.idx[k] = idx[k];
+    }
+    hipLaunchKernelGGL(k_set_few, dim3(1), dim3(64), 0, ctx->stream, ctx->d_x + h.poff, ctx->d_y + h.poff,
+                       ctx->d_z + h.poff, f, m);
+    HSMC_HIP(ctx, hipGetLastError());
+    ctx->version++;
+    return HSMC_OK;
   }
   int *didx = (int *)scratch(ctx, 21, sizeof(int) * m);
   double *dq = (double *)scratch(ctx, 22, sizeof(double) * 3 * m);

@@ -168,3 +168,32 @@ def test_uniform_insertions_filed_in_lds_or_memory(n, rho):
     for m in (1, 511, 5000):
         assert ctx.widom_uniform(31 + (n << 33), 0, 0, m) == int((near[:m] >= 1.0).sum())
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 64, 257, 1025, 16384, 16385])
+def test_few_queries_and_moves_by_value(n):
+    """Overlap queries up to 8 at a time take no grid, more do; one call after
+    another on a configuration changed by set_particles (up to 8 by value)."""
+    L = max(4.2, (n / 0.6) ** (1 / 3))
+    rng = np.random.default_rng(n)
+    xyz = rng.random((n, 3)) * L
+    ctx = _context(xyz, (L, L, L))
+    for m in (1, 7, 8, 9, 40):
+        idx = rng.integers(0, n, m).astype(np.int32)
+        q = rng.random((m, 3)) * L
+        q[0] = (0.0, L, 0.5 * L)
+        want = []
+        for k in range(m):
+            d = _image(q[k] - xyz, L)
+            s = d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]
+            s[idx[k]] = 9.0
+            want.append(np.any(s < 1.0))
+        assert np.array_equal(ctx.overlap_batch(idx, q), np.array(want, dtype=np.uint8)), m
+        # the same particle twice among few: its last place stands
+        moved = np.concatenate([idx[:min(m, n)], idx[:1]]) if m < 8 else np.unique(idx)
+        to = rng.random((len(moved), 3)) * L
+        ctx.set_particles(moved, to)
+        for i, t in zip(moved, to):
+            xyz[i] = t
+        assert np.array_equal(ctx.download()[:, 1:], xyz), m
+    ctx.close()
