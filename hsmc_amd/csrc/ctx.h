@@ -124,9 +124,10 @@ struct hsmc_gpu_ctx {
   static constexpr int kPinned = 3;
   void *pin[kPinned] = {};
   size_t pin_bytes[kPinned] = {};
-  // the move counters are all in the host totals and sweep_now is the sweep
-  // counter: nothing has swept since they were last read
+  // the move counters are all in the host totals: nothing has swept since
+  // they were last read
   bool folded = false;
+  // the sweep counter once every sweep enqueued is done (*d_sweep then)
   unsigned long long sweep_now = 0;
   // results of an observable, stored by its last kernel in pinned memory
   unsigned long long *h_acc = nullptr;
@@ -208,13 +209,13 @@ size_t phase_lds_bytes(int cap, int lcap, int cpb);
 // n checkerboard sweeps of every replica (enqueued on the context stream)
 int run_sweeps(hsmc_gpu_ctx *ctx, int n);
 // Resident sweeps (resident.hip): whether the context's replicas run that
-// way, in what shape, and n sweeps of all of them.
+// way, in what shape, and n sweeps of all of them from sweep number `base` on.
 struct ResidentShape {
   int lpc = 0, threads = 0;
   size_t bytes = 0;
 };
 bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape);
-int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, int n);
+int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, unsigned long long base, int n);
 // File the current by-id positions into the cell slots of the last sweep's
 // grid (the cell list the volume-move scan reads after positions changed).
 int rebin_last_sweep(hsmc_gpu_ctx *ctx);

@@ -80,12 +80,10 @@ void drop_graph(hsmc_gpu_ctx *ctx) {
 
 // One replica per workgroup: its move counters summed over its active cells
 // (cells / 8 entries from aoff on; the padding behind them is never written)
-// into out[2 r], out[2 r + 1], and cleared; the sweep counter and the sticky
-// error bits behind them.
+// into out[2 r], out[2 r + 1], and cleared; the sticky error bits behind them.
 __global__ void __launch_bounds__(256)
 k_fold_counters(const RepDev *__restrict__ reps, int R, unsigned int *__restrict__ cacc,
-                unsigned int *__restrict__ cleft, const unsigned long long *__restrict__ sweep,
-                const unsigned int *__restrict__ err, unsigned long long *__restrict__ out) {
+                unsigned int *__restrict__ cleft, const unsigned int *__restrict__ err, unsigned long long *__restrict__ out) {
   __shared__ unsigned long long s[2][4];
   const int r = blockIdx.x, a0 = reps[r].aoff, a1 = a0 + reps[r].gx * reps[r].gy * reps[r].gz / 8;
   unsigned long long sa = 0, sl = 0;
@@ -107,7 +105,7 @@ k_fold_counters(const RepDev *__restrict__ reps, int R, unsigned int *__restrict
   if (threadIdx.x < 2) {
     const unsigned long long *v = s[threadIdx.x];
     out[2 * r + threadIdx.x] = v[0] + v[1] + v[2] + v[3];
-    if (r == 0) out[2 * R + threadIdx.x] = threadIdx.x ? (unsigned long long)*err : *sweep;
+    if (r == 0 && threadIdx.x == 0) out[2 * R] = *err;
   }
 }
 
@@ -115,10 +113,10 @@ k_fold_counters(const RepDev *__restrict__ reps, int R, unsigned int *__restrict
 // while nothing has swept since.
 int fold_counters(hsmc_gpu_ctx *ctx) {
   if (ctx->folded || !ctx->d_cacc || ctx->Atot == 0) return HSMC_OK;
-  unsigned long long *out = (unsigned long long *)pinned(ctx, P_COUNTERS, sizeof(unsigned long long) * (2 * (size_t)ctx->R + 2));
+  unsigned long long *out = (unsigned long long *)pinned(ctx, P_COUNTERS, sizeof(unsigned long long) * (2 * (size_t)ctx->R + 1));
   if (!out) return HSMC_ERR_NO_MEMORY;
   hipLaunchKernelGGL(k_fold_counters, dim3((unsigned)ctx->R), dim3(256), 0, ctx->stream, ctx->d_reps, ctx->R, ctx->d_cacc,
-                     ctx->d_cleft, ctx->d_sweep, ctx->d_err, out);
+                     ctx->d_cleft, ctx->d_err, out);
   HSMC_HIP(ctx, hipGetLastError());
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   for (int r = 0; r < ctx->R; ++r) {
@@ -126,8 +124,7 @@ int fold_counters(hsmc_gpu_ctx *ctx) {
     ctx->tot_left[r] += out[2 * r + 1];
   }
   ctx->resident_sweeps = 0;
-  ctx->sweep_now = out[2 * ctx->R];
-  ctx->folded = out[2 * ctx->R + 1] == 0;  // with an error pending, the next reader reports it
+  ctx->folded = out[2 * ctx->R] == 0;  // with an error pending, the next reader reports it
   return HSMC_OK;
 }
 

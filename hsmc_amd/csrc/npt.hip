@@ -166,7 +166,7 @@ k_vol_apply(const int *__restrict__ blk, const int *__restrict__ prep, const Vol
 // of the published table (40 us with a scan per move); a sweep's volume moves
 // took about 400 us as rounds of transfers and waits.
 constexpr int kVolDepth = 4;               // moves per launch at most
-constexpr int kVolThreads = 1024;
+constexpr int kVolThreads = 1024;         // threads at most: one per sphere, 256 at least
 constexpr int kVolPer = 4;                 // spheres per thread at most
 constexpr int kVolSpheres = kVolThreads * kVolPer;
 constexpr int kVolAxis = 16;               // search-grid cells per axis at most
@@ -191,12 +191,12 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
   __shared__ int tot[kVolThreads / 64];
   __shared__ double low[kVolThreads / 64];
   __shared__ VolNode tree[(1 << kVolDepth) - 1];
-  const int r = blockIdx.x, t = threadIdx.x, w = t >> 6;
+  const int r = blockIdx.x, T = blockDim.x, t = threadIdx.x, w = t >> 6;
   const int steps = plan[r].steps;
   if (steps == 0) return;
   // the moves lie in host memory: read once, side by side
   constexpr int words = sizeof(VolNode) / 8;
-  static_assert(sizeof(VolNode) % 8 == 0 && words * ((1 << kVolDepth) - 1) <= kVolThreads, "one read");
+  static_assert(sizeof(VolNode) % 8 == 0 && words * ((1 << kVolDepth) - 1) <= 256, "one read");
   const int count = (1 << steps) - 1;
   if (t < words * count)
     reinterpret_cast<unsigned long long *>(tree)[t] =
@@ -206,7 +206,7 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
   double x[kVolPer], y[kVolPer], z[kVolPer];
 #pragma unroll
   for (int u = 0; u < kVolPer; ++u) {
-    const int i = min(t + u * kVolThreads, N - 1);
+    const int i = min(t + u * T, N - 1);
     x[u] = gx[poff + i];
     y[u] = gy[poff + i];
     z[u] = gz[poff + i];
@@ -226,18 +226,18 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
     iz = nz / lz;
     const int C = nx * ny * nz;
     __syncthreads();  // an earlier filing is no longer read
-    for (int c = t; c < C; c += kVolThreads) cnt[c] = 0;
+    for (int c = t; c < C; c += T) cnt[c] = 0;
     __syncthreads();
     int ci[kVolPer], at[kVolPer];
 #pragma unroll
     for (int u = 0; u < kVolPer; ++u) {
-      if (t + u * kVolThreads < N) {
+      if (t + u * T < N) {
         ci[u] = (search_cell(x[u], ix, nx) * ny + search_cell(y[u], iy, ny)) * nz + search_cell(z[u], iz, nz);
         at[u] = atomicAdd(&cnt[ci[u]], 1);
       }
     }
     __syncthreads();
-    const int per = (C + kVolThreads - 1) / kVolThreads, c0 = min(t * per, C), c1 = min(c0 + per, C);
+    const int per = (C + T - 1) / T, c0 = min(t * per, C), c1 = min(c0 + per, C);
     int s = 0;
     for (int c = c0; c < c1; ++c) s += cnt[c];
     const int incl = group_inclusive_sum<64>(s);
@@ -252,7 +252,7 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kVolPer; ++u) {
-      if (t + u * kVolThreads < N) {
+      if (t + u * T < N) {
         const int p = (ci[u] ? cnt[ci[u] - 1] : 0) + at[u];
         px[p] = x[u];
         py[p] = y[u];
@@ -265,7 +265,7 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
   // spheres after p in filed order), in every thread
   auto least = [&](auto &&f) {
     double m = 1e300;
-    for (int p = t; p < N; p += kVolThreads) {
+    for (int p = t; p < N; p += T) {
       const double ax = px[p], ay = py[p], az = pz[p];
       const int cx = search_cell(ax, ix, nx), cy = search_cell(ay, iy, ny), cz = search_cell(az, iz, nz);
       for (int d = 0; d < 27; ++d) {
@@ -280,7 +280,7 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
     __syncthreads();  // low is no longer read
     if ((t & 63) == 0) low[w] = m;
     __syncthreads();
-    for (int k = 0; k < kVolThreads / 64; ++k) m = fmin(m, low[k]);
+    for (int k = 0; k < T / 64; ++k) m = fmin(m, low[k]);
     return m;
   };
   double sf_min = 1.0;  // along any path: at most kVolDepth compressions in a row
@@ -328,7 +328,7 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
   if (moved) {
 #pragma unroll
     for (int u = 0; u < kVolPer; ++u) {
-      const int i = t + u * kVolThreads;
+      const int i = t + u * T;
       if (i < N) {
         gx[poff + i] = x[u];
         gy[poff + i] = y[u];
@@ -484,6 +484,7 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
   const int R = ctx->R;
   int n_max = 0;
   for (const RepHost &h : ctx->reps) n_max = std::max(n_max, h.p.n_part);
+  const int threads = std::min(kVolThreads, (n_max + 255) / 256 * 256);
   const size_t lds = sizeof(double) * 3 * n_max + sizeof(int) * kVolAxis * kVolAxis * kVolAxis;
   if (lds > 60 * 1024)  // with the kernel's own few KB above 64 KB
     HSMC_HIP(ctx, hipFuncSetAttribute((const void *)k_volume_moves, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -512,7 +513,7 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
     memcpy(host, plan.data(), sizeof(VolPlan) * R);
     memcpy(host + o_node, nodes.data(), sizeof(VolNode) * nodes.size());
     const int *res = (const int *)(host + o_res);
-    hipLaunchKernelGGL(k_volume_moves, dim3((unsigned)R), dim3(kVolThreads), lds, ctx->stream, ctx->d_reps,
+    hipLaunchKernelGGL(k_volume_moves, dim3((unsigned)R), dim3((unsigned)threads), lds, ctx->stream, ctx->d_reps,
                        (const VolPlan *)host, (const VolNode *)(host + o_node), ctx->d_x, ctx->d_y, ctx->d_z,
                        (int *)(host + o_res));
     HSMC_HIP(ctx, hipGetLastError());
@@ -671,9 +672,7 @@ int hsmc_gpu_npt_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, const double *press,
   for (int r = 0; r < R; ++r)
     if (!(press[r] >= 0.0) || !(dv_max[r] > 0.0) || !std::isfinite(press[r])) return HSMC_ERR_BAD_ARG;
   if (n_sweeps == 0) return HSMC_OK;
-  unsigned long long sweep0 = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&sweep0, ctx->d_sweep, sizeof(sweep0), hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  const unsigned long long sweep0 = ctx->sweep_now;
   bool small = true;
   for (const RepHost &h : ctx->reps) small = small && h.p.n_part <= kVolSpheres;
   std::vector<int> steps(R);

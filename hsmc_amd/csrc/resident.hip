@@ -91,10 +91,10 @@ __host__ __device__ inline Layout resident_layout(int N, int C, int cap, int gro
 template <int CAP, int LPC, int RC>
 __global__ void __launch_bounds__(1024)
 k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict__ x,
-                  double *__restrict__ y, double *__restrict__ z,
-                  const unsigned long long *__restrict__ sweep_base, int n_sweeps,
+                  double *__restrict__ y, double *__restrict__ z, unsigned long long base,
+                  unsigned long long *__restrict__ sweep_counter, int n_sweeps,
                   unsigned int *__restrict__ cacc, unsigned int *__restrict__ cleft,
-                  unsigned int *__restrict__ err) {
+                  unsigned int *__restrict__ err, unsigned int *__restrict__ host_err) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const RepDev rp = reps[blockIdx.x];
   const int T = blockDim.x, tid = threadIdx.x, groups = T / LPC;
@@ -139,7 +139,7 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
     jok[q] = j < 27 && stencil_axis_ok(jx[q], rp.gx) && stencil_axis_ok(jy[q], rp.gy) &&
              stencil_axis_ok(jz[q], rp.gz);
   }
-  const unsigned long long base = *sweep_base;
+  unsigned bad = 0;  // sticky error bits
   unsigned n_acc = 0, n_left = 0;
   auto in_cell = [&](double px_, double py_, double pz_, const SweepDev &sw) {
     return (shifted_cell(px_, sw.shx, rp.lx, rp.ix, rp.gx) * rp.gy +
@@ -180,7 +180,7 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
           occ[c * CAP + sl] = (uint16_t)i;
           ci[u] = c;
         } else {
-          atomicOr(err, kErrOverflow);
+          bad |= kErrOverflow;
         }
       }
     }
@@ -257,7 +257,7 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
         const int incl = lane_sum<LPC>(mine);
         const int total = __shfl(incl, LPC - 1, LPC);
         if (total > lcap) {  // above the host's packing bound: overlapping spheres
-          if (lane == 0) atomicOr(err, kErrListFull);
+          bad |= kErrListFull;
           continue;
         }
         int o = incl - mine;
@@ -335,14 +335,21 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
     y[rp.poff + i] = py[i];
     z[rp.poff + i] = pz[i];
   }
+  if (bad) {  // for the device's readers, and the host's copy at once
+    atomicOr(err, bad);
+    *host_err = bad;
+  }
+  // the first sweep's number came by value, so the counter is only written
+  if (blockIdx.x == 0 && tid == 0) *sweep_counter = base + (unsigned long long)n_sweeps;
   if (lane == 0 && grp < A) {
     if (n_acc) atomicAdd(&cacc[rp.aoff + grp], n_acc);
     if (n_left) atomicAdd(&cleft[rp.aoff + grp], n_left);
   }
 }
 
-using ResidentFn = void (*)(const RepDev *, int, double *, double *, double *, const unsigned long long *, int,
-                            unsigned int *, unsigned int *, unsigned int *);
+using ResidentFn = void (*)(const RepDev *, int, double *, double *, double *, unsigned long long,
+                            unsigned long long *, int, unsigned int *, unsigned int *, unsigned int *,
+                            unsigned int *);
 
 // Lanes per active cell: 32 while a phase's cells fit the workgroup's 32 such
 // groups (us per sweep at N = 108 and 256, 8 and 27 cells a phase: 15.3 and
@@ -353,10 +360,6 @@ constexpr int kWide = 32, kNarrow = 16;
 ResidentFn resident_fn(int cap, int lpc) {
   if (lpc == kWide) return cap == 8 ? k_sweeps_resident<8, kWide, 2> : k_sweeps_resident<16, kWide, 2>;
   return cap == 8 ? k_sweeps_resident<8, kNarrow, 3> : k_sweeps_resident<16, kNarrow, 3>;
-}
-
-__global__ void k_add_sweeps(unsigned long long *sweep_base, int n) {
-  if (threadIdx.x == 0) *sweep_base += (unsigned long long)n;
 }
 
 }  // namespace
@@ -395,13 +398,13 @@ bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape) {
   return shape->bytes <= 160 * 1024;
 }
 
-int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, int n) {
+int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, unsigned long long base, int n) {
   ResidentFn fn = resident_fn(ctx->cap, shape.lpc);
   if (shape.bytes > 64 * 1024)
     HSMC_HIP(ctx, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.bytes));
   hipLaunchKernelGGL(fn, dim3((unsigned)ctx->R), dim3((unsigned)shape.threads), shape.bytes, ctx->stream, ctx->d_reps,
-                     ctx->lcap, ctx->d_x, ctx->d_y, ctx->d_z, ctx->d_sweep, n, ctx->d_cacc, ctx->d_cleft, ctx->d_err);
-  hipLaunchKernelGGL(k_add_sweeps, dim3(1), dim3(64), 0, ctx->stream, ctx->d_sweep, n);
+                     ctx->lcap, ctx->d_x, ctx->d_y, ctx->d_z, base, ctx->d_sweep, n, ctx->d_cacc, ctx->d_cleft,
+                     ctx->d_err, (unsigned int *)ctx->h_err);
   HSMC_HIP(ctx, hipGetLastError());
   return HSMC_OK;
 }

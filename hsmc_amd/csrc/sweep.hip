@@ -914,11 +914,10 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
         int st = fold_counters(ctx);
         if (st) return st;
       }
-      int st = launch_resident(ctx, shape, k);
+      int st = launch_resident(ctx, shape, ctx->sweep_now, k);
       if (st) return st;
+      ctx->sweep_now += k;
       ctx->resident_sweeps += k;
-      HSMC_HIP(ctx, hipMemcpyAsync((void *)ctx->h_err, ctx->d_err, sizeof(unsigned int),
-                                   hipMemcpyDeviceToHost, ctx->stream));
     }
     ctx->cells_version = 0;  // no cell list in memory
     ctx->counts_stale = true;
@@ -931,6 +930,7 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
       if (*ctx->h_err) return check_device_errors(ctx);
       int st = launch_persistent(ctx, std::min(per, n - done));
       if (st) return st;
+      ctx->sweep_now += std::min(per, n - done);
       ctx->swp_last = std::min(per, n - done) - 1;
       HSMC_HIP(ctx, hipMemcpyAsync((void *)ctx->h_err, ctx->d_err, sizeof(unsigned int),
                                    hipMemcpyDeviceToHost, ctx->stream));
@@ -948,6 +948,7 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
     for (; done + K <= n; done += K) {
       if (*ctx->h_err) return check_device_errors(ctx);
       HSMC_HIP(ctx, hipGraphLaunch(ctx->gexec, ctx->stream));
+      ctx->sweep_now += K;
       HSMC_HIP(ctx, hipMemcpyAsync((void *)ctx->h_err, ctx->d_err, sizeof(unsigned int),
                                    hipMemcpyDeviceToHost, ctx->stream));
       ctx->swp_last = can_chain(ctx) ? K - 1 : 0;  // the last sweep's table entry
@@ -967,6 +968,7 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
       hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, ctx->stream, ctx->d_sweep, rem);
       HSMC_HIP(ctx, hipGetLastError());
     }
+    ctx->sweep_now += rem;
     HSMC_HIP(ctx, hipMemcpyAsync((void *)ctx->h_err, ctx->d_err, sizeof(unsigned int),
                                  hipMemcpyDeviceToHost, ctx->stream));
     ctx->swp_last = can_chain(ctx) && rem < kSweepTable ? rem - 1 : 0;
@@ -1051,6 +1053,7 @@ int hsmc_gpu_time_phase_kernel(hsmc_gpu_ctx *ctx, int n_sweeps, float *avg_ms, i
   for (int s = 0; s < n_sweeps; ++s) {
     enqueue_sweep(ctx, 0, ctx->stream, ev);
     hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, ctx->stream, ctx->d_sweep, 1);
+    ctx->sweep_now += 1;
     HSMC_HIP(ctx, hipEventSynchronize(ev[15]));
     float ms = 0.f;
     HSMC_HIP(ctx, hipEventElapsedTime(&ms, ev[0], ev[15]));
@@ -1111,19 +1114,16 @@ int hsmc_gpu_reset_counters(hsmc_gpu_ctx *ctx) {
 
 int hsmc_gpu_set_sweep_counter(hsmc_gpu_ctx *ctx, uint64_t sweep) {
   if (!ctx) return HSMC_ERR_BAD_ARG;
-  unsigned long long now = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&now, ctx->d_sweep, sizeof(now), hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   const unsigned long long want = (unsigned long long)sweep;
   HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_sweep, &want, sizeof(want), hipMemcpyHostToDevice, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   // attempts are N * (sweep - sweep_at_reset): move the origin with the counter
-  ctx->sweep_at_reset += want - now;
+  ctx->sweep_at_reset += want - ctx->sweep_now;
+  ctx->sweep_now = want;
   // the last sweep's cell list is found by the counter's parity: refile it
   // before anything reads it, and clear it before it is filled again
   ctx->cells_version = 0;
   ctx->counts_stale = true;
-  ctx->folded = false;
   return HSMC_OK;
 }
 
@@ -1147,7 +1147,7 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
   // save positions, sweep counter and move counters; restore afterwards
   double *save = (double *)scratch(ctx, 23, sizeof(double) * 3 * P);
   if (!save) return HSMC_ERR_NO_MEMORY;
-  unsigned long long sweep0 = 0;
+  const unsigned long long sweep0 = ctx->sweep_now;
   {
     int st0 = fold_counters(ctx);
     if (st0) return st0;
@@ -1156,7 +1156,6 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
   HSMC_HIP(ctx, hipMemcpyAsync(save, ctx->d_x, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
   HSMC_HIP(ctx, hipMemcpyAsync(save + P, ctx->d_y, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
   HSMC_HIP(ctx, hipMemcpyAsync(save + 2 * P, ctx->d_z, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
-  HSMC_HIP(ctx, hipMemcpyAsync(&sweep0, ctx->d_sweep, sizeof(sweep0), hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
   const hsmc_gpu_tuning start = ctx->tune;
   const bool start_set = ctx->tune_set;
@@ -1217,6 +1216,7 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
   HSMC_HIP(ctx, hipMemsetAsync(ctx->d_cleft, 0, sizeof(unsigned int) * ctx->cell_alloc, ctx->stream));
   HSMC_HIP(ctx, hipMemsetAsync(ctx->d_cnt, 0, sizeof(int) * 2 * ctx->cell_alloc, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->sweep_now = sweep0;
   ctx->version++;  // positions restored, cell lists cleared
   ctx->tot_acc = acc0;
   ctx->tot_left = left0;
