@@ -803,10 +803,13 @@ k_free_tiles(Vox vx, const unsigned char *__restrict__ flag, int *__restrict__ s
 }
 
 // Pack the tiles' free voxels into one list: tile t's cnt[t] entries go to
-// list[off[t] ...] (off: exclusive prefix sum of cnt); one wave per tile.
+// list[off[t] ...] (off: exclusive prefix sum of cnt); one wave per tile.  The
+// number of free voxels goes to the host.
 __global__ void __launch_bounds__(256)
 k_gather_free(const int *__restrict__ slots, const int *__restrict__ cnt,
-              const int *__restrict__ off, int *__restrict__ list, long tiles) {
+              const int *__restrict__ off, int *__restrict__ list, long tiles,
+              unsigned long long *__restrict__ host) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *host = (unsigned long long)off[tiles];
   const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= tiles) return;
   const int n = cnt[t], o = off[t];
@@ -838,42 +841,43 @@ k_voxel_scores_list(NGrid g, Vox vx, float far2, const MlpDev *__restrict__ net,
 
 // Network part of the proposal mass of a free voxel v:
 // mix * softmax(f)_v = mix * exp(f_v - fmax) / sumexp, with st[0] = fmax and
-// st[1] = sumexp (on the device, written by k_reduce_parts).
+// st[1] = sumexp (on the device, written by k_cdf_local).
 __device__ __forceinline__ double network_mass(const float *__restrict__ f, long v,
                                                const double *__restrict__ st, double mix) {
   return mix * exp((double)f[v] - st[0]) / st[1];
 }
 
 // st[0] = max of the blocks' maxima, st[1] = sum of their sums of
-// exp(f - max) rescaled to st[0], each in a fixed order (strided partials,
-// then a tree); st[2] = 0.
-__global__ void __launch_bounds__(256)
-k_reduce_parts(const float *__restrict__ bmax, const float *__restrict__ bsum, long nb,
-               double *__restrict__ st) {
+// exp(f - max) rescaled to st[0], each in a fixed order (256 strided
+// partials, then a tree), for the whole workgroup (at least 256 threads).
+__device__ __forceinline__ void softmax_stats(const float *__restrict__ bmax,
+                                              const float *__restrict__ bsum, long nb, double st[2]) {
   __shared__ double s[256];
+  const int t = threadIdx.x;
   double m = -INFINITY;
-  for (long b = threadIdx.x; b < nb; b += 256) m = fmax(m, (double)bmax[b]);
-  s[threadIdx.x] = m;
+  if (t < 256) {
+    for (long b = t; b < nb; b += 256) m = fmax(m, (double)bmax[b]);
+    s[t] = m;
+  }
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] = fmax(s[threadIdx.x], s[threadIdx.x + w]);
+    if (t < w) s[t] = fmax(s[t], s[t + w]);
     __syncthreads();
   }
   const double fm = s[0];
   __syncthreads();
-  double e = 0.0;
-  for (long b = threadIdx.x; b < nb; b += 256) e += (double)bsum[b] * exp((double)bmax[b] - fm);
-  s[threadIdx.x] = e;
+  if (t < 256) {
+    double e = 0.0;
+    for (long b = t; b < nb; b += 256) e += (double)bsum[b] * exp((double)bmax[b] - fm);
+    s[t] = e;
+  }
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+    if (t < w) s[t] += s[t + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    st[0] = fm;
-    st[1] = s[0];
-    st[2] = 0.0;
-  }
+  st[0] = fm;
+  st[1] = s[0];
 }
 
 // The statistics of a proposal with no free voxel (every voxel keeps the
@@ -886,37 +890,57 @@ __global__ void k_empty_stats(double *__restrict__ st) {
   }
 }
 
-// Cumulative network mass over the free-voxel list (list order), in three
-// passes: inclusive sums within blocks of 4096 entries (+ block totals), an
-// exclusive scan of the block totals (one workgroup; its last entry is the
-// total), then the block offsets added.
+// Cumulative network mass over the free-voxel list (list order): inclusive
+// sums within blocks of 4096 entries (+ block totals), then the blocks'
+// exclusive offsets added, the total behind the block totals.  The offsets
+// are a scan of the totals, of up to kScanWave of them by every workgroup of
+// the adding kernel for itself, of more by a kernel in between (the same
+// additions either way): with the totals, the hits and the number of free
+// voxels also going to the host from the kernels that know them, one insertion
+// call at N = 108000 takes 292 us, 342 with a kernel for each of these steps,
+// two copies and two waits.  With bmax the softmax totals are taken from the
+// scoring kernel's nparts block partials first (each workgroup for itself,
+// the first stores them); otherwise st holds them already.
+constexpr int kScanWave = 64;
+
 __global__ void __launch_bounds__(1024)
-k_cdf_local(const float *__restrict__ f, const int *__restrict__ list, long V,
-            const double *__restrict__ st, double mix, double *__restrict__ cdf,
+k_cdf_local(const float *__restrict__ f, const int *__restrict__ list, long V, const float *__restrict__ bmax,
+            long nparts, double *__restrict__ stats, double mix, double *__restrict__ cdf,
             double *__restrict__ bsum) {
-  __shared__ double s[1024];
+  __shared__ double s[2][1024];
   const long base = (long)blockIdx.x * 4096;
+  double st[2];
+  if (bmax) {
+    softmax_stats(bmax, bmax + nparts, nparts, st);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      stats[0] = st[0];
+      stats[1] = st[1];
+      stats[2] = 0.0;
+    }
+  } else {
+    st[0] = stats[0];
+    st[1] = stats[1];
+  }
   double v[4], tot = 0.0;
   for (int j = 0; j < 4; ++j) {
     const long i = base + threadIdx.x * 4 + j;
     v[j] = i < V ? network_mass(f, list[i], st, mix) : 0.0;
     tot += v[j];
   }
-  s[threadIdx.x] = tot;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {
-    const double t = (int)threadIdx.x >= d ? s[threadIdx.x - d] : 0.0;
+  // s[0] and s[1] in turn: one barrier a step
+  double incl = tot;
+  for (int d = 1, b = 0; d < 1024; d <<= 1, b ^= 1) {
+    s[b][threadIdx.x] = incl;
     __syncthreads();
-    s[threadIdx.x] += t;
-    __syncthreads();
+    incl += (int)threadIdx.x >= d ? s[b][threadIdx.x - d] : 0.0;
   }
-  double run = s[threadIdx.x] - tot;
+  double run = incl - tot;
   for (int j = 0; j < 4; ++j) {
     const long i = base + threadIdx.x * 4 + j;
     run += v[j];
     if (i < V) cdf[i] = run;
   }
-  if (threadIdx.x == 1023) bsum[blockIdx.x] = s[1023];
+  if (threadIdx.x == 1023) bsum[blockIdx.x] = incl;
 }
 
 __global__ void __launch_bounds__(1024) k_cdf_blocks(double *__restrict__ b, int nb) {
@@ -942,9 +966,28 @@ __global__ void __launch_bounds__(1024) k_cdf_blocks(double *__restrict__ b, int
   if (t == 1023) b[nb] = part[1023];
 }
 
-__global__ void k_cdf_add(double *__restrict__ cdf, long V, const double *__restrict__ boff) {
+// SCAN: b holds the nb <= kScanWave block totals, scanned here (k_cdf_blocks'
+// additions: steps of 1, 2, 4, ... and the own total taken off again).
+template <bool SCAN>
+__global__ void __launch_bounds__(256)
+k_cdf_add(double *__restrict__ cdf, long V, double *__restrict__ b, int nb, double *__restrict__ total) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < V) cdf[i] += boff[i / 4096];
+  double off = 0.0;
+  const int mine = (int)((long)blockIdx.x * blockDim.x / 4096);  // 4096 is a multiple of the workgroup's entries
+  if constexpr (SCAN) {
+    const int lane = threadIdx.x & 63;
+    const double own = lane < nb ? b[lane] : 0.0;
+    double incl = own;
+    for (int d = 1; d < 64; d <<= 1) {
+      const double v = __shfl_up(incl, d, 64);
+      incl += lane >= d ? v : 0.0;
+    }
+    off = __shfl(incl - own, mine, 64);
+    if (blockIdx.x == 0 && threadIdx.x == 63) *total = incl;
+  } else {
+    off = b[mine];
+  }
+  if (i < V) cdf[i] += off;
 }
 
 // No sphere centre closer than 1 to q in the 27 cells around it (the
@@ -1009,7 +1052,7 @@ k_insert(NGrid g1, Vox vx, const double *__restrict__ cdf, const int *__restrict
          const float *__restrict__ f, const unsigned char *__restrict__ flag,
          const double *__restrict__ st, double mix, uint32_t k0, uint32_t k1,
          unsigned long long sample, double *__restrict__ part,
-         unsigned long long *__restrict__ hits) {
+         unsigned int *__restrict__ hits) {
   __shared__ double rs[4];
   __shared__ unsigned long long rh[4];
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1059,28 +1102,42 @@ k_insert(NGrid g1, Vox vx, const double *__restrict__ cdf, const int *__restrict
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    // the block's weight goes to its own slot and is summed in a fixed order
-    // afterwards (k_sum_fixed), so an estimate never depends on block timing
+    // the block's weight and hits go to their own slots; the weights are summed
+    // in a fixed order afterwards (k_sum_fixed), so an estimate never depends
+    // on block timing
     part[blockIdx.x] = rs[0] + rs[1] + rs[2] + rs[3];
-    const unsigned long long sh = rh[0] + rh[1] + rh[2] + rh[3];
-    if (sh) atomicAdd(hits, sh);
+    hits[blockIdx.x] = (unsigned int)(rh[0] + rh[1] + rh[2] + rh[3]);
   }
 }
 
-// out = sum of part[0..n) in an order fixed by n alone: 256 strided partial
-// sums, then a pairwise tree.
-__global__ void __launch_bounds__(256) k_sum_fixed(const double *__restrict__ part, long n,
-                                                   double *__restrict__ out) {
+// host[0] = sum of part[0..n), as bits, in an order fixed by n alone (256
+// strided partial sums, then a pairwise tree), host[1] = sum of hits[0..n).
+__global__ void __launch_bounds__(256) k_sum_fixed(const double *__restrict__ part,
+                                                   const unsigned int *__restrict__ hits, long n,
+                                                   unsigned long long *__restrict__ host) {
   __shared__ double s[256];
+  __shared__ unsigned long long sh[256];
   double a = 0.0;
-  for (long i = threadIdx.x; i < n; i += 256) a += part[i];
+  unsigned long long h = 0;
+#pragma unroll 4
+  for (long i = threadIdx.x; i < n; i += 256) {
+    a += part[i];
+    h += hits[i];
+  }
   s[threadIdx.x] = a;
+  sh[threadIdx.x] = h;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+    if ((int)threadIdx.x < w) {
+      s[threadIdx.x] += s[threadIdx.x + w];
+      sh[threadIdx.x] += sh[threadIdx.x + w];
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = s[0];
+  if (threadIdx.x == 0) {
+    host[0] = (unsigned long long)__double_as_longlong(s[0]);
+    host[1] = sh[0];
+  }
 }
 
 // Build a CSR grid of one replica (side >= cut) into the given scratch slots.
@@ -1155,28 +1212,24 @@ __device__ __forceinline__ int cell_in(const CellDims &d, double x, double y, do
 
 __global__ void k_grid_count_pair(const double *__restrict__ x, const double *__restrict__ y,
                                   const double *__restrict__ z, int n, CellDims a, CellDims b,
-                                  int ca, int *__restrict__ cnt, int *__restrict__ cellof) {
+                                  int ca, int *__restrict__ cnt, int4 *__restrict__ at) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const double xi = x[i], yi = y[i], zi = z[i];
   const int c0 = cell_in(a, xi, yi, zi), c1 = ca + cell_in(b, xi, yi, zi);
-  cellof[i] = c0;
-  cellof[n + i] = c1;
-  atomicAdd(&cnt[c0], 1);
-  atomicAdd(&cnt[c1], 1);
+  at[i] = make_int4(c0, c1, atomicAdd(&cnt[c0], 1), atomicAdd(&cnt[c1], 1));
 }
 
 __global__ void k_grid_scatter_pair(const double *__restrict__ x, const double *__restrict__ y,
                                     const double *__restrict__ z, int n,
-                                    const int *__restrict__ cellof, const int *__restrict__ start,
-                                    int *__restrict__ fill, double *__restrict__ px,
-                                    double *__restrict__ py, double *__restrict__ pz) {
+                                    const int4 *__restrict__ at, const int *__restrict__ start,
+                                    double *__restrict__ px, double *__restrict__ py,
+                                    double *__restrict__ pz) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const double xi = x[i], yi = y[i], zi = z[i];
-  const int c0 = cellof[i], c1 = cellof[n + i];
-  const int s0 = start[c0], s1 = start[c1];
-  const int p0 = s0 + atomicAdd(&fill[c0], 1), p1 = s1 + atomicAdd(&fill[c1], 1);
+  const int4 a = at[i];
+  const int p0 = start[a.x] + a.z, p1 = start[a.y] + a.w;
   px[p0] = xi;
   py[p0] = yi;
   pz[p0] = zi;
@@ -1196,11 +1249,11 @@ int grid_cells_for2(double L, double cut) {
 // ctx.hip 21..22, sweep.hip 23): descriptor grid 24..26, the insertion call's
 // descriptor and overlap grids built together 27..29,
 // rows / scores 30, targets / block partials 31, cumulative mass 32, gradient
-// sums of the training workgroups 33, sums 34, per-block insertion weights 35, cumulative-mass block sums 36,
+// sums of the training workgroups 33, per-block insertion weights and hits 35, cumulative-mass block sums 36,
 // grid-scan partials 37, voxel scores 38, score block reductions 39,
 // free-voxel tile slots and list 40, tile counts, offsets and scan space 41,
 // blocked-voxel flags 42, softmax statistics 43.
-enum { L_GRID_A = 24, L_GRID_PAIR = 27, L_X = 30, L_T = 31, L_CDF = 32, L_GRAD = 33, L_ACC = 34, L_PART = 35,
+enum { L_GRID_A = 24, L_GRID_PAIR = 27, L_X = 30, L_T = 31, L_CDF = 32, L_GRAD = 33, L_PART = 35,
        L_BSUM = 36, L_SCANP = 37, L_F = 38, L_FRED = 39, L_LIST = 40, L_NFREE = 41, L_FLAG = 42,
        L_STATS = 43 };
 
@@ -1232,13 +1285,13 @@ int build_ngrid_pair(hsmc_gpu_ctx *ctx, int replica, double cut_a, double cut_b,
   if (C + 1 > (1L << 31) - 1 || 2L * N > (1L << 31) - 1) return HSMC_ERR_NOT_SUPPORTED;
   const bool cached = ctx->ngrid_replica[1] == replica && ctx->ngrid_version[1] == ctx->version &&
                       ctx->ngrid_cut[1] == cut_a + cut_b;
-  int *cnt = (int *)scratch(ctx, L_GRID_PAIR + 0, sizeof(int) * 2 * (C + 1) + sizeof(int) * 2 * N);
+  const size_t cells = ((size_t)C + 4) & ~(size_t)3;  // keeps the int4 behind the counts aligned
+  int *cnt = (int *)scratch(ctx, L_GRID_PAIR + 0, sizeof(int) * cells + sizeof(int4) * N);
   double *pos = (double *)scratch(ctx, L_GRID_PAIR + 1, sizeof(double) * 6 * (size_t)N);
   int *start = (int *)scratch(ctx, L_GRID_PAIR + 2, sizeof(int) * (C + 1));
   int *part = (int *)scratch(ctx, L_SCANP, sizeof(int) * scan_workspace_ints(C));
   if (!cnt || !pos || !start || !part) return HSMC_ERR_NO_MEMORY;
-  int *fill = cnt + (C + 1);
-  int *cellof = fill + (C + 1);
+  int4 *at = (int4 *)(cnt + cells);  // each sphere's two cells and its rank in each
   const size_t stride = 2 * (size_t)N;
   set_grid(ga, h, cut_a, start, pos, stride);
   set_grid(gb, h, cut_b, start + Ca, pos, stride);
@@ -1246,12 +1299,12 @@ int build_ngrid_pair(hsmc_gpu_ctx *ctx, int replica, double cut_a, double cut_b,
   const CellDims da{ga.nx, ga.ny, ga.nz, ga.ix, ga.iy, ga.iz};
   const CellDims db{gb.nx, gb.ny, gb.nz, gb.ix, gb.iy, gb.iz};
   const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
-  HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * 2 * (C + 1), ctx->stream));
+  HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * (C + 1), ctx->stream));
   hipLaunchKernelGGL(k_grid_count_pair, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z,
-                     N, da, db, (int)Ca, cnt, cellof);
+                     N, da, db, (int)Ca, cnt, at);
   exclusive_scan(ctx->stream, cnt, (int)C, start, part, false);
   hipLaunchKernelGGL(k_grid_scatter_pair, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y,
-                     z, N, cellof, start, fill, pos, pos + stride, pos + 2 * stride);
+                     z, N, at, start, pos, pos + stride, pos + 2 * stride);
   HSMC_HIP(ctx, hipGetLastError());
   ctx->ngrid_replica[1] = replica;
   ctx->ngrid_version[1] = ctx->version;
@@ -1360,21 +1413,26 @@ __global__ void k_mask_blocked(float *__restrict__ f, const unsigned char *__res
 
 // The proposal of one configuration: the byte flags of blocked voxels
 // (k_mark_blocked), the list of free voxels (k_free_tiles, k_gather_free),
-// the network's scores of the free voxels in f (k_voxel_scores_list), and
-// in stats[0], stats[1] (device) fmax and sumexp over them (0 and 1 when none is
-// free, so every voxel keeps the uniform part alone).  Where a voxel is too
+// the network's scores of the free voxels in f (k_voxel_scores_list), and the
+// block partials of their softmax totals (with no free voxel the totals
+// themselves: 0 and 1, so every voxel keeps the uniform part alone).  Where a voxel is too
 // large for any exclusion, or too small for the marking kernel's 8
 // candidates per axis, every voxel is free and scored.  Only the number of
 // free voxels comes back to the host (it sizes the later launches).
 struct Proposal {
   unsigned char *flag = nullptr;
   int *list = nullptr;
-  double *stats = nullptr;
+  const float *parts = nullptr;  // the scoring kernel's block partials
+  long nparts = 0;
   long nfree = 0;
 };
 
-int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, const NGrid &g, const Vox &vx,
+// `grid` builds the search grids and gives the descriptors' one; its launches
+// run while the host waits for the number of free voxels.
+template <class MakeGrid>
+int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, MakeGrid &&grid, const Vox &vx,
                            const MlpDev *net, float *f, Proposal *pr) {
+  NGrid g;
   const double h = 0.5 * sqrt(vx.vx * vx.vx + vx.vy * vx.vy + vx.vz * vx.vz);
   const double r = 1.0 - h - 1e-9;
   // the marking kernel's 8 candidate voxels per axis must cover the centres
@@ -1395,18 +1453,19 @@ int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, const NGrid &g, const
   int *list = slots + (size_t)tiles * 256;
   pr->flag = flag;
   pr->list = list;
-  pr->stats = stats;
   HSMC_HIP(ctx, hipMemsetAsync(flag, 0, (size_t)vx.V, ctx->stream));
   if (!(r > 0.0) || !span_ok) {
     float *bred = nullptr;
     long nblk = 0;
-    int st = launch_scores(ctx, g, vx, net, f, &bred, &nblk);
+    int st = grid(&g);
+    if (st) return st;
+    st = launch_scores(ctx, g, vx, net, f, &bred, &nblk);
     if (st) return st;
     hipLaunchKernelGGL(k_iota, dim3((unsigned)((vx.V + 255) / 256)), dim3(256), 0, ctx->stream, list,
                        vx.V);
-    hipLaunchKernelGGL(k_reduce_parts, dim3(1), dim3(256), 0, ctx->stream, bred, bred + nblk, nblk,
-                       stats);
     HSMC_HIP(ctx, hipGetLastError());
+    pr->parts = bred;
+    pr->nparts = nblk;
     pr->nfree = vx.V;
     return HSMC_OK;
   }
@@ -1421,11 +1480,13 @@ int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, const NGrid &g, const
                      flag, slots, cnt, tiles);
   exclusive_scan(ctx->stream, cnt, (int)tiles, off, part, false);
   hipLaunchKernelGGL(k_gather_free, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, ctx->stream,
-                     slots, cnt, off, list, tiles);
+                     slots, cnt, off, list, tiles, ctx->h_acc);
   HSMC_HIP(ctx, hipGetLastError());
-  int nf = 0;
-  HSMC_HIP(ctx, hipMemcpyAsync(&nf, off + tiles, sizeof(nf), hipMemcpyDeviceToHost, ctx->stream));
-  HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  HSMC_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+  int st = grid(&g);
+  if (st) return st;
+  HSMC_HIP(ctx, hipEventSynchronize(ctx->ev0));
+  const int nf = (int)ctx->h_acc[0];
   pr->nfree = nf;
   if (nf == 0) {
     hipLaunchKernelGGL(k_empty_stats, dim3(1), dim3(64), 0, ctx->stream, stats);
@@ -1435,13 +1496,14 @@ int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, const NGrid &g, const
   const long nb = ((long)nf + 255) / 256;
   float *b = (float *)scratch(ctx, L_FRED, sizeof(float) * 2 * (size_t)nb);
   if (!b) return HSMC_ERR_NO_MEMORY;
-  // the softmax totals from the scoring kernel's per-block max and sum of
+  // the softmax totals come from the scoring kernel's per-block max and sum of
   // exp(f - max) (each block's 256 list entries reduced in a fixed order),
   // combined in a fixed order: they depend only on the scores and the list
   hipLaunchKernelGGL(k_voxel_scores_list, dim3((unsigned)nb), dim3(256), 0, ctx->stream, g, vx,
                      far2_of(g), net, list, (int)nf, f, b, b + nb);
-  hipLaunchKernelGGL(k_reduce_parts, dim3(1), dim3(256), 0, ctx->stream, b, b + nb, nb, stats);
   HSMC_HIP(ctx, hipGetLastError());
+  pr->parts = b;
+  pr->nparts = nb;
   return HSMC_OK;
 }
 
@@ -1633,22 +1695,26 @@ int hsmc_gpu_widom_learned(hsmc_gpu_mlp *m, int replica, double voxel, double mi
     return HSMC_ERR_BAD_ARG;
   hsmc_gpu_ctx *ctx = m->ctx;
   if (replica < 0 || replica >= ctx->R) return HSMC_ERR_BAD_ARG;
-  NGrid g, g1;
-  int st = build_ngrid_pair(ctx, replica, kDescCut, 1.0 + 1e-9, g, g1);
-  if (st) return st;
   const Vox vx = make_vox(ctx->reps[replica], voxel);
   if (vx.V > (1L << 31) - 1) return HSMC_ERR_NOT_SUPPORTED;
+  NGrid g1;
+  auto grids = [&](NGrid *g) { return build_ngrid_pair(ctx, replica, kDescCut, 1.0 + 1e-9, *g, g1); };
   float *f = (float *)scratch(ctx, L_F, sizeof(float) * (size_t)vx.V);
-  double *acc = (double *)scratch(ctx, L_ACC, sizeof(double) * 2);
   const long nblk_ins = (long)((n + 255) / 256);
-  double *part = (double *)scratch(ctx, L_PART, sizeof(double) * (size_t)nblk_ins);
-  if (!f || !acc || !part) return HSMC_ERR_NO_MEMORY;
+  double *part = (double *)scratch(ctx, L_PART, (sizeof(double) + sizeof(unsigned int)) * (size_t)nblk_ins);
+  if (!f || !part) return HSMC_ERR_NO_MEMORY;
+  unsigned int *hpart = (unsigned int *)(part + nblk_ins);
   const bool scores_ok = m->sc_replica == replica && m->sc_version == ctx->version &&
                          m->sc_step == m->step && m->sc_voxel == voxel &&
                          m->sc_stamp == ctx->score_stamp;
   Proposal pr;
-  if (!scores_ok) {
-    st = launch_proposal_scores(ctx, replica, g, vx, m->net, f, &pr);
+  int st = HSMC_OK;
+  if (scores_ok) {
+    NGrid g;
+    st = grids(&g);
+    if (st) return st;
+  } else {
+    st = launch_proposal_scores(ctx, replica, grids, vx, m->net, f, &pr);
     if (st) return st;
     m->sc_replica = replica;
     m->sc_version = ctx->version;
@@ -1672,11 +1738,17 @@ int hsmc_gpu_widom_learned(hsmc_gpu_mlp *m, int replica, double voxel, double mi
   double *bsum = (double *)scratch(ctx, L_BSUM, sizeof(double) * (size_t)(ncdf + 1));
   if (!cdf || !bsum) return HSMC_ERR_NO_MEMORY;
   if (m->sc_mix != mix && nfree > 0) {
-    hipLaunchKernelGGL(k_cdf_local, dim3((unsigned)ncdf), dim3(1024), 0, ctx->stream, f, list,
-                       nfree, stats, mix, cdf, bsum);
-    hipLaunchKernelGGL(k_cdf_blocks, dim3(1), dim3(1024), 0, ctx->stream, bsum, (int)ncdf);
-    hipLaunchKernelGGL(k_cdf_add, dim3((unsigned)((nfree + 255) / 256)), dim3(256), 0, ctx->stream,
-                       cdf, nfree, bsum);
+    hipLaunchKernelGGL(k_cdf_local, dim3((unsigned)ncdf), dim3(1024), 0, ctx->stream, f, list, nfree,
+                       pr.parts, pr.nparts, stats, mix, cdf, bsum);
+    const dim3 add_blocks((unsigned)((nfree + 255) / 256));
+    if (ncdf <= kScanWave) {
+      hipLaunchKernelGGL(k_cdf_add<true>, add_blocks, dim3(256), 0, ctx->stream, cdf, nfree, bsum, (int)ncdf,
+                         bsum + ncdf);
+    } else {
+      hipLaunchKernelGGL(k_cdf_blocks, dim3(1), dim3(1024), 0, ctx->stream, bsum, (int)ncdf);
+      hipLaunchKernelGGL(k_cdf_add<false>, add_blocks, dim3(256), 0, ctx->stream, cdf, nfree, bsum, (int)ncdf,
+                         bsum + ncdf);
+    }
     HSMC_HIP(ctx, hipGetLastError());
   }
   if (m->sc_mix != mix) {
@@ -1690,19 +1762,15 @@ int hsmc_gpu_widom_learned(hsmc_gpu_mlp *m, int replica, double voxel, double mi
   philox4x32_10(0u, 0u, (uint32_t)sample, 0x4C530000u | (uint32_t)((sample >> 32) & 0xFFFFu),
                 (uint32_t)seed, (uint32_t)(seed >> 32), u);
   const double u0 = (double)u[0] * 0x1p-32;
-  HSMC_HIP(ctx, hipMemsetAsync(acc, 0, sizeof(double) * 2, ctx->stream));
   hipLaunchKernelGGL(k_insert, dim3((unsigned)nblk_ins), dim3(256), 0, ctx->stream, g1, vx,
                      cdf, list, nfree, total, (long)n, u0, f, flag, stats, mix,
-                     (uint32_t)seed, (uint32_t)(seed >> 32), (unsigned long long)sample, part,
-                     reinterpret_cast<unsigned long long *>(acc + 1));
-  hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, ctx->stream, part, nblk_ins, acc);
+                     (uint32_t)seed, (uint32_t)(seed >> 32), (unsigned long long)sample, part, hpart);
+  hipLaunchKernelGGL(k_sum_fixed, dim3(1), dim3(256), 0, ctx->stream, part, hpart, nblk_ins, ctx->h_acc);
   HSMC_HIP(ctx, hipGetLastError());
-  double ha[2] = {0, 0};
-  HSMC_HIP(ctx, hipMemcpyAsync(ha, acc, sizeof(double) * 2, hipMemcpyDeviceToHost, ctx->stream));
   HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  *estimate = ha[0];
+  *estimate = __builtin_bit_cast(double, ctx->h_acc[0]);
   if (n_done) *n_done = n;
-  if (hits) *hits = (int64_t)__builtin_bit_cast(unsigned long long, ha[1]);
+  if (hits) *hits = (int64_t)ctx->h_acc[1];
   return HSMC_OK;
 }
 
@@ -1742,16 +1810,14 @@ int hsmc_gpu_proposal_scores(hsmc_gpu_mlp *m, int replica, double voxel, float *
   if (!scores) return HSMC_OK;
   if (cap < vx.V) return HSMC_ERR_BAD_ARG;
   if (vx.V > (1L << 31) - 1) return HSMC_ERR_NOT_SUPPORTED;
-  NGrid g;
-  int st = build_ngrid(ctx, replica, kDescCut, L_GRID_A, g);
-  if (st) return st;
   float *f = (float *)scratch(ctx, L_F, sizeof(float) * (size_t)vx.V);
   if (!f) return HSMC_ERR_NO_MEMORY;
   // the shared score buffer is overwritten: no network's cache stays valid
   ++ctx->score_stamp;
   m->sc_replica = -1;
   Proposal pr;
-  st = launch_proposal_scores(ctx, replica, g, vx, m->net, f, &pr);
+  int st = launch_proposal_scores(
+      ctx, replica, [&](NGrid *g) { return build_ngrid(ctx, replica, kDescCut, L_GRID_A, *g); }, vx, m->net, f, &pr);
   if (st) return st;
   hipLaunchKernelGGL(k_mask_blocked, dim3((unsigned)((vx.V + 255) / 256)), dim3(256), 0,
                      ctx->stream, f, pr.flag, vx.V);

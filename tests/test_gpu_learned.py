@@ -146,6 +146,27 @@ def test_systematic_sampler_weights():
     assert r["n"] == 54321 and r["hits"] > 0
 
 
+@pytest.mark.parametrize("m", [8, 20, 64, 66])
+def test_cumulative_mass_over_few_and_many_blocks(m):
+    """The cumulative mass in 1, 2, 64 and about 70 blocks of 4096 voxels (up to 64
+    are scanned by the adding kernel itself, more by a kernel of their own):
+    three spheres in a box of edge 20 leave P_ins = 1 - 3 (4 pi / 3) / 20^3.
+    A weight is at most 1 / (1 - mix) = 10, so its variance is at most 10 and
+    the estimate's deviation sqrt(10 / n).  A mix changed on kept scores gives
+    the same estimate as on fresh ones."""
+    L, n = 20.0, 200000
+    ctx = gpu.Context([dict(n=3, box=(L, L, L), dr_max=0.1, seed=4)])
+    ctx.upload(np.array([[0, 3.0, 3.0, 3.0], [1, 10.0, 12.0, 9.0], [2, 17.0, 5.0, 16.0]]))
+    net = gpu.Mlp(ctx, seed=6)
+    got = net.widom(L / m, 0.9, 8, 0, n)
+    want = 1.0 - 3 * (4.0 * math.pi / 3.0) / L ** 3
+    assert abs(got["estimate"] - want) <= 5.0 * math.sqrt(10.0 / n)
+    kept = net.widom(L / m, 0.5, 8, 1, n)
+    fresh = gpu.Mlp(ctx, seed=6).widom(L / m, 0.5, 8, 1, n)
+    assert kept["estimate"] == fresh["estimate"] and kept["hits"] == fresh["hits"]
+    ctx.close()
+
+
 @pytest.mark.parametrize("n,rho", [(10, 0.8), (3, 0.6)])
 def test_voxel_scores_match_point_path(n, rho):
     """Voxel scores (tiled kernel for the N = 4000 box of edge 17.1, per-voxel
