@@ -159,7 +159,7 @@ __global__ void k_grid_scatter(const double *__restrict__ x, const double *__res
   if (i >= n) return;
   const int2 c = cellof[i];
   const int pos = start[c.x] + c.y;
-  ids[pos] = i;
+  if (ids) ids[pos] = i;
   px[pos] = x[i];
   py[pos] = y[i];
   pz[pos] = z[i];
@@ -1047,13 +1047,30 @@ bool cells_at_least(const hsmc_gpu_replica &p, double side, int n) {
          grid_cells_for(p.lz, side) >= n;
 }
 
-// First double at which the monotone condition holds, from a guess a few
-// units in the last place away.
+// First non-negative double at which the monotone condition holds (infinity
+// if it holds nowhere), from a guess: usually a few units in the last place
+// away, but the bound between "-1" and "above" of a bin width near 1 lies
+// anywhere, so the steps double until they pass it and halve from there.
 template <class Cond>
 double first_double(double guess, Cond &&holds) {
-  while (guess > 0.0 && holds(guess)) guess = nextafter(guess, 0.0);
-  while (!holds(guess)) guess = nextafter(guess, INFINITY);
-  return guess;
+  constexpr long long kInf = 0x7ff0000000000000LL;
+  auto at = [&](long long bits) { return holds(__builtin_bit_cast(double, bits)); };
+  long long lo = -1, hi = kInf;  // it holds not at lo (below every double) and at hi, or nowhere
+  const long long g = std::min(__builtin_bit_cast(long long, guess), kInf);
+  for (long long step = 1, p = g; step > 0 && p > lo && p < hi; step *= 2) {
+    if (at(p)) {
+      hi = p;
+      p = g - step;
+    } else {
+      lo = p;
+      p = step < kInf - g ? g + step : kInf;
+    }
+  }
+  while (hi - lo > 1) {
+    const long long mid = lo + (hi - lo) / 2;
+    (at(mid) ? hi : lo) = mid;
+  }
+  return __builtin_bit_cast(double, hi);
 }
 
 // Edges of the bins (int)((dr - 1.0) / dr_bin) in squared distance, on the
@@ -1091,10 +1108,11 @@ __global__ void k_zero_words(unsigned int *__restrict__ p, long n) {
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Workspace layout of the scan: counts and starts of the grid's C cells, cell
-// (and place in it) and id of the N spheres, their sorted positions and
-// the workgroups' result masks, each region 256-B aligned.
+// (and place in it) of the N spheres and their sorted positions, each region
+// 256-B aligned; 32 bytes a sphere and 8 a cell.  The workgroups' result masks
+// lie over the cells, which are read no more once the spheres are sorted.
 struct ScanLayout {
-  size_t cnt, start, cellof, ids, px, py, pz, mask, part, bytes;
+  size_t cnt, start, cellof, px, py, pz, part, bytes;
 };
 
 ScanLayout scan_layout(long N, long C) {
@@ -1108,11 +1126,9 @@ ScanLayout scan_layout(long N, long C) {
   l.cnt = take(sizeof(int) * C);
   l.start = take(sizeof(int) * (C + 1));
   l.cellof = take(sizeof(int2) * N);
-  l.ids = take(sizeof(int) * N);
   l.px = take(sizeof(double) * N);
   l.py = take(sizeof(double) * N);
   l.pz = take(sizeof(double) * N);
-  l.mask = take(sizeof(unsigned long long) * ((N + 255) / 256));  // one per workgroup
   l.part = take(sizeof(int) * scan_workspace_ints(C));
   l.bytes = o;
   return l;
@@ -1166,10 +1182,9 @@ int overlap_scan_in_workspace(hsmc_gpu_ctx *ctx, int replica, const double *sf, 
   }
   int *cnt = (int *)(ws + l.cnt), *start = (int *)(ws + l.start);
   int2 *cellof = (int2 *)(ws + l.cellof);
-  int *ids = (int *)(ws + l.ids);
   double *px = (double *)(ws + l.px), *py = (double *)(ws + l.py), *pz = (double *)(ws + l.pz);
-  unsigned long long *dmask = (unsigned long long *)(ws + l.mask);
-  g.start = start; g.ids = ids; g.px = px; g.py = py; g.pz = pz;
+  unsigned long long *dmask = (unsigned long long *)(ws + l.cellof);
+  g.start = start; g.ids = nullptr; g.px = px; g.py = py; g.pz = pz;
   const long zero_words = C;
   hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((zero_words + 255) / 256)), dim3(256), 0, ctx->stream,
                      (unsigned int *)cnt, zero_words);
@@ -1181,7 +1196,7 @@ int overlap_scan_in_workspace(hsmc_gpu_ctx *ctx, int replica, const double *sf, 
                      nz, g.ix, g.iy, g.iz, cnt, cellof);
   exclusive_scan(ctx->stream, cnt, (int)C, start, (int *)(ws + l.part), false);
   hipLaunchKernelGGL(k_grid_scatter, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, cellof,
-                     start, ids, px, py, pz);
+                     start, (int *)nullptr, px, py, pz);
   hipLaunchKernelGGL(k_scaled_spheres, dim3(blocks), dim3(256), 0, ctx->stream, g, N, t, n_sf,
                      cut * cut, dmask);
   hipLaunchKernelGGL(k_sum_all<true>, dim3(1), dim3(1024), 0, ctx->stream, dmask, (int)blocks,

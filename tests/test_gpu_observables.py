@@ -107,6 +107,20 @@ def test_histogram_bins_at_their_edges():
     ctx.close()
 
 
+@pytest.mark.parametrize("dr_bin", [5e-324, 1e-9, 1.0 - 1e-12, 1.0, 1.0 + 1e-12, 1e300, math.inf])
+def test_histogram_of_extreme_bin_widths(dr_bin):
+    """Widths at which the bins' edges fall together, onto zero or nowhere."""
+    rng = np.random.default_rng(12)
+    box = np.array([8.0, 8.0, 8.0])
+    xyz = np.vstack([rng.random((60, 3)) * box, [[1.0, 1.0, 1.0], [1.0, 1.0, 2.0], [1.0, 1.0, 1.0]]])
+    i, j, s = _near_pairs(xyz, box, 3.0)
+    ctx = _context(xyz, box)
+    want = _histogram(s, dr_bin, 40, 2.9)
+    got = ctx.rdf_counts(dr_bin, 40, 2.9)
+    assert np.array_equal(got[0], want[0]) and got[1] == want[1]
+    ctx.close()
+
+
 @pytest.mark.parametrize("shape,drop", [((4, 4, 4), 1), ((8, 8, 16), 0), ((16, 16, 16), 0),
                                         ((16, 16, 17), 5), ((16, 16, 20), 0), ((16, 16, 21), 3),
                                         ((4, 45, 50), 2), ((6, 38, 40), 7)])
