@@ -518,29 +518,99 @@ k_point_descriptors(NGrid g, const double *__restrict__ q, int m, float far2,
   for (int k = 0; k < NIN; ++k) out[(size_t)i * NIN + k] = d[k];
 }
 
-// Training rows from uniform points of Philox stream (key, sample): input =
-// descriptor of the voxel holding the point, target = -beta * max(0, 1 - d).
+__device__ __forceinline__ int cell_of(const NGrid &g, double x, double y, double z) {
+  return (search_cell(x, g.ix, g.nx) * g.ny + search_cell(y, g.iy, g.ny)) * g.nz + search_cell(z, g.iz, g.nz);
+}
+
+// Uniform point i of Philox stream (key, sample), and the centre of the voxel
+// that holds it.
+struct TrainingPoints {
+  uint32_t k0, k1;
+  unsigned long long sample;
+  __device__ __forceinline__ void operator()(const NGrid &g, const Vox &vx, long long i, double q[3],
+                                             double c[3]) const {
+    uint32_t u[4];
+    philox4x32_10((uint32_t)i, (uint32_t)((unsigned long long)i >> 32), (uint32_t)sample,
+                  0x57490000u | (uint32_t)((sample >> 32) & 0xFFFFu), k0, k1, u);
+    q[0] = u32_unit_closed(u[0]) * g.lx;
+    q[1] = u32_unit_closed(u[1]) * g.ly;
+    q[2] = u32_unit_closed(u[2]) * g.lz;
+    int ix = (int)(q[0] / vx.vx), iy = (int)(q[1] / vx.vy), iz = (int)(q[2] / vx.vz);
+    ix = min(ix, vx.mx - 1);
+    iy = min(iy, vx.my - 1);
+    iz = min(iz, vx.mz - 1);
+    const long v = ((long)ix * vx.my + iy) * vx.mz + iz;
+    voxel_centre(vx, v, c[0], c[1], c[2]);
+  }
+};
+
+// Points are worked on in the order of their voxels' cells, so that a wave
+// reads the spheres of one or two cells instead of 64 cells' (each of these
+// scattered lines takes the compute unit's address path a cycle, which
+// bounded the rows).  The rows stay where they were: only which lane makes
+// which row changes.  rank[i] = place of point i among its cell's; cnt = the
+// cells' counts.  Up to kLdsCells cells a workgroup counts its points in LDS
+// first: on a grid of few cells its one addition a cell takes the place of
+// hundreds to the same few words.
+constexpr int kLdsCells = 8192;
+constexpr int kSortThreads = 1024;
+
+template <bool LDS>
+__global__ void __launch_bounds__(kSortThreads)
+k_training_count(NGrid g, Vox vx, TrainingPoints point, long long first, int n, int *__restrict__ cnt,
+                 int *__restrict__ rank) {
+  __shared__ int own[LDS ? kLdsCells : 1];
+  const int i = blockIdx.x * kSortThreads + threadIdx.x;
+  const int C = g.nx * g.ny * g.nz;
+  if constexpr (LDS) {
+    for (int c = threadIdx.x; c < C; c += kSortThreads) own[c] = 0;
+    __syncthreads();
+  }
+  int cell = 0, r = 0;
+  if (i < n) {
+    double q[3], c[3];
+    point(g, vx, first + i, q, c);
+    cell = cell_of(g, c[0], c[1], c[2]);
+    r = atomicAdd(LDS ? &own[cell] : &cnt[cell], 1);
+  }
+  if constexpr (LDS) {
+    __syncthreads();
+    for (int c = threadIdx.x; c < C; c += kSortThreads) {
+      const int k = own[c];
+      if (k) own[c] = atomicAdd(&cnt[c], k);
+    }
+    __syncthreads();
+    r += own[cell];
+  }
+  if (i < n) rank[i] = r;
+}
+
 __global__ void __launch_bounds__(256)
-k_training_rows(NGrid g, Vox vx, uint32_t k0, uint32_t k1, unsigned long long sample, long long n,
-                float far2, float beta, float *__restrict__ X, float *__restrict__ T) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+k_training_order(NGrid g, Vox vx, TrainingPoints point, long long first, int n,
+                 const int *__restrict__ start, const int *__restrict__ rank, int *__restrict__ order) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  uint32_t u[4];
-  philox4x32_10((uint32_t)i, (uint32_t)((unsigned long long)i >> 32), (uint32_t)sample,
-                0x57490000u | (uint32_t)((sample >> 32) & 0xFFFFu), k0, k1, u);
-  const double qx = u32_unit_closed(u[0]) * g.lx, qy = u32_unit_closed(u[1]) * g.ly,
-               qz = u32_unit_closed(u[2]) * g.lz;
-  const float dmin = sqrtf(nearest1(g, qx, qy, qz, far2));
+  double q[3], c[3];
+  point(g, vx, first + i, q, c);
+  order[start[cell_of(g, c[0], c[1], c[2])] + rank[i]] = i;
+}
+
+// Training rows of points first .. first + n - 1, in the given order (any
+// without one): input = descriptor of the voxel holding the point, target
+// = -beta * max(0, 1 - d).
+__global__ void __launch_bounds__(256)
+k_training_rows(NGrid g, Vox vx, TrainingPoints point, long long first, long long n,
+                const int *__restrict__ order, float far2, float beta, float *__restrict__ X,
+                float *__restrict__ T) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const long long i = first + (order ? order[t] : t);
+  double q[3], c[3];
+  point(g, vx, i, q, c);
+  const float dmin = sqrtf(nearest1(g, q[0], q[1], q[2], far2));
   T[i] = -beta * fmaxf(0.f, 1.f - dmin);
-  int ix = (int)(qx / vx.vx), iy = (int)(qy / vx.vy), iz = (int)(qz / vx.vz);
-  ix = min(ix, vx.mx - 1);
-  iy = min(iy, vx.my - 1);
-  iz = min(iz, vx.mz - 1);
-  const long v = ((long)ix * vx.my + iy) * vx.mz + iz;
-  double cx, cy, cz;
-  voxel_centre(vx, v, cx, cy, cz);
   float d[NIN];
-  descriptor(g, cx, cy, cz, far2, d);
+  descriptor(g, c[0], c[1], c[2], far2, d);
   for (int k = 0; k < NIN; ++k) X[(size_t)i * NIN + k] = d[k];
 }
 
@@ -1249,11 +1319,12 @@ int grid_cells_for2(double L, double cut) {
 // ctx.hip 21..22, sweep.hip 23): descriptor grid 24..26, the insertion call's
 // descriptor and overlap grids built together 27..29,
 // rows / scores 30, targets / block partials 31, cumulative mass 32, gradient
-// sums of the training workgroups 33, per-block insertion weights and hits 35, cumulative-mass block sums 36,
+// sums of the training workgroups 33, order of the training points 34,
+// per-block insertion weights and hits 35, cumulative-mass block sums 36,
 // grid-scan partials 37, voxel scores 38, score block reductions 39,
 // free-voxel tile slots and list 40, tile counts, offsets and scan space 41,
 // blocked-voxel flags 42, softmax statistics 43.
-enum { L_GRID_A = 24, L_GRID_PAIR = 27, L_X = 30, L_T = 31, L_CDF = 32, L_GRAD = 33, L_PART = 35,
+enum { L_GRID_A = 24, L_GRID_PAIR = 27, L_X = 30, L_T = 31, L_CDF = 32, L_GRAD = 33, L_ORDER = 34, L_PART = 35,
        L_BSUM = 36, L_SCANP = 37, L_F = 38, L_FRED = 39, L_LIST = 40, L_NFREE = 41, L_FLAG = 42,
        L_STATS = 43 };
 
@@ -1347,6 +1418,47 @@ int build_ngrid(hsmc_gpu_ctx *ctx, int replica, double cut, int slot0, NGrid &g)
   ctx->ngrid_replica[which] = replica;
   ctx->ngrid_version[which] = ctx->version;
   ctx->ngrid_cut[which] = cut;
+  return HSMC_OK;
+}
+
+// The rows of n points.  From kSortRows points on, and at least one for each
+// cell, in the order of their cells, kSortChunk points at a time (which bounds
+// the workspace); their ranks lie where their targets will be.  A call with
+// one pass over n points at N = 4000, unsorted and sorted: 2^15 points 104 and
+// 118 us (the sort's three launches), 2^17 273 and 163, 2^20 1911 and 648; at
+// N = 32000 128 and 121, 378 and 173, 2794 and 700; at N = 108, where the few
+// cells' spheres stay in the first cache either way, 89 and 119, 154 and 162,
+// 788 and 628.
+constexpr long long kSortRows = 65536, kSortChunk = 1 << 20;
+
+int launch_training_rows(hsmc_gpu_ctx *ctx, const NGrid &g, const Vox &vx, const TrainingPoints &point,
+                         long long n, float far2, float beta, float *X, float *T) {
+  const long C = (long)g.nx * g.ny * g.nz;
+  if (n < kSortRows || C > n) {
+    hipLaunchKernelGGL(k_training_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, g, vx,
+                       point, 0LL, n, (const int *)nullptr, far2, beta, X, T);
+    HSMC_HIP(ctx, hipGetLastError());
+    return HSMC_OK;
+  }
+  const size_t chunk = (size_t)std::min(n, kSortChunk);
+  int *order = (int *)scratch(ctx, L_ORDER, sizeof(int) * (chunk + 2 * (size_t)C + 1 + (size_t)scan_workspace_ints(C)));
+  if (!order) return HSMC_ERR_NO_MEMORY;
+  int *cnt = order + chunk, *start = cnt + C, *part = start + C + 1;
+  for (long long first = 0; first < n; first += kSortChunk) {
+    const int m = (int)std::min(kSortChunk, n - first);
+    int *rank = (int *)T + first;
+    HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * C, ctx->stream));
+    hipLaunchKernelGGL(C <= kLdsCells ? k_training_count<true> : k_training_count<false>,
+                       dim3((unsigned)((m + kSortThreads - 1) / kSortThreads)), dim3(kSortThreads), 0, ctx->stream,
+                       g, vx, point, first, m, cnt, rank);
+    exclusive_scan(ctx->stream, cnt, (int)C, start, part, false);
+    const dim3 blocks((unsigned)((m + 255) / 256));
+    hipLaunchKernelGGL(k_training_order, blocks, dim3(256), 0, ctx->stream, g, vx, point, first, m, start, rank,
+                       order);
+    hipLaunchKernelGGL(k_training_rows, blocks, dim3(256), 0, ctx->stream, g, vx, point, first, (long long)m,
+                       order, far2, beta, X, T);
+    HSMC_HIP(ctx, hipGetLastError());
+  }
   return HSMC_OK;
 }
 
@@ -1659,10 +1771,9 @@ int hsmc_gpu_mlp_train(hsmc_gpu_mlp *m, int replica, double voxel, uint64_t seed
   float *X = (float *)scratch(ctx, L_X, sizeof(float) * NIN * (size_t)n_points);
   float *T = (float *)scratch(ctx, L_T, sizeof(float) * (size_t)n_points);
   if (!X || !T) return HSMC_ERR_NO_MEMORY;
-  hipLaunchKernelGGL(k_training_rows, dim3((unsigned)((n_points + 255) / 256)), dim3(256), 0,
-                     ctx->stream, g, vx, (uint32_t)seed, (uint32_t)(seed >> 32),
-                     (unsigned long long)sample, (long long)n_points, far2_of(g), beta, X, T);
-  HSMC_HIP(ctx, hipGetLastError());
+  st = launch_training_rows(ctx, g, vx, TrainingPoints{(uint32_t)seed, (uint32_t)(seed >> 32), sample},
+                            n_points, far2_of(g), beta, X, T);
+  if (st) return st;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const int gb = grad_blocks((int)std::min<int64_t>(batch, n_points));
   float *part = (float *)scratch(ctx, L_GRAD, sizeof(float) * kGradStride * gb);

@@ -146,6 +146,48 @@ def test_systematic_sampler_weights():
     assert r["n"] == 54321 and r["hits"] > 0
 
 
+def _uniform_points(seed, sample, n):
+    """Points 0..n-1 of the Philox4x32-10 stream (key, sample), in units of the
+    box: word / (2^32 - 1)."""
+    k0, k1 = seed & 0xFFFFFFFF, seed >> 32
+    i = np.arange(n, dtype=np.uint64)
+    c = [i & 0xFFFFFFFF, i >> 32, np.full(n, sample, np.uint64), np.full(n, 0x57490000, np.uint64)]
+    for _ in range(10):
+        a, b = c[0] * np.uint64(0xD2511F53), c[2] * np.uint64(0xCD9E8D57)
+        c = [(b >> 32) ^ c[1] ^ np.uint64(k0), b & 0xFFFFFFFF, (a >> 32) ^ c[3] ^ np.uint64(k1), a & 0xFFFFFFFF]
+        k0, k1 = (k0 + 0x9E3779B9) & 0xFFFFFFFF, (k1 + 0xBB67AE85) & 0xFFFFFFFF
+    return np.stack(c[:3], axis=1) / float(2 ** 32 - 1)
+
+
+@pytest.mark.parametrize("L,points", [(6.3, 65535), (6.3, 65536), (17.0, 70001), (32.0, 65536),
+                                      (17.0, (1 << 20) + 65)])
+def test_training_rows_in_any_order(L, points):
+    """Rows made point by point and in the order of their cells (from 65536
+    points on, 2^20 at a time), counted in LDS or, above 8192 cells (a box of
+    edge 32), in memory.  With a learning rate of 0 the loss is the mean of
+    (y - t)^2 over the rows; each y is within the forward pass's bound e of
+    the oracle's, so the loss is within mean(2 |y - t| e + e^2) and FP32 sums'
+    rounding, 1e-5 of it."""
+    rng = np.random.default_rng(3)
+    n = 400
+    conf = np.column_stack([np.arange(n), rng.random((n, 3)) * L])
+    ctx = gpu.Context([dict(n=n, box=(L, L, L), dr_max=0.1, seed=4)])
+    ctx.upload(conf)
+    net = gpu.Mlp(ctx, seed=6)
+    p = (rng.standard_normal(M.NPARAM) * 0.2).astype(np.float32)
+    net.set(p)
+    got = net.train(0.25, 5, 3, points, epochs=1, batch=8192, lr=0.0, beta=10.0)
+    u = _uniform_points(5, 3, points) * L
+    side = L / math.ceil(L / 0.25)
+    centre = (np.minimum(np.floor(u / side), math.ceil(L / 0.25) - 1) + 0.5) * side
+    t = -10.0 * np.maximum(0.0, -gpu.point_descriptors(ctx, u)[:, 0].astype(np.float64))
+    y, _ = M.forward(p.astype(np.float64), gpu.point_descriptors(ctx, centre).astype(np.float64), bf=True)
+    e = 2e-3 * max(1.0, np.max(np.abs(y)))
+    want = np.mean((y - t) ** 2)
+    assert abs(got - want) <= np.mean(2 * np.abs(y - t) * e + e * e) + 1e-5 * want
+    ctx.close()
+
+
 @pytest.mark.parametrize("m", [8, 20, 64, 66])
 def test_cumulative_mass_over_few_and_many_blocks(m):
     """The cumulative mass in 1, 2, 64 and about 70 blocks of 4096 voxels (up to 64
