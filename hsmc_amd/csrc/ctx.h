@@ -19,6 +19,7 @@
 //   aoff             int32[R+1]  prefix of active cells per phase, each
 //                                replica's range padded to a multiple of 8
 //   arep             int32[A]    replica owning each active cell
+//   bricks           Brick[...]  bricks of active cells (large contexts)
 //   sweep            uint64      sweeps done (read by every sweep kernel)
 //   cacc, cleft      uint32[C]   accepted moves / moves rejected for leaving
 //                                the cell, per sweep cell; each cell is
@@ -75,6 +76,12 @@ struct __attribute__((aligned(32))) SlotRec {
   int pad;
 };
 
+// A brick of one replica's active cells (bricks.hip): the first one's indices
+// along each axis (the same for every sublattice) and how many.
+struct Brick {
+  int r, x0, y0, z0, nx, ny, nz, pad;
+};
+
 struct RepHost {
   hsmc_gpu_replica p;
   int gx, gy, gz;
@@ -101,6 +108,10 @@ struct hsmc_gpu_ctx {
   int *d_arep = nullptr;  // replica of each active cell (Atot entries)
   size_t arep_alloc = 0;
   int lcap = 128;         // LDS candidate-list capacity of the phase kernel
+  // bricks of all replicas; none where the sweeps run cell by cell
+  hsmc::Brick *d_bricks = nullptr;
+  size_t brick_alloc = 0;
+  int n_bricks = 0;
   int *d_prep = nullptr;
   double *d_x = nullptr, *d_y = nullptr, *d_z = nullptr;
   int *d_cnt = nullptr;
@@ -216,6 +227,17 @@ struct ResidentShape {
 };
 bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape);
 int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, unsigned long long base, int n);
+// Brick phases (bricks.hip): the bricks of the present layout, whether the
+// context's launched sweeps run that way, and one phase of them.
+// From kBrickCells active cells of all replicas on: a sweep by bricks and cell
+// by cell takes 110 and 47 us at 4000 active cells, 122 and 73 at 14000, 135
+// and 139 at 33000 (8 replicas of N = 32000), 138 and 136 at 36000 (one of
+// N = 256000, whose cell phases file the next sweep), 207 and 246 at 70000,
+// 253 and 557 at 187000.
+constexpr long kBrickCells = 40000;
+int build_bricks(hsmc_gpu_ctx *ctx);
+bool bricks_run(const hsmc_gpu_ctx *ctx);
+void enqueue_brick_phase(hsmc_gpu_ctx *ctx, int phase, int k, hipStream_t s);
 // File the current by-id positions into the cell slots of the last sweep's
 // grid (the cell list the volume-move scan reads after positions changed).
 int rebin_last_sweep(hsmc_gpu_ctx *ctx);

@@ -280,6 +280,10 @@ int layout(hsmc_gpu_ctx *ctx) {
     ctx->cell_alloc = alloc;
     ctx->cap = cap;
   }
+  {
+    int st = build_bricks(ctx);
+    if (st) return st;
+  }
   // keep the phase kernel's LDS staging within 64 KiB per workgroup
   {
     while (ctx->tune.cells_per_block > 1 &&
@@ -499,7 +503,7 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
   if (!ctx) return HSMC_OK;
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   drop_graph(ctx);
-  void *bufs[] = {ctx->d_reps, ctx->d_swp, ctx->d_aoff, ctx->d_arep, ctx->d_prep, ctx->d_x, ctx->d_y, ctx->d_z,
+  void *bufs[] = {ctx->d_reps, ctx->d_swp, ctx->d_aoff, ctx->d_arep, ctx->d_bricks, ctx->d_prep, ctx->d_x, ctx->d_y, ctx->d_z,
                   ctx->d_cnt, ctx->d_slot, ctx->d_sweep,
                   ctx->d_cacc, ctx->d_cleft, ctx->d_err, ctx->d_bar};
   for (void *b : bufs)

@@ -14,6 +14,9 @@
 //      (moves.c:52-54), wrapped by apply_pbc (moves.c:215-226) and tested
 //      for overlap with every other sphere in the 27 neighbouring cells with
 //      the reference's FP64 arithmetic (moves.c:400-431).
+// Contexts of many active cells run the phases by bricks of cells (bricks.hip)
+// with the same results; small replicas run whole sweeps in one launch
+// (resident.hip).
 // With one replica, the sweeps of a batch after the first are chained: the
 // last phase of each sweep files every sphere into the next sweep's shifted
 // grid (at its final position), so those sweeps need no k_rebin, and the
@@ -35,18 +38,6 @@
 using namespace hsmc;
 
 namespace {
-
-// Vector store at agent scope: written through the XCD's L2 (the next
-// phase's workgroups read it from other XCDs).
-__device__ __forceinline__ void store_through(double *p, double v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Work item i of a sweep's rebin: clear cell i of the next sweep's count
 // buffer, file particle i into its cell of the shifted grid, and draw
@@ -810,6 +801,14 @@ void enqueue_sweep(hsmc_gpu_ctx *ctx, int k, hipStream_t s, hipEvent_t *phase_ev
                        ctx->rep0, ctx->d_swp, ctx->R, kt, nsw, ctx->d_prep, (int)ctx->Ptot,
                        (int)ctx->Ctot, ctx->d_x, ctx->d_y, ctx->d_z, ctx->d_cnt, ctx->d_slot,
                        ctx->cap, ctx->d_sweep, k, ctx->d_err);
+  if (bricks_run(ctx)) {
+    for (int p = 0; p < 8; ++p) {
+      if (phase_events && p == 0) (void)hipEventRecord(phase_events[0], s);
+      enqueue_brick_phase(ctx, p, k, s);
+      if (phase_events && p == 7) (void)hipEventRecord(phase_events[15], s);
+    }
+    return;
+  }
   const int lpc = ctx->tune.lanes_per_cell, cpb = ctx->tune.cells_per_block;
   const int bs = lpc * cpb;
   const unsigned blocks = (unsigned)((ctx->Atot + cpb - 1) / cpb);
@@ -833,7 +832,7 @@ void enqueue_sweep(hsmc_gpu_ctx *ctx, int k, hipStream_t s, hipEvent_t *phase_ev
 bool can_chain(const hsmc_gpu_ctx *ctx) {
   const int lpc = ctx->tune.lanes_per_cell, cpb = ctx->tune.cells_per_block;
   const long lanes = (ctx->Atot + cpb - 1) / cpb * lpc * cpb;
-  return ctx->R == 1 && lanes >= ctx->Ctot && lanes >= ctx->Ptot;
+  return ctx->R == 1 && !bricks_run(ctx) && lanes >= ctx->Ctot && lanes >= ctx->Ptot;
 }
 
 // Capture K sweeps (and the counter advance) into one graph: the main graph
@@ -1161,13 +1160,15 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
   const bool start_set = ctx->tune_set;
   hsmc_gpu_tuning winner = start;
   float best_ms = 1e30f;
-  // the resident kernel, where the replicas fit it, stands beside the launch
-  // shapes; when it wins the tuning stays as it was and is not in force
-  bool resident = false;
+  // the resident kernel or the bricks, where the context has them, stand
+  // beside the launch shapes; when they win the tuning stays as it was and is
+  // not in force
+  bool own_route = false;
   {
     ResidentShape shape;
-    if (resident_shape(ctx, &shape)) {
-      ctx->tune_set = false;
+    ctx->tune_set = false;
+    if (resident_shape(ctx, &shape) || bricks_run(ctx)) {
+      drop_graph(ctx);
       float ms = 0.f;
       int st = hsmc_gpu_time_sweeps(ctx, std::max(2, sweeps_per_trial / 4), &ms);
       if (st == HSMC_OK) st = hsmc_gpu_time_sweeps(ctx, sweeps_per_trial, &ms);
@@ -1176,7 +1177,7 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
         return st;
       }
       best_ms = ms;
-      resident = true;
+      own_route = true;
     }
   }
   ctx->tune_set = true;
@@ -1202,11 +1203,11 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
         if (ms < best_ms) {
           best_ms = ms;
           winner = t;
-          resident = false;
+          own_route = false;
         }
       }
   ctx->tune = winner;
-  ctx->tune_set = !resident;
+  ctx->tune_set = !own_route;
   drop_graph(ctx);
   HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_x, save, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
   HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_y, save + P, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
