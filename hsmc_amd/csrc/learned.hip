@@ -788,16 +788,18 @@ k_voxel_scores_tiled(NGrid g, Vox vx, float far2, double smin, const MlpDev *__r
 // written for free voxels only; the flags tell the others apart.
 struct Box3 {
   double lx, ly, lz;
+  double ux, uy, uz;  // voxels per unit length
 };
 
 // First candidate voxel index for centres (i + 0.5) * v within r of p: the
 // centres within r have i in the open interval (x, x + 2r/v) with
 // x = (p - r)/v - 0.5, and the 8 indices from floor(x - 1e-9) cover it when
 // 2r/v + 1 < 8 - 1e-6 (the host checks; 6.27 for voxels of edge 0.25), also
-// where rounding puts x on the other side of an integer.  The distance test
-// then decides each candidate.
-__device__ __forceinline__ int voxel_first(double p, double r, double v) {
-  return (int)floor((p - r) / v - 0.5 - 1e-9);
+// where rounding, of 1/v too, puts x on the other side of an integer.  The
+// distance test then decides each candidate.  (Three divisions a sphere were
+// a third of the kernel's instructions, which bound it: 42 us for N = 108000.)
+__device__ __forceinline__ int voxel_first(double p, double r, double per_unit) {
+  return (int)floor((p - r) * per_unit - 0.5 - 1e-9);
 }
 
 __device__ __forceinline__ int wrap_voxel(int i, int m) {
@@ -820,8 +822,7 @@ k_mark_blocked(const double *__restrict__ x, const double *__restrict__ y,
   const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (p >= N) return;  // the whole wave
   const double px = x[p], py = y[p], pz = z[p];
-  const int lx = voxel_first(px, r, vx.vx), ly = voxel_first(py, r, vx.vy),
-            lz = voxel_first(pz, r, vx.vz);
+  const int lx = voxel_first(px, r, b.ux), ly = voxel_first(py, r, b.uy), lz = voxel_first(pz, r, b.uz);
   const double r2 = r * r;
   // 8 x 8 x 8 candidates: lane's (y, z) column, 8 x-layers.  The squared
   // distance is compute_dist's (dx^2 + dy^2) + dz^2 with the minimum image
@@ -1585,7 +1586,7 @@ int launch_proposal_scores(hsmc_gpu_ctx *ctx, int replica, MakeGrid &&grid, cons
   int *off = cnt + tiles;
   int *part = off + tiles + 1;
   const int N = rh.p.n_part;
-  Box3 b3{rh.p.lx, rh.p.ly, rh.p.lz};
+  Box3 b3{rh.p.lx, rh.p.ly, rh.p.lz, 1.0 / vx.vx, 1.0 / vx.vy, 1.0 / vx.vz};
   hipLaunchKernelGGL(k_mark_blocked, dim3((unsigned)((N + 3) / 4)), dim3(256), 0, ctx->stream,
                      ctx->d_x + rh.poff, ctx->d_y + rh.poff, ctx->d_z + rh.poff, N, vx, b3, r, flag);
   hipLaunchKernelGGL(k_free_tiles, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, ctx->stream, vx,

@@ -101,9 +101,9 @@ __global__ void __launch_bounds__(1024) k_scan1(int *__restrict__ cnt, int n, in
 // offset.  Three short launches in place of one workgroup walking the whole
 // array.
 constexpr int kScanTile = 4096;
-// Up to here k_scan1 alone: one pass over n entries takes 3 us, the three
-// launches 9 us.
-constexpr int kScanOne = 32 * 1024;
+// Up to here k_scan1 alone: 3 us for up to 2000 entries, 5 for 5500, 8 for
+// 11700, 16 for 16000 and 25 for 31000, against 9 to 11 for the three launches.
+constexpr int kScanOne = 12 * 1024;
 
 template <bool CLEAR>
 __global__ void __launch_bounds__(256) k_scan_tile(int *__restrict__ in, int n,
