@@ -468,107 +468,181 @@ k_widom_uniform_lds(Grid gg, int N, const double *__restrict__ x, const double *
 // One wave per cell: lanes j < 27 read the neighbour cells' ranges, and the
 // spheres of the 27 cells are staged once in LDS in the order own cell, 6
 // faces, 12 edges, 8 corners (the likeliest overlaps first).  The wave then
-// takes 64 points at a time, one per lane, and walks the list in lockstep
-// (every lane reads entry e together: an LDS broadcast) with the
-// reference's FP64 distance (moves.c:400-431 order, minimum image), leaving
-// the walk as soon as a ballot shows every point overlapping.
+// takes 128 points at a time, two to a lane, and walks the list in lockstep
+// (every lane reads entry e together: an LDS broadcast), leaving the walk as
+// soon as a ballot shows every point overlapping.
+//
+// Bounded by instructions: per cell the points' draws (20 32 x 32-bit
+// products each) and 26 tests of up to 128 points.  The list therefore holds
+// positions relative to the cell, image applied, in FP32: a test is 6.5
+// instructions and one 16-byte read, where the FP64 one is 9 (or 15 with the
+// minimum image) and three reads.  A smallest squared distance within
+// kWidomBand of 1 is decided again by the reference's FP64 arithmetic
+// (moves.c:400-431 order, minimum image) on the FP64 positions, so every
+// decision is the FP64 one: cells are less than 2 wide (floor(L) of them), so
+// a sphere less than 2 away lies within 4 of the cell's corner, each
+// coordinate within 3e-7 of its value, a difference within 7e-7 and the
+// squared distance within 3e-6 of its own near 1.  Axes of fewer than 3 cells,
+// where a neighbour cell's image depends on the point, take the FP64 test.
+// A call of 10^7 insertions at N = 108000 on a grid that is there: 82 us, 100
+// with FP64 tests, 139 with 64-bit cell arithmetic and a wave's set-up for
+// every cell besides (6144 workgroups take several cells a wave; 2048 of them
+// 84 us, a wave for each cell 103); 1000 a cell at N = 4000 39, 68 and 67.
 constexpr int kWidomCellsLcap = 256;   // bound of spheres in a 27-cell stencil (host-checked)
 constexpr int kWidomCellsWaves = 4;    // waves per workgroup
-constexpr int kWidomCellsBlocks = 1 << 16;
+constexpr int kWidomCellsBlocks = 6144;
+constexpr float kWidomBand = 1e-5f;
 
+template <bool FAST>
 __global__ void __launch_bounds__(64 * kWidomCellsWaves)
 k_widom_cells(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, int per_cell,
               unsigned long long *__restrict__ part, unsigned *__restrict__ err) {
-  __shared__ double sx_[kWidomCellsWaves][kWidomCellsLcap];
-  __shared__ double sy_[kWidomCellsWaves][kWidomCellsLcap];
-  __shared__ double sz_[kWidomCellsWaves][kWidomCellsLcap];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  double *Lx = sx_[w], *Ly = sy_[w], *Lz = sz_[w];
-  const long C = (long)g.nx * g.ny * g.nz;
+  __shared__ float4 list[FAST ? kWidomCellsWaves : 1][FAST ? kWidomCellsLcap : 1];
+  __shared__ double exact[FAST ? 1 : kWidomCellsWaves][3][FAST ? 1 : kWidomCellsLcap];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int C = g.nx * g.ny * g.nz;  // at most 2^28 (build_grid)
+  int dx = 0, dy = 0, dz = 0;        // lane < 27: its neighbour cell (distinct cells only)
+  if (lane < 27) stencil_by_distance(lane, dx, dy, dz);
+  const bool near = lane < 27 && stencil_axis_ok(dx, g.nx) && stencil_axis_ok(dy, g.ny) && stencil_axis_ok(dz, g.nz);
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
   const uint32_t c3 = 0x57430000u | (uint32_t)((sample >> 32) & 0xFFFFu);
+  const float sfx = (float)(g.sx * 0x1p-32), sfy = (float)(g.sy * 0x1p-32), sfz = (float)(g.sz * 0x1p-32);
   unsigned long long h = 0;
-  for (long c = (long)blockIdx.x * kWidomCellsWaves + w; c < C; c += (long)gridDim.x * kWidomCellsWaves) {
-    const int iz = (int)(c % g.nz);
-    const long t2 = c / g.nz;
-    const int iy = (int)(t2 % g.ny), ix = (int)(t2 / g.ny);
-    // A cell with every index in [1, g - 2] and its neighbours hold positions
-    // and points within 2 sides of each other, under half the box when
-    // g >= 8: compute_dist's minimum image (moves.c:414-427) changes no
-    // difference there and is left out (the same FP64 operations remain).
-    // The cell is the wave's, so the choice is uniform.
-    const bool inner = g.nx >= 8 && g.ny >= 8 && g.nz >= 8 && ix >= 1 && ix <= g.nx - 2 &&
-                       iy >= 1 && iy <= g.ny - 2 && iz >= 1 && iz <= g.nz - 2;
-    // neighbour ranges (distinct cells only on axes of fewer than 3 cells)
+  for (int c = blockIdx.x * kWidomCellsWaves + w; c < C; c += gridDim.x * kWidomCellsWaves) {
+    const int t2 = c / g.nz, iz = c - t2 * g.nz, ix = t2 / g.ny, iy = t2 - ix * g.ny;
     int b = 0, n = 0;
-    if (lane < 27) {
-      int dx = 0, dy = 0, dz = 0;
-      stencil_by_distance(lane, dx, dy, dz);
-      if (stencil_axis_ok(dx, g.nx) && stencil_axis_ok(dy, g.ny) && stencil_axis_ok(dz, g.nz)) {
-        const int nc = (wrap_index(ix + dx, g.nx) * g.ny + wrap_index(iy + dy, g.ny)) * g.nz +
-                       wrap_index(iz + dz, g.nz);
-        b = g.start[nc];
-        n = g.start[nc + 1] - b;
-      }
+    if (near) {
+      const int jx = ix + dx, jy = iy + dy, jz = iz + dz;
+      const int nc = (wrap_index(jx, g.nx) * g.ny + wrap_index(jy, g.ny)) * g.nz + wrap_index(jz, g.nz);
+      b = g.start[nc];
+      n = g.start[nc + 1] - b;
     }
-    int incl = n;
-    for (int d = 1; d < 32; d <<= 1) {
-      const int v = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += v;
-    }
+    const int incl = group_inclusive_sum<32>(n);
     // the list length, read into a scalar register so that the point loop
     // below is a uniform loop; padded to a multiple of 4 with positions no
     // point can overlap (the loop tests 4 entries between its exit checks)
-    const int T = __builtin_amdgcn_readfirstlane(__shfl(incl, 26, 64));
+    const int T = __builtin_amdgcn_readlane(incl, 26);
     const int T4 = (T + 3) & ~3;
     if (T4 > kWidomCellsLcap) {  // above the packing bound the host checks: cannot happen
       if (lane == 0) atomicOr(err, kErrListFull);
       continue;
     }
-    for (int q = 0, o = incl - n; q < n; ++q) {
-      Lx[o + q] = g.px[b + q];
-      Ly[o + q] = g.py[b + q];
-      Lz[o + q] = g.pz[b + q];
+    const int o = incl - n;
+    if constexpr (FAST) {
+      // the entries' places first, by cells; then an entry to a lane, so that
+      // three loads fetch the list and not three for each sphere of a cell
+#pragma unroll 1
+      for (int q = 0; q < n; ++q) list[w][o + q].w = __int_as_float(b + q);
+      wave_sync();
+      const double cx = (ix + 0.5) * g.sx, cy = (iy + 0.5) * g.sy, cz = (iz + 0.5) * g.sz;
+      auto from_corner = [](double v, double centre, double side, double L) {
+        const double d = v - centre;
+        return (float)(d - (__builtin_fabs(d) > 0.5 * L ? __builtin_copysign(L, d) : 0.0) + 0.5 * side);
+      };
+#pragma unroll 1
+      for (int e = lane; e < T4; e += 64) {
+        const int s = e < T ? __float_as_int(list[w][e].w) : 0;
+        const double px = g.px[s], py = g.py[s], pz = g.pz[s];
+        list[w][e].x = e < T ? from_corner(px, cx, g.sx, g.lx) : 1e18f;
+        list[w][e].y = from_corner(py, cy, g.sy, g.ly);
+        list[w][e].z = from_corner(pz, cz, g.sz, g.lz);
+      }
+    } else {
+      for (int q = 0; q < n; ++q) {
+        exact[w][0][o + q] = g.px[b + q];
+        exact[w][1][o + q] = g.py[b + q];
+        exact[w][2][o + q] = g.pz[b + q];
+      }
+      if (lane < T4 - T) exact[w][0][T + lane] = exact[w][1][T + lane] = exact[w][2][T + lane] = 1e300;
     }
-    if (lane < T4 - T) {
-      Lx[T + lane] = 1e300;
-      Ly[T + lane] = 1e300;
-      Lz[T + lane] = 1e300;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // 64 points at a time: point base + lane of the cell
-    for (int base = 0; base < per_cell; base += 64) {
-      const int jj = base + lane;
-      const bool mine = jj < per_cell;
-      uint32_t u[4];
+    wave_sync();
+    // point jj of the cell
+    auto draw = [&](int jj, uint32_t u[4]) {
       philox4x32_10((uint32_t)c, (uint32_t)jj, (uint32_t)sample, c3, k0, k1, u);
-      const double qx = ((double)ix + ((double)u[0] + 0.5) * 0x1p-32) * g.sx;
-      const double qy = ((double)iy + ((double)u[1] + 0.5) * 0x1p-32) * g.sy;
-      const double qz = ((double)iz + ((double)u[2] + 0.5) * 0x1p-32) * g.sz;
-      // the smallest squared distance so far: a point overlaps a sphere iff
-      // it is below 1 (one v_min per pair in place of a compare and a merge)
-      double m = 1e300;
-      if (inner) {
+    };
+    auto coord = [](int i, uint32_t u, double side) { return ((double)i + ((double)u + 0.5) * 0x1p-32) * side; };
+    auto walk = [&](auto points, int base) {
+      constexpr int P = decltype(points)::value;
+      bool mine[P];
+      if constexpr (FAST) {
+        float q[P][3], m[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const int jj = base + 64 * p + lane;
+          uint32_t u[4];
+          draw(jj, u);
+          q[p][0] = (float)u[0] * sfx;
+          q[p][1] = (float)u[1] * sfy;
+          q[p][2] = (float)u[2] * sfz;
+          mine[p] = jj < per_cell;
+          m[p] = mine[p] ? 9.0f : 0.0f;
+        }
         for (int e = 0; e < T4; e += 4) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const double dx = qx - Lx[e + i], dy = qy - Ly[e + i], dz = qz - Lz[e + i];
-            m = fmin(m, dx * dx + dy * dy + dz * dz);
+          for (int i = 0; i < 4; i += 2) {
+            const float4 a = list[w][e + i], d = list[w][e + i + 1];
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+              const float ax = q[p][0] - a.x, ay = q[p][1] - a.y, az = q[p][2] - a.z;
+              const float bx = q[p][0] - d.x, by = q[p][1] - d.y, bz = q[p][2] - d.z;
+              m[p] = fminf(m[p], fminf(__builtin_fmaf(az, az, __builtin_fmaf(ay, ay, ax * ax)),
+                                       __builtin_fmaf(bz, bz, __builtin_fmaf(by, by, bx * bx))));
+            }
           }
-          if (__all(m < 1.0 || !mine)) break;
+          float far = m[0];
+          if constexpr (P == 2) far = fmaxf(m[0], m[1]);
+          if (__all(far < 1.0f - kWidomBand)) break;
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          bool free = m[p] >= 1.0f + kWidomBand;
+          const bool undecided = m[p] >= 1.0f - kWidomBand && !free;
+          if (__any(undecided)) {
+            uint32_t u[4];
+            draw(base + 64 * p + lane, u);
+            const double x = coord(ix, u[0], g.sx), y = coord(iy, u[1], g.sy), z = coord(iz, u[2], g.sz);
+            if (undecided)
+              free = true;
+#pragma unroll 1
+            for (int e = 0; e < T; ++e) {
+              const int s = __float_as_int(list[w][e].w);
+              if (undecided && dist2(x, y, z, g.px[s], g.py[s], g.pz[s], g.lx, g.ly, g.lz) < 1.0) free = false;
+            }
+          }
+          if (free && mine[p]) ++h;
         }
       } else {
-        for (int e = 0; e < T4; e += 4) {
-#pragma unroll 1
-          for (int i = 0; i < 4; ++i)
-            m = fmin(m, dist2(qx, qy, qz, Lx[e + i], Ly[e + i], Lz[e + i], g.lx, g.ly, g.lz));
-          if (__all(m < 1.0 || !mine)) break;
+        double q[P][3], m[P];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const int jj = base + 64 * p + lane;
+          uint32_t u[4];
+          draw(jj, u);
+          q[p][0] = coord(ix, u[0], g.sx);
+          q[p][1] = coord(iy, u[1], g.sy);
+          q[p][2] = coord(iz, u[2], g.sz);
+          mine[p] = jj < per_cell;
+          m[p] = mine[p] ? 1e300 : 0.0;
         }
+        for (int e = 0; e < T4; ++e) {
+#pragma unroll
+          for (int p = 0; p < P; ++p)
+            m[p] = fmin(m[p], dist2(q[p][0], q[p][1], q[p][2], exact[w][0][e], exact[w][1][e], exact[w][2][e], g.lx,
+                                    g.ly, g.lz));
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          if (m[p] >= 1.0) ++h;
       }
-      const bool ov = m < 1.0;
-      if (mine && !ov) ++h;
-    }
+    };
+    int base = 0;
+    if constexpr (FAST)
+      for (; base + 64 < per_cell; base += 128) walk(std::integral_constant<int, 2>{}, base);
+    for (; base < per_cell; base += 64) walk(std::integral_constant<int, 1>{}, base);
     __builtin_amdgcn_wave_barrier();  // the list is rewritten for the next cell
   }
   const unsigned long long s = block_sum_u64(h);
@@ -1590,7 +1664,8 @@ int hsmc_gpu_widom_cells(hsmc_gpu_ctx *ctx, int replica, uint64_t seed, uint64_t
   const long blocks = std::min((C + kWidomCellsWaves - 1) / kWidomCellsWaves, (long)kWidomCellsBlocks);
   unsigned long long *part = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * blocks);
   if (!part) return HSMC_ERR_NO_MEMORY;
-  hipLaunchKernelGGL(k_widom_cells, dim3((unsigned)blocks), dim3(64 * kWidomCellsWaves), 0, ctx->stream, g,
+  const bool fast = g.nx >= 3 && g.ny >= 3 && g.nz >= 3;
+  hipLaunchKernelGGL(fast ? k_widom_cells<true> : k_widom_cells<false>, dim3((unsigned)blocks), dim3(64 * kWidomCellsWaves), 0, ctx->stream, g,
                      (uint32_t)seed, (uint32_t)(seed >> 32), (unsigned long long)sample, (int)per_cell,
                      part, ctx->d_err);
   hipLaunchKernelGGL(k_sum_all<false>, dim3(1), dim3(1024), 0, ctx->stream, part, (int)blocks, ctx->d_err,

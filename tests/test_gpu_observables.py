@@ -211,3 +211,37 @@ def test_few_queries_and_moves_by_value(n):
             xyz[i] = t
         assert np.array_equal(ctx.download()[:, 1:], xyz), m
     ctx.close()
+
+
+@pytest.mark.parametrize("box,n,per_cell", [((4.3, 5.0, 6.7), 60, 300), ((2.5, 9.1, 4.9), 50, 129), ((2.2, 2.9, 2.6), 5, 1000),
+                                            ((11.3, 12.9, 10.2), 300, 64), ((11.3, 12.9, 10.2), 300, 65),
+                                            ((30.2, 31.7, 29.9), 4000, 20), ((40.0, 4.5, 30.0), 200, 128)])
+def test_stratified_insertions_match_all_pairs(box, n, per_cell):
+    """Grids of 2 cells an axis (the FP64 test) and of 4 and more (FP32 with a
+    band), one and two points a lane with their remainders; spheres overlap at
+    random, so lists of every length occur.  About 2e-4 of the points have a
+    sphere whose squared distance is within the band."""
+    rng = np.random.default_rng(per_cell)
+    xyz = rng.random((n, 3)) * np.array(box)
+    ctx = _context(xyz, box)
+    hits, points, grid = ctx.widom_cells(9, 4, per_cell)
+    assert grid == tuple(int(b / (1.0 + 1e-9)) for b in box)
+    mask = np.uint64(0xFFFFFFFF)
+    cells = int(np.prod(grid))
+    w = [np.repeat(np.arange(cells, dtype=np.uint64), per_cell), np.tile(np.arange(per_cell, dtype=np.uint64), cells),
+         np.full(cells * per_cell, 4, np.uint64), np.full(cells * per_cell, 0x57430000, np.uint64)]
+    index = w[0].astype(np.int64)
+    k0, k1 = 9, 0
+    for _ in range(10):
+        a, b = np.uint64(0xD2511F53) * w[0], np.uint64(0xCD9E8D57) * w[2]
+        w = [(b >> np.uint64(32)) ^ w[1] ^ np.uint64(k0), b & mask, (a >> np.uint64(32)) ^ w[3] ^ np.uint64(k1), a & mask]
+        k0, k1 = (k0 + 0x9E3779B9) & 0xFFFFFFFF, (k1 + 0xBB67AE85) & 0xFFFFFFFF
+    at = np.stack([index // (grid[1] * grid[2]), index // grid[2] % grid[1], index % grid[2]], 1)
+    q = (at + (np.stack(w[:3], 1).astype(np.float64) + 0.5) * 2.0 ** -32) * (np.array(box) / np.array(grid))
+    free = np.ones(len(q), bool)
+    for c in xyz:
+        d = np.abs(q - c)
+        d = np.minimum(d, np.array(box) - d)
+        free &= ~((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2] < 1.0)
+    assert points == len(q) and hits == int(free.sum())
+    ctx.close()
