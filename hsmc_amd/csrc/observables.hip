@@ -1183,7 +1183,7 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Workspace layout of the scan: counts and starts of the grid's C cells, cell
 // (and place in it) of the N spheres and their sorted positions, each region
-// 256-B aligned; 32 bytes a sphere and 8 a cell.  The workgroups' result masks
+// 256-B aligned; 32 bytes a sphere and 12 a cell.  The workgroups' result masks
 // lie over the cells, which are read no more once the spheres are sorted.
 struct ScanLayout {
   size_t cnt, start, cellof, px, py, pz, part, bytes;
@@ -1204,6 +1204,11 @@ ScanLayout scan_layout(long N, long C) {
   l.py = take(sizeof(double) * N);
   l.pz = take(sizeof(double) * N);
   l.part = take(sizeof(int) * scan_workspace_ints(C));
+  // room this build does without (a second count of the cells, the scale table
+  // and a mask): the size asked for, and so the call that is refused, stays
+  take(sizeof(int) * C);
+  take(sizeof(double) * 64);
+  take(sizeof(unsigned long long));
   l.bytes = o;
   return l;
 }

@@ -63,7 +63,10 @@ typedef struct hsmc_gpu_replica {
  * launch of resident workgroups runs sweeps_per_graph whole sweeps (64 when
  * 0), with a grid barrier between the rebin and each sublattice phase in
  * place of a kernel boundary; the trajectory is the same.  Other values
- * give HSMC_ERR_BAD_ARG. */
+ * give HSMC_ERR_BAD_ARG.  A shape set by hand is used as it is; without one,
+ * replicas small enough run whole sweeps in one launch and contexts of
+ * 40000 active cells and more run by bricks of cells, on the same
+ * trajectory. */
 typedef struct hsmc_gpu_tuning {
   int32_t lanes_per_cell;
   int32_t cells_per_block;
@@ -150,7 +153,9 @@ int hsmc_gpu_occupant_picks(int device, uint64_t seed, uint32_t cell, uint64_t s
 int hsmc_gpu_set_tuning(hsmc_gpu_ctx *ctx, const hsmc_gpu_tuning *t);
 int hsmc_gpu_get_tuning(const hsmc_gpu_ctx *ctx, hsmc_gpu_tuning *t);
 /* Time the candidate launch shapes on this context's own replicas (their
- * state is saved and restored) and keep the fastest.  *best receives it. */
+ * state is saved and restored), and the context's own way of running where it
+ * has one, and keep the fastest.  *best receives the launch shape (the one in
+ * force before, not used, where the own way wins). */
 int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *best);
 /* Average duration (ms) of one launch of the sweep's dominant kernel (the
  * sublattice-phase kernel), measured with HIP events around each launch
