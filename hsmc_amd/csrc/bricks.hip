@@ -103,19 +103,33 @@ k_brick_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev 
   SlotRec *slot = slot_all + (size_t)(one ? par : 0) * CAP * C + rp.coff;
   const int colour = (int)((sw.order >> (4 * phase)) & 0xFu);
   const int ox = colour & 1, oy = (colour >> 1) & 1, oz = (colour >> 2) & 1;
-  // the brick at once, or its cells one by one if it or its neighbourhood
-  // holds more spheres than fit (overlapping configurations)
-  int nx = br.nx, ny = br.ny, nz = br.nz, parts = 1;
-  for (int part = 0; part < parts; ++part) {
+  // The brick at once; where it or its neighbourhood holds more spheres than
+  // fit (a lattice's layers, an uneven configuration), half of it after the
+  // other along its longest side, and a half that does not fit cell by cell.
+  int half = -1, single = -1;
+  for (bool again = false;; again = true) {
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));  // as here(), for what is derived from the lane
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int x0 = br.x0, y0 = br.y0, z0 = br.z0;
-    if (parts > 1) {
-      const int by = here(br.ny), bz = here(br.nz);
-      x0 += part / (by * bz);
-      y0 += part / bz % by;
-      z0 += part % bz;
+    int x0 = br.x0, y0 = br.y0, z0 = br.z0, nx = br.nx, ny = br.ny, nz = br.nz;
+    if (half >= 0) {
+      const int axis = nx >= ny && nx >= nz ? 0 : (ny >= nz ? 1 : 2);
+      const int n = axis == 0 ? nx : (axis == 1 ? ny : nz), first = (n + 1) / 2;
+      const int skip = half ? first : 0, take = half ? n - first : first;
+      x0 += axis == 0 ? skip : 0;
+      y0 += axis == 1 ? skip : 0;
+      z0 += axis == 2 ? skip : 0;
+      nx = axis == 0 ? take : nx;
+      ny = axis == 1 ? take : ny;
+      nz = axis == 2 ? take : nz;
+    }
+    const int cells = nx * ny * nz;
+    if (single >= 0) {
+      const int by = here(ny), bz = here(nz);
+      x0 += single / (by * bz);
+      y0 += single / bz % by;
+      z0 += single % bz;
+      nx = ny = nz = 1;
     }
     const int na = nx * ny * nz;
     const int ry = 2 * ny + 1, rz = 2 * nz + 1, ncell = (2 * nx + 1) * ry * rz;
@@ -132,7 +146,7 @@ k_brick_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev 
       iy = t - ix * ry;
     };
 
-    if (part > 0) __syncthreads();  // the last part's lists are no longer read
+    if (again) __syncthreads();  // the last part's lists are no longer read
     if (tid < 3 * kSide) {
       const int d = tid / kSide, i = tid - d * kSide;
       const int first = d == 0 ? lx : d == 1 ? ly : lz, g = d == 0 ? rp.gx : d == 1 ? rp.gy : rp.gz;
@@ -169,10 +183,10 @@ k_brick_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev 
     const int all = __builtin_amdgcn_readlane(upto, 63);  // a scalar: the brick's shape stays one
     const int total = all & 0xFFFF, attempts = all >> 16;
     if (total > kSpheres || attempts > kAttempts) {  // the same in every thread; not a single cell's stencil
-      parts = na;
-      nx = ny = nz = 1;
-      part = -1;
-      __syncthreads();
+      if (half < 0)
+        half = 0;
+      else
+        single = 0;
       continue;
     }
 #pragma unroll 1
@@ -415,6 +429,10 @@ k_brick_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev 
         if (n_left) atomicAdd(&cleft[ai], n_left);
       }
     }
+    if (half < 0) break;
+    if (single >= 0 && ++single < cells) continue;
+    single = -1;
+    if (++half == 2) break;
   }
 }
 

@@ -73,15 +73,32 @@ def test_one_large_replica(box):
     _same(*_both([_sites(np.random.default_rng(2), box, 0.85)], [box]))
 
 
-def test_uneven_density_and_overlaps():
-    """Bricks with more spheres than their list holds go cell by cell: one
-    replica's spheres lie in an eighth of its box, another's overlap at random."""
+@pytest.mark.parametrize("wide", [False, True])
+def test_uneven_density_and_overlaps(wide):
+    """Bricks with more spheres than their list holds go half by half: one
+    replica's spheres lie in an eighth of its box, another's overlap at random.
+    With 16 slots a cell (a replica of wide cells beside them), halves that
+    hold too many go cell by cell: a cluster of 3.4 spheres a cell."""
     rng = np.random.default_rng(3)
     box = (24.0, 24.0, 24.0)
-    confs, boxes = _with_bulk(rng, [box, box], [1.0, 1.0])
+    confs, boxes = _with_bulk(rng, [box, box, (4.7, 4.7, 4.7) if wide else box], [1.0, 1.0, 0.5])
     confs[0] = np.vstack([_sites(rng, (12.0, 12.0, 12.0), 1.0), 12.0 + 12.0 * rng.random((40, 3))])
     confs[1] = rng.random((6000, 3)) * np.array([24.0, 24.0, 12.0])
+    if wide:
+        confs[1] = np.vstack([11.0 * rng.random((3460, 3)), 12.0 + 12.0 * rng.random((40, 3))])
     _same(*_both(confs, boxes))
+
+
+def test_lattice_starts():
+    """Perfect lattices, whose layers fill some bricks beyond the mean."""
+    confs, boxes = [], []
+    for n, rho in ((6, 0.93), (9, 0.9), (10, 0.8), (11, 1.0), (12, 0.6), (13, 0.93), (30, 0.9)):
+        L = (4 * n ** 3 / rho) ** (1 / 3)
+        g = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 1, 3)
+        basis = np.array([(0, 0, 0), (.5, .5, 0), (.5, 0, .5), (0, .5, .5)])
+        confs.append(((g + basis) * (L / n)).reshape(-1, 3))
+        boxes.append((L, L, L))
+    _same(*_both(confs * 3, boxes * 3, sweeps=(1, 1)))
 
 
 def test_positions_outside_the_box():
