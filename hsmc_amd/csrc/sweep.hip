@@ -135,6 +135,20 @@ struct FileReq {
 template <int M>
 using dvec = double __attribute__((ext_vector_type(M)));
 
+// n / d and, in rem, n % d of 0 <= n < 2^31, with m = ceil(2^32 / d) from the
+// host (d = 1: 2^32 - 1): the product's upper word is the quotient or one
+// beside it.  The divisions stood before the counts' loads, 20 dependent
+// instructions each.
+__device__ __forceinline__ int quotient(int n, int d, uint32_t m, int &rem) {
+  int q = (int)__umulhi((uint32_t)n, m);
+  rem = n - q * d;
+  if (rem < 0) --q, rem += d;
+  if (rem >= d) ++q, rem -= d;
+  return q;
+}
+
+uint32_t quotient_word(int d) { return d == 1 ? 0xFFFFFFFFu : (uint32_t)(((1ull << 32) + d - 1) / d); }
+
 // One active cell's attempts in one sublattice phase: the work of one group
 // of LPC lanes.  a is the active-cell index, a0 the first active cell of the
 // group's workgroup (of cells_per_block consecutive cells), Lm the group's
@@ -146,7 +160,7 @@ template <int CAP, int LPC, int LCAP, bool ONE, bool FILE>
 __device__ __forceinline__ void phase_cell(
     int a, int a0, int lane, int *Lm, const RepDev *__restrict__ reps, const RepDev &rp0,
     const SweepDev *__restrict__ swp, const SweepDev &sw0, const int *__restrict__ arep, int R,
-    int A, int phase, unsigned long long sweep,
+    int A, uint32_t mz, uint32_t my, int phase, unsigned long long sweep,
     double *__restrict__ x, double *__restrict__ y, double *__restrict__ z,
     int *__restrict__ cnt, int C, SlotRec *__restrict__ slot_all,
     unsigned int *__restrict__ cacc, unsigned int *__restrict__ cleft,
@@ -184,11 +198,17 @@ __device__ __forceinline__ void phase_cell(
   // and leaves with them (nc = 0).
   const int hz2 = rp.gz >> 1, hy2 = rp.gy >> 1;
   const int la = a - rp.aoff;
-  const bool live = a < A && la < hz2 * hy2 * (rp.gx >> 1);
-  const int iz2 = la % hz2;
-  const int t2 = la / hz2;
-  const int iy2 = t2 % hy2;
-  const int ix2 = t2 / hy2;
+  const int live = (int)(a < A) & (int)(la < hz2 * hy2 * (rp.gx >> 1));  // no branch
+  int iz2, iy2, t2, ix2;
+  if constexpr (ONE) {
+    t2 = quotient(la, hz2, mz, iz2);
+    ix2 = quotient(t2, hy2, my, iy2);
+  } else {
+    t2 = la / hz2;
+    iz2 = la % hz2;
+    ix2 = t2 / hy2;
+    iy2 = t2 % hy2;
+  }
   const int cx = 2 * ix2 + (colour & 1);
   const int cy = 2 * iy2 + ((colour >> 1) & 1);
   const int cz = 2 * iz2 + ((colour >> 2) & 1);
@@ -201,12 +221,11 @@ __device__ __forceinline__ void phase_cell(
   // j%3-1), 13 being the active cell itself; the other lanes read the count
   // of cell 0 and discard it.
   const int sdx = lane / 9 - 1, sdy = (lane / 3) % 3 - 1, sdz = lane % 3 - 1;
-  const bool owner = lane < 27 && live && stencil_axis_ok(sdx, rp.gx) &&
-                     stencil_axis_ok(sdy, rp.gy) && stencil_axis_ok(sdz, rp.gz);
-  const int ncell =
-      owner ? rp.coff + (wrap_index(cx + sdx, rp.gx) * rp.gy + wrap_index(cy + sdy, rp.gy)) * rp.gz +
-                  wrap_index(cz + sdz, rp.gz)
-            : 0;
+  auto axis_ok = [](int d, int g) { return (int)(g > 2) | (int)(d >= 0); };  // stencil_axis_ok for g = 2, 4, ...
+  const bool owner = (int)(lane < 27) & live & axis_ok(sdx, rp.gx) & axis_ok(sdy, rp.gy) & axis_ok(sdz, rp.gz);
+  const int stencil_cell = rp.coff + (wrap_index(cx + sdx, rp.gx) * rp.gy + wrap_index(cy + sdy, rp.gy)) * rp.gz +
+                           wrap_index(cz + sdz, rp.gz);
+  const int ncell = owner ? stencil_cell : 0;
   const int n_loaded = cntb[ncell];
 
   // draw block of attempt t = lane for every attempt a cell can make (t <
@@ -215,6 +234,13 @@ __device__ __forceinline__ void phase_cell(
   if (lane < CAP)
     philox4x32_10((uint32_t)cid, (uint32_t)lane, (uint32_t)sweep, (uint32_t)(sweep >> 32), rp.k0,
                   rp.k1, w);
+
+  // the parameters' scalar loads end here, beside the counts', and not each
+  // before the load that would wait for them
+  if constexpr (ONE) {
+    asm volatile("" ::"s"(rp.lx), "s"(rp.ly), "s"(rp.lz), "s"(rp.ix), "s"(rp.iy), "s"(rp.iz), "s"(rp.dr_max));
+    asm volatile("" ::"s"(shx), "s"(shy), "s"(shz), "s"(x), "s"(y), "s"(z), "s"(cacc), "s"(cleft));
+  }
 
   const int nj = owner ? (n_loaded < CAP ? n_loaded : CAP) : 0;
   const int incl = group_inclusive_sum<LPC>(nj);
@@ -234,11 +260,15 @@ __device__ __forceinline__ void phase_cell(
   const SlotRec *orec = slot + (size_t)(lane < nc ? lane : 0) * C + rp.coff + cid;
   const int my_id = orec->id;
   const double o_x = orec->x, o_y = orec->y, o_z = orec->z;
-  // stage the stencil list: the slot of every entry into LDS, then each
+  // stage the stencil list: the slot of every entry into LDS (most cells hold
+  // two at most), then each
   // lane loads its entries' FP64 positions into registers, all loads of the
   // work item in flight together.  Entries past T read entry 0's record (T
   // >= nc >= 1 here); copies past T are never tested.
-  for (int q = 0; q < nj; ++q) Lm[off + q] = q * C + ncell;
+  if (nj > 0) Lm[off] = ncell;
+  if (nj > 1) Lm[off + 1] = C + ncell;
+#pragma unroll 1
+  for (int q = 2; q < nj; ++q) Lm[off + q] = q * C + ncell;
   wave_lds_sync();
   dvec<M> px, py, pz;
 #pragma unroll
@@ -522,25 +552,30 @@ __device__ __forceinline__ void file_next_sweep(int g, int P, int C, int phase, 
 // rebin): lane g files particle g and its cell's occupant into the next
 // sweep's list.  The host checks that the lanes cover C and P.  Each mode is
 // its own kernel, so the plain phases carry none of this code.
+// What the first loads need comes first among the arguments (the launch brings
+// the first 14 words in scalar registers; phase and cells per workgroup share
+// one): the sweep counter, the table entry and the record's load then leave
+// together, and nothing branches or divides before the counts' loads.  One
+// replica, per sweep of 8 phases: N = 4000 36.4 -> 34.6 us, N = 32000 41.0 ->
+// 39.4, N = 108000 73.0 -> 68.9, with the loops over the slots short too.
 // Occupancy: at least 6 waves per SIMD (at most 80 VGPRs) for stencil lists
 // of up to 192 entries, 4 for the longest lists and for one replica (whose
 // few active cells never fill the device).
 template <int CAP, int LPC, int LCAP, bool ONE, int MODE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!ONE && LCAP <= 192 ? 6 : 4)))
 k_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev *__restrict__ swp,
-        const RepDev *__restrict__ reps, const RepDev rp0, const int *__restrict__ arep, int R,
-        int P, int A, int phase, int k, int kt,
+        int *__restrict__ cnt, SlotRec *__restrict__ slot, int k, int phase_cpb, int A, int C, uint32_t mz, uint32_t my,
+        const RepDev rp0, const RepDev *__restrict__ reps, const int *__restrict__ arep, int R, int P,
         double *__restrict__ x, double *__restrict__ y, double *__restrict__ z,
-        int *__restrict__ cnt, int C, SlotRec *__restrict__ slot,
         unsigned int *__restrict__ cacc, unsigned int *__restrict__ cleft,
         unsigned int *__restrict__ err) {
   extern __shared__ __attribute__((aligned(16))) int smem_i[];
   SweepDev sw0{}, swn0{};
-  if constexpr (ONE) sw0 = swp[kt];
-  if constexpr (ONE && MODE == 2) swn0 = swp[kt + 1];
+  if constexpr (ONE) sw0 = swp[0];
+  if constexpr (ONE && MODE == 2) swn0 = swp[1];
   const unsigned long long sweep = *sweep_base + (unsigned long long)k;
-  const int cpb = blockDim.x / LPC;
-  const int g = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const int phase = phase_cpb & 15, cpb = phase_cpb >> 4;
+  const int g = (int)(blockIdx.x * cpb * LPC + threadIdx.x);
   double ax = 0.0, ay = 0.0, az = 0.0;
   if constexpr (ONE && MODE == 2) {  // particle g's position, loaded first
     const int gp = g < P ? g : 0;
@@ -553,7 +588,7 @@ k_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev *__res
   FileReq req{};
   phase_cell<CAP, LPC, LCAP, ONE, MODE == 2>(blockIdx.x * cpb + sub, blockIdx.x * cpb, lane,
                                              smem_i + (size_t)sub * (LCAP + 14 * CAP), reps, rp0,
-                                             swp, sw0, arep, R, A, phase, sweep, x, y, z, cnt, C,
+                                             swp, sw0, arep, R, A, mz, my, phase, sweep, x, y, z, cnt, C,
                                              slot, cacc, cleft, err, req);
   if constexpr (ONE && MODE == 1) {
     if (g < C) cnt[(size_t)((sweep & 1ull) ^ 1ull) * C + g] = 0;
@@ -612,7 +647,7 @@ template <int CAP, int LPC, int LCAP, bool ONE>
 __global__ void __launch_bounds__(256)
 k_sweeps_persistent(const RepDev *__restrict__ reps, const RepDev rp0, SweepDev *__restrict__ swp,
                     const int *__restrict__ arep, const int *__restrict__ prep, int R, int P, int C,
-                    int A, double *__restrict__ x, double *__restrict__ y, double *__restrict__ z,
+                    int A, uint32_t mz, uint32_t my, double *__restrict__ x, double *__restrict__ y, double *__restrict__ z,
                     int *__restrict__ cnt, SlotRec *__restrict__ slot, int cap,
                     const unsigned long long *__restrict__ sweep_base, int n_sweeps,
                     unsigned int *__restrict__ cacc, unsigned int *__restrict__ cleft,
@@ -636,7 +671,7 @@ k_sweeps_persistent(const RepDev *__restrict__ reps, const RepDev rp0, SweepDev 
         const SweepDev sw0 = ONE ? swp[s] : SweepDev{};
         FileReq req{};
         phase_cell<CAP, LPC, LCAP, ONE, false>(a0 + sub, a0, lane, Lm, reps, rp0, swp, sw0, arep,
-                                               R, A, p, sweep, x, y, z, cnt, C, slot, cacc, cleft,
+                                               R, A, mz, my, p, sweep, x, y, z, cnt, C, slot, cacc, cleft,
                                                err, req);
       }
       if (!grid_barrier(bar, err)) return;
@@ -669,10 +704,9 @@ k_occupant_picks(uint32_t k0, uint32_t k1, uint32_t cell, unsigned long long swe
   out[t] = occupant_pick(w[0], n, cell, (uint32_t)t, sweep, k0, k1);
 }
 
-using PhaseFn = void (*)(const unsigned long long *, const SweepDev *, const RepDev *, const RepDev,
-                         const int *, int, int, int, int, int, int, double *,
-                         double *, double *, int *, int, SlotRec *, unsigned int *, unsigned int *,
-                         unsigned int *);
+using PhaseFn = void (*)(const unsigned long long *, const SweepDev *, int *, SlotRec *, int, int, int, int,
+                         uint32_t, uint32_t, const RepDev, const RepDev *, const int *, int, int, double *,
+                         double *, double *, unsigned int *, unsigned int *, unsigned int *);
 
 template <int CAP, int LCAP, bool ONE, int MODE>
 PhaseFn phase_fn_l(int lpc) {
@@ -700,7 +734,7 @@ PhaseFn phase_fn(int cap, int lpc, int lcap, bool one, int mode = 0) {
 }
 
 using PersistentFn = void (*)(const RepDev *, const RepDev, SweepDev *, const int *, const int *,
-                              int, int, int, int, double *, double *, double *, int *, SlotRec *,
+                              int, int, int, int, uint32_t, uint32_t, double *, double *, double *, int *, SlotRec *,
                               int, const unsigned long long *, int, unsigned int *,
                               unsigned int *, unsigned int *, GridBarrier *);
 
@@ -762,7 +796,8 @@ int launch_persistent(hsmc_gpu_ctx *ctx, int n) {
   int ns = n;
   unsigned int *cacc = ctx->d_cacc, *cleft = ctx->d_cleft, *err = ctx->d_err;
   GridBarrier *bar = reinterpret_cast<GridBarrier *>(ctx->d_bar);
-  void *args[] = {&reps, &rp0, &swp, &arep, &prep, &R, &P, &C, &A, &x, &y, &z, &cnt, &slot,
+  uint32_t mz = quotient_word(rp0.gz >> 1), my = quotient_word(rp0.gy >> 1);
+  void *args[] = {&reps, &rp0, &swp, &arep, &prep, &R, &P, &C, &A, &mz, &my, &x, &y, &z, &cnt, &slot,
                   &cap, &sweep, &ns, &cacc, &cleft, &err, &bar};
   HSMC_HIP(ctx, hipLaunchCooperativeKernel((const void *)fn, dim3((unsigned)grid), dim3(lpc * cpb),
                                            args, (unsigned)lds, ctx->stream));
@@ -813,15 +848,14 @@ void enqueue_sweep(hsmc_gpu_ctx *ctx, int k, hipStream_t s, hipEvent_t *phase_ev
   const int bs = lpc * cpb;
   const unsigned blocks = (unsigned)((ctx->Atot + cpb - 1) / cpb);
   const size_t lds = phase_lds_bytes(ctx->cap, ctx->lcap, cpb);
+  const uint32_t mz = quotient_word(ctx->rep0.gz >> 1), my = quotient_word(ctx->rep0.gy >> 1);
   for (int p = 0; p < 8; ++p) {
     const int mode = p == 0 && chained ? 1 : p == 7 && file_next ? 2 : 0;
     PhaseFn fn = phase_fn(ctx->cap, lpc, ctx->lcap, ctx->R == 1, mode);
     if (phase_events && p == 0) (void)hipEventRecord(phase_events[0], s);
-    hipLaunchKernelGGL(fn, dim3(blocks), dim3(bs), lds, s, ctx->d_sweep, ctx->d_swp,
-                       ctx->d_reps, ctx->rep0, ctx->d_arep, ctx->R, (int)ctx->Ptot,
-                       (int)ctx->Atot, p, k, kt, ctx->d_x, ctx->d_y, ctx->d_z,
-                       ctx->d_cnt, (int)ctx->Ctot, ctx->d_slot, ctx->d_cacc,
-                       ctx->d_cleft, ctx->d_err);
+    hipLaunchKernelGGL(fn, dim3(blocks), dim3(bs), lds, s, ctx->d_sweep, ctx->d_swp + kt, ctx->d_cnt, ctx->d_slot,
+                       k, p | cpb << 4, (int)ctx->Atot, (int)ctx->Ctot, mz, my, ctx->rep0, ctx->d_reps, ctx->d_arep, ctx->R,
+                       (int)ctx->Ptot, ctx->d_x, ctx->d_y, ctx->d_z, ctx->d_cacc, ctx->d_cleft, ctx->d_err);
     if (phase_events && p == 7) (void)hipEventRecord(phase_events[15], s);
   }
 }
