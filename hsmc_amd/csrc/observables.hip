@@ -396,8 +396,8 @@ k_widom_uniform(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, lon
   uniform_points(g, k0, k1, sample, first, n, part);
 }
 
-// The same for systems whose grid and positions fit in 64 KB of LDS: every
-// workgroup files the spheres itself (a few us, beside the three launches of
+// The same for systems whose grid and positions fit in LDS: every workgroup
+// files the spheres itself (a few us, beside the three launches of
 // a grid in memory) and its points' scattered reads stay on the chip.
 constexpr int kWidomLdsThreads = 512, kWidomLdsBlocks = 1024;
 
@@ -412,26 +412,27 @@ struct LdsGrid {  // after filing, last[c] is the end of cell c and so the start
 
 size_t widom_lds_bytes(long N, long C) { return sizeof(double) * 3 * N + sizeof(int) * C; }
 
-__global__ void __launch_bounds__(kWidomLdsThreads)
+template <int THREADS>
+__global__ void __launch_bounds__(THREADS)
 k_widom_uniform_lds(Grid gg, int N, const double *__restrict__ x, const double *__restrict__ y,
                     const double *__restrict__ z, uint32_t k0, uint32_t k1,
                     unsigned long long sample, long long first, long long n,
                     unsigned long long *__restrict__ part) {
   extern __shared__ double lds_pos[];
-  __shared__ int tot[kWidomLdsThreads / 64];
+  __shared__ int tot[THREADS / 64];
   double *px = lds_pos, *py = px + N, *pz = py + N;
   int *cnt = reinterpret_cast<int *>(pz + N);
   const int t = threadIdx.x, C = gg.nx * gg.ny * gg.nz;
-  for (int c = t; c < C; c += kWidomLdsThreads) cnt[c] = 0;
+  for (int c = t; c < C; c += THREADS) cnt[c] = 0;
   __syncthreads();
   auto cell = [&](double a, double b, double c) {
     return (search_cell(a, gg.ix, gg.nx) * gg.ny + search_cell(b, gg.iy, gg.ny)) * gg.nz +
            search_cell(c, gg.iz, gg.nz);
   };
-  for (int i = t; i < N; i += kWidomLdsThreads) atomicAdd(&cnt[cell(x[i], y[i], z[i])], 1);
+  for (int i = t; i < N; i += THREADS) atomicAdd(&cnt[cell(x[i], y[i], z[i])], 1);
   __syncthreads();
   // counts to starts: a run of consecutive cells per thread
-  const int per = (C + kWidomLdsThreads - 1) / kWidomLdsThreads, c0 = min(t * per, C), c1 = min(c0 + per, C);
+  const int per = (C + THREADS - 1) / THREADS, c0 = min(t * per, C), c1 = min(c0 + per, C);
   int s = 0;
   for (int c = c0; c < c1; ++c) s += cnt[c];
   const int incl = group_inclusive_sum<64>(s);
@@ -445,7 +446,7 @@ k_widom_uniform_lds(Grid gg, int N, const double *__restrict__ x, const double *
     run += k;
   }
   __syncthreads();
-  for (int i = t; i < N; i += kWidomLdsThreads) {
+  for (int i = t; i < N; i += THREADS) {
     const double a = x[i], b = y[i], c = z[i];
     const int p = atomicAdd(&cnt[cell(a, b, c)], 1);
     px[p] = a;
@@ -1089,6 +1090,15 @@ int build_grid(hsmc_gpu_ctx *ctx, int replica, double cut, Grid &g) {
 }
 
 constexpr int kWidomLdsSpheres = 2048;
+// Above that, or with more cells than 64 KB take, one workgroup of 1024 a
+// compute unit files them while grid and positions fit in LDS, the box is not
+// so dilute that most of the LDS is empty cells, and filing is not more work
+// than the points on a grid that is there already (us a call, grid to be built
+// / there / LDS, N = 4000 at density 0.8: 10^5 points 42 / 29 / 31, 10^6 72 /
+// 57 / 51, 10^7 302 / 287 / 236; N = 2048 at density 0.3, 2.8 cells a sphere:
+// 10^7 661 / 650 / 709).
+constexpr size_t kWidomLdsBytes = 158 * 1024;  // and some static words
+constexpr long long kWidomLdsPoints = 400000;
 constexpr int kSmallRuns = 4096;   // all_pairs: shorter runs for the smallest systems
 constexpr double kRowSide = 2.0;   // row_pairs: smallest cell side worth a workgroup
 
@@ -1617,13 +1627,21 @@ int hsmc_gpu_widom_uniform(hsmc_gpu_ctx *ctx, int replica, uint64_t seed, uint64
   Grid g;
   set_grid(h, 1.0 + 1e-9, g);
   const size_t lds = widom_lds_bytes(N, (long)g.nx * g.ny * g.nz);
-  const bool in_lds = N <= kWidomLdsSpheres && lds <= 64 * 1024;
-  const long long wg = in_lds ? kWidomLdsThreads : 256, most = in_lds ? kWidomLdsBlocks : kWidomUniformBlocks;
+  const bool small = N <= kWidomLdsSpheres && lds <= 64 * 1024;
+  const bool kept = ctx->aux_replica == replica && ctx->aux_version == ctx->version && ctx->aux_n[0] == g.nx &&
+                    ctx->aux_n[1] == g.ny && ctx->aux_n[2] == g.nz;
+  const bool in_lds = small || (lds <= kWidomLdsBytes && (long)g.nx * g.ny * g.nz <= 2L * N &&
+                                !(kept && n < kWidomLdsPoints));
+  const long long wg = in_lds ? (small ? kWidomLdsThreads : 1024) : 256;
+  const long long most = in_lds ? (small ? kWidomLdsBlocks : ctx->n_cu) : kWidomUniformBlocks;
   const long long blocks = std::min((n + wg - 1) / wg, most);
   unsigned long long *part = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * blocks);
   if (!part) return HSMC_ERR_NO_MEMORY;
   if (in_lds) {
-    hipLaunchKernelGGL(k_widom_uniform_lds, dim3((unsigned)blocks), dim3((unsigned)wg), lds, ctx->stream, g, N,
+    auto fn = small ? k_widom_uniform_lds<kWidomLdsThreads> : k_widom_uniform_lds<1024>;
+    if (lds > 64 * 1024)
+      HSMC_HIP(ctx, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)wg), lds, ctx->stream, g, N,
                        ctx->d_x + h.poff, ctx->d_y + h.poff, ctx->d_z + h.poff, (uint32_t)seed,
                        (uint32_t)(seed >> 32), (unsigned long long)sample, (long long)first, (long long)n, part);
   } else {

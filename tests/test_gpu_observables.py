@@ -184,6 +184,30 @@ def test_uniform_insertions_filed_in_lds_or_memory(n, rho):
     ctx.close()
 
 
+@pytest.mark.parametrize("n,rho", [(2049, 0.6), (4000, 0.8), (5200, 0.9), (5400, 0.9), (3000, 0.4)])
+def test_uniform_insertions_of_larger_systems(n, rho):
+    """One workgroup of 1024 with up to 158 KB of LDS, or the grid in memory
+    (larger, dilute, or few points on a grid that is there): the same hits, and
+    the points' own over all spheres in numpy."""
+    rng = np.random.default_rng(n)
+    L = (n / rho) ** (1 / 3)
+    xyz = rng.random((n, 3)) * L
+    ctx = _context(xyz, (L, L, L))
+    fresh = ctx.widom_uniform(5, 0, 0, 3000)
+    ctx.widom_cells(1, 1, 1)                      # builds the grid
+    assert ctx.widom_uniform(5, 0, 0, 3000) == fresh
+    many = ctx.widom_uniform(5, 0, 0, 450000)
+    assert many == sum(ctx.widom_uniform(5, 0, first, 150000) for first in (0, 150000, 300000))
+    q = _uniform(5, 3000) * L
+    free = np.ones(len(q), bool)
+    for c in xyz:
+        d = np.abs(q - c)
+        d = np.minimum(d, L - d)
+        free &= ~((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2] < 1.0)
+    assert fresh == int(free.sum())
+    ctx.close()
+
+
 @pytest.mark.parametrize("n", [1, 64, 257, 1025, 16384, 16385])
 def test_few_queries_and_moves_by_value(n):
     """Overlap queries up to 8 at a time take no grid, more do; one call after
