@@ -215,6 +215,9 @@ void fill_repdev(const RepHost &h, RepDev &d);
 // if so their records go to rd (when given), the host's copy of replica 0's
 // follows, and a one-replica graph that carries another one is dropped.
 bool layout_keeps(hsmc_gpu_ctx *ctx, std::vector<RepDev> *rd = nullptr);
+// Whether a replica in the box of record d keeps its sweep grid and the
+// layout's capacities suffice for it.
+bool box_fits_layout(const hsmc_gpu_ctx *ctx, const RepHost &h, const RepDev &d);
 // LDS bytes of one sublattice-phase workgroup of cpb cells
 size_t phase_lds_bytes(int cap, int lcap, int cpb);
 // n checkerboard sweeps of every replica (enqueued on the context stream)

@@ -163,6 +163,11 @@ void fill_repdev(const RepHost &h, RepDev &d) {
 bool needs_big_cells(const RepDev &d) { return d.sx >= 1.1547 || d.sy >= 1.1547 || d.sz >= 1.1547; }
 bool cells_too_wide(const RepDev &d) { return d.sx >= 1.5 || d.sy >= 1.5 || d.sz >= 1.5; }
 
+bool box_fits_layout(const hsmc_gpu_ctx *ctx, const RepHost &h, const RepDev &d) {
+  return sweep_grid_cells(d.lx) == h.gx && sweep_grid_cells(d.ly) == h.gy && sweep_grid_cells(d.lz) == h.gz &&
+         !cells_too_wide(d) && (ctx->cap == 16 || !needs_big_cells(d)) && lcap_for(stencil_list_bound(d)) <= ctx->lcap;
+}
+
 bool layout_keeps(hsmc_gpu_ctx *ctx, std::vector<RepDev> *out) {
   if (!ctx->d_cnt || !ctx->d_reps) return false;
   std::vector<RepDev> rd(ctx->R);

@@ -478,9 +478,15 @@ int boxes_changed(hsmc_gpu_ctx *ctx) {
 }
 
 // The volume moves of one sweep, steps[r] of replica r, for replicas that
-// fit k_volume_moves.
+// fit k_volume_moves.  With *ahead set, the next sweep is enqueued behind the
+// last of them where the layout serves every outcome (the resident kernel
+// reads boxes and positions on the device), so that it runs while the host
+// takes the decisions in and draws the next moves (32 replicas of N = 256: 57
+// -> 52 us a sweep); *ahead tells whether it was.
 int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::vector<int> &steps, int rounds,
-                       const double *press, const double *dv_max, uint64_t *vol_counts) {
+                       const double *press, const double *dv_max, uint64_t *vol_counts, bool *ahead) {
+  const bool may = *ahead;
+  *ahead = false;
   const int R = ctx->R;
   int n_max = 0;
   for (const RepHost &h : ctx->reps) n_max = std::max(n_max, h.p.n_part);
@@ -493,6 +499,7 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
     std::vector<VolNode> nodes;
     std::vector<VolPlan> plan(R);
     std::vector<Box> at;
+    bool keeps = may && t0 + kVolDepth >= rounds;
     for (int r = 0; r < R; ++r) {
       const RepHost &h = ctx->reps[r];
       const int k = std::max(0, std::min(kVolDepth, steps[r] - t0));
@@ -503,6 +510,7 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
       for (int i = 0, depth = 0; i < n; ++i) {
         if (i == (2 << depth) - 1) ++depth;
         nodes.push_back(propose(h, at[i], sweep, t0 + depth, press[r], dv_max[r], &at[2 * i + 1]));
+        keeps = keeps && box_fits_layout(ctx, h, nodes.back().rec);
         at[2 * i + 2] = at[i];
       }
     }
@@ -517,7 +525,15 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
                        (const VolPlan *)host, (const VolNode *)(host + o_node), ctx->d_x, ctx->d_y, ctx->d_z,
                        (int *)(host + o_res));
     HSMC_HIP(ctx, hipGetLastError());
-    HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (keeps) {
+      HSMC_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
+      int st = run_sweeps(ctx, 1);
+      if (st) return st;
+      *ahead = true;
+      HSMC_HIP(ctx, hipEventSynchronize(ctx->ev0));
+    } else {
+      HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    }
     bool any = false;
     for (int r = 0; r < R; ++r) {
       int cur = 0;
@@ -676,8 +692,10 @@ int hsmc_gpu_npt_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, const double *press,
   bool small = true;
   for (const RepHost &h : ctx->reps) small = small && h.p.n_part <= kVolSpheres;
   std::vector<int> steps(R);
+  ResidentShape shape;
+  bool ahead = false;  // the sweep was enqueued behind the last one's volume moves
   for (int sw = 0; sw < n_sweeps; ++sw) {
-    int st = run_sweeps(ctx, 1);
+    int st = ahead ? HSMC_OK : run_sweeps(ctx, 1);
     if (st) return st;
     const unsigned long long s = sweep0 + (unsigned long long)sw;  // the sweep just done
     int rounds = 0;
@@ -687,7 +705,9 @@ int hsmc_gpu_npt_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, const double *press,
       steps[r] = volume_steps(ctx->reps[r].p.n_part, u[0]);
       rounds = std::max(rounds, steps[r]);
     }
-    st = small ? volume_moves_small(ctx, s, steps, rounds, press, dv_max, vol_counts)
+    ahead = small && sw + 1 < n_sweeps && !ctx->tune_set && resident_shape(ctx, &shape);
+    if (rounds == 0) ahead = false;
+    st = small ? volume_moves_small(ctx, s, steps, rounds, press, dv_max, vol_counts, &ahead)
                : volume_moves_rounds(ctx, s, steps, rounds, press, dv_max, vol_counts);
     if (st) return st;
   }

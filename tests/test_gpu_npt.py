@@ -307,3 +307,22 @@ def test_npt_moves_in_one_launch_equal_moves_in_rounds():
     assert all(one.any_overlap_scaled_batch(1.0) == 1)
     one.close()
     rounds.close()
+
+
+@pytest.mark.parametrize("dv", [0.004, 0.05, 0.3])
+def test_npt_sweeps_in_one_call_equal_single_sweeps(dv):
+    """Inside a call the next sweep is enqueued behind the volume moves where
+    the layout serves all their outcomes; a call of one sweep never does.  Small
+    steps keep the grids, wide ones change them, between them some sweeps do."""
+    spec = [(2, 0.35, 900 + k, 0.2) for k in range(4)] + [(4, 0.7, 80 + k, 0.1) for k in range(3)]
+    press = [0.6] * 4 + [4.0] * 3
+    a, b = make(spec), make(spec)
+    one = a.npt_sweeps(60, press, [dv] * 7)
+    many = sum(b.npt_sweeps(1, press, [dv] * 7) for _ in range(60))
+    assert np.array_equal(one, many) and one[:, 1].sum() > 0
+    for r in range(a.R):
+        assert a.box(r) == b.box(r), r
+        assert np.array_equal(a.download(r), b.download(r)), r
+        assert a.counters(r) == b.counters(r), r
+    a.close()
+    b.close()
