@@ -381,11 +381,19 @@ __global__ void k_pack_net(const float *__restrict__ P, MlpDev *__restrict__ net
 }
 
 // ---- descriptors -------------------------------------------------------------
+// A sphere's position, one aligned record: a wave's lanes read 64 spheres, and
+// two loads of it occupy the compute unit's address path two thirds as long as
+// three of an array each (scores of 50260 free voxels 51 -> 39 us, 2^20 sorted
+// training rows at N = 4000 648 -> 566).
+struct __attribute__((aligned(32))) Pos {
+  double x, y, z, pad;
+};
+
 struct NGrid {  // CSR observable grid (side >= 1.5) over one replica
   int nx, ny, nz;
   double sx, sy, sz, ix, iy, iz, lx, ly, lz;  // ix = 1.0 / sx ...
   const int *start;
-  const double *px, *py, *pz;
+  const Pos *p;
 };
 
 // Candidate range of one row (dx, dy) of the 27-cell stencil: the row's z
@@ -446,9 +454,10 @@ __device__ __forceinline__ void scan_rows(const NGrid &g, double qx, double qy, 
       for (int u = 0; u < CH; ++u) {
         const int e = min(u0 + u, len - 1);
         const int q = e + (e < la ? pa : pb);
-        ox[u] = g.px[q];
-        oy[u] = g.py[q];
-        oz[u] = g.pz[q];
+        const Pos &o = g.p[q];
+        ox[u] = o.x;
+        oy[u] = o.y;
+        oz[u] = o.z;
       }
 #pragma unroll
       for (int u = 0; u < CH; ++u)
@@ -728,9 +737,9 @@ k_voxel_scores_tiled(NGrid g, Vox vx, float far2, double smin, const MlpDev *__r
     const int c = (wrap_index(lo[0] + kx, g.nx) * g.ny + wrap_index(lo[1] + ky, g.ny)) * g.nz +
                   wrap_index(lo[2] + kz, g.nz);
     for (int p = g.start[c]; p < g.start[c + 1]; ++p) {
-      const double dx = min_image(g.px[p] - ccx, g.lx, g.lx / 2.0);
-      const double dy = min_image(g.py[p] - ccy, g.ly, g.ly / 2.0);
-      const double dz = min_image(g.pz[p] - ccz, g.lz, g.lz / 2.0);
+      const double dx = min_image(g.p[p].x - ccx, g.lx, g.lx / 2.0);
+      const double dy = min_image(g.p[p].y - ccy, g.ly, g.ly / 2.0);
+      const double dz = min_image(g.p[p].z - ccz, g.lz, g.lz / 2.0);
       if (fabs(dx) <= ex && fabs(dy) <= ey && fabs(dz) <= ez) {
         const int slot = atomicAdd(&ncand, 1);
         if (slot < TCAP) {
@@ -1080,7 +1089,7 @@ __device__ __forceinline__ bool widom_free(const NGrid &g1, double qx, double qy
   };
   auto hit = [&](int b, int e) {
     for (int p = b; p < e; ++p)
-      if (dist2(qx, qy, qz, g1.px[p], g1.py[p], g1.pz[p], g1.lx, g1.ly, g1.lz) < 1.0)
+      if (dist2(qx, qy, qz, g1.p[p].x, g1.p[p].y, g1.p[p].z, g1.lx, g1.ly, g1.lz) < 1.0)
         return true;
     return false;
   };
@@ -1256,15 +1265,12 @@ __global__ void k_grid_count2(const double *__restrict__ x, const double *__rest
 __global__ void k_grid_scatter2(const double *__restrict__ x, const double *__restrict__ y,
                                 const double *__restrict__ z, int n, const int *__restrict__ cellof,
                                 const int *__restrict__ start, int *__restrict__ fill,
-                                double *__restrict__ px, double *__restrict__ py,
-                                double *__restrict__ pz) {
+                                Pos *__restrict__ p) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int c = cellof[i];
   const int pos = start[c] + atomicAdd(&fill[c], 1);
-  px[pos] = x[i];
-  py[pos] = y[i];
-  pz[pos] = z[i];
+  p[pos] = Pos{x[i], y[i], z[i], 0.0};
 }
 
 // Two CSR grids of one replica filed in one pass: grid a's cells are the
@@ -1294,19 +1300,13 @@ __global__ void k_grid_count_pair(const double *__restrict__ x, const double *__
 __global__ void k_grid_scatter_pair(const double *__restrict__ x, const double *__restrict__ y,
                                     const double *__restrict__ z, int n,
                                     const int4 *__restrict__ at, const int *__restrict__ start,
-                                    double *__restrict__ px, double *__restrict__ py,
-                                    double *__restrict__ pz) {
+                                    Pos *__restrict__ p) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const double xi = x[i], yi = y[i], zi = z[i];
   const int4 a = at[i];
   const int p0 = start[a.x] + a.z, p1 = start[a.y] + a.w;
-  px[p0] = xi;
-  py[p0] = yi;
-  pz[p0] = zi;
-  px[p1] = xi;
-  py[p1] = yi;
-  pz[p1] = zi;
+  p[p0] = p[p1] = Pos{xi, yi, zi, 0.0};
 }
 
 int grid_cells_for2(double L, double cut) {
@@ -1329,8 +1329,7 @@ enum { L_GRID_A = 24, L_GRID_PAIR = 27, L_X = 30, L_T = 31, L_CDF = 32, L_GRAD =
        L_BSUM = 36, L_SCANP = 37, L_F = 38, L_FRED = 39, L_LIST = 40, L_NFREE = 41, L_FLAG = 42,
        L_STATS = 43 };
 
-void set_grid(NGrid &g, const RepHost &h, double cut, const int *start, const double *pos,
-              size_t stride) {
+void set_grid(NGrid &g, const RepHost &h, double cut, const int *start, const Pos *pos) {
   g.nx = grid_cells_for2(h.p.lx, cut);
   g.ny = grid_cells_for2(h.p.ly, cut);
   g.nz = grid_cells_for2(h.p.lz, cut);
@@ -1338,7 +1337,7 @@ void set_grid(NGrid &g, const RepHost &h, double cut, const int *start, const do
   g.ix = 1.0 / g.sx; g.iy = 1.0 / g.sy; g.iz = 1.0 / g.sz;
   g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
   g.start = start;
-  g.px = pos; g.py = pos + stride; g.pz = pos + 2 * stride;
+  g.p = pos;
 }
 
 // Descriptor grid (cut_a) and overlap grid (cut_b) of `replica` in one set
@@ -1359,14 +1358,13 @@ int build_ngrid_pair(hsmc_gpu_ctx *ctx, int replica, double cut_a, double cut_b,
                       ctx->ngrid_cut[1] == cut_a + cut_b;
   const size_t cells = ((size_t)C + 4) & ~(size_t)3;  // keeps the int4 behind the counts aligned
   int *cnt = (int *)scratch(ctx, L_GRID_PAIR + 0, sizeof(int) * cells + sizeof(int4) * N);
-  double *pos = (double *)scratch(ctx, L_GRID_PAIR + 1, sizeof(double) * 6 * (size_t)N);
+  Pos *pos = (Pos *)scratch(ctx, L_GRID_PAIR + 1, sizeof(Pos) * 2 * (size_t)N);
   int *start = (int *)scratch(ctx, L_GRID_PAIR + 2, sizeof(int) * (C + 1));
   int *part = (int *)scratch(ctx, L_SCANP, sizeof(int) * scan_workspace_ints(C));
   if (!cnt || !pos || !start || !part) return HSMC_ERR_NO_MEMORY;
   int4 *at = (int4 *)(cnt + cells);  // each sphere's two cells and its rank in each
-  const size_t stride = 2 * (size_t)N;
-  set_grid(ga, h, cut_a, start, pos, stride);
-  set_grid(gb, h, cut_b, start + Ca, pos, stride);
+  set_grid(ga, h, cut_a, start, pos);
+  set_grid(gb, h, cut_b, start + Ca, pos);
   if (cached) return HSMC_OK;
   const CellDims da{ga.nx, ga.ny, ga.nz, ga.ix, ga.iy, ga.iz};
   const CellDims db{gb.nx, gb.ny, gb.nz, gb.ix, gb.iy, gb.iz};
@@ -1376,7 +1374,7 @@ int build_ngrid_pair(hsmc_gpu_ctx *ctx, int replica, double cut_a, double cut_b,
                      N, da, db, (int)Ca, cnt, at);
   exclusive_scan(ctx->stream, cnt, (int)C, start, part, false);
   hipLaunchKernelGGL(k_grid_scatter_pair, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y,
-                     z, N, at, start, pos, pos + stride, pos + 2 * stride);
+                     z, N, at, start, pos);
   HSMC_HIP(ctx, hipGetLastError());
   ctx->ngrid_replica[1] = replica;
   ctx->ngrid_version[1] = ctx->version;
@@ -1394,7 +1392,7 @@ int build_ngrid(hsmc_gpu_ctx *ctx, int replica, double cut, int slot0, NGrid &g)
   const bool cached = ctx->ngrid_replica[which] == replica &&
                       ctx->ngrid_version[which] == ctx->version && ctx->ngrid_cut[which] == cut;
   int *cnt = (int *)scratch(ctx, slot0 + 0, sizeof(int) * 2 * (C + 1) + sizeof(int) * N);
-  double *pos = (double *)scratch(ctx, slot0 + 1, sizeof(double) * 3 * N);
+  Pos *pos = (Pos *)scratch(ctx, slot0 + 1, sizeof(Pos) * (size_t)N);
   int *start = (int *)scratch(ctx, slot0 + 2, sizeof(int) * (C + 1));
   int *part = (int *)scratch(ctx, L_SCANP, sizeof(int) * scan_workspace_ints(C));
   if (!cnt || !pos || !start || !part) return HSMC_ERR_NO_MEMORY;
@@ -1407,14 +1405,14 @@ int build_ngrid(hsmc_gpu_ctx *ctx, int replica, double cut, int slot0, NGrid &g)
   g.ix = 1.0 / sx; g.iy = 1.0 / sy; g.iz = 1.0 / sz;
   g.lx = h.p.lx; g.ly = h.p.ly; g.lz = h.p.lz;
   g.start = start;
-  g.px = pos; g.py = pos + N; g.pz = pos + 2 * (size_t)N;
+  g.p = pos;
   if (cached) return HSMC_OK;
   HSMC_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * 2 * (C + 1), ctx->stream));
   hipLaunchKernelGGL(k_grid_count2, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z, N,
                      nx, ny, nz, g.ix, g.iy, g.iz, cnt, cellof);
   exclusive_scan(ctx->stream, cnt, (int)C, start, part, false);
   hipLaunchKernelGGL(k_grid_scatter2, dim3((N + 255) / 256), dim3(256), 0, ctx->stream, x, y, z,
-                     N, cellof, start, fill, pos, pos + N, pos + 2 * (size_t)N);
+                     N, cellof, start, fill, pos);
   HSMC_HIP(ctx, hipGetLastError());
   ctx->ngrid_replica[which] = replica;
   ctx->ngrid_version[which] = ctx->version;
@@ -1425,7 +1423,8 @@ int build_ngrid(hsmc_gpu_ctx *ctx, int replica, double cut, int slot0, NGrid &g)
 // The rows of n points.  From kSortRows points on, and at least one for each
 // cell, in the order of their cells, kSortChunk points at a time (which bounds
 // the workspace); their ranks lie where their targets will be.  A call with
-// one pass over n points at N = 4000, unsorted and sorted: 2^15 points 104 and
+// one pass over n points at N = 4000, unsorted and sorted (with the positions
+// in three arrays; both 5 to 15 % faster as records): 2^15 points 104 and
 // 118 us (the sort's three launches), 2^17 273 and 163, 2^20 1911 and 648; at
 // N = 32000 128 and 121, 378 and 173, 2794 and 700; at N = 108, where the few
 // cells' spheres stay in the first cache either way, 89 and 119, 154 and 162,
