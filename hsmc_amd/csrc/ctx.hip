@@ -39,13 +39,20 @@ void *scratch(hsmc_gpu_ctx *ctx, int slot, size_t bytes) {
   return ctx->scratch[slot];
 }
 
+// Two chunks of rows and an error word.
+static size_t rows_bytes(int chunk) { return 32 * 2 * (size_t)chunk + sizeof(unsigned long long); }
+
+static void free_pinned(hsmc_gpu_ctx *ctx, int slot) {
+  if (ctx->pin[slot] != ctx->first_rows) (void)hipHostFree(ctx->pin[slot]);
+  ctx->pin[slot] = nullptr;
+  ctx->pin_bytes[slot] = 0;
+}
+
 void *pinned(hsmc_gpu_ctx *ctx, PinnedSlot slot, size_t bytes) {
   if (ctx->pin_bytes[slot] >= bytes) return ctx->pin[slot];
   if (ctx->pin[slot]) {
     (void)hipStreamSynchronize(ctx->stream);
-    (void)hipHostFree(ctx->pin[slot]);
-    ctx->pin[slot] = nullptr;
-    ctx->pin_bytes[slot] = 0;
+    free_pinned(ctx, slot);
   }
   const size_t want = bytes + bytes / 4;
   if (hipHostMalloc(&ctx->pin[slot], want, hipHostMallocDefault) != hipSuccess) {
@@ -476,19 +483,23 @@ int hsmc_gpu_create(hsmc_gpu_ctx **out, int device, int n_replicas,
       hipMalloc(&ctx->d_z, sizeof(double) * ptot) != hipSuccess ||
       hipMalloc(&ctx->d_sweep, sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc(&ctx->d_err, sizeof(unsigned int)) != hipSuccess ||
-      hipMalloc(&ctx->d_bar, 2 * sizeof(unsigned int)) != hipSuccess ||
-      hipHostMalloc((void **)&ctx->h_acc, sizeof(unsigned long long) * kResults,
-                    hipHostMallocDefault) != hipSuccess)
+      hipMalloc(&ctx->d_bar, 2 * sizeof(unsigned int)) != hipSuccess)
     return fail(HSMC_ERR_NO_MEMORY);
+  {
+    int n_max = 0;
+    for (int r = 0; r < n_replicas; ++r) n_max = std::max(n_max, (int)replicas[r].n_part);
+    const size_t o_err = (sizeof(unsigned long long) * kResults + 63) / 64 * 64, o_rows = o_err + 64;
+    const size_t first = rows_bytes(std::min(n_max, kRowChunk));
+    if (hipHostMalloc((void **)&ctx->pin_first, o_rows + first, hipHostMallocDefault) != hipSuccess)
+      return fail(HSMC_ERR_NO_MEMORY);
+    ctx->h_acc = (unsigned long long *)ctx->pin_first;
+    ctx->h_err = (volatile unsigned int *)(ctx->pin_first + o_err);
+    *ctx->h_err = 0u;
+    ctx->pin[P_ROWS] = ctx->first_rows = ctx->pin_first + o_rows;
+    ctx->pin_bytes[P_ROWS] = first;
+  }
   if (hipDeviceGetAttribute(&ctx->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
     return fail(HSMC_ERR_HIP);
-  {
-    void *pinned = nullptr;
-    if (hipHostMalloc(&pinned, sizeof(unsigned int), hipHostMallocDefault) != hipSuccess)
-      return fail(HSMC_ERR_NO_MEMORY);
-    ctx->h_err = (volatile unsigned int *)pinned;
-    *ctx->h_err = 0u;
-  }
   if (hipMemcpy(ctx->d_prep, prep.data(), sizeof(int) * ptot, hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(ctx->d_sweep, 0, sizeof(unsigned long long)) != hipSuccess ||
       hipMemset(ctx->d_swp, 0, sizeof(SweepDev) * std::max(n_replicas, kSweepTable)) != hipSuccess ||
@@ -515,10 +526,9 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
     if (b) (void)hipFree(b);
   for (int i = 0; i < hsmc_gpu_ctx::kScratch; ++i)
     if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
-  if (ctx->h_err) (void)hipHostFree((void *)ctx->h_err);
-  if (ctx->h_acc) (void)hipHostFree(ctx->h_acc);
-  for (void *p : ctx->pin)
-    if (p) (void)hipHostFree(p);
+  for (int i = 0; i < hsmc_gpu_ctx::kPinned; ++i)
+    if (ctx->pin[i]) free_pinned(ctx, i);
+  if (ctx->pin_first) (void)hipHostFree(ctx->pin_first);
   if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
   if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -544,7 +554,7 @@ int hsmc_gpu_upload(hsmc_gpu_ctx *ctx, int replica, const double *conf4) {
     }
   }
   const int chunk = std::min(n, kRowChunk);
-  double4 *rows = (double4 *)pinned(ctx, P_ROWS, sizeof(double4) * 2 * (size_t)chunk + sizeof(unsigned long long));
+  double4 *rows = (double4 *)pinned(ctx, P_ROWS, rows_bytes(chunk));
   if (!rows) return HSMC_ERR_NO_MEMORY;
   const hipEvent_t ev[2] = {ctx->ev0, ctx->ev1};
   for (int first = 0, c = 0; first < n; first += chunk, ++c) {
@@ -566,7 +576,7 @@ int hsmc_gpu_download(hsmc_gpu_ctx *ctx, int replica, double *conf4) {
   if (!ctx || replica < 0 || replica >= ctx->R || !conf4) return HSMC_ERR_BAD_ARG;
   const RepHost &h = ctx->reps[replica];
   const int n = h.p.n_part, chunk = std::min(n, kRowChunk);
-  double4 *rows = (double4 *)pinned(ctx, P_ROWS, sizeof(double4) * 2 * (size_t)chunk + sizeof(unsigned long long));
+  double4 *rows = (double4 *)pinned(ctx, P_ROWS, rows_bytes(chunk));
   if (!rows) return HSMC_ERR_NO_MEMORY;
   unsigned long long *err = (unsigned long long *)(rows + 2 * (size_t)chunk);
   const hipEvent_t ev[2] = {ctx->ev0, ctx->ev1};
