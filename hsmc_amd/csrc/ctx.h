@@ -163,6 +163,10 @@ struct hsmc_gpu_ctx {
   // far as the resident kernel made them (a counter takes at most
   // 2^32 attempts)
   unsigned long long resident_sweeps = 0;
+  // and how many of them make it fold: an entry gathers the attempts of
+  // C / 8 / groups cells, below 256 a sweep, so 2^24 sweeps stay below 2^32
+  // (a test lowers it)
+  unsigned long long fold_sweeps = 1ull << 24;
   // the launched sweeps' count buffers may hold an earlier sweep's counts
   // (the resident kernel ran, or the sweep counter moved)
   bool counts_stale = false;

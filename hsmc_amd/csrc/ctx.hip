@@ -536,6 +536,14 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
   return HSMC_OK;
 }
 
+// For tests, not part of the interface (include/hsmc_gpu.h): the number of
+// resident sweeps after which the move counters are folded.
+int hsmc_gpu_test_fold_sweeps(hsmc_gpu_ctx *ctx, uint64_t sweeps) {
+  if (!ctx || sweeps == 0) return HSMC_ERR_BAD_ARG;
+  ctx->fold_sweeps = sweeps;
+  return HSMC_OK;
+}
+
 int hsmc_gpu_sync(hsmc_gpu_ctx *ctx) {
   if (!ctx) return HSMC_ERR_BAD_ARG;
   return check_device_errors(ctx);  // waits for the stream

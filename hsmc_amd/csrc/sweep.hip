@@ -941,11 +941,10 @@ int run_sweeps(hsmc_gpu_ctx *ctx, int n) {
     for (int done = 0; done < n; done += per) {
       if (*ctx->h_err) return check_device_errors(ctx);
       const int k = std::min(per, n - done);
-      // a counter entry gathers the attempts of C / 8 / groups cells, below
-      // 256 a sweep: 2^24 sweeps stay below 2^32
-      if (ctx->resident_sweeps + k > (1u << 24)) {
+      if (ctx->resident_sweeps + k > ctx->fold_sweeps) {
         int st = fold_counters(ctx);
         if (st) return st;
+        ctx->folded = false;  // the sweeps launched now are not in the totals
       }
       int st = launch_resident(ctx, shape, ctx->sweep_now, k);
       if (st) return st;

@@ -1,6 +1,8 @@
 """Sweeps of small systems in one launch (a system per workgroup, in LDS):
 the trajectory, counters and errors of the oracle's restatement and of the
 launched kernels, over the shapes the kernel treats apart."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -128,3 +130,32 @@ def test_overfull_cells_are_reported(tuned):
     other.sync()
     other.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("calls,fold", [((60, 60, 60), 100), ((9000,), 5000)])
+def test_counters_across_a_fold_between_launches(calls, fold):
+    """The 32-bit counters are folded into the totals before they could
+    overflow (every 2^24 sweeps; lowered here): sweeps launched after that,
+    in the same call, count too, and a reset takes them along."""
+    systems = [_melted((3, 3, 3), 0.7, 6), _melted((2, 2, 6), 0.42, 7)]
+    reps = [dict(n=len(c), box=b, dr_max=0.15, seed=40 + k) for k, (c, b) in enumerate(systems)]
+    ctxs = [gpu.Context(reps) for _ in range(2)]
+    resident, launched = ctxs
+    launched.set_tuning(32, 4, 64)
+    assert gpu.load().hsmc_gpu_test_fold_sweeps(resident.h, C.c_uint64(fold)) == 0
+    for ctx in ctxs:
+        for r, (conf, _) in enumerate(systems):
+            ctx.upload(conf, r)
+        for n in calls:
+            ctx.sweeps(n)
+    for r in (0, 1):
+        assert resident.counters(r) == launched.counters(r), r
+    for ctx in ctxs:
+        for n in calls:
+            ctx.sweeps(n)
+        ctx.reset_counters()
+        ctx.sweeps(3)
+    for r in (0, 1):
+        assert resident.counters(r) == launched.counters(r), r
+    for ctx in ctxs:
+        ctx.close()
