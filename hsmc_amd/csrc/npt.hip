@@ -525,11 +525,13 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
                        (const VolPlan *)host, (const VolNode *)(host + o_node), ctx->d_x, ctx->d_y, ctx->d_z,
                        (int *)(host + o_res));
     HSMC_HIP(ctx, hipGetLastError());
+    // a sweep that cannot be enqueued (an error of the last one, say) is
+    // reported once the moves above are taken in: they are done on the device
+    int sweep_status = HSMC_OK;
     if (keeps) {
       HSMC_HIP(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-      int st = run_sweeps(ctx, 1);
-      if (st) return st;
-      *ahead = true;
+      sweep_status = run_sweeps(ctx, 1);
+      *ahead = sweep_status == HSMC_OK;
       HSMC_HIP(ctx, hipEventSynchronize(ctx->ev0));
     } else {
       HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -555,6 +557,7 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
       int st = boxes_changed(ctx);
       if (st) return st;
     }
+    if (sweep_status) return sweep_status;
   }
   return HSMC_OK;
 }

@@ -326,3 +326,35 @@ def test_npt_sweeps_in_one_call_equal_single_sweeps(dv):
         assert a.counters(r) == b.counters(r), r
     a.close()
     b.close()
+
+
+def test_boxes_after_a_call_that_fails():
+    """A cell overflow of one replica ends the call; the volume moves done on
+    the device by then are in the boxes that the host reports: a configuration
+    uploaded in them is swept as in a fresh context of those boxes."""
+    specs = [(4, 0.60, 60 + k, 0.1) for k in range(8)]
+    ctx = make(specs)
+    conf, box0 = gpu.lattice(2, 4, 0.60)
+    over = conf.copy()
+    over[:40, 1:] = 3.0 + 0.1 * np.random.default_rng(1).random((40, 3))
+    ctx.upload(over, 0)
+    with pytest.raises(gpu.HsmcError) as e:
+        ctx.npt_sweeps(20, 3.0, 0.05)
+    assert e.value.code == -1
+    boxes = [ctx.box(r) for r in range(ctx.R)]
+    assert any(b != tuple(box0) for b in boxes)
+    fresh = gpu.Context([dict(n=256, box=b, dr_max=0.1, seed=60 + r) for r, b in enumerate(boxes)])
+    fresh.set_sweep_counter(ctx.counters()["sweeps"])
+    for r, b in enumerate(boxes):
+        scaled = conf.copy()
+        scaled[:, 1:] *= np.array(b) / np.array(box0)
+        ctx.upload(scaled, r)
+        fresh.upload(scaled, r)
+    for sweeps in (lambda c: c.sweeps(5), lambda c: c.npt_sweeps(5, 3.0, 0.02)):
+        for c in (ctx, fresh):
+            sweeps(c)
+        for r in range(ctx.R):
+            assert ctx.box(r) == fresh.box(r), r
+            assert np.array_equal(ctx.download(r), fresh.download(r)), r
+    ctx.close()
+    fresh.close()
