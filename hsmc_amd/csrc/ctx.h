@@ -206,6 +206,7 @@ struct hsmc_gpu_ctx {
   static constexpr int kScratch = 44;
   void *scratch[kScratch] = {};
   size_t scratch_bytes[kScratch] = {};
+  size_t scratch_limit = ~(size_t)0;  // a larger one counts as refused (a test lowers it)
 };
 
 namespace hsmc {

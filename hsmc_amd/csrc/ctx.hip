@@ -31,7 +31,7 @@ void *scratch(hsmc_gpu_ctx *ctx, int slot, size_t bytes) {
     ctx->scratch_bytes[slot] = 0;
   }
   size_t want = bytes + bytes / 4;
-  if (hipMalloc(&ctx->scratch[slot], want) != hipSuccess) {
+  if (bytes > ctx->scratch_limit || hipMalloc(&ctx->scratch[slot], want) != hipSuccess) {
     ctx->last_error = "scratch allocation failed";
     return nullptr;
   }
@@ -537,10 +537,17 @@ int hsmc_gpu_destroy(hsmc_gpu_ctx *ctx) {
 }
 
 // For tests, not part of the interface (include/hsmc_gpu.h): the number of
-// resident sweeps after which the move counters are folded.
+// resident sweeps after which the move counters are folded, and the largest
+// device workspace that is not refused.
 int hsmc_gpu_test_fold_sweeps(hsmc_gpu_ctx *ctx, uint64_t sweeps) {
   if (!ctx || sweeps == 0) return HSMC_ERR_BAD_ARG;
   ctx->fold_sweeps = sweeps;
+  return HSMC_OK;
+}
+
+int hsmc_gpu_test_scratch_limit(hsmc_gpu_ctx *ctx, uint64_t bytes) {
+  if (!ctx) return HSMC_ERR_BAD_ARG;
+  ctx->scratch_limit = bytes;
   return HSMC_OK;
 }
 

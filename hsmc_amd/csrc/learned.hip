@@ -1825,15 +1825,12 @@ int hsmc_gpu_widom_learned(hsmc_gpu_mlp *m, int replica, double voxel, double mi
     st = grids(&g);
     if (st) return st;
   } else {
+    // the shared buffers are overwritten: no network's cache stays valid, and
+    // this one's holds again once its last kernel is launched
+    m->sc_replica = -1;
+    ++ctx->score_stamp;
     st = launch_proposal_scores(ctx, replica, grids, vx, m->net, f, &pr);
     if (st) return st;
-    m->sc_replica = replica;
-    m->sc_version = ctx->version;
-    m->sc_step = m->step;
-    m->sc_voxel = voxel;
-    m->sc_nfree = pr.nfree;
-    m->sc_mix = -1.0;  // the cumulative mass is rebuilt below
-    m->sc_stamp = ++ctx->score_stamp;
   }
   // the cached proposal's flags and free list (the same scratch the scoring
   // wrote; the stamp check above guarantees nobody rewrote it since)
@@ -1843,12 +1840,14 @@ int hsmc_gpu_widom_learned(hsmc_gpu_mlp *m, int replica, double voxel, double mi
   double *stats = (double *)scratch(ctx, L_STATS, sizeof(double) * 3);
   if (!slots || !flag || !stats) return HSMC_ERR_NO_MEMORY;
   const int *list = slots + (size_t)tiles * 256;
-  const long nfree = m->sc_nfree;
+  const long nfree = scores_ok ? m->sc_nfree : pr.nfree;
   const long ncdf = std::max(1L, (nfree + 4095) / 4096);
   double *cdf = (double *)scratch(ctx, L_CDF, sizeof(double) * (size_t)std::max(1L, nfree));
   double *bsum = (double *)scratch(ctx, L_BSUM, sizeof(double) * (size_t)(ncdf + 1));
   if (!cdf || !bsum) return HSMC_ERR_NO_MEMORY;
-  if (m->sc_mix != mix && nfree > 0) {
+  const bool new_mass = !scores_ok || m->sc_mix != mix;
+  if (new_mass) m->sc_replica = -1;
+  if (new_mass && nfree > 0) {
     hipLaunchKernelGGL(k_cdf_local, dim3((unsigned)ncdf), dim3(1024), 0, ctx->stream, f, list, nfree,
                        pr.parts, pr.nparts, stats, mix, cdf, bsum);
     const dim3 add_blocks((unsigned)((nfree + 255) / 256));
@@ -1862,10 +1861,13 @@ int hsmc_gpu_widom_learned(hsmc_gpu_mlp *m, int replica, double voxel, double mi
     }
     HSMC_HIP(ctx, hipGetLastError());
   }
-  if (m->sc_mix != mix) {
-    m->sc_mix = mix;
-    m->sc_stamp = ++ctx->score_stamp;
-  }
+  m->sc_replica = replica;
+  m->sc_version = ctx->version;
+  m->sc_step = m->step;
+  m->sc_voxel = voxel;
+  m->sc_nfree = nfree;
+  m->sc_mix = mix;
+  if (new_mass) m->sc_stamp = ++ctx->score_stamp;
   // the network mass's total: the scan's last entry, or 0 with no free voxel
   const double *total = nfree > 0 ? bsum + ncdf : stats + 2;
   // one uniform offset per call for the systematic sample

@@ -2,6 +2,7 @@
 FP64 oracle (with the kernels' BF16 rounding points), descriptors against
 brute force, unbiasedness of the importance-weighted estimate, and the gain of
 the trained network over uniform insertion."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -401,4 +402,42 @@ def test_learned_widom_at_full_size():
     scale = max(1.0, float(np.max(np.abs(ref))))
     assert np.quantile(diff, 0.99) <= 1e-4 * scale, np.quantile(diff, 0.99)
     assert diff.max() <= 0.05 * scale, diff.max()
+    ctx.close()
+
+
+@pytest.mark.parametrize("voxel", [0.25, 0.15])
+def test_estimate_after_a_refused_workspace(voxel):
+    """A call that is refused the workspace of its cumulative mass leaves no
+    half-made proposal behind: the next call's estimate is a fresh context's,
+    also right after a call on another configuration (and where every voxel is
+    scored, voxel 0.15)."""
+    conf, box = gpu.lattice(2, 3, 0.9)
+    dilute, dbox = gpu.lattice(2, 4, 0.45)
+
+    def make():
+        ctx = gpu.Context([dict(n=len(conf), box=box, dr_max=0.05, seed=1),
+                           dict(n=len(dilute), box=dbox, dr_max=0.1, seed=2)])
+        ctx.upload(conf, 0)
+        ctx.upload(dilute, 1)
+        ctx.sweeps(30)
+        return ctx, gpu.Mlp(ctx, seed=4)
+
+    fresh, net = make()
+    want = net.widom(voxel, 0.9, 5, 1, 20000, r=1)
+    assert want["hits"] > 0
+    fresh.close()
+    ctx, net = make()
+    net.widom(0.25, 0.9, 5, 1, 20000, r=0)
+    _, n_free = net.proposal_scores(voxel, r=1)   # every other workspace is there now
+    limit = 30000
+    assert 8 * n_free > limit
+    refuse = gpu.load().hsmc_gpu_test_scratch_limit
+    for _ in range(2):
+        assert refuse(ctx.h, C.c_uint64(limit)) == 0
+        with pytest.raises(gpu.HsmcError) as e:
+            net.widom(voxel, 0.9, 5, 1, 20000, r=1)
+        assert e.value.code == -7
+    refuse(ctx.h, C.c_uint64(2 ** 63))
+    assert net.widom(voxel, 0.9, 5, 1, 20000, r=1) == want
+    assert net.widom(voxel, 0.9, 5, 1, 20000, r=1) == want
     ctx.close()
