@@ -33,6 +33,11 @@ void *scratch(hsmc_gpu_ctx *ctx, int slot, size_t bytes) {
   size_t want = bytes + bytes / 4;
   if (bytes > ctx->scratch_limit || hipMalloc(&ctx->scratch[slot], want) != hipSuccess) {
     ctx->last_error = "scratch allocation failed";
+    // what the slot held is gone: nothing kept in workspaces stays valid
+    // (grids, cell lists and proposals are kept by version)
+    ctx->version++;
+    ctx->edge_bins = 0;
+    ctx->counts_bytes = 0;
     return nullptr;
   }
   ctx->scratch_bytes[slot] = want;

@@ -1164,6 +1164,7 @@ int bin_edges(hsmc_gpu_ctx *ctx, double dr_bin, int nbins, const double **edge) 
   double *d = (double *)scratch(ctx, S_BINS, sizeof(double) * (nbins + 1));
   if (!d) return HSMC_ERR_NO_MEMORY;
   if (ctx->edge_bins < nbins || ctx->edge_dr != dr_bin) {
+    ctx->edge_bins = 0;  // until they are there
     std::vector<double> e(nbins + 1);
     for (int b = 0; b <= nbins; ++b) {
       const double r = b == 0 ? std::max(0.0, 1.0 - dr_bin) : 1.0 + b * dr_bin;

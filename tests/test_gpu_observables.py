@@ -3,6 +3,7 @@ where their kernels change: with and without a neighbour grid, tile edges of
 the all-pairs kernels, the 3^3 and 5^3 stencils and their fallback on thin
 boxes, bins by formula and by edges, spheres filed in LDS or in memory.
 Every result is compared with FP64 numpy over all pairs, bit for bit."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -268,4 +269,62 @@ def test_stratified_insertions_match_all_pairs(box, n, per_cell):
         d = np.minimum(d, np.array(box) - d)
         free &= ~((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2] < 1.0)
     assert points == len(q) and hits == int(free.sum())
+    ctx.close()
+
+
+def _refuse_above(ctx, limit):
+    assert gpu.load().hsmc_gpu_test_scratch_limit(ctx.h, C.c_uint64(limit)) == 0
+
+
+def _refused(call):
+    with pytest.raises(gpu.HsmcError) as e:
+        call()
+    assert e.value.code == -7
+
+
+def test_bin_edges_after_a_refused_workspace():
+    """Edges lost to a workspace that could not grow are made again (another
+    context's edges lie in the freed memory meanwhile)."""
+    conf, box = gpu.lattice(2, 6, 0.8)
+    ctx = gpu.Context([dict(n=len(conf), box=box, dr_max=0.1)])
+    ctx.upload(conf)
+    ctx.sweeps(20)
+    want, oor = ctx.rdf_counts(0.01, 100, 2.5)
+    assert want.sum() > 0 and oor > 0
+    _refuse_above(ctx, 4000)
+    _refused(lambda: ctx.rdf_counts(0.01, 1000, 2.5))
+    other = gpu.Context([dict(n=len(conf), box=box, dr_max=0.1)])
+    other.upload(conf)
+    other.rdf_counts(0.02, 100, 2.5)
+    other.close()
+    _refuse_above(ctx, 2 ** 63)
+    got, out = ctx.rdf_counts(0.01, 100, 2.5)
+    assert np.array_equal(got, want) and out == oor
+    ctx.close()
+
+
+def test_grids_after_a_refused_workspace():
+    """A grid that a larger replica's refused one has displaced is built again:
+    search grid, its cleared counts, and the descriptors' grid."""
+    small, sbox = gpu.lattice(2, 3, 0.7)
+    large, lbox = gpu.lattice(2, 12, 0.7)
+    ctx = gpu.Context([dict(n=len(small), box=sbox), dict(n=len(large), box=lbox)])
+    ctx.upload(small, 0)
+    ctx.upload(large, 1)
+    q = np.random.default_rng(3).random((500, 3)) * np.array(sbox)
+    free, desc = ctx.widom_points(q, 0), gpu.point_descriptors(ctx, q, 0)
+    part_cell, _ = ctx.cell_list((4, 4, 4), 12, 0)
+    ctx.widom_points(q, 0)
+    # each limit lets some of the larger grid's buffers through
+    for limit in (3000, 9000, 20000, 40000, 50000):
+        _refuse_above(ctx, limit)
+        _refused(lambda: ctx.widom_points(q, 1))
+        _refused(lambda: gpu.point_descriptors(ctx, q, 1))
+        _refused(lambda: ctx.cell_list((20, 20, 20), 12, 1))
+        _refuse_above(ctx, 2 ** 63)
+        assert np.array_equal(ctx.widom_points(q, 0), free)
+        assert np.array_equal(gpu.point_descriptors(ctx, q, 0), desc)
+        assert np.array_equal(ctx.cell_list((4, 4, 4), 12, 0)[0], part_cell)
+        assert np.array_equal(ctx.widom_points(q, 0), free)
+    assert ctx.any_overlap_scaled([0.999], 1)[0] == 1
     ctx.close()
