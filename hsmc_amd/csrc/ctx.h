@@ -51,8 +51,8 @@ struct RepDev {
 };
 
 // Results of an observable: a histogram's bins (at most 8192) and its
-// out-of-range count.
-constexpr int kResults = 8192 + 1;
+// out-of-range count (two words).
+constexpr int kResults = 8192 + 2;
 
 // Entries of the one-replica sweep table: one per sweep of a batch (at most
 // 512 sweeps per graph) and one past the last.

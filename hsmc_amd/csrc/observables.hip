@@ -714,7 +714,7 @@ __device__ __forceinline__ void hist_begin(const Bins &bn, unsigned int *hist) {
 
 template <bool EDGES>
 __device__ __forceinline__ void bin_pair(const Bins &bn, unsigned int *hist, double s,
-                                         unsigned int &bad) {
+                                         unsigned long long &bad) {
   if (!(s < bn.smax)) return;
   int b;
   bool in;
@@ -739,13 +739,18 @@ __device__ __forceinline__ void bin_pair(const Bins &bn, unsigned int *hist, dou
     ++bad;
 }
 
-// The workgroup's counts, and its pairs out of the bins' range, in its row.
-__device__ __forceinline__ void hist_end(const Bins &bn, const unsigned int *hist, unsigned int bad,
+// The workgroup's counts, and its pairs out of the bins' range, in its row:
+// these in two words, as one workgroup can meet more than 2^32 of them (a cell
+// of a cutoff of 0.4 box edges at N = 2 * 10^6).
+__device__ __forceinline__ void hist_end(const Bins &bn, const unsigned int *hist, unsigned long long bad,
                                          unsigned int *__restrict__ part) {
-  unsigned int *row = part + (size_t)blockIdx.x * (bn.n + 1);
+  unsigned int *row = part + (size_t)blockIdx.x * (bn.n + 2);
   const unsigned long long out = block_sum_u64(bad);  // with the barrier before the counts are read
   for (int b = threadIdx.x; b < bn.n; b += blockDim.x) row[b] = hist[b];
-  if (threadIdx.x == 0) row[bn.n] = (unsigned int)out;
+  if (threadIdx.x == 0) {
+    row[bn.n] = (unsigned int)out;
+    row[bn.n + 1] = (unsigned int)(out >> 32);
+  }
 }
 
 // Scale factors of one scan, passed by value (no host-to-device copy).
@@ -826,7 +831,7 @@ k_hist_all(const double *__restrict__ x, const double *__restrict__ y, const dou
            int n, double lx, double ly, double lz, Bins bn, unsigned int *__restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) unsigned int hist[];
   hist_begin(bn, hist);
-  unsigned int bad = 0;
+  unsigned long long bad = 0;
   all_pairs<JC>(x, y, z, n, lx, ly, lz, [&](double s, double, double, double, double, double, double) {
     bin_pair<EDGES>(bn, hist, s, bad);
   });
@@ -934,7 +939,7 @@ __global__ void __launch_bounds__(kRowThreads)
 k_hist_rows(Grid g, Bins bn, unsigned int *__restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) unsigned int hist[];
   hist_begin(bn, hist);
-  unsigned int bad = 0;
+  unsigned long long bad = 0;
   row_pairs<S>(g, [&](double s, double, double, double, double, double, double) {
     bin_pair<EDGES>(bn, hist, s, bad);
   });
@@ -973,7 +978,7 @@ __global__ void __launch_bounds__(256)
 k_hist_spheres(Grid g, int n, Bins bn, unsigned int *__restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) unsigned int hist[];
   hist_begin(bn, hist);
-  unsigned int bad = 0;
+  unsigned long long bad = 0;
   sphere_pairs(g, n, [&](double s, double, double, double, double, double, double) {
     bin_pair<EDGES>(bn, hist, s, bad);
   });
@@ -1534,7 +1539,7 @@ static int pair_hist(hsmc_gpu_ctx *ctx, int replica, double dr_bin, int nbins, d
                      (edges ? sizeof(double) * ((size_t)nbins + 1) : 0);
   unsigned blocks;
   auto rows_of = [&]() {
-    return (unsigned int *)scratch(ctx, S_OUT0, sizeof(unsigned int) * ((size_t)nbins + 1) * blocks);
+    return (unsigned int *)scratch(ctx, S_OUT0, sizeof(unsigned int) * ((size_t)nbins + 2) * blocks);
   };
   unsigned int *part;
   if (N <= (rmax_eff < kWide ? kAllPairs : kAllPairsWide)) {
@@ -1569,10 +1574,10 @@ static int pair_hist(hsmc_gpu_ctx *ctx, int replica, double dr_bin, int nbins, d
     }
   }
   HSMC_HIP(ctx, hipGetLastError());
-  int st = sum_rows(ctx, part, (int)blocks, nbins + 1);
+  int st = sum_rows(ctx, part, (int)blocks, nbins + 2);
   if (st) return st;
   for (int b = 0; b < nbins; ++b) counts[b] = (int64_t)ctx->h_acc[b];
-  if (oor) *oor = (int64_t)ctx->h_acc[nbins];
+  if (oor) *oor = (int64_t)(ctx->h_acc[nbins] + (ctx->h_acc[nbins + 1] << 32));
   return HSMC_OK;
 }
 

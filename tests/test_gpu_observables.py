@@ -328,3 +328,25 @@ def test_grids_after_a_refused_workspace():
         assert np.array_equal(ctx.widom_points(q, 0), free)
     assert ctx.any_overlap_scaled([0.999], 1)[0] == 1
     ctx.close()
+
+
+def test_out_of_range_pairs_beyond_32_bits_in_one_workgroup():
+    """N = 128^3 on a lattice, cutoff 0.4 of the edge: each of the 125 cells'
+    workgroups meets 4.7 * 10^9 pairs within the cutoff, nearly all beyond the
+    bins.  Every site sees the same distances, so the pairs of one make the
+    count."""
+    n, a = 128, 1.05
+    L = n * a
+    cells = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    ctx = _context(cells * a, (L, L, L))
+    rmax, nbins, dr_bin = 0.39991 * L, 20, 0.02   # bins to 1.4: the first neighbours, at 1.05
+    counts, oor = ctx.rdf_counts(dr_bin, nbins, rmax)
+    m = np.minimum(np.arange(n), n - np.arange(n)).astype(float) * a
+    r = np.sqrt(m[:, None, None] ** 2 + m[None, :, None] ** 2 + m[None, None, :] ** 2).ravel()
+    assert np.abs(r - rmax).min() > 1e-6
+    within = int((r < rmax).sum()) - 1
+    assert counts[2] == 3 * n ** 3 and counts.sum() == 3 * n ** 3
+    total = n ** 3 * within // 2
+    assert total // 125 > 2 ** 32
+    assert oor == total - 3 * n ** 3
+    ctx.close()
