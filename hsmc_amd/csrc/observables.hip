@@ -862,6 +862,7 @@ k_scaled_all(const double *__restrict__ x, const double *__restrict__ y, const d
 // per pair of cells 5 wide and each pair binned by square root and division).
 // (Four cells a workgroup of 1024 left fewer counts to add up but 75 us of
 // uneven work where single cells take 53.)
+// At most kRowBlocks workgroups, and so rows of counts: 67 MB with 8192 bins.
 constexpr int kRowThreads = 256, kRowBlocks = 2048;
 
 template <int S, class F>
@@ -960,17 +961,17 @@ k_scaled_rows(Grid g, SfTable sf, int nsf, double cut2,
 // thread per sphere walks the distinct cells of its 27-cell stencil.
 template <class F>
 __device__ __forceinline__ void sphere_pairs(const Grid &g, int n, F &&f) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
-  const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
-  for_stencil(g, cx, cy, cz, [&](int b, int e) {
-    for (int q = max(b, p + 1); q < e; ++q) {  // each unordered pair once
-      const double bx = g.px[q], by = g.py[q], bz = g.pz[q];
-      f(dist2(ax, ay, az, bx, by, bz, g.lx, g.ly, g.lz), ax, ay, az, bx, by, bz);
-    }
-    return false;
-  });
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
+    const double ax = g.px[p], ay = g.py[p], az = g.pz[p];
+    const int cx = search_cell(ax, g.ix, g.nx), cy = search_cell(ay, g.iy, g.ny), cz = search_cell(az, g.iz, g.nz);
+    for_stencil(g, cx, cy, cz, [&](int b, int e) {
+      for (int q = max(b, p + 1); q < e; ++q) {  // each unordered pair once
+        const double bx = g.px[q], by = g.py[q], bz = g.pz[q];
+        f(dist2(ax, ay, az, bx, by, bz, g.lx, g.ly, g.lz), ax, ay, az, bx, by, bz);
+      }
+      return false;
+    });
+  }
 }
 
 template <bool EDGES>
@@ -1471,7 +1472,7 @@ int hsmc_gpu_any_overlap_scaled(hsmc_gpu_ctx *ctx, int replica, const double *sf
     int st = build_grid(ctx, replica, rows ? side : cut, g);
     if (st) return st;
     const long C = (long)g.nx * g.ny * g.nz;
-    blocks = rows ? (unsigned)std::min(C, (long)kRowBlocks) : (unsigned)((N + 255) / 256);
+    blocks = (unsigned)std::min(rows ? C : ((long)N + 255) / 256, (long)kRowBlocks);
     part = (unsigned long long *)scratch(ctx, S_OUT0, sizeof(unsigned long long) * blocks);
     if (!part) return HSMC_ERR_NO_MEMORY;
     if (rows)
@@ -1561,7 +1562,7 @@ static int pair_hist(hsmc_gpu_ctx *ctx, int replica, double dr_bin, int nbins, d
     int st = build_grid(ctx, replica, rows ? side : cut, g);
     if (st) return st;
     const long C = (long)g.nx * g.ny * g.nz;
-    blocks = rows ? (unsigned)std::min(C, (long)kRowBlocks) : (unsigned)((N + 255) / 256);
+    blocks = (unsigned)std::min(rows ? C : ((long)N + 255) / 256, (long)kRowBlocks);
     part = rows_of();
     if (!part) return HSMC_ERR_NO_MEMORY;
     if (rows) {

@@ -350,3 +350,17 @@ def test_out_of_range_pairs_beyond_32_bits_in_one_workgroup():
     assert total // 125 > 2 ** 32
     assert oor == total - 3 * n ** 3
     ctx.close()
+
+
+def test_rows_of_counts_are_bounded_on_thin_boxes():
+    """N = 528000 on a box of 2 search cells across (a thread per sphere): the
+    workgroups' rows of 8192 bins stay within 2048, and every sphere is
+    reached."""
+    n, a = 33000, 1.05
+    cells = np.stack(np.meshgrid(np.arange(4), np.arange(4), np.arange(n), indexing="ij"), -1).reshape(-1, 3)
+    ctx = _context(cells * a, (4 * a, 4 * a, n * a))
+    _refuse_above(ctx, 2048 * 8194 * 4)
+    counts, oor = ctx.rdf_counts(0.0001, 8192, 1.3)
+    assert counts[500] + counts[499] == 3 * len(cells) == counts.sum() and oor == 0
+    assert ctx.any_overlap_scaled([1.0, 0.96, 0.95]).tolist() == [1, 1, 0]
+    ctx.close()
