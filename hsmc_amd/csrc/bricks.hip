@@ -338,9 +338,20 @@ k_brick_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev 
       const int p1 = b1 - l0, p2 = b2 + ql - 4 * l01;
       int T = len + __shfl_xor(len, 1, 4);
       T += __shfl_xor(T, 2, 4);
-      if (T > lcap) {  // the capacity of the other kernels' stencil list
-        if (ql == 0) atomicOr(err, kErrListFull);
-        nc = 0;
+      if (T > lcap) {
+        // the capacity of the other kernels' stencil list, which holds a cell
+        // once where an axis has two (the region has it before and after)
+        int once = 0;
+#pragma unroll 1
+        for (int j = 0; j < 27; ++j) {
+          const int dx = j / 9 - 1, dy = j / 3 % 3 - 1, dz = j % 3 - 1, i = i0 + (dx * ry + dy) * rz + dz;
+          if (stencil_axis_ok(dx, rp.gx) && stencil_axis_ok(dy, rp.gy) && stencil_axis_ok(dz, rp.gz))
+            once += start[i + 1] - start[i];
+        }
+        if (once > lcap) {
+          if (ql == 0) atomicOr(err, kErrListFull);
+          nc = 0;
+        }
       }
       unsigned n_acc = 0, n_left = 0, moved = 0;
 #pragma unroll 1

@@ -133,3 +133,15 @@ def test_autotune_times_the_bricks():
     rng = np.random.default_rng(6)
     confs, boxes = _with_bulk(rng, [(9.0, 9.0, 9.0)], [0.8])
     _same(*_both(confs, boxes, after=lambda ctx: ctx.autotune(4)))
+
+
+def test_full_stencils_on_two_cell_axes():
+    """2 x 2 x 2 cells: a stencil has each cell once, and no more spheres than
+    there are, though the brick's neighbourhood meets a cell up to 8 times.  16
+    spheres of 20 lie in one cell and 4 in the one across the corner (they
+    overlap, so that they stay): 128 + 4 meetings of 20 spheres, for a list of
+    128."""
+    rng = np.random.default_rng(7)
+    confs, boxes = _with_bulk(rng, [(2.9, 2.9, 2.9)] * 8, [0.5] * 8)
+    confs[:8] = [np.vstack([0.1 * rng.random((16, 3)), 1.45 + 0.1 * rng.random((4, 3))]) for _ in range(8)]
+    _same(*_both(confs, boxes, sweeps=(10, 2)))
