@@ -23,9 +23,9 @@
 //
 // LDS holds each sphere's position in the brick's own frame in FP32, one
 // 16-byte read a test and no minimum image.  A squared distance outside
-// 1 -+ kBand decides; one inside, or any where a sphere lies outside its cell
-// (and so outside the box), is decided by the reference's FP64 arithmetic on
-// the FP64 positions, so every decision is the FP64 one: coordinates in the
+// 1 -+ kBand decides; one inside, or any where a sphere lies (or a step may
+// lead) outside the box, is decided by the reference's FP64 arithmetic on the
+// FP64 positions, so every decision is the FP64 one: coordinates in the
 // frame stay below 32 diameters, so each is within 9.6e-7 of its value, a
 // difference within 2e-6 (with its rounding), and the squared distance
 // within 2 (|dx| + |dy| + |dz|) 2e-6 < 7.2e-6 of its own near 1.
@@ -61,6 +61,12 @@ static_assert(kRegion <= 2048, "a region cell's index has 11 bits");
 __device__ __forceinline__ int here(int v) {
   asm volatile("" : "+s"(v));
   return v;
+}
+
+// Whether v lies outside [0, L] by more than 2^-20 of L (a step wider than two
+// boxes leads there), by the high words: a negative number's is the larger.
+__device__ __forceinline__ bool outside(double v, double L) {
+  return (unsigned)__double2hiint(v) > (unsigned)__double2hiint(L);
 }
 
 template <int CAP>
@@ -155,7 +161,7 @@ k_brick_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev 
       cell_at[d][i] = wrap_index(first + i, g) * (d == 0 ? rp.gy * rp.gz : d == 1 ? rp.gz : 1);
     }
     if (tid < 4) bin[tid] = put_in[tid] = 0;
-    if (tid == 4) odd = 0;
+    if (tid == 4) odd = rp.dr_max > 2.0 * fmin(rp.lx, fmin(rp.ly, rp.lz));  // steps may end outside the box
     __syncthreads();
     // prefix sums of the region's counts, a cell to a lane: within chunks of
     // 64, then over the chunks; spheres in the low 16 bits and those of
@@ -222,16 +228,16 @@ k_brick_phase(const unsigned long long *__restrict__ sweep_base, const SweepDev 
         at = (m >> 11) * C + grid_cell(ix, iy, iz);
         return slot[(unsigned)at];
       };
-      auto place = [&](double v, int d, int i, double side, double L) {
+      auto place = [&](double v, int d, int i, double L) {
         const double off = v - centre[d][i], wrap = __builtin_fabs(off) > 0.5 * L ? __builtin_copysign(L, off) : 0.0;
-        if (!(__builtin_fabs(off - wrap) <= 0.75 * side)) odd = 1;
+        if (outside(v, L)) odd = 1;  // all others lie within half a side of the centre, or an edge from there
         return (float)(v - centre[d][0] - wrap);
       };
       auto put = [&](int e, const SlotRec &r, int ix, int iy, int iz, int at) {
         float4 v;
-        v.x = place(r.x, 0, ix, rp.sx, rp.lx);
-        v.y = place(r.y, 1, iy, rp.sy, rp.ly);
-        v.z = place(r.z, 2, iz, rp.sz, rp.lz);
+        v.x = place(r.x, 0, ix, rp.lx);
+        v.y = place(r.y, 1, iy, rp.ly);
+        v.z = place(r.z, 2, iz, rp.lz);
         v.w = __int_as_float(at);
         if (ix & iy & iz & 1) {
           const int a = first_att[((ix >> 1) * ny + (iy >> 1)) * nz + (iz >> 1)] + (map[e] >> 11);

@@ -145,3 +145,20 @@ def test_full_stencils_on_two_cell_axes():
     confs, boxes = _with_bulk(rng, [(2.9, 2.9, 2.9)] * 8, [0.5] * 8)
     confs[:8] = [np.vstack([0.1 * rng.random((16, 3)), 1.45 + 0.1 * rng.random((4, 3))]) for _ in range(8)]
     _same(*_both(confs, boxes, sweeps=(10, 2)))
+
+
+def test_steps_wider_than_the_box():
+    """A step of up to two box edges either way leaves spheres outside the box
+    (the wrap is a single one), some an edge away from where the reference's
+    minimum image sees them."""
+    rng = np.random.default_rng(8)
+    confs, boxes = _with_bulk(rng, [(4.2, 4.2, 4.2)] * 24, [0.2] * 24)
+    confs = [c if len(c) else np.zeros((1, 3)) for c in confs]
+
+    def wide(ctx):
+        for r in range(24):
+            ctx.set_dr_max(16.5, r)
+
+    a, b = _both(confs, boxes, sweeps=(2, 400), after=wide)
+    assert any((x[:, 1:] > 4.2).any() for x, _ in b[:24])
+    _same(a, b)
