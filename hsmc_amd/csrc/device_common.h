@@ -137,6 +137,15 @@ __host__ __device__ __forceinline__ int shifted_cell(double x, double shift, dou
   return c < g ? c : g - 1;
 }
 
+// The cell of that grid a sphere is filed in.  A position a side and more
+// below the shifted origin's image is left of the grid (steps wider than four
+// box edges lead there: the wrap is a single one) and goes to the first cell.
+__host__ __device__ __forceinline__ int filed_cell(double x, double shift, double L,
+                                                   double inv_side, int g) {
+  const int c = shifted_cell(x, shift, L, inv_side, g);
+  return c < 0 ? 0 : c;
+}
+
 // Cell of coordinate x on an unshifted grid (cell_part_idx, cell_list.c:244-246),
 // clamped into [0, g-1].
 __host__ __device__ __forceinline__ int plain_cell(double x, double side, int g) {

@@ -840,11 +840,13 @@ k_mark_blocked(const double *__restrict__ x, const double *__restrict__ y,
   const int kx = lane & 7;
   const int ixk = wrap_voxel(lx + kx, vx.mx);
   const double dxk = image_mag((ixk + 0.5) * vx.vx - px, b.lx);
-  const double dx2k = dxk * dxk;
+  const double dx2k = (unsigned)ixk < (unsigned)vx.mx ? dxk * dxk : INFINITY;
   const int iy = wrap_voxel(ly + (lane >> 3), vx.my), iz = wrap_voxel(lz + (lane & 7), vx.mz);
   const double dy = image_mag((iy + 0.5) * vx.vy - py, b.ly);
   const double dz = image_mag((iz + 0.5) * vx.vz - pz, b.lz);
-  const double dy2 = dy * dy, dz2 = dz * dz;
+  // (a sphere outside the box has candidates off the voxels: none of them)
+  const double dy2 = (unsigned)iy < (unsigned)vx.my ? dy * dy : INFINITY,
+               dz2 = (unsigned)iz < (unsigned)vx.mz ? dz * dz : INFINITY;
   const long col = (long)iy * vx.mz + iz, layer = (long)vx.my * vx.mz;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {

@@ -76,9 +76,9 @@ k_vol_overlap(const RepDev *__restrict__ reps, const SweepDev *__restrict__ swp,
   // last sweep's entry when there is one replica)
   const double shx = swp[r].shx, shy = swp[r].shy, shz = swp[r].shz;
   const double ax = x[i], ay = y[i], az = z[i];
-  const int cx = shifted_cell(ax, shx, rp.lx, rp.ix, rp.gx);
-  const int cy = shifted_cell(ay, shy, rp.ly, rp.iy, rp.gy);
-  const int cz = shifted_cell(az, shz, rp.lz, rp.iz, rp.gz);
+  const int cx = filed_cell(ax, shx, rp.lx, rp.ix, rp.gx);
+  const int cy = filed_cell(ay, shy, rp.ly, rp.iy, rp.gy);
+  const int cz = filed_cell(az, shz, rp.lz, rp.iz, rp.gz);
   const int me = i - rp.poff;
   // d = 13 is the own cell; d = 14..26 are the forward offsets.  The
   // answer does not depend on the order of the tests, so the 14 cells'

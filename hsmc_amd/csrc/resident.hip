@@ -141,10 +141,16 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
   }
   unsigned bad = 0;  // sticky error bits
   unsigned n_acc = 0, n_left = 0;
+  // the cell a position lies in, -1 left of the grid
   auto in_cell = [&](double px_, double py_, double pz_, const SweepDev &sw) {
-    return (shifted_cell(px_, sw.shx, rp.lx, rp.ix, rp.gx) * rp.gy +
-            shifted_cell(py_, sw.shy, rp.ly, rp.iy, rp.gy)) * rp.gz +
-           shifted_cell(pz_, sw.shz, rp.lz, rp.iz, rp.gz);
+    const int cx = shifted_cell(px_, sw.shx, rp.lx, rp.ix, rp.gx), cy = shifted_cell(py_, sw.shy, rp.ly, rp.iy, rp.gy),
+              cz = shifted_cell(pz_, sw.shz, rp.lz, rp.iz, rp.gz);
+    return (cx | cy | cz) < 0 ? -1 : (cx * rp.gy + cy) * rp.gz + cz;
+  };
+  auto file_cell = [&](double px_, double py_, double pz_, const SweepDev &sw) {
+    return (filed_cell(px_, sw.shx, rp.lx, rp.ix, rp.gx) * rp.gy +
+            filed_cell(py_, sw.shy, rp.ly, rp.iy, rp.gy)) * rp.gz +
+           filed_cell(pz_, sw.shz, rp.lz, rp.iz, rp.gz);
   };
   // an attempt's draw applied to its sphere at (bx, by, bz)
   auto trial = [&](uint32_t w1, uint32_t w2, uint32_t w3, double bx, double by, double bz,
@@ -174,7 +180,7 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
       const int i = tid + u * T;
       ci[u] = -1;
       if (i < N) {
-        const int c = in_cell(px[i], py[i], pz[i], sw);
+        const int c = file_cell(px[i], py[i], pz[i], sw);
         const int sl = atomicAdd(&cnt[c], 1);
         if (sl < CAP) {
           occ[c * CAP + sl] = (uint16_t)i;

@@ -65,9 +65,9 @@ __device__ __forceinline__ void rebin_one(int i, const RepDev *__restrict__ reps
     const RepDev rp = ONE ? rp0 : reps[rr];
     double shx, shy, shz;
     sweep_shift(rp, sweep, shx, shy, shz);
-    const int cx = shifted_cell(px, shx, rp.lx, rp.ix, rp.gx);
-    const int cy = shifted_cell(py, shy, rp.ly, rp.iy, rp.gy);
-    const int cz = shifted_cell(pz, shz, rp.lz, rp.iz, rp.gz);
+    const int cx = filed_cell(px, shx, rp.lx, rp.ix, rp.gx);
+    const int cy = filed_cell(py, shy, rp.ly, rp.iy, rp.gy);
+    const int cz = filed_cell(pz, shz, rp.lz, rp.iz, rp.gz);
     const int c = rp.coff + (cx * rp.gy + cy) * rp.gz + cz;
     const int sl = atomicAdd(&cnt[(size_t)buf * C + c], 1);
     if (sl < cap) {
@@ -508,16 +508,16 @@ __device__ __forceinline__ void file_next_sweep(int g, int P, int C, int phase, 
   int *cntn = cnt + (size_t)(par ^ 1) * C;
   SlotRec *slotn = slot_all + (size_t)(par ^ 1) * CAP * C;
   const int colour = (int)((cur.order >> (4 * phase)) & 0xFu);
-  const int cx = shifted_cell(ax, cur.shx, rp.lx, rp.ix, rp.gx);
-  const int cy = shifted_cell(ay, cur.shy, rp.ly, rp.iy, rp.gy);
-  const int cz = shifted_cell(az, cur.shz, rp.lz, rp.iz, rp.gz);
+  const int cx = filed_cell(ax, cur.shx, rp.lx, rp.ix, rp.gx);
+  const int cy = filed_cell(ay, cur.shy, rp.ly, rp.iy, rp.gy);
+  const int cz = filed_cell(az, cur.shz, rp.lz, rp.iz, rp.gz);
   const bool active = (((cx ^ colour) | (cy ^ (colour >> 1)) | (cz ^ (colour >> 2))) & 1) == 0;
   const bool af = g < P && !active;
   auto next_cell = [&](double px, double py, double pz) {
     return rp.coff +
-           (shifted_cell(px, nxt.shx, rp.lx, rp.ix, rp.gx) * rp.gy +
-            shifted_cell(py, nxt.shy, rp.ly, rp.iy, rp.gy)) * rp.gz +
-           shifted_cell(pz, nxt.shz, rp.lz, rp.iz, rp.gz);
+           (filed_cell(px, nxt.shx, rp.lx, rp.ix, rp.gx) * rp.gy +
+            filed_cell(py, nxt.shy, rp.ly, rp.iy, rp.gy)) * rp.gz +
+           filed_cell(pz, nxt.shz, rp.lz, rp.iz, rp.gz);
   };
   const int ca = next_cell(ax, ay, az), ct = next_cell(req.x, req.y, req.z);
   int s1 = 0, s2 = 0;

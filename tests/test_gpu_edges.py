@@ -138,3 +138,44 @@ def test_counters_are_current_after_every_kind_of_sweep():
     ctx.sweeps(2)
     assert ctx.counters()["attempts"] == 1000 and ctx.counters()["sweeps"] == sweeps + 2
     ctx.close()
+
+
+def _wide_steps(reps, confs, tuning):
+    ctx = gpu.Context(reps)
+    for r, c in enumerate(confs):
+        ctx.upload(c, r)
+    if tuning:
+        ctx.set_tuning(*tuning)
+    out = []
+    for _ in range(20):
+        ctx.sweeps(50)
+        out += [ctx.download(r) for r in range(len(reps))]
+    return ctx, out, [ctx.counters(r) for r in range(len(reps))], \
+        [ctx.any_overlap_scaled_batch(sf).tolist() for sf in (0.99, 0.9)]
+
+
+@pytest.mark.parametrize("replicas", [1, 3])
+def test_steps_of_many_box_edges(replicas):
+    """Steps of up to 5 box edges either way leave spheres far outside the box
+    and left of the sweep grid: they are filed in a cell of it all the same,
+    alike by every route, and the calls that follow read them in range."""
+    conf, box = gpu.lattice(2, 3, 0.45)
+    conf = conf[::18].copy()   # 6 spheres: no cell can hold too many
+    conf[:, 0] = np.arange(6)
+    reps = [dict(n=6, box=box, dr_max=10.0 * box[0], seed=3 + r) for r in range(replicas)]
+    runs = [_wide_steps(reps, [conf] * replicas, t) for t in (None, (32, 2, 0), (32, 8, 16), (64, 4, 0, 1))]
+    x = np.array(runs[0][1])[:, :, 1:]
+    assert x.min() < -box[0] and x.max() > 2 * box[0]
+    for run in runs[1:]:
+        assert np.array_equal(np.array(run[1])[:, :, 1:], x)
+        assert run[2:] == runs[0][2:]
+    ctx = runs[0][0]
+    net = gpu.Mlp(ctx, seed=1)
+    f, n_free = net.proposal_scores(0.25)
+    assert np.isneginf(f).sum() == len(f) - n_free
+    assert net.widom(0.25, 0.9, 1, 1, 20000)["n"] == 20000
+    ctx.widom_cells(1, 1, 100)
+    ctx.widom_uniform(1, 1, 0, 10000)
+    ctx.contact_counts(0.01, 5, 1.05)
+    for run in runs:
+        run[0].close()
