@@ -159,10 +159,11 @@ k_vol_apply(const int *__restrict__ blk, const int *__restrict__ prep, const Vol
 // One scan serves all the moves: the smallest squared distance s of any pair,
 // on a search grid filed in LDS whose cells cover the strongest compression
 // of the tree.  A move by sf makes an overlap when s sf^2 < 1, and an
-// accepted one scales s by sf^2; the rounding of coordinates and products
-// moves s by less than kNear (a coordinate's is 2^-53 of the box edge), and
-// only where s sf^2 lies within kNear of 1 are the pairs tested one by one
-// with the reference's arithmetic.  Latency-bound, 23 us for the 32 x N = 256
+// accepted one scales s by sf^2; only where s sf^2 lies within kNear, or
+// kNearEdge of the longest edge, of 1 are the pairs tested one by one with
+// the reference's arithmetic.  The rounding of the coordinates in up to 3
+// accepted moves (2^-53 of the edge each) and of the products moves s by less:
+// by 2 (|dx| + |dy| + |dz|) 6 2^-53 < 2.4e-15 of the edge near 1.  Latency-bound, 23 us for the 32 x N = 256
 // of the published table (40 us with a scan per move); a sweep's volume moves
 // took about 400 us as rounds of transfers and waits.
 constexpr int kVolDepth = 4;               // moves per launch at most
@@ -170,7 +171,7 @@ constexpr int kVolThreads = 1024;         // threads at most: one per sphere, 25
 constexpr int kVolPer = 4;                 // spheres per thread at most
 constexpr int kVolSpheres = kVolThreads * kVolPer;
 constexpr int kVolAxis = 16;               // search-grid cells per axis at most
-constexpr double kNear = 1e-9;             // for box edges up to 10^5
+constexpr double kNear = 1e-9, kNearEdge = 1e-14;
 
 struct VolPlan {
   int steps, first;  // moves of this launch and the replica's first node
@@ -297,11 +298,12 @@ k_volume_moves(RepDev *__restrict__ reps, const VolPlan *__restrict__ plan,
                   (1.0 + 1e-6) / (sf_min * sf_min));
   int cur = 0, bits = 0, moved = 0;
   for (int k = 0; k < steps; ++k) {
+    const double near = fmax(kNear, kNearEdge * fmax(lx, fmax(ly, lz)));
     const double sf = tree[cur].sf, after = s * sf * sf;
     bool hit = false;
     if (sf < 1.0) {  // an expansion makes no overlap
       hit = after < 1.0;
-      if (fabs(after - 1.0) < kNear) {
+      if (fabs(after - 1.0) < near) {
         file((1.0 / sf) * (1.0 + 1e-6));
         hit = least([&](double ax, double ay, double az, double bx, double by, double bz) {
                 return dist2_scaled(ax, ay, az, bx, by, bz, lx, ly, lz, sf);

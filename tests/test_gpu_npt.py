@@ -358,3 +358,109 @@ def test_boxes_after_a_call_that_fails():
             assert np.array_equal(ctx.download(r), fresh.download(r)), r
     ctx.close()
     fresh.close()
+
+
+def _philox(ctr, key):
+    c, (k0, k1) = list(ctr), key
+    for _ in range(10):
+        a, b = 0xD2511F53 * c[0], 0xCD9E8D57 * c[2]
+        c = [(b >> 32) ^ c[1] ^ k0, b & 0xFFFFFFFF, (a >> 32) ^ c[3] ^ k1, a & 0xFFFFFFFF]
+        k0, k1 = (k0 + 0x9E3779B9) & 0xFFFFFFFF, (k1 + 0xBB67AE85) & 0xFFFFFFFF
+    return c
+
+
+def _first_moves(seed, n, dv, box):
+    """Scale factors of the first sweep's volume moves of a replica of n
+    spheres, to the bit if every one is accepted."""
+    word = _philox((0, 0, 0, 0x4E505400), (seed, 0))[0]
+    p, k = 1.0 / (n + 1.0), 0
+    pk = cdf = (1.0 - p) ** n
+    while word * 2.0 ** -32 > cdf and k < n:
+        pk *= (n - k) / (k + 1) * p / (1.0 - p)
+        k += 1
+        cdf += pk
+    lx, ly, lz = box
+    out = []
+    for t in range(k):
+        u = _philox((0, 0, t + 1, 0x4E505400), (seed, 0))[0] / 4294967295.0
+        vol = lx * ly * lz
+        out.append(math.pow(math.exp(math.log(vol) + (u - 0.5) * dv) / vol, 1.0 / 3.0))
+        lx, ly, lz = lx * out[-1], ly * out[-1], lz * out[-1]
+    return out
+
+
+def _tie_contexts(confs, box, seed, dv, press):
+    """One sweep of the replicas by moves in one launch, and by rounds (beside
+    a replica of more than 4096 spheres).  The spheres do not move (dr_max 0)."""
+    big, bbox = gpu.lattice(2, 11, 0.5)
+    out = []
+    for rounds in (False, True):
+        reps = [dict(n=len(c), box=box, dr_max=0.0, seed=seed) for c in confs]
+        data = list(confs)
+        if rounds:
+            reps.append(dict(n=len(big), box=bbox, dr_max=0.1, seed=9))
+            data.append(big[:, 1:])
+        ctx = gpu.Context(reps)
+        for r, c in enumerate(data):
+            ctx.upload(np.column_stack([np.arange(len(c)), c]), r)
+        moves = ctx.npt_sweeps(1, [press] * len(reps), [dv] * len(reps))[:len(confs)]
+        out.append((moves, [ctx.box(r) for r in range(len(confs))], [ctx.download(r) for r in range(len(confs))]))
+        ctx.close()
+    for a, b in zip(*out):
+        assert np.array_equal(np.array(a), np.array(b))
+    return out[0][0]
+
+
+@pytest.mark.parametrize("moves", [1, 2, 3])
+def test_volume_moves_at_contact(moves):
+    """Two spheres at 1 / sf within a few units in the last place, sf the
+    product of the first moves' factors, the last of them a compression: the
+    decision is the reference's arithmetic on the positions that the moves
+    before it left.  Across the box edge too, where the minimum image rounds."""
+    n, dv = 6, 0.06
+    box = (7.3, 8.1, 9.7)
+
+    def fits(f):   # the last one is a compression beyond all before it
+        return len(f) == moves and f[-1] < 0.999 and all(np.prod(f[:k + 1]) > np.prod(f) * 1.001
+                                                         for k in range(moves - 1))
+
+    seed = next(s for s in range(1, 4000) if fits(_first_moves(s, n, dv, box)))
+    sf = float(np.prod(_first_moves(seed, n, dv, box)))
+    rng = np.random.default_rng(4)
+    others = np.array([(1.0, 1.0, 1.0), (1.0, 5.0, 7.0), (5.5, 5.0, 1.0), (5.5, 1.0, 8.0)])
+    confs = []
+    for k in range(-12, 13):
+        d = (1.0 / sf) * (1.0 + k * 2.0 ** -52)
+        x0 = (3.0 + 0.3 * rng.random(), 7.3 - 0.4 * rng.random())[k % 2]
+        a = np.array([x0, 3.0, 4.0])
+        b = a + np.array([d, 0.0, 0.0])
+        b[0] = b[0] - box[0] if b[0] > box[0] else b[0]
+        confs.append(np.vstack([a, b, others]))
+    counts = _tie_contexts(confs, box, seed, dv, 50.0)   # a pressure that the rule lets any compression pass
+    assert np.all(counts[:, 0] == moves)
+    assert 0 < (counts[:, 2] > 0).sum() < len(confs), counts
+
+
+@pytest.mark.parametrize("seed,overlap", [(1181, True), (1020, False)])
+def test_volume_moves_at_contact_in_a_long_box(seed, overlap):
+    """Coordinates above 2^22 are rounded by up to 2^-31 in an accepted move,
+    so the second move's decision lies further from what the first scan's
+    distance says than in a short box: beyond 1e-9 of the squared distance, on
+    the other side of contact."""
+    box = (4.3e6, 2.2, 2.3)
+    f1, f2 = _first_moves(seed, 2, 1e-3, box)
+    assert f1 < 1.0 and f2 < 1.0
+    unit = 2.0 ** -30   # of the coordinates there
+    d = round(1.0 / (f1 * f2) / unit) * unit
+    rng = np.random.default_rng(5)
+    found = None
+    for _ in range(20000):
+        a = 4.25e6 + round(rng.random() * 1e4 / unit) * unit
+        b = a + d + int(rng.integers(-3, 4)) * unit
+        said, is_ = ((b - a) * f1 * f2) ** 2, ((b * f1 - a * f1) * f2) ** 2
+        if abs(said - 1.0) > 1.05e-9 and abs(is_ - 1.0) > 1e-13 and (is_ < 1.0) == overlap == (said > 1.0):
+            found = a, b
+            break
+    conf = np.array([(found[0], 1.0, 1.0), (found[1], 1.0, 1.0)])
+    counts = _tie_contexts([conf], box, seed, 1e-3, 1e-3)
+    assert counts[0].tolist() == [2, 1 if overlap else 2, int(overlap), 0]
