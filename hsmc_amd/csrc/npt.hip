@@ -171,6 +171,8 @@ constexpr int kVolThreads = 1024;         // threads at most: one per sphere, 25
 constexpr int kVolPer = 4;                 // spheres per thread at most
 constexpr int kVolSpheres = kVolThreads * kVolPer;
 constexpr int kVolAxis = 16;               // search-grid cells per axis at most
+
+constexpr size_t vol_lds_bytes(int N) { return sizeof(double) * 3 * N + sizeof(int) * kVolAxis * kVolAxis * kVolAxis; }
 constexpr double kNear = 1e-9, kNearEdge = 1e-14;
 
 struct VolPlan {
@@ -493,9 +495,12 @@ int volume_moves_small(hsmc_gpu_ctx *ctx, unsigned long long sweep, const std::v
   int n_max = 0;
   for (const RepHost &h : ctx->reps) n_max = std::max(n_max, h.p.n_part);
   const int threads = std::min(kVolThreads, (n_max + 255) / 256 * 256);
-  const size_t lds = sizeof(double) * 3 * n_max + sizeof(int) * kVolAxis * kVolAxis * kVolAxis;
-  if (lds > 60 * 1024)  // with the kernel's own few KB above 64 KB
-    HSMC_HIP(ctx, hipFuncSetAttribute((const void *)k_volume_moves, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  const size_t lds = vol_lds_bytes(n_max);
+  // with the kernel's own few KB above 64 KB; always the same value: contexts
+  // of other threads launch this kernel too
+  if (lds > 60 * 1024)
+    HSMC_HIP(ctx, hipFuncSetAttribute((const void *)k_volume_moves, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)vol_lds_bytes(kVolSpheres)));
   for (int t0 = 0; t0 < rounds; t0 += kVolDepth) {
     // each replica's tree of this launch's moves
     std::vector<VolNode> nodes;

@@ -1646,8 +1646,8 @@ int hsmc_gpu_widom_uniform(hsmc_gpu_ctx *ctx, int replica, uint64_t seed, uint64
   if (!part) return HSMC_ERR_NO_MEMORY;
   if (in_lds) {
     auto fn = small ? k_widom_uniform_lds<kWidomLdsThreads> : k_widom_uniform_lds<1024>;
-    if (lds > 64 * 1024)
-      HSMC_HIP(ctx, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (lds > 64 * 1024)  // always the same value: contexts of other threads launch this kernel too
+      HSMC_HIP(ctx, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWidomLdsBytes));
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)wg), lds, ctx->stream, g, N,
                        ctx->d_x + h.poff, ctx->d_y + h.poff, ctx->d_z + h.poff, (uint32_t)seed,
                        (uint32_t)(seed >> 32), (unsigned long long)sample, (long long)first, (long long)n, part);

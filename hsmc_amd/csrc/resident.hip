@@ -38,6 +38,7 @@ namespace {
 constexpr int kDrawTable = 64;  // sweeps whose shift and order are drawn together
 constexpr int kMaxPer = 4;      // spheres per thread at most
 constexpr unsigned kStays = 0x8000u;
+constexpr size_t kMaxLds = 160 * 1024;
 
 __device__ __forceinline__ void lds_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -401,13 +402,14 @@ bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape) {
     const Layout l = resident_layout(h.p.n_part, h.gx * h.gy * h.gz, ctx->cap, shape->threads / shape->lpc, ctx->lcap);
     shape->bytes = std::max(shape->bytes, (size_t)l.bytes);
   }
-  return shape->bytes <= 160 * 1024;
+  return shape->bytes <= kMaxLds;
 }
 
 int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, unsigned long long base, int n) {
   ResidentFn fn = resident_fn(ctx->cap, shape.lpc);
+  // always the same value: contexts of other threads launch this kernel too
   if (shape.bytes > 64 * 1024)
-    HSMC_HIP(ctx, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shape.bytes));
+    HSMC_HIP(ctx, hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
   hipLaunchKernelGGL(fn, dim3((unsigned)ctx->R), dim3((unsigned)shape.threads), shape.bytes, ctx->stream, ctx->d_reps,
                      ctx->lcap, ctx->d_x, ctx->d_y, ctx->d_z, base, ctx->d_sweep, n, ctx->d_cacc, ctx->d_cleft,
                      ctx->d_err, (unsigned int *)ctx->h_err);

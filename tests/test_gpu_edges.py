@@ -3,6 +3,8 @@ out of range, and the conditions the reference turns into print-and-exit
 (cell_list.c:126-129 cells narrower than a diameter, cell_list.c:229-232 a
 cell over max_part).  Every error is a status code; the context stays usable
 after it."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -179,3 +181,31 @@ def test_steps_of_many_box_edges(replicas):
     ctx.contact_counts(0.01, 5, 1.05)
     for run in runs:
         run[0].close()
+
+
+def test_contexts_of_threads_share_kernels():
+    """Two threads, each with its own contexts, launch the kernels that keep a
+    system in more than 64 KB of LDS with different sizes: no launch is refused
+    for the other's, and the results are those of one thread."""
+    def work(n):
+        conf, box = gpu.lattice(2, n, 0.6)
+        out = []
+        ctx = gpu.Context([dict(n=len(conf), box=box, dr_max=0.1, seed=r) for r in range(64)])
+        for r in range(64):
+            ctx.upload(conf, r)
+        big, bbox = gpu.lattice(2, n + 3, 0.8)
+        wide = gpu.Context([dict(n=len(big), box=bbox, dr_max=0.1, seed=1)])
+        wide.upload(big)
+        for k in range(40):
+            ctx.sweeps(2)
+            ctx.npt_sweeps(2, 2.0, 0.01)
+            out.append(wide.widom_uniform(1, k, 0, 500000))
+        out += [ctx.download(r).tobytes() for r in range(64)]
+        for c in (ctx, wide):
+            c.close()
+        return out
+
+    want = [work(6), work(7)]
+    with ThreadPoolExecutor(2) as pool:
+        got = list(pool.map(work, (6, 7)))
+    assert got == want
