@@ -962,6 +962,18 @@ __device__ __forceinline__ void softmax_stats(const float *__restrict__ bmax,
   st[1] = s[0];
 }
 
+// The same by one workgroup, for a proposal of many free voxels.
+__global__ void __launch_bounds__(256)
+k_softmax_stats(const float *__restrict__ bmax, long nb, double *__restrict__ stats) {
+  double st[2];
+  softmax_stats(bmax, bmax + nb, nb, st);
+  if (threadIdx.x == 0) {
+    stats[0] = st[0];
+    stats[1] = st[1];
+    stats[2] = 0.0;
+  }
+}
+
 // The statistics of a proposal with no free voxel (every voxel keeps the
 // uniform part alone).
 __global__ void k_empty_stats(double *__restrict__ st) {
@@ -984,6 +996,11 @@ __global__ void k_empty_stats(double *__restrict__ st) {
 // scoring kernel's nparts block partials first (each workgroup for itself,
 // the first stores them); otherwise st holds them already.
 constexpr int kScanWave = 64;
+// Up to here every workgroup of k_cdf_local takes the totals for itself, above
+// one workgroup does before them: a call at N = 108000 with 4520 partials 483
+// and 488 us, with 9985 664 and 647, with 58864 2163 and 1425, with 82004 4543
+// and 2749 (the work of the first grows with the square of the free voxels).
+constexpr long kStatsParts = 8192;
 
 __global__ void __launch_bounds__(1024)
 k_cdf_local(const float *__restrict__ f, const int *__restrict__ list, long V, const float *__restrict__ bmax,
@@ -1850,8 +1867,13 @@ int hsmc_gpu_widom_learned(hsmc_gpu_mlp *m, int replica, double voxel, double mi
   const bool new_mass = !scores_ok || m->sc_mix != mix;
   if (new_mass) m->sc_replica = -1;
   if (new_mass && nfree > 0) {
+    const float *parts = pr.parts;
+    if (parts && pr.nparts > kStatsParts) {
+      hipLaunchKernelGGL(k_softmax_stats, dim3(1), dim3(256), 0, ctx->stream, parts, pr.nparts, stats);
+      parts = nullptr;
+    }
     hipLaunchKernelGGL(k_cdf_local, dim3((unsigned)ncdf), dim3(1024), 0, ctx->stream, f, list, nfree,
-                       pr.parts, pr.nparts, stats, mix, cdf, bsum);
+                       parts, pr.nparts, stats, mix, cdf, bsum);
     const dim3 add_blocks((unsigned)((nfree + 255) / 256));
     if (ncdf <= kScanWave) {
       hipLaunchKernelGGL(k_cdf_add<true>, add_blocks, dim3(256), 0, ctx->stream, cdf, nfree, bsum, (int)ncdf,

@@ -441,3 +441,40 @@ def test_estimate_after_a_refused_workspace(voxel):
     assert net.widom(voxel, 0.9, 5, 1, 20000, r=1) == want
     assert net.widom(voxel, 0.9, 5, 1, 20000, r=1) == want
     ctx.close()
+
+
+@pytest.mark.parametrize("m", [128, 136])
+def test_totals_of_few_and_many_partials(m):
+    """8192 and 9826 partials of the softmax totals (up to 8192 each workgroup
+    of the cumulative mass takes them for itself): the hits and the estimate of
+    the systematic sample that numpy draws from the same scores.  A voxel's
+    bound moved by rounding past an insertion changes it by one weight, 10 / n
+    at most; two such are allowed for."""
+    L, n, mix, seed, sample = 20.0, 50000, 0.9, 8, 3
+    spheres = np.array([[3.0, 3.0, 3.0], [10.0, 12.0, 9.0], [17.0, 5.0, 16.0]])
+    ctx = gpu.Context([dict(n=3, box=(L, L, L), dr_max=0.1, seed=4)])
+    ctx.upload(np.column_stack([np.arange(3), spheres]))
+    net = gpu.Mlp(ctx, seed=6)
+    got = net.widom(L / m, mix, seed, sample, n)
+    f, n_free = net.proposal_scores(L / m)
+    V = len(f)
+    m = round(V ** (1 / 3))
+    assert n_free == V == m ** 3
+    e = np.exp(f.astype(np.float64) - f.max())
+    mass = mix * e / e.sum()
+    cdf = np.cumsum(mass)
+    un = 1.0 - mix
+    T = un + cdf[-1]
+    u0 = O.philox((0, 0, sample, 0x4C530000), (seed, 0))[0] * 2.0 ** -32
+    t = (np.arange(n) + u0) / n * T
+    v = np.where(t < un, np.minimum((t / un * V).astype(np.int64), V - 1),
+                 np.minimum(np.searchsorted(cdf, t - un, side="right"), V - 1))
+    u = np.array([O.philox((i, 0, sample, 0x4C490000), (seed, 0))[:3] for i in range(n)], dtype=np.float64)
+    q = (np.stack([v // (m * m), v // m % m, v % m], axis=1) + (u + 0.5) * 2.0 ** -32) * (L / m)
+    d = np.abs(q[:, None, :] - spheres[None, :, :])
+    free = (np.minimum(d, L - d) ** 2).sum(-1).min(1) >= 1.0
+    w = 1.0 / (V * n * ((un / V + mass[v]) / T))
+    assert abs(got["hits"] - int(free.sum())) <= 2
+    assert abs(got["estimate"] - w[free].sum()) <= 2 * 10.0 / n
+    assert abs(w[free].sum() - (1.0 - 4.0 * math.pi / L ** 3)) < 0.05   # the restatement itself
+    ctx.close()
