@@ -472,8 +472,10 @@ int build_bricks(hsmc_gpu_ctx *ctx) {
   ctx->n_bricks = 0;
   if (ctx->Atot < kBrickCells) return HSMC_OK;
   std::vector<Brick> v;
+  long active = 0;  // without the padding of small replicas
   for (int r = 0; r < ctx->R; ++r) {
     const RepHost &h = ctx->reps[r];
+    active += (long)h.gx * h.gy * h.gz / 8;
     // the shape that costs least: a workgroup's own work and its region's
     const double in_cell = h.p.n_part / ((double)h.gx * h.gy * h.gz);
     auto fits = [&](long cells, int room) {  // with room for uneven density
@@ -512,6 +514,7 @@ int build_bricks(hsmc_gpu_ctx *ctx) {
       x0 = x1;
     }
   }
+  if (active < kBrickMean * (long)v.size()) return HSMC_OK;  // cell by cell
   if (v.size() > ctx->brick_alloc) {
     (void)hipFree(ctx->d_bricks);
     ctx->d_bricks = nullptr;

@@ -249,6 +249,11 @@ int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, unsigned long
 // N = 256000, whose cell phases file the next sweep), 207 and 246 at 70000,
 // 253 and 557 at 187000.
 constexpr long kBrickCells = 40000;
+// And with this many active cells a brick on average: a workgroup takes as
+// long for a small replica's few cells.  60000 active cells in replicas of 8,
+// 12, 16, 18, 24 and 27: a sweep by bricks 390, 243, 251, 199, 215 and 190 us,
+// cell by cell 217, 216, 219, 198, 221 and 219.
+constexpr long kBrickMean = 20;
 int build_bricks(hsmc_gpu_ctx *ctx);
 bool bricks_run(const hsmc_gpu_ctx *ctx);
 void enqueue_brick_phase(hsmc_gpu_ctx *ctx, int phase, int k, hipStream_t s);

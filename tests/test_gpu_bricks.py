@@ -162,3 +162,30 @@ def test_steps_wider_than_the_box():
     a, b = _both(confs, boxes, sweeps=(2, 400), after=wide)
     assert any((x[:, 1:] > 4.2).any() for x, _ in b[:24])
     _same(a, b)
+
+
+@pytest.mark.parametrize("cells,replicas", [(4, 5100), (6, 1500)])
+def test_many_small_replicas(cells, replicas):
+    """40800 active cells in replicas of 8 (too few for a brick each: cell by
+    cell), 42000 of 27 beside a larger one (bricks): each replica as alone."""
+    L = 1.07 * cells
+    xyz = _sites(np.random.default_rng(9), (L, L, L), 0.7)
+    systems = [(xyz, (L, L, L))] * replicas
+    if cells == 6:   # beside a replica that no workgroup can keep in LDS
+        systems.append((_sites(np.random.default_rng(9), (24.0, 24.0, 24.0), 0.7), (24.0, 24.0, 24.0)))
+
+    def run(which):
+        ctx = gpu.Context([dict(n=len(systems[k][0]), box=systems[k][1], dr_max=0.2, seed=3 + k) for k in which])
+        for r, k in enumerate(which):
+            ctx.upload(np.column_stack([np.arange(len(systems[k][0])), systems[k][0]]), r)
+        ctx.sweeps(9)
+        return ctx
+
+    every = list(range(len(systems)))
+    ctx = run(every)
+    for k in (0, 1, replicas // 2, len(systems) - 1):
+        alone = run([k])
+        assert np.array_equal(ctx.download(k), alone.download()), k
+        assert ctx.counters(k) == alone.counters(), k
+        alone.close()
+    ctx.close()
