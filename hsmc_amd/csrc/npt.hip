@@ -13,8 +13,8 @@
 // samples it.  In rounds, round t holds the t-th move of every replica that
 // draws more than t, and one kernel checks every compression of the round.
 //
-// Replicas of up to 4096 spheres make all of a sweep's moves in one launch
-// (k_volume_moves), larger ones round by round with the scan below.
+// Small replicas make all of a sweep's moves in one launch (k_volume_moves;
+// moves_in_one_launch says which), others round by round with the scan below.
 //
 // That scan reads the cell list the last sweep left (the sweep grid: cells of
 // side > 1 holding every sphere, filed by the sweep's rebin and kept by its
@@ -171,6 +171,14 @@ constexpr int kVolThreads = 1024;         // threads at most: one per sphere, 25
 constexpr int kVolPer = 4;                 // spheres per thread at most
 constexpr int kVolSpheres = kVolThreads * kVolPer;
 constexpr int kVolAxis = 16;               // search-grid cells per axis at most
+
+// Where one launch of a workgroup a replica is faster than a round of kernels
+// on the whole device and a wait for each move (of which some replica of many
+// makes more).  us per NpT sweep at density 0.6, one launch / rounds (the waits
+// take one of two durations in a process): a single replica of 864 spheres 67 /
+// 63 to 75, 2048 75 / 62 to 75, 4000 93 / 62 to 75; four of 864 79 / 106, 2048
+// 99 / 96 to 104, 4000 131 / 98 to 105; 16 of 2916 125 / 148, 4000 155 / 157.
+constexpr bool moves_in_one_launch(int R, int n_max) { return n_max <= kVolSpheres && n_max <= 1500 + 250L * R; }
 
 constexpr size_t vol_lds_bytes(int N) { return sizeof(double) * 3 * N + sizeof(int) * kVolAxis * kVolAxis * kVolAxis; }
 constexpr double kNear = 1e-9, kNearEdge = 1e-14;
@@ -699,8 +707,9 @@ int hsmc_gpu_npt_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, const double *press,
     if (!(press[r] >= 0.0) || !(dv_max[r] > 0.0) || !std::isfinite(press[r])) return HSMC_ERR_BAD_ARG;
   if (n_sweeps == 0) return HSMC_OK;
   const unsigned long long sweep0 = ctx->sweep_now;
-  bool small = true;
-  for (const RepHost &h : ctx->reps) small = small && h.p.n_part <= kVolSpheres;
+  int n_max = 0;
+  for (const RepHost &h : ctx->reps) n_max = std::max(n_max, (int)h.p.n_part);
+  const bool small = moves_in_one_launch(R, n_max);
   std::vector<int> steps(R);
   ResidentShape shape;
   bool ahead = false;  // the sweep was enqueued behind the last one's volume moves

@@ -464,3 +464,32 @@ def test_volume_moves_at_contact_in_a_long_box(seed, overlap):
     conf = np.array([(found[0], 1.0, 1.0), (found[1], 1.0, 1.0)])
     counts = _tie_contexts([conf], box, seed, 1e-3, 1e-3)
     assert counts[0].tolist() == [2, 1 if overlap else 2, int(overlap), 0]
+
+
+@pytest.mark.parametrize("R,n", [(1, 1750), (1, 1751), (2, 2000), (2, 2001), (11, 4096), (11, 4097)])
+def test_npt_route_by_size_and_number(R, n):
+    """On both sides of the rule for the moves in one launch (1500 + 250 R
+    spheres, 4096 at most): replicas of a batch equal the same replicas beside
+    one of 5324 spheres, whose moves go in rounds."""
+    conf, _ = gpu.lattice(2, 11, 0.55)
+    rng = np.random.default_rng(n)
+    box = tuple(1.0 + (4 * 11 ** 3 / 0.55) ** (1 / 3) for _ in range(3))
+    confs = []
+    for _ in range(R):
+        c = conf[np.sort(rng.permutation(len(conf))[:n])].copy()
+        c[:, 0] = np.arange(n)
+        confs.append(c)
+    spec = [dict(n=n, box=box, dr_max=0.1, seed=70 + r) for r in range(R)]
+    a = gpu.Context(spec)
+    b = gpu.Context(spec + [dict(n=len(conf), box=box, dr_max=0.1, seed=1)])
+    for r, c in enumerate(confs):
+        a.upload(c, r)
+        b.upload(c, r)
+    b.upload(conf, R)
+    press, dv = [0.2] * R, [0.01] * R
+    m = a.npt_sweeps(12, press, dv)
+    assert np.array_equal(m, b.npt_sweeps(12, press + [1.0], dv + [0.001])[:R]) and m[:, 1].sum() > 0
+    for r in range(R):
+        assert a.box(r) == b.box(r) and np.array_equal(a.download(r), b.download(r)), r
+    a.close()
+    b.close()
