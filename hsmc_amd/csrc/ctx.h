@@ -243,11 +243,11 @@ bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape);
 int launch_resident(hsmc_gpu_ctx *ctx, const ResidentShape &shape, unsigned long long base, int n);
 // Brick phases (bricks.hip): the bricks of the present layout, whether the
 // context's launched sweeps run that way, and one phase of them.
-// From kBrickCells active cells of all replicas on: a sweep by bricks and cell
-// by cell takes 110 and 47 us at 4000 active cells, 122 and 73 at 14000, 135
-// and 139 at 33000 (8 replicas of N = 32000), 138 and 136 at 36000 (one of
-// N = 256000, whose cell phases file the next sweep), 207 and 246 at 70000,
-// 253 and 557 at 187000.
+// From kBrickCells active cells of all replicas on.  A sweep by bricks and cell
+// by cell takes, for one replica, whose cell phases file the next sweep, 122
+// and 118 us at 38000 active cells, 125 and 134 at 44000, 146 and 153 at 46700
+// (densities 0.6, 0.6 and 0.9), 165 and 211 at 69000; for several, 138 and 96 at
+// 22000, 134 and 134 at 33000, 141 and 157 at 41000, 159 and 227 at 65500.
 constexpr long kBrickCells = 40000;
 // And with this many active cells a brick on average: a workgroup takes as
 // long for a small replica's few cells.  60000 active cells in replicas of 8,

@@ -375,11 +375,13 @@ namespace hsmc {
 
 // Shape of the resident kernel for the context's replicas; false where they
 // do not fit in LDS or launched sweeps are faster.  Measured per sweep: the
-// resident kernel takes about 9 + 0.24 A us with A active cells a phase in
-// its largest replica, for as many replicas as there are compute units; the
-// launched phases take 38 us and 0.0026 us for each active cell of all
-// replicas (N = 256: 18.5 against 38 us for one replica, 48 for 32, 68 for
-// 256; N = 864: 42 against 35, 45 and 137; N = 1372: 58 against 43, 57, 180).
+// resident kernel takes about 12 + 0.11 A + 0.0225 N us with A active cells a
+// phase and N spheres in its largest replica, for as many replicas as there are
+// compute units; the launched phases (in their default shape) take 35 us for
+// one replica, 42 for several, and 0.0029 us for each active cell of all (A =
+// 64 and N = 500 at density 0.85: 26 us against 34 for one replica, 44 for 32,
+// 89 for 256; 125 and 864: 43 against 34, 47, 135; 125 and 1372: 57 against 41,
+// 58, 176).
 bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape) {
   long n_max = 0, a_max = 0;
   for (int r = 0; r < ctx->R; ++r) {
@@ -390,7 +392,8 @@ bool resident_shape(const hsmc_gpu_ctx *ctx, ResidentShape *shape) {
   }
   if (n_max > 1024 * kMaxPer || a_max > 1024) return false;
   const double turns = (double)((ctx->R + ctx->n_cu - 1) / ctx->n_cu);
-  if (turns * (9.0 + 0.24 * a_max) > 38.0 + 0.0026 * (double)ctx->Atot) return false;
+  if (turns * (12.0 + 0.11 * a_max + 0.0225 * n_max) > (ctx->R == 1 ? 35.0 : 42.0) + 0.0029 * (double)ctx->Atot)
+    return false;
   shape->lpc = a_max <= 1024 / kWide ? kWide : kNarrow;
   shape->threads = 256;
   while (shape->threads < 1024 &&
