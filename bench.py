@@ -299,6 +299,8 @@ def batched(args) -> None:
     if args.tuning:
         ctx.set_tuning(*(int(v) for v in args.tuning.split(",")))
         tuning = ctx.get_tuning()
+    if not ctx.tuning_in_force():
+        tuning = "not in force: the context's own route is faster"
     print(f"[bench] batched: {len(reps)} replicas, {total} spheres, tuning {tuning}",
           file=sys.stderr, flush=True)
     ctx.sweeps(args.warmup)
@@ -347,7 +349,8 @@ def npt(args) -> None:
     del confs
     if not args.tuning and not args.no_autotune:
         ctx.autotune(16)  # NVT trials of the same phase kernels; positions are restored
-    print(f"[bench] npt: {R} replicas, {total} spheres, tuning {ctx.get_tuning()}",
+    tuning = ctx.get_tuning() if ctx.tuning_in_force() else "not in force: the context's own route is faster"
+    print(f"[bench] npt: {R} replicas, {total} spheres, tuning {tuning}",
           file=sys.stderr, flush=True)
     ctx.npt_sweeps(args.warmup, press, dv)
     ctx.sync()
@@ -374,7 +377,7 @@ def npt(args) -> None:
         "data": "synthetic (fcc 4*40^3 starts at the Carnahan-Starling density, Philox proposals)",
         "config": {"workload": "64 NpT replicas (21 at beta P = 5, 21 at 8, 22 at 11), N = 256000 "
                                "each, max ln-volume step 0.001, dr_max 0.1",
-                   "total_spheres": total, "tuning": ctx.get_tuning(),
+                   "total_spheres": total, "tuning": tuning,
                    "acceptance": sum(a["accepted"] for a in acc) / attempts},
         "volume_moves": {"proposed": int(vol[:, 0].sum()), "accepted": int(vol[:, 1].sum()),
                          "rejected_overlap": int(vol[:, 2].sum()),

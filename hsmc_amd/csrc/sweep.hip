@@ -1173,6 +1173,12 @@ int hsmc_gpu_get_tuning(const hsmc_gpu_ctx *ctx, hsmc_gpu_tuning *t) {
   return HSMC_OK;
 }
 
+int hsmc_gpu_tuning_in_force(const hsmc_gpu_ctx *ctx) {
+  if (!ctx) return HSMC_ERR_BAD_ARG;
+  ResidentShape shape;
+  return ctx->tune_set || !(resident_shape(ctx, &shape) || bricks_run(ctx));
+}
+
 int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *best) {
   if (!ctx || sweeps_per_trial <= 0) return HSMC_ERR_BAD_ARG;
   const size_t P = (size_t)ctx->Ptot;
@@ -1194,9 +1200,9 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
   hsmc_gpu_tuning winner = start;
   float best_ms = 1e30f;
   // the resident kernel or the bricks, where the context has them, stand
-  // beside the launch shapes; when they win the tuning stays as it was and is
-  // not in force
-  bool own_route = false;
+  // beside the launch shapes; when they win, the fastest shape is kept and
+  // returned all the same, but not in force
+  float own_ms = 1e30f;
   {
     ResidentShape shape;
     ctx->tune_set = false;
@@ -1209,8 +1215,7 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
         ctx->tune_set = start_set;
         return st;
       }
-      best_ms = ms;
-      own_route = true;
+      own_ms = ms;
     }
   }
   ctx->tune_set = true;
@@ -1236,11 +1241,10 @@ int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *
         if (ms < best_ms) {
           best_ms = ms;
           winner = t;
-          own_route = false;
         }
       }
   ctx->tune = winner;
-  ctx->tune_set = !own_route;
+  ctx->tune_set = best_ms <= own_ms;
   drop_graph(ctx);
   HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_x, save, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));
   HSMC_HIP(ctx, hipMemcpyAsync(ctx->d_y, save + P, sizeof(double) * P, hipMemcpyDeviceToDevice, ctx->stream));

@@ -29,7 +29,7 @@ EXPORTS = [
     "hsmc_gpu_counters", "hsmc_gpu_reset_counters", "hsmc_gpu_set_sweep_counter",
     "hsmc_gpu_set_tuning", "hsmc_gpu_box", "hsmc_gpu_npt_sweeps",
     "hsmc_gpu_any_overlap_scaled_batch",
-    "hsmc_gpu_get_tuning", "hsmc_gpu_autotune", "hsmc_gpu_time_phase_kernel",
+    "hsmc_gpu_get_tuning", "hsmc_gpu_tuning_in_force", "hsmc_gpu_autotune", "hsmc_gpu_time_phase_kernel",
     "hsmc_gpu_cell_list", "hsmc_gpu_overlap_batch", "hsmc_gpu_overlap_scaled",
     "hsmc_gpu_any_overlap_scaled", "hsmc_gpu_pair_dist", "hsmc_gpu_rdf_counts",
     "hsmc_gpu_contact_counts", "hsmc_gpu_widom_points", "hsmc_gpu_widom_uniform",
@@ -115,6 +115,7 @@ def load() -> C.CDLL:
         "hsmc_gpu_any_overlap_scaled_batch": (i32, [vp, P(f64), P(C.c_uint8)]),
         "hsmc_gpu_set_tuning": (i32, [vp, P(Tuning)]),
         "hsmc_gpu_get_tuning": (i32, [vp, P(Tuning)]),
+        "hsmc_gpu_tuning_in_force": (i32, [vp]),
         "hsmc_gpu_autotune": (i32, [vp, i32, P(Tuning)]),
         "hsmc_gpu_time_phase_kernel": (i32, [vp, i32, P(C.c_float), P(i32)]),
         "hsmc_gpu_cell_list": (i32, [vp, i32, i32, i32, i32, i32, P(i32), P(i32)]),
@@ -295,6 +296,9 @@ class Context:
         t = Tuning()
         self._ck(self.L.hsmc_gpu_get_tuning(self.h, C.byref(t)), "get_tuning")
         return t.as_dict()
+
+    def tuning_in_force(self) -> bool:
+        return self.L.hsmc_gpu_tuning_in_force(self.h) == 1
 
     def autotune(self, sweeps_per_trial: int = 64) -> dict:
         t = Tuning()

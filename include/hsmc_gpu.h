@@ -152,10 +152,15 @@ int hsmc_gpu_occupant_picks(int device, uint64_t seed, uint32_t cell, uint64_t s
                             int32_t count, uint32_t *out);
 int hsmc_gpu_set_tuning(hsmc_gpu_ctx *ctx, const hsmc_gpu_tuning *t);
 int hsmc_gpu_get_tuning(const hsmc_gpu_ctx *ctx, hsmc_gpu_tuning *t);
+/* 1 if the context's sweeps run in its launch shape, 0 if they go its own way
+ * (whole sweeps in one launch, or bricks of cells; see hsmc_gpu_tuning). */
+int hsmc_gpu_tuning_in_force(const hsmc_gpu_ctx *ctx);
 /* Time the candidate launch shapes on this context's own replicas (their
  * state is saved and restored), and the context's own way of running where it
- * has one, and keep the fastest.  *best receives the launch shape (the one in
- * force before, not used, where the own way wins). */
+ * has one, and keep the fastest.  *best receives the fastest launch shape,
+ * also where the own way is faster and stays: the shape is not in force then
+ * (hsmc_gpu_tuning_in_force), and a context like this one is as fast only
+ * without set_tuning. */
 int hsmc_gpu_autotune(hsmc_gpu_ctx *ctx, int sweeps_per_trial, hsmc_gpu_tuning *best);
 /* Average duration (ms) of one launch of the sweep's dominant kernel (the
  * sublattice-phase kernel), measured with HIP events around each launch

@@ -239,3 +239,29 @@ def test_persistent_batched_sweeps_equal_launched_sweeps():
     for r in range(len(reps)):
         assert np.array_equal(outs[0][r][0], outs[1][r][0]), r
         assert outs[0][r][1] == outs[1][r][1], r
+
+
+@pytest.mark.parametrize("n", [4, 7])
+def test_autotune_returns_a_shape_to_pass_on(n):
+    """The shape returned is the fastest of those tried, also where the
+    context's own way of running is faster still and stays (N = 256); whether
+    the shape is in force can be asked.  Another context takes it."""
+    conf, box = gpu.lattice(2, n, 0.7)
+    ctx, other = (gpu.Context([dict(n=len(conf), box=box, dr_max=0.1, seed=5)]) for _ in range(2))
+    for c in (ctx, other):
+        c.upload(conf)
+        c.sweeps(100)
+    assert ctx.tuning_in_force() == (n == 7)
+    ctx.set_tuning(64, 1, 0)   # some ten times slower than graphs
+    assert ctx.tuning_in_force()
+    best = ctx.autotune(64)
+    assert best["sweeps_per_graph"] > 0
+    assert best == ctx.get_tuning()
+    assert ctx.tuning_in_force() == (n == 7)
+    other.set_tuning(*best.values())
+    assert other.tuning_in_force()
+    for c in (ctx, other):
+        c.sweeps(20)
+    assert np.array_equal(ctx.download(), other.download())
+    ctx.close()
+    other.close()
