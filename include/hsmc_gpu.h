@@ -93,7 +93,10 @@ int hsmc_gpu_upload(hsmc_gpu_ctx *ctx, int replica, const double *conf4);
 /* Copy the replica's configuration out as N x {id,x,y,z}. */
 int hsmc_gpu_download(hsmc_gpu_ctx *ctx, int replica, double *conf4);
 /* Overwrite the coordinates of m particles: idx[k] moves to
- * xyz[3k..3k+2] (the part_conf update of an accepted move, moves.c:52-54). */
+ * xyz[3k..3k+2] (the part_conf update of an accepted move, moves.c:52-54).
+ * Up to 8 particles are set by a kernel enqueued on the context's stream: the
+ * call returns before it has run, every later call on the context sees it, and
+ * an error of its own is reported by one of them (hsmc_gpu_sync waits). */
 int hsmc_gpu_set_particles(hsmc_gpu_ctx *ctx, int replica, const int32_t *idx,
                            const double *xyz, int m);
 /* Replace the box edges without moving particles. */
@@ -117,7 +120,8 @@ int hsmc_gpu_box(const hsmc_gpu_ctx *ctx, int replica, double out[3]);
  * grid and a random order of the 8 sublattices; each active cell makes as
  * many displacement attempts as it has occupants, on uniformly chosen
  * occupants; a move that leaves its cell is rejected.  N attempts per
- * replica per sweep, like sweep_nvt. */
+ * replica per sweep, like sweep_nvt.  Enqueued: the call returns before the
+ * sweeps are done, and their errors are reported by a later call. */
 int hsmc_gpu_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps);
 /* Same, bracketed by HIP events on the context's stream; *ms = elapsed. */
 int hsmc_gpu_time_sweeps(hsmc_gpu_ctx *ctx, int n_sweeps, float *ms);
