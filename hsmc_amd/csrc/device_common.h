@@ -215,6 +215,13 @@ __host__ __device__ __forceinline__ int wrap_index(int i, int g) {
   return i;
 }
 
+// LDS written by one lane of a wave is read by its others after this.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Inclusive sum of v over each group of LPC (32 or 64) consecutive lanes of
 // a full wave, in DPP moves with no LDS round trip: shifts by 1, 2, 4 and 8
 // within each row of 16 lanes, then lane 15 of each even row added to the

@@ -92,12 +92,6 @@ __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ bf16x4 to_bf16x4(f32x4 v) {
   bf16x4 r;
 #pragma unroll
@@ -637,7 +631,7 @@ __device__ void score_block(const MlpDev *__restrict__ net, uint16_t (*X)[64 * K
       if (k + i < NIN) c[i] = d[k + i];
     *reinterpret_cast<bf16x4 *>(&X[w][lane * KIN + k]) = to_bf16x4(c);
   }
-  wave_sync();
+  wave_lds_sync();
   float val = 0.f;
   {
     const NetRegs nr(net);
@@ -1179,7 +1173,7 @@ k_insert(NGrid g1, Vox vx, const double *__restrict__ cdf, const int *__restrict
     const int iz = (int)(v % vx.mz);
     const long tv = v / vx.mz;
     const int iy = (int)(tv % vx.my), ix = (int)(tv / vx.my);
-  uint32_t u[4];
+    uint32_t u[4];
     philox4x32_10((uint32_t)i, (uint32_t)(i >> 32), (uint32_t)sample,
                   0x4C490000u | (uint32_t)((sample >> 32) & 0xFFFFu), k0, k1, u);
     const double qx = (ix + ((double)u[0] + 0.5) * 0x1p-32) * vx.vx;

@@ -273,7 +273,9 @@ __global__ void k_overlap_batch(Grid g, const int *__restrict__ idx, const doubl
 // all N, the same tests in another order.  The queries come by value, the
 // answers go to pinned memory: one launch and one wait, where a grid of a
 // configuration not seen before costs three launches and the queries two
-// copies (a move of the serial chain at N = 256: 40 -> 13 us).
+// copies.  A call after a move of one sphere, by grid and so: 82 and 24 us at N
+// = 256 (18 of them the query), 82 and 28 at 16384; on a grid that is there 44
+// and 18, 44 and 23.  (Workgroups of 256 take as long up to N = 256.)
 constexpr int kFewQueries = 8;
 constexpr int kFewSpheres = 16384;
 
@@ -505,11 +507,6 @@ k_widom_cells(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, int p
   int dx = 0, dy = 0, dz = 0;        // lane < 27: its neighbour cell (distinct cells only)
   if (lane < 27) stencil_by_distance(lane, dx, dy, dz);
   const bool near = lane < 27 && stencil_axis_ok(dx, g.nx) && stencil_axis_ok(dy, g.ny) && stencil_axis_ok(dz, g.nz);
-  auto wave_sync = [] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  };
   const uint32_t c3 = 0x57430000u | (uint32_t)((sample >> 32) & 0xFFFFu);
   const float sfx = (float)(g.sx * 0x1p-32), sfy = (float)(g.sy * 0x1p-32), sfz = (float)(g.sz * 0x1p-32);
   unsigned long long h = 0;
@@ -538,7 +535,7 @@ k_widom_cells(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, int p
       // three loads fetch the list and not three for each sphere of a cell
 #pragma unroll 1
       for (int q = 0; q < n; ++q) list[w][o + q].w = __int_as_float(b + q);
-      wave_sync();
+      wave_lds_sync();
       const double cx = (ix + 0.5) * g.sx, cy = (iy + 0.5) * g.sy, cz = (iz + 0.5) * g.sz;
       auto from_corner = [](double v, double centre, double side, double L) {
         const double d = v - centre;
@@ -560,7 +557,7 @@ k_widom_cells(Grid g, uint32_t k0, uint32_t k1, unsigned long long sample, int p
       }
       if (lane < T4 - T) exact[w][0][T + lane] = exact[w][1][T + lane] = exact[w][2][T + lane] = 1e300;
     }
-    wave_sync();
+    wave_lds_sync();
     // point jj of the cell
     auto draw = [&](int jj, uint32_t u[4]) {
       philox4x32_10((uint32_t)c, (uint32_t)jj, (uint32_t)sample, c3, k0, k1, u);
@@ -1331,8 +1328,8 @@ int hsmc_gpu_cell_list(hsmc_gpu_ctx *ctx, int replica, int nx, int ny, int nz, i
       return HSMC_ERR_NO_MEMORY;
     ctx->aux_replica = -1;  // the CSR scratch now holds this grid
     const double *x = ctx->d_x + h.poff, *y = ctx->d_y + h.poff, *z = ctx->d_z + h.poff;
-  long clear = 0;
-  if (clear_counts(ctx, cnt, C, &clear)) return HSMC_ERR_HIP;
+    long clear = 0;
+    if (clear_counts(ctx, cnt, C, &clear)) return HSMC_ERR_HIP;
     const unsigned blocks = (unsigned)((N + 255) / 256);
     hipLaunchKernelGGL(k_grid_count<true>, dim3(blocks), dim3(256), 0, ctx->stream, x, y, z, N, nx, ny,
                        nz, sx, sy, sz, cnt, cellof);
@@ -1389,8 +1386,7 @@ int hsmc_gpu_overlap_batch(hsmc_gpu_ctx *ctx, int replica, const int32_t *idx, c
     f.idx[k] = idx[k];
   }
   if (few) {
-    const unsigned threads = h.p.n_part <= 256 ? 256 : 1024;
-    hipLaunchKernelGGL(k_overlap_few, dim3((unsigned)m), dim3(threads), 0, ctx->stream, f, ctx->d_x + h.poff,
+    hipLaunchKernelGGL(k_overlap_few, dim3((unsigned)m), dim3(1024), 0, ctx->stream, f, ctx->d_x + h.poff,
                        ctx->d_y + h.poff, ctx->d_z + h.poff, h.p.n_part, h.p.lx, h.p.ly, h.p.lz, ctx->h_acc);
     HSMC_HIP(ctx, hipGetLastError());
     HSMC_HIP(ctx, hipStreamSynchronize(ctx->stream));

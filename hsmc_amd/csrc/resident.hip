@@ -40,12 +40,6 @@ constexpr int kMaxPer = 4;      // spheres per thread at most
 constexpr unsigned kStays = 0x8000u;
 constexpr size_t kMaxLds = 160 * 1024;
 
-__device__ __forceinline__ void lds_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Inclusive sum over groups of LPC (16 or 32) lanes.  A group of 16 is a DPP
 // row: shifts by 1, 2, 4 and 8 within it, a shifted-in lane reading 0.
 template <int LPC>
@@ -278,7 +272,7 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
           o += nn[q];
         }
         double nx = tx[it], ny = ty[it], nz = tz[it];
-        lds_wave_sync();
+        wave_lds_sync();
         // the list's first RC * LPC spheres in registers; a lane past its end
         // holds a sphere no trial can meet
         int id[RC];
@@ -329,7 +323,7 @@ k_sweeps_resident(const RepDev *__restrict__ reps, int lcap, double *__restrict_
               word = (unsigned)m | (in_cell(nx, ny, nz, sw) == c0 ? kStays : 0u);
             }
           }
-          lds_wave_sync();
+          wave_lds_sync();
         }
       }
       __syncthreads();

@@ -12,12 +12,6 @@ __device__ __forceinline__ void store_through(double *p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Shift of the sweep grid for one sweep: 3 uniform draws in [0, side).
 __device__ __forceinline__ void sweep_shift(const RepDev &rp, unsigned long long sweep,
                                             double &shx, double &shy, double &shz) {
