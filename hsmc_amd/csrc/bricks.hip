@@ -11,8 +11,8 @@
 // into a list in LDS; a lane draws an attempt; 4 lanes test an active cell's
 // attempts one after another.
 //
-// 256 replicas of N = 4000 at density 0.6: 27 us a phase, 65 us cell by cell
-// (a sweep 253 and 557 us); N = 10^6 at density 0.9: a sweep 274 and 419 us.
+// 256 replicas of N = 4000 at density 0.6: 30 us a phase, 65 us cell by cell
+// (a sweep 256 and 525 us); N = 10^6 at density 0.9: a sweep 270 and 383 us.
 // Bounded by instruction issue (about 1100 vector instructions a wave: a
 // third the counts and list, a third the pair tests) and by what a workgroup
 // waits for on its way (10 us alone on the device), which 5 workgroups a

@@ -20,9 +20,9 @@
 // cells' spheres into a list and its first RC * LPC positions into registers,
 // then make the cell's attempts one after the other, each broadcast from the
 // lane that holds it.  What bounds it is the instructions of these steps on
-// the four SIMDs of one compute unit and their latency: of 18.5 us per sweep
+// the four SIMDs of one compute unit and their latency: of 18.9 us per sweep
 // at N = 256, filing and drawing take 1.5, gathering 5.7 and the attempts the
-// rest (18.5 us against 38 with a launch per phase).
+// rest (34 us with a launch per phase).
 #include <stdio.h>
 
 #include <algorithm>
@@ -353,9 +353,9 @@ using ResidentFn = void (*)(const RepDev *, int, double *, double *, double *, u
                             unsigned int *);
 
 // Lanes per active cell: 32 while a phase's cells fit the workgroup's 32 such
-// groups (us per sweep at N = 108 and 256, 8 and 27 cells a phase: 15.3 and
-// 18.5, against 19.3 and 20.7 with 16), else 16 (N = 500, 864 and 1372, 64,
-// 125 and 216 cells: 25.1, 42.3 and 57.9, against 30.8, 52.9 and 69.3).
+// groups (us per sweep at N = 108 and 256, 8 and 27 cells a phase: 17.0 and
+// 18.9, against 19.6 and 19.9 with 16), else 16 (N = 500, 864 and 1372, 64,
+// 125 and 216 cells: 25.3, 43.4 and 67.5, against 32.2, 55.0 and 83.9).
 constexpr int kWide = 32, kNarrow = 16;
 
 ResidentFn resident_fn(int cap, int lpc) {
