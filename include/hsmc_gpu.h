@@ -65,8 +65,8 @@ typedef struct hsmc_gpu_replica {
  * place of a kernel boundary; the trajectory is the same.  Other values
  * give HSMC_ERR_BAD_ARG.  A shape set by hand is used as it is; without one,
  * replicas small enough run whole sweeps in one launch and contexts of
- * 40000 active cells and more run by bricks of cells, on the same
- * trajectory. */
+ * 40000 active cells and more (at least 20 to a brick on average) run by
+ * bricks of cells, on the same trajectory. */
 typedef struct hsmc_gpu_tuning {
   int32_t lanes_per_cell;
   int32_t cells_per_block;
